@@ -111,6 +111,14 @@ int tpq_int8_mm_dequant_ws(const int8_t* a, const int8_t* w, const float* row_sc
                            void* stream);
 
 /*
+ * Copies of int8 rows with zeros behind K: a [M,K] -> a_out [M,K_padded] and w [N,K] -> w_out [N,K_padded] in one launch
+ * (a_out or w_out NULL: not that one).  For products with K % 16 != 0 and many rows, whose tiled kernels want 16-byte
+ * aligned rows: the products above on the copies with K_padded give the same sums.  No counterpart in the reference.
+ */
+int tpq_int8_pad_rows(const int8_t* a, int64_t M, const int8_t* w, int64_t N, int64_t K, int8_t* a_out,
+                      int8_t* w_out, int64_t K_padded, void* stream);
+
+/*
  * tpq_int8_mm_dequant_ws without the workspace argument, for callers that cannot allocate device memory
  * (code under HIP graph capture, serving loops and harnesses that forbid hipMalloc).  No counterpart in the
  * reference.  The slice matrices live in a buffer built into the library, tpq_int8_mm_noalloc_max_bytes()
@@ -196,8 +204,9 @@ int tpq_ternary_mm(const int8_t* x, const float* row_scale, const uint8_t* packe
 /*
  * The same product (same reference lines) with an optional device workspace.  From 33 rows on with
  * K > 2560 the fastest kernel cuts K into splits whose exact int32 partial sums go to the workspace
- * ([splits][M][N]) and are added by a second kernel: bit-identical results.  tpq_ternary_mm_workspace_bytes
- * says how many bytes the shape can use (0: none needed); a NULL or smaller workspace runs
+ * ([splits][M][N]) and are added by a second kernel: bit-identical results.  From about 650 rows on, and for
+ * K that no kernel of the packed weight takes, the weight is written out as int8 in the workspace for the int8 GEMM (same
+ * result bits; not with acc_out).  tpq_ternary_mm_workspace_bytes says how many bytes the shape can use (0: none needed); a NULL or smaller workspace runs
  * tpq_ternary_mm's kernels.  Nothing has to be cleared between calls.
  */
 int64_t tpq_ternary_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);

@@ -40,7 +40,10 @@
 // Four extra wavefronts that do nothing but request (one per SIMD, 168 registers per wavefront) were built and measured:
 // the loop drops from 1085 to 1064 clocks per stage, the first stage arrives 1000 clocks later, same time; not kept.
 //
-// Requires K % 128 == 0, K < 2^23 and 16-byte aligned operands.  Edges in M and N: source rows are clamped, stores masked.
+// Requires rows of k of a multiple of 16 bytes, below 2^23, and 16-byte aligned operands.  Edges in M and N: source rows
+// are clamped, stores masked.  Edge in k (row_bytes % 128 != 0): in the last stage a lane whose chunk lies behind the end of
+// its row fetches the row's last chunk instead, and once its loads have landed writes zeros over what it fetched, ahead of
+// the barrier that publishes the stage.  The steady loop ends in front of that stage, so nothing in it asks about the edge.
 #pragma once
 
 #include "int8_gemm_dma.h"
@@ -120,12 +123,15 @@ struct ArithF32 {  // 32 k per stage, four v_mfma_f32_16x16x4_f32 per fragment: 
     }
 };
 
+// The kernel's building blocks are lambdas that have to be inlined: a call would put the accumulators in memory.
+#define TPQ_INLINED __attribute__((always_inline))
+
 // A, W: row-major [M][K], [N][K] with K contiguous; row_bytes = K * sizeof(element).
 // MB: blocks of 16 rows per wavefront: 4 (tile of 256 rows, what the description above and the numbers are about) or 2
 // (tile of 128 rows for problems with few rows or few tiles: per stage 32 wave-level loads against 16 MFMAs per
 // wavefront, so the vector memory path bounds it at about 700 clocks per stage; int8, 4096 x 4096: 15.4 .. 18.8 us at
 // 256 .. 1024 rows, where the 256-row tiles take 21 .. 22 and the sliced launches 21 .. 32).
-template <class Tile, class Arith, int MB>
+template <class Tile, class Arith, int MB, bool EDGE>
 __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restrict__ A, const char* __restrict__ W, int M, int N,
                                                                          int row_bytes, Tile tile, int vector_stores, int slices) {
     using out_t = typename Tile::out_t;
@@ -164,9 +170,13 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
         }
     }
     const int m0 = tile_m * BM, n0 = tile_n * BN;
-    const int nk_all = row_bytes / kDmaRowBytes, nk_slice = (nk_all + slices - 1) / slices;
+    const int nk_all = (row_bytes + kDmaRowBytes - 1) / kDmaRowBytes, nk_slice = (nk_all + slices - 1) / slices;
     const int kt0 = blockIdx.y * nk_slice;
     const int nk = nk_all - kt0 < nk_slice ? nk_all - kt0 : nk_slice;
+    // 16-byte chunks of k in the partial last stage, 0 if this workgroup has none; the steady loops run over nk_steady stages
+    const int edge_chunks = EDGE && kt0 + nk == nk_all ? (row_bytes % kDmaRowBytes) / 16 : 0;
+    const int nk_steady = EDGE && edge_chunks ? nk - 1 : nk;
+    constexpr int kTail = EDGE ? 1 : 0;  // stages that the steady loops leave to the checked steps for the edge's sake
 
     // ---- requests -----------------------------------------------------------------------------------------------
     // Wavefront r owns row blocks of eight rows: kLoadsA of the activations, kLoadsW of
@@ -191,15 +201,28 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
     const uint32_t ring_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_ptr)ring));
     const char* const base_a = A + static_cast<size_t>(m0) * row_bytes + static_cast<size_t>(kt0) * kDmaRowBytes;
     const char* const base_w = W + static_cast<size_t>(n0) * row_bytes + static_cast<size_t>(kt0) * kDmaRowBytes;
+    // the chunk of its row that this lane fetches with load i (what the swizzle above makes of it)
+    auto chunk_of = [&](int i) TPQ_INLINED {
+        const int block = i < kLoadsA ? rq * kLoadsA + i : BM / 8 + rq * kLoadsW + (i - kLoadsA);
+        return (lane & 7) ^ (((block * 8 + (lane >> 3)) >> 1) & 7);
+    };
     // loads [FIRST, FIRST + COUNT) of stage kt into ring slot SLOT: scalar base, constant per-lane offset, no vector ALU
-    auto request = [&](auto first, auto count, auto slot_c, int kt) {
+    // edge_c: kt may be the partial stage
+    auto request = [&](auto first, auto count, auto slot_c, int kt, auto edge_c) TPQ_INLINED {
         constexpr int FIRST = decltype(first)::value, COUNT = decltype(count)::value, SLOT = decltype(slot_c)::value;
-        const char* const sa = base_a + static_cast<size_t>(kt) * kDmaRowBytes;
-        const char* const sw = base_w + static_cast<size_t>(kt) * kDmaRowBytes;
+        constexpr bool kMayBeEdge = EDGE && decltype(edge_c)::value;
+        const int last_chunk = kMayBeEdge && kt == nk - 1 && edge_chunks ? edge_chunks - 1 : 7;
+        const size_t k_bytes = static_cast<size_t>(kt) * kDmaRowBytes;
+        const char* const sa = base_a + k_bytes;
+        const char* const sw = base_w + k_bytes;
 #pragma unroll
         for (int i = FIRST; i < FIRST + COUNT; ++i) {
             const uint32_t dst = ring_addr + SLOT * kStageBytes + lds_of_load[i];
-            const uint32_t off = voff[i];
+            uint32_t off = voff[i];
+            if constexpr (kMayBeEdge) {  // (arithmetic, not a branch)
+                const int behind = chunk_of(i) - last_chunk;
+                off -= static_cast<uint32_t>(behind > 0 ? behind : 0) * 16;
+            }
             if (i < kLoadsA) {
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(sa) : "memory", "m0");
             } else {
@@ -209,7 +232,18 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
     };
     constexpr std::integral_constant<int, 0> c0{};
     constexpr std::integral_constant<int, kLoads> cAll{};
-        auto request_stage = [&](auto slot_c, int kt) { request(c0, cAll, slot_c, kt); };
+    auto request_stage = [&](auto slot_c, int kt, auto edge_c) TPQ_INLINED { request(c0, cAll, slot_c, kt, edge_c); };
+    // the partial stage has landed in SLOT: zeros over what this lane fetched in place of chunks behind the row's end
+    auto clear_behind_edge = [&](auto slot_c) TPQ_INLINED {
+        constexpr int SLOT = decltype(slot_c)::value;
+        const v4i zero = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const uint32_t where = ring_addr + SLOT * kStageBytes + lds_of_load[i] + lane * 16;
+            if (chunk_of(i) >= edge_chunks) asm volatile("ds_write_b128 %0, %1" ::"v"(where), "v"(zero) : "memory");
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
 
     // ---- fragment reads -----------------------------------------------------------------------------------------
     // v_mfma_i32_16x16x64_i8: lane (r = lane % 16, c = lane / 16) holds row r, 16-byte chunk c of a k-half of 64 bytes.
@@ -229,7 +263,7 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
             addr_b[s][kh] = ring_addr + s * kStageBytes + (BM + wn * WN + frag_row) * kDmaRowBytes + chunk;
         }
     v4i fa[2][MB], fb[2][4];  // [k-half][block of 16 rows]
-    auto read_half = [&](auto slot_c, auto half_c) {
+    auto read_half = [&](auto slot_c, auto half_c) TPQ_INLINED {
         constexpr int SLOT = decltype(slot_c)::value;
 #pragma unroll
         for (int kh = decltype(half_c)::value; kh < decltype(half_c)::value + 1; ++kh) {
@@ -246,7 +280,7 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
             asm volatile("ds_read_b128 %0, %1 offset:6144" : "=v"(b3) : "v"(ab) : "memory");
         }
     };
-    auto read_stage = [&](auto slot_c) {
+    auto read_stage = [&](auto slot_c) TPQ_INLINED {
         read_half(slot_c, std::integral_constant<int, 0>{});
         read_half(slot_c, std::integral_constant<int, 1>{});
     };
@@ -255,20 +289,20 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
 #endif
     // memory phase of a wavefront that also requests: TPQ_STAGGER_INTERLEAVE 0: the reads, then the requests; 1: a third
     // of the requests ahead of each half of the reads and behind them, so that the memory path has work from the start
-    auto read_and_request = [&](auto read_slot, auto fill_slot, int kt_new) {
+    auto read_and_request = [&](auto read_slot, auto fill_slot, int kt_new, auto edge_c) TPQ_INLINED {
         if constexpr (TPQ_STAGGER_INTERLEAVE == 0) {
             read_stage(read_slot);
-            request_stage(fill_slot, kt_new);
+            request_stage(fill_slot, kt_new, edge_c);
         } else {
             constexpr int kFirst = (kLoads + 2) / 3, kSecond = (kLoads - kFirst + 1) / 2, kThird = kLoads - kFirst - kSecond;  // 2 2 2 (2 1 1)
-            request(std::integral_constant<int, 0>{}, std::integral_constant<int, kFirst>{}, fill_slot, kt_new);
+            request(std::integral_constant<int, 0>{}, std::integral_constant<int, kFirst>{}, fill_slot, kt_new, edge_c);
             read_half(read_slot, std::integral_constant<int, 0>{});
-            request(std::integral_constant<int, kFirst>{}, std::integral_constant<int, kSecond>{}, fill_slot, kt_new);
+            request(std::integral_constant<int, kFirst>{}, std::integral_constant<int, kSecond>{}, fill_slot, kt_new, edge_c);
             read_half(read_slot, std::integral_constant<int, 1>{});
-            request(std::integral_constant<int, kFirst + kSecond>{}, std::integral_constant<int, kThird>{}, fill_slot, kt_new);
+            request(std::integral_constant<int, kFirst + kSecond>{}, std::integral_constant<int, kThird>{}, fill_slot, kt_new, edge_c);
         }
     };
-    auto stage_ready = [&]() {  // every fragment read has delivered; the MFMAs that use them stay behind this point
+    auto stage_ready = [&]() TPQ_INLINED {  // every fragment read has delivered; the MFMAs that use them stay behind this point
         // (every register must appear once: a register named twice would be copied in front of the wait)
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[0][0]), "+v"(fa[0][1]), "+v"(fb[0][0]), "+v"(fb[0][1]), "+v"(fb[0][2]), "+v"(fb[0][3]));
         asm volatile("" : "+v"(fa[1][0]), "+v"(fa[1][1]), "+v"(fb[1][0]), "+v"(fb[1][1]), "+v"(fb[1][2]), "+v"(fb[1][3]));
@@ -282,7 +316,7 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
         for (int j = 0; j < 4; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
     // W fragment first: a lane ends up with 4 consecutive n for one m.  Column blocks in snake order, so that one operand
     // changes from one instruction to the next.
-    auto multiply_stage = [&]() {
+    auto multiply_stage = [&]() TPQ_INLINED {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(kPhasePrio);
 #pragma unroll
@@ -303,7 +337,7 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
     // behind the scales with a bare instruction, copied out at the end
     uint4* phase_lds = reinterpret_cast<uint4*>(lds_bytes + kRingBytes + (2 * BN + BM) * sizeof(float)) + wave * 64;
     int phase_index = 0;
-    auto phase_end = [&]() {
+    auto phase_end = [&]() TPQ_INLINED {
         __builtin_amdgcn_sched_barrier(0);
         if (phase_index > 0) {
             uint32_t t0, t1, t2, t3;
@@ -321,15 +355,15 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
         __builtin_amdgcn_sched_barrier(0);
     };
 #else
-    auto phase_end = [&]() {
+    auto phase_end = [&]() TPQ_INLINED {
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
 #endif
-    auto wait_loads = [&](auto allowed) { __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(allowed)::value)); };
+    auto wait_loads = [&](auto allowed) TPQ_INLINED { __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(allowed)::value)); };
     // at most `stages` (0 .. S - 1, wave-uniform) whole stages of this wavefront's requests may still be outstanding
-    auto wait_stages = [&](int stages) {
+    auto wait_stages = [&](int stages) TPQ_INLINED {
         bool done = false;
         static_for<0, S>([&](auto i) {
             constexpr int N = S - 1 - decltype(i)::value;  // S - 1 down to 0
@@ -366,38 +400,41 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
     {
         const int mine = wave < 4 ? (nk < S ? nk : S) : (nk < S - 1 ? nk : S - 1);  // stages this wavefront requests here
         static_for<0, S>([&](auto st) {
-            if (decltype(st)::value < mine) request_stage(st, decltype(st)::value);
+            if (decltype(st)::value < mine) request_stage(st, decltype(st)::value, std::true_type{});
         });
         wait_stages(mine - 1);  // stage 0 (and the scales in front of it) landed
+        if (EDGE && edge_chunks && nk == 1) clear_behind_edge(c0);
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     TPQ_STAGGER_STAMP(1);
 
     // one phase pair of a wavefront; SLOT = slot of stage kt.  STEADY: every stage named exists, no conditions.
     // group 0: multiply kt | read kt + 1, request kt + S into SLOT
-    auto group0_step = [&](auto slot_c, auto steady, int kt) {
+    auto group0_step = [&](auto slot_c, auto steady, int kt) TPQ_INLINED {
         constexpr int SLOT = decltype(slot_c)::value, NEXT = (SLOT + 1) % S;
         constexpr bool STEADY = decltype(steady)::value;
         multiply_stage();
         if (STEADY) wait_loads(kSteadyWait);  // own share of kt + 1 landed (kt + 2 .. may be in flight)
         else wait_stages(nk - kt - 2 < 0 ? 0 : nk - kt - 2 < S - 2 ? nk - kt - 2 : S - 2);
+        if (EDGE && !STEADY && edge_chunks && kt + 1 == nk - 1) clear_behind_edge(std::integral_constant<int, NEXT>{});
         phase_end();
         if (STEADY || kt + 1 < nk) {
-            if (STEADY || kt + S < nk) read_and_request(std::integral_constant<int, NEXT>{}, slot_c, kt + S);
+            if (STEADY || kt + S < nk) read_and_request(std::integral_constant<int, NEXT>{}, slot_c, kt + S, std::integral_constant<bool, !STEADY>{});
             else read_stage(std::integral_constant<int, NEXT>{});
             stage_ready();
             phase_end();
         }
     };
     // group 1: read kt, request kt + S - 1 into the slot of kt - 1 | multiply kt
-    auto group1_step = [&](auto slot_c, auto steady, int kt) {
-        constexpr int SLOT = decltype(slot_c)::value, PREV = (SLOT + S - 1) % S;
+    auto group1_step = [&](auto slot_c, auto steady, int kt) TPQ_INLINED {
+        constexpr int SLOT = decltype(slot_c)::value, PREV = (SLOT + S - 1) % S, NEXT = (SLOT + 1) % S;
         constexpr bool STEADY = decltype(steady)::value;
-        if (STEADY || kt + S - 1 < nk) read_and_request(slot_c, std::integral_constant<int, PREV>{}, kt + S - 1);
+        if (STEADY || kt + S - 1 < nk) read_and_request(slot_c, std::integral_constant<int, PREV>{}, kt + S - 1, std::integral_constant<bool, !STEADY>{});
         else read_stage(slot_c);
         stage_ready();
         if (STEADY) wait_loads(kSteadyWait);  // own share of kt + 1 landed (kt + 2 .. may be in flight)
         else wait_stages(nk - kt - 2 < 0 ? 0 : nk - kt - 2 < S - 2 ? nk - kt - 2 : S - 2);
+        if (EDGE && !STEADY && edge_chunks && kt + 1 == nk - 1) clear_behind_edge(std::integral_constant<int, NEXT>{});
         phase_end();
         multiply_stage();
         if (STEADY || kt + 1 < nk) phase_end();
@@ -406,22 +443,22 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
     constexpr std::false_type kChecked{};
 
     // The steady loops are unrolled S times so that the ring slot is a constant; what is left behind them (at most
-    // 2 S - 1 stages) is nested straight-line code with the conditions of the ends (a loop with a runtime slot made
+    // 2 S - 1 stages, one more with an edge) is nested straight-line code with the conditions of the ends (a loop with a runtime slot made
     // the compiler copy the accumulators between its arms).
     int kt = 0;
     if (wave < 4) {
         read_stage(c0);
         stage_ready();
-        for (; kt + 2 * S - 1 < nk; kt += S)
+        for (; kt + 2 * S - 1 < nk_steady; kt += S)
             static_for<0, S>([&](auto i) { group0_step(i, kSteady, kt + decltype(i)::value); });
-        nested_while_below<0, 2 * S - 1>(kt, nk, [&](auto d) {  // the first of them in slot 0
+        nested_while_below<0, 2 * S - 1 + kTail>(kt, nk, [&](auto d) {  // the first of them in slot 0
             group0_step(std::integral_constant<int, decltype(d)::value % S>{}, kChecked, kt + decltype(d)::value);
         });
     } else {
         group1_step(c0, kChecked, 0);
-        for (kt = 1; kt + 2 * S - 2 < nk; kt += S)
+        for (kt = 1; kt + 2 * S - 2 < nk_steady; kt += S)
             static_for<0, S>([&](auto i) { group1_step(std::integral_constant<int, (1 + decltype(i)::value) % S>{}, kSteady, kt + decltype(i)::value); });
-        nested_while_below<0, 2 * S - 2>(kt, nk, [&](auto d) {  // the first of them in slot 1
+        nested_while_below<0, 2 * S - 2 + kTail>(kt, nk, [&](auto d) {  // the first of them in slot 1
             group1_step(std::integral_constant<int, (1 + decltype(d)::value) % S>{}, kChecked, kt + decltype(d)::value);
         });
     }
@@ -503,21 +540,27 @@ __global__ __launch_bounds__(512) void gemm_stagger_kernel(const char* __restric
     TPQ_STAGGER_STAMP(3);
 }
 
-// row_bytes = K * sizeof(element): a multiple of 128 below 2^23
-template <class Arith, int MB, class Tile>
-int launch_stagger_bytes(const void* a, const void* w, int64_t M, int64_t N, int64_t row_bytes, Tile tile, hipStream_t s, int slices, const char* what) {
+// row_bytes = K * sizeof(element): below 2^23, a multiple of 128 or (EDGE) of 16.  Two instantiations: with the edge's code in
+// it the kernel without an edge loses 0.3 us (2048 x 4096 x 4096 33.6 -> 33.9 with the quantizer).
+template <class Arith, int MB, bool EDGE, class Tile>
+int launch_stagger_as(const void* a, const void* w, int64_t M, int64_t N, int64_t row_bytes, Tile tile, hipStream_t s, int slices, const char* what) {
     constexpr int BM = 64 * MB;
     constexpr size_t smem = static_cast<size_t>(kDmaStages) * (BM + 128) * kDmaRowBytes + (2 * 128 + BM) * sizeof(float) + kStaggerStampBytes;
     const int64_t tiles = ((M + BM - 1) / BM) * ((N + 127) / 128);
     TPQ_REQUIRE(tiles <= 0x7FFFFFFF, TPQ_ERR_INVALID_VALUE, "staggered gemm: too many tiles");
-    TPQ_REQUIRE(row_bytes % kDmaRowBytes == 0 && row_bytes < (1 << 23), TPQ_ERR_INVALID_VALUE, "staggered gemm: a row of k must be a multiple of 128 bytes below 2^23");
-    auto kernel = gemm_stagger_kernel<Tile, Arith, MB>;
+    TPQ_REQUIRE(row_bytes > 0 && row_bytes % (EDGE ? 16 : kDmaRowBytes) == 0 && row_bytes < (1 << 23), TPQ_ERR_INVALID_VALUE, "staggered gemm: a row of k must be a multiple of %d bytes below 2^23", EDGE ? 16 : kDmaRowBytes);
+    auto kernel = gemm_stagger_kernel<Tile, Arith, MB, EDGE>;
     static std::atomic<uint64_t> configured{0};  // per instantiation
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), smem, configured, what)) return rc;
     const int vector_stores = (N * sizeof(typename Tile::out_t)) % 16 == 0 && aligned(tile.out, 16);
     kernel<<<dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(slices)), 512, smem, s>>>(
         static_cast<const char*>(a), static_cast<const char*>(w), static_cast<int>(M), static_cast<int>(N), static_cast<int>(row_bytes), tile, vector_stores, slices);
     return check_launch(what);
+}
+
+template <class Arith, int MB, class Tile>
+int launch_stagger_bytes(const void* a, const void* w, int64_t M, int64_t N, int64_t row_bytes, Tile tile, hipStream_t s, int slices, const char* what) {
+    return launch_stagger_as<Arith, MB, false>(a, w, M, N, row_bytes, tile, s, slices, what);
 }
 
 template <class Tile>

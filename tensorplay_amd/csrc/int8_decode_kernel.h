@@ -18,14 +18,16 @@
 namespace tpq {
 namespace {
 
-template <int NB, int MB, int WAVES, class Epilogue>
+// RAGGED: any K >= 1 and any alignment.  Rows that are no multiple of 128 bytes start anywhere in a cache line, so a load
+// touches more of them, but the weight is still read once, in place.
+template <int NB, int MB, int WAVES, class Epilogue, bool RAGGED = false>
 __global__ __launch_bounds__(WAVES * kWave) void int8_decode_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ w,
                                                                    int M, int N, int K, Epilogue ep) {
     __shared__ int red[WAVES][NB * MB][4][kWave];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = lane & 15, q = lane >> 4;
-    const int steps = K / 128;
+    const int steps = RAGGED ? (K + 127) / 128 : K / 128;
     const int n0 = blockIdx.x * (16 * NB);
     const uint4* w_base[NB];
 #pragma unroll
@@ -46,6 +48,19 @@ __global__ __launch_bounds__(WAVES * kWave) void int8_decode_kernel(const int8_t
         uint4 xv[MB][2];
     };
     auto load = [&](int s, Step& st) {
+        if constexpr (RAGGED) {
+            const int left = K - s * 128 - q * 32;  // bytes of the row at and behind this lane's 32
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) st.w[b][h] = load_k16_ragged(reinterpret_cast<const int8_t*>(w_base[b] + s * 8 + h), left - 16 * h);
+#pragma unroll
+            for (int r = 0; r < MB; ++r)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (row_live[r]) st.xv[r][h] = load_k16_ragged(reinterpret_cast<const int8_t*>(x_base[r] + s * 8 + h), left - 16 * h);
+            return;
+        }
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             st.w[b][0] = nt_load(w_base[b] + s * 8);
@@ -287,6 +302,22 @@ bool launch_int8_flight(const int8_t* x, const int8_t* w, int rows, int N, int K
 #undef TPQ_I8F_ROWS
 #undef TPQ_I8F
     return true;
+}
+
+// Any K and alignment, in slabs of 32 rows (16 for what is left).
+template <class Epilogue, class Rebase>
+int launch_int8_decode_ragged(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t K, Epilogue ep, Rebase rebase, hipStream_t s) {
+    const int n = static_cast<int>(N), k = static_cast<int>(K);
+    const dim3 grid(static_cast<unsigned>((N + 15) / 16));
+    for (int64_t m0 = 0; m0 < M;) {
+        const int rows = static_cast<int>(M - m0 < 32 ? M - m0 : 32);
+        const Epilogue slab = rebase(ep, m0);
+        const int8_t* xs = a + m0 * K;
+        if (rows > 16) int8_decode_kernel<1, 2, 8, Epilogue, true><<<grid, 8 * kWave, 0, s>>>(xs, w, rows, n, k, slab);
+        else int8_decode_kernel<1, 1, 8, Epilogue, true><<<grid, 8 * kWave, 0, s>>>(xs, w, rows, n, k, slab);
+        m0 += rows;
+    }
+    return check_launch("int8 decode gemm (any K)");
 }
 
 // slabs of 32 rows (16 for what is left); the epilogue sees row indices of the whole problem through `rebase`

@@ -36,7 +36,7 @@ struct TiledPlan {
     int slices;
 };
 inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, bool may_slice) {
-    const double nk = static_cast<double>(K / kDmaRowBytes);
+    const double nk = static_cast<double>((K + kDmaRowBytes - 1) / kDmaRowBytes);
     const int64_t cols = (N + 127) / 128, t256 = ((M + 255) / 256) * cols, t128 = ((M + 127) / 128) * cols;
     const double stream = 128.0 * static_cast<double>(K) / 12.5;  // a tile's weight bytes at what one compute unit pulls from HBM
     const double tall_tile = nk * 1080.0 + 9000.0, short_tile = nk * 690.0 + 8000.0;
@@ -74,6 +74,10 @@ int launch_tiled(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t
     }
     if (K >= (1 << 23) || (env && env[0] == 'd')) return launch_dma(a, w, M, N, K, tile, s, 1);
     const bool use_short = env ? env[0] == 'h' : plan_tiled(M, N, K, false).form == kShort;
+    if (K % kDmaRowBytes != 0) {
+        if (use_short) return launch_stagger_as<ArithI8, 2, true>(a, w, M, N, K, tile, s, 1, "int8 mfma gemm (staggered, 128 rows, edge in k)");
+        return launch_stagger_as<ArithI8, 4, true>(a, w, M, N, K, tile, s, 1, "int8 mfma gemm (staggered, edge in k)");
+    }
     if (use_short) return launch_stagger_bytes<ArithI8, 2>(a, w, M, N, K, tile, s, 1, "int8 mfma gemm (staggered, 128 rows)");
     return launch_stagger(a, w, M, N, K, tile, s, 1);
 }
@@ -97,6 +101,12 @@ template <int DT>
 EpilogueDequant<DT> rebase_rows(const EpilogueDequant<DT>& ep, int64_t m0, int64_t N) {
     return EpilogueDequant<DT>{ep.out + m0 * N, ep.rs + m0, ep.cs, ep.bias};
 }
+
+// Rows of k that the aligned decode kernel does not take: up to this many activation rows the same kernel with loads from
+// any address.  Measured (us, this kernel / what ran before, one output per thread for K % 16 != 0): 5284 -> 2944 at 2 rows
+// 6.5 / 136, 3640 -> 1280 at 16 and 32 rows 6.7 and 9.2 / 107; 1328 -> 3113 (K % 16 == 0) at 16 rows 4.4 / 7.6.
+constexpr int64_t kRaggedRows = 32;
+inline bool int8_decode_ragged_ok(int64_t M, int64_t N, int64_t K) { return M >= 1 && K >= 1 && N <= 0x7FFFFFF0 && K <= 0x7FFFFF00; }
 
 // Up to this many rows the decode kernel streams the weight once per 32 rows.
 inline int int8_decode_rows(int64_t N) {
@@ -193,11 +203,30 @@ int launch_best(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t 
     const int decode_rows = int8_decode_rows(N);
     if (M <= decode_rows && int8_decode_ok(a, w, M, N, K) && !(force && force[0] == 'r'))
         return launch_int8_decode(a, w, M, N, K, ep, [N](const Epilogue& e, int64_t m0) { return rebase_rows(e, m0, N); }, s);
+    if (M <= kRaggedRows && int8_decode_ragged_ok(M, N, K) && !(force && force[0] == 'r'))
+        return launch_int8_decode_ragged(a, w, M, N, K, ep, [N](const Epilogue& e, int64_t m0) { return rebase_rows(e, m0, N); }, s);
     // The ring-buffered kernel also wins when its 256 x 128 tiles fill only part of the chip: at K = N = 4096,
     // M = 512 / 1024 it takes 27.9 / 29.5 us against 33.9 / 39.4 us for the register-staged kernel on 128 x 64 tiles.
     // (65 .. 128 rows included: on 128 x 128 tiles 128 rows of 4096 x 4096 take 15 us, 24.6 on the register-staged kernel)
-    if (K % kDmaRowBytes == 0 && !(force && force[0] == 'r')) return launch_tiled(a, w, M, N, K, to_tile(ep), s);
+    // Rows that are no multiple of the 128-byte stage (K % 16 == 0 still) take the staggered kernel's edge stage from 65 rows
+    // on: 473 rows of 1328 -> 3113 12.5 us (register-staged kernel 37.8); below, the 64 x 32 tiles of that one have the more
+    // workgroups (48 rows of the same 8.7 us, staggered 9.6).
+    if ((K % kDmaRowBytes == 0 || (M > 64 && K < (1 << 23))) && !(force && force[0] == 'r')) return launch_tiled(a, w, M, N, K, to_tile(ep), s);
     return launch_mfma(a, w, M, N, K, ep, s);
+}
+
+// Copies of both operands with rows of K_padded bytes, zeros behind K (the tiled kernels want rows that start at 16-byte
+// addresses): one 16-byte chunk of a destination per thread.
+__global__ __launch_bounds__(256) void int8_pad_rows_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ w, int64_t chunks_a,
+                                                            int64_t chunks, int K, int chunks_per_row, uint4* __restrict__ a_out,
+                                                            uint4* __restrict__ w_out) {
+    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < chunks; i += gridDim.x * 256ll) {
+        const bool of_a = i < chunks_a;
+        const int64_t j = of_a ? i : i - chunks_a;
+        const int64_t row = j < 0x7FFFFFFF ? static_cast<uint32_t>(j) / static_cast<uint32_t>(chunks_per_row) : j / chunks_per_row;
+        const int k = static_cast<int>(j - row * chunks_per_row) * 16;
+        (of_a ? a_out : w_out)[j] = load_k16_ragged((of_a ? a : w) + row * K + k, K - k);
+    }
 }
 
 // Any strides, any K, signed or unsigned left operand: 16x16 outputs per
@@ -283,8 +312,11 @@ TPQ_EXPORT int tpq_int_mm(const void* a, int a_unsigned, const int8_t* b, int64_
     }
     TPQ_REQUIRE(a && b, TPQ_ERR_INVALID_VALUE, "_int_mm: null operand");
     const EpilogueInt32 ep{c};
-    if (!a_unsigned && b_stride_k == 1 && b_stride_n == K && mfma_path_ok(a, b, M, N, K))
-        return launch_best(static_cast<const int8_t*>(a), b, M, N, K, ep, s);
+    if (!a_unsigned && b_stride_k == 1 && b_stride_n == K) {
+        if (mfma_path_ok(a, b, M, N, K)) return launch_best(static_cast<const int8_t*>(a), b, M, N, K, ep, s);
+        if (M <= kRaggedRows && int8_decode_ragged_ok(M, N, K))
+            return launch_int8_decode_ragged(static_cast<const int8_t*>(a), b, M, N, K, ep, [N](const EpilogueInt32& e, int64_t m0) { return rebase_rows(e, m0, N); }, s);
+    }
     return launch_generic(a, a_unsigned, b, b_stride_k, b_stride_n, M, K, N, ep, s);
 }
 
@@ -299,11 +331,13 @@ TPQ_EXPORT int tpq_int8_mm_dequant(const int8_t* a, const int8_t* w, const float
                 "int8_mm_dequant: null pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool fast = K > 0 && mfma_path_ok(a, w, M, N, K);
+    const bool ragged = M <= kRaggedRows && int8_decode_ragged_ok(M, N, K);
 #define TPQ_DISPATCH(DT)                                                                            \
     {                                                                                               \
         const EpilogueDequant<DT> ep{static_cast<typename Elem<DT>::storage*>(out), row_scale,      \
                                      col_scale, bias};                                              \
         if (fast) return launch_best(a, w, M, N, K, ep, s);                                         \
+        if (ragged) return launch_int8_decode_ragged(a, w, M, N, K, ep, [N](const EpilogueDequant<DT>& e, int64_t m0) { return rebase_rows(e, m0, N); }, s); \
         return launch_generic(a, 0, w, 1, K, M, K, N, ep, s);                                       \
     }
     switch (out_dtype) {
@@ -312,6 +346,20 @@ TPQ_EXPORT int tpq_int8_mm_dequant(const int8_t* a, const int8_t* w, const float
         default: TPQ_DISPATCH(TPQ_DTYPE_BF16)
     }
 #undef TPQ_DISPATCH
+}
+
+TPQ_EXPORT int tpq_int8_pad_rows(const int8_t* a, int64_t M, const int8_t* w, int64_t N, int64_t K, int8_t* a_out, int8_t* w_out,
+                                 int64_t K_padded, void* stream) {
+    TPQ_REQUIRE(M >= 0 && N >= 0 && K >= 0 && K_padded >= K && K_padded % 16 == 0, TPQ_ERR_INVALID_VALUE,
+                "int8_pad_rows: K_padded must be a multiple of 16, at least K");
+    const int64_t chunks_a = a_out ? M * (K_padded / 16) : 0, chunks_w = w_out ? N * (K_padded / 16) : 0;
+    if (chunks_a + chunks_w == 0) return TPQ_OK;
+    TPQ_REQUIRE(K == 0 || ((a || !chunks_a) && (w || !chunks_w)), TPQ_ERR_INVALID_VALUE, "int8_pad_rows: null pointer");
+    TPQ_REQUIRE(aligned(a_out, 16) && aligned(w_out, 16) && K_padded <= 0x7FFFFFF0, TPQ_ERR_INVALID_VALUE, "int8_pad_rows: destinations must be 16-byte aligned");
+    const int64_t blocks = (chunks_a + chunks_w + 255) / 256;
+    int8_pad_rows_kernel<<<static_cast<unsigned>(blocks > 16384 ? 16384 : blocks), 256, 0, static_cast<hipStream_t>(stream)>>>(
+        a, w, chunks_a, chunks_a + chunks_w, static_cast<int>(K), static_cast<int>(K_padded / 16), reinterpret_cast<uint4*>(a_out), reinterpret_cast<uint4*>(w_out));
+    return check_launch("int8_pad_rows");
 }
 
 TPQ_EXPORT int64_t tpq_int8_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {

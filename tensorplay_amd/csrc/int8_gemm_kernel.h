@@ -33,6 +33,20 @@ constexpr int kChunksPerRow = 4;    // 16-byte chunks per row per stage
 
 __device__ __forceinline__ int swz(int row) { return (((row >> 1) ^ (row >> 3)) & 1) | (((row >> 2) & 1) << 1); }
 
+// 16 bytes of k from any address (global_load_dwordx4 takes unaligned ones), `left` of them inside the row: the rest are zeros
+__device__ __forceinline__ uint4 load_k16_ragged(const int8_t* p, int left) {
+    typedef uint32_t u4_unaligned __attribute__((ext_vector_type(4), aligned(1)));
+    if (left >= 16) {
+        const u4_unaligned v = *reinterpret_cast<const u4_unaligned*>(p);
+        return make_uint4(v.x, v.y, v.z, v.w);
+    }
+    uint32_t d[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 15; ++e)
+        if (e < left) d[e >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(p[e])) << (8 * (e & 3));
+    return make_uint4(d[0], d[1], d[2], d[3]);
+}
+
 struct EpilogueInt32 {
     int32_t* c;
     __device__ __forceinline__ void store(int64_t idx, int m, int n, int v) const { c[idx] = v; }
