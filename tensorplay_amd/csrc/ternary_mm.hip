@@ -119,6 +119,97 @@ __global__ __launch_bounds__(256) void ternary_generic_kernel(const int8_t* __re
     }
 }
 
+// ---- the expanded route --------------------------------------------------------------------------------
+// The packed weight written out once per call as int8 rows of kp bytes (zeros behind K), the weight's one scale as a column
+// of scales, and, where K is no multiple of the tile stage, the activation codes copied to rows of kp bytes as well; the
+// int8 GEMM does the rest with the same sums and the same float operations.  It pays where the GEMM's rate is worth more
+// than the pass (N K bytes written: 7 us at 2560 x 6912), and wherever K fits none of the packed kernels.  Measured (us,
+// expanded / packed kernels): 2560 -> 6912 at 384, 777, 2048 rows 24.5 / 22.3, 31 / 42, 51 / 90; 6912 -> 2560 33 / 21,
+// 40 / 45, 45 / 81; 1024 -> 2048 11 / 6, 12.5 / 10.5, 13 / 19.  K that is no multiple of 256 (the tile kernel's stage):
+// 1920 -> 5504 at 256 rows 20 / 45; K % 64 != 0, where one thread computed an output: 3412 <-> 7872 at 759 rows (both
+// linears) 0.1 ms / 90 ms.
+inline int64_t ternary_padded_k(int64_t K) { return (K + 127) / 128 * 128; }
+inline int64_t round_up_256(int64_t v) { return (v + 255) / 256 * 256; }
+
+struct ExpandedPlan {
+    int64_t kp, x_at, scale_at, gemm_at, gemm_bytes, total;  // byte offsets into the workspace, the weight at 0
+};
+inline ExpandedPlan plan_expanded(int64_t M, int64_t N, int64_t K) {
+    ExpandedPlan p;
+    p.kp = ternary_padded_k(K);
+    p.x_at = round_up_256(N * p.kp);
+    p.scale_at = p.x_at + (p.kp == K ? 0 : round_up_256(M * p.kp));
+    p.gemm_at = p.scale_at + round_up_256(N * 4);
+    p.gemm_bytes = tpq_int8_mm_workspace_bytes(M, N, p.kp);
+    p.total = p.gemm_at + p.gemm_bytes;
+    return p;
+}
+
+// Does a kernel that reads the packed weight take this shape (operands aligned)?
+inline bool ternary_packed_kernel_takes(int64_t M, int64_t N, int64_t K) {
+    if (M == 1 && ternary_row_rows_per_workgroup(M, N, K)) return true;
+    if (M <= 32) return K % 256 == 0 || (M <= 8 && K % 64 == 0);
+    return ternary_slab_splits(M, N, K) >= 1 || K % kTgStage == 0;
+}
+
+inline bool ternary_wants_expanded(int64_t M, int64_t N, int64_t K) {
+    if (M < 1 || N < 1 || K < 1 || M > 0x7FFFFFFF || N > 0x7FFFFFF0 || K > 0x7FFFFF00) return false;
+    if (!ternary_packed_kernel_takes(M, N, K)) return true;
+    if (const char* e = tuning_env("TPQ_TERNARY_EXPAND")) return M >= std::atoll(e);
+    return M >= 1280 || (M > 640 && N * K >= (int64_t{1} << 23));
+}
+
+// grid-stride over 16-byte chunks: first the weight's (a packed 32-bit word each), then the activations' (if x_out)
+__global__ __launch_bounds__(256) void ternary_expand_kernel(const uint8_t* __restrict__ packed, const int8_t* __restrict__ x, int64_t chunks_w,
+                                                             int64_t chunks, int N, int K, int chunks_per_row, float w_scale, uint4* __restrict__ w_out,
+                                                             uint4* __restrict__ x_out, float* __restrict__ scales) {
+    typedef uint32_t word_unaligned __attribute__((aligned(1)));
+    const int64_t bpr = (K + 3) >> 2;
+    const int64_t first = blockIdx.x * 256ll + threadIdx.x, stride = gridDim.x * 256ll;
+    for (int64_t i = first; i < N; i += stride) scales[i] = w_scale;
+    for (int64_t i = first; i < chunks; i += stride) {
+        const bool of_w = i < chunks_w;
+        const int64_t j = of_w ? i : i - chunks_w;
+        const int64_t row = j < 0x7FFFFFFF ? static_cast<uint32_t>(j) / static_cast<uint32_t>(chunks_per_row) : j / chunks_per_row;
+        const int k = static_cast<int>(j - row * chunks_per_row) * 16, left = K - k;
+        if (!of_w) {
+            x_out[j] = load_k16_ragged(x + row * K + k, left);
+            continue;
+        }
+        uint4 codes = make_uint4(0, 0, 0, 0);
+        if (left >= 16) {
+            codes = ternary_word_to_i8x16(*reinterpret_cast<const word_unaligned*>(packed + row * bpr + (k >> 2)));
+        } else if (left > 0) {
+            uint32_t word = 0;
+            for (int b = 0; 4 * b < left; ++b) {
+                uint32_t byte = packed[row * bpr + (k >> 2) + b];
+                const int live = left - 4 * b;  // codes of this byte inside the row
+                if (live < 4) byte &= 0xFFu << (8 - 2 * live);
+                word |= (byte & 0xFFu) << (8 * b);
+            }
+            codes = ternary_word_to_i8x16(word);
+        }
+        w_out[j] = codes;
+    }
+}
+
+int launch_ternary_expanded(const int8_t* x, const float* row_scale, const uint8_t* packed, float w_scale, const float* bias, int64_t M, int64_t N,
+                            int64_t K, void* out, int out_dtype, const ExpandedPlan& p, void* workspace, hipStream_t s) {
+    char* const ws = static_cast<char*>(workspace);
+    const bool copy_x = p.kp != K;
+    const int64_t chunks_w = N * (p.kp / 16), chunks = chunks_w + (copy_x ? M * (p.kp / 16) : 0);
+    int8_t* const w8 = reinterpret_cast<int8_t*>(ws);
+    int8_t* const x8 = reinterpret_cast<int8_t*>(ws + p.x_at);
+    float* const scales = reinterpret_cast<float*>(ws + p.scale_at);
+    const int64_t blocks = (chunks + 255) / 256;
+    ternary_expand_kernel<<<static_cast<unsigned>(blocks > 16384 ? 16384 : blocks), 256, 0, s>>>(
+        packed, x, chunks_w, chunks, static_cast<int>(N), static_cast<int>(K), static_cast<int>(p.kp / 16), w_scale, reinterpret_cast<uint4*>(w8),
+        reinterpret_cast<uint4*>(x8), scales);
+    if (int rc = check_launch("tpq_ternary_mm (expand)")) return rc;
+    return tpq_int8_mm_dequant_ws(copy_x ? x8 : x, w8, row_scale, scales, bias, out, out_dtype, M, N, p.kp, p.gemm_bytes ? ws + p.gemm_at : nullptr,
+                                  p.gemm_bytes, s);
+}
+
 template <class Epilogue>
 int launch_ternary(const int8_t* x, const uint8_t* packed, int64_t M, int64_t N, int64_t K,
                    Epilogue ep, hipStream_t s, void* workspace, int64_t workspace_bytes) {
@@ -179,6 +270,7 @@ int launch_ternary(const int8_t* x, const uint8_t* packed, int64_t M, int64_t N,
 using namespace tpq;
 
 TPQ_EXPORT int64_t tpq_ternary_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (ternary_wants_expanded(M, N, K)) return plan_expanded(M, N, K).total;
     const int splits = M > 0 && N > 0 && K > 0 ? ternary_slab_splits(M, N, K) : 0;
     return splits > 1 ? static_cast<int64_t>(splits) * M * N * 4 : 0;
 }
@@ -201,6 +293,12 @@ TPQ_EXPORT int tpq_ternary_mm_ws(const int8_t* x, const float* row_scale, const 
     TPQ_REQUIRE((K == 0 || (x && packed)) && (!out || row_scale), TPQ_ERR_INVALID_VALUE,
                 "bitnet_linear_packed: null pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // (the raw sums are an output of the packed kernels only)
+    if (workspace != nullptr && !acc_out && K > 0 && aligned(workspace, 16) && aligned(x, 16) && ternary_wants_expanded(M, N, K)) {
+        const ExpandedPlan plan = plan_expanded(M, N, K);
+        if (workspace_bytes >= plan.total)
+            return launch_ternary_expanded(x, row_scale, packed, w_scale, bias, M, N, K, out, out_dtype, plan, workspace, s);
+    }
     switch (out_dtype) {
         case TPQ_DTYPE_F32: {
             const EpilogueTernary<TPQ_DTYPE_F32> ep{static_cast<float*>(out), acc_out, row_scale, bias, w_scale};

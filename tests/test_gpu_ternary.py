@@ -156,3 +156,22 @@ def test_ternary_one_row_kernel_arbitrary_bytes(ops, K, N):
     _, want_neg = oracle.ternary_mm(flipped, rs, packed, 0.03, K)
     _, neg = ops.ternary_mm(dev(flipped), dev(rs), dev(packed), 0.03, K, return_acc=True)
     np.testing.assert_array_equal(host(neg), want_neg)
+
+
+@pytest.mark.parametrize("M,K,N", [
+    # K that no kernel of the packed weight takes: whole bytes, part of a byte, part of a word, one code
+    (1, 3788, 40), (2, 5196, 33), (7, 1023, 24), (33, 1, 9), (40, 130, 17), (249, 3364, 66), (20, 1180, 136),
+    # many rows: the weight expanded for the int8 GEMM, K a multiple of its stage and not
+    (1300, 512, 72), (700, 6912, 1216), (700, 320, 100), (40, 1920, 5504)])
+def test_ternary_expanded(ops, M, K, N):
+    """The weight written out as int8 rows: any byte value (0b10 decodes to -2, codes behind K in the last byte ignored),
+    scaled output with bias equal to the oracle's bit for bit."""
+    rng = np.random.default_rng(M + K + N)
+    packed = rng.integers(0, 256, size=(N, (K + 3) // 4)).astype(np.uint8)
+    x = rng.integers(-127, 128, size=(M, K)).astype(np.int8)
+    rs = (rng.random(M) * 0.01 + 1e-3).astype(np.float32)
+    bias = rng.normal(0, 0.05, N).astype(np.float32)
+    for name in ("f32", "bf16"):
+        want, _ = oracle.ternary_mm(x, rs, packed, 0.03, K, bias=bias, out_dtype=name)
+        got = ops.ternary_mm(dev(x), dev(rs), dev(packed), 0.03, K, bias=dev(bias), out_dtype=TORCH_DT[name])
+        np.testing.assert_array_equal(host(got), want)
