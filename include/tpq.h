@@ -215,6 +215,22 @@ int tpq_ternary_mm_ws(const int8_t* x, const float* row_scale, const uint8_t* pa
                       int32_t* acc_out, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * The int4 and n-bit weight-only products for a block of activation rows (about 17 .. 500; any count is taken), float32 /
+ * float16 / bfloat16, groups of any multiple of 32 (int4: 32, 64 or 128, innerKTiles = 2), K % 32 == 0; anything else
+ * returns TPQ_ERR_UNSUPPORTED.  Same operations and reference lines as tpq_int4_mm and tpq_lowbit_mm (1, 2, 4, 8 bits); the
+ * dequantized weight is rounded to the activation type once.  x, packed: 16-byte aligned; out: 8 bytes (float32: 16);
+ * lowbit: N % 4 == 0.  workspace (16-byte aligned, contents undefined, may be NULL): with
+ * tpq_packed_rows_workspace_bytes bytes the k range can be cut into slices where the channels do not fill the chip; the
+ * slices are added in a fixed order.
+ */
+int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
+int tpq_int4_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, int64_t N, int64_t group,
+                     const void* scales_and_zeros, void* out, void* workspace, int64_t workspace_bytes, void* stream);
+int tpq_lowbit_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const uint8_t* packed, int bits, int lsb_first,
+                       int64_t N, int64_t group, const float* scales_and_zeros, const float* bias, void* out,
+                       void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Two fusions around the decode matmul for the MLP of a decoder layer (float16 / bfloat16
  * activations, innerKTiles = 2, group 128, K % 128 == 0; anything else returns TPQ_ERR_UNSUPPORTED
  * and the caller runs the separate ops).  Both round exactly where the separate ops would.

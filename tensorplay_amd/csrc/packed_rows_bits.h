@@ -1,0 +1,39 @@
+// Call of the n-bit packed product for a block of activation rows, between its entry point and the translation units of
+// the activation types.
+#pragma once
+
+#include "packed_rows_kernel.h"
+
+namespace tpq {
+
+struct PackedRowsBits {
+    const void *x, *packed, *sz;
+    const float* bias;
+    void *out, *workspace;
+    int64_t M, N, K, group, room_floats;
+    int bits, lsb_first;
+    hipStream_t stream;
+};
+
+int packed_rows_bits_f32(const PackedRowsBits& call);
+int packed_rows_bits_f16(const PackedRowsBits& call);
+int packed_rows_bits_bf16(const PackedRowsBits& call);
+
+namespace {
+
+template <int DT>
+int run_packed_rows_bits(const PackedRowsBits& c) {
+    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats);
+    PackedRowsArgs a{};
+    a.x = c.x; a.w = c.packed; a.sz = c.sz; a.bias = c.bias; a.y = c.out; a.partial = static_cast<float*>(c.workspace);
+    a.M = static_cast<int>(c.M); a.N = static_cast<int>(c.N); a.K = static_cast<int>(c.K); a.tiles_per_group = static_cast<int>(c.group / 32);
+    switch (c.bits) {
+        case 1: return c.lsb_first ? launch_packed_rows<DT, SourceBits<1, true>>(a, p, c.stream) : launch_packed_rows<DT, SourceBits<1, false>>(a, p, c.stream);
+        case 2: return launch_packed_rows<DT, SourceBits<2, false>>(a, p, c.stream);
+        case 4: return launch_packed_rows<DT, SourceBits<4, false>>(a, p, c.stream);
+        default: return launch_packed_rows<DT, SourceBits<8, false>>(a, p, c.stream);  // one code per byte: the bit order does not matter
+    }
+}
+
+}  // namespace
+}  // namespace tpq

@@ -1,0 +1,583 @@
+// Weight-only product of a block of activation rows (a prompt, a decode batch: 9 .. a few hundred rows) with a packed
+// weight, float16 / bfloat16 / float32, groups of any multiple of 32, K % 32 == 0:
+//   y[m][n] = sum_k x[m][k] w[n][k],  w dequantized in registers, once per 16 MB rows, on its way into the matrix cores.
+// The weight comes from one of two sources: the int4 device layout (tiles of 8 channels x 32 k) or rows of n-bit codes.
+//
+// What bounds it: with few rows the stream of the weight and the latency of its first bytes; from about 48 rows on what a
+// compute unit does per step of 128 k and 32 channels, of which four things cost about the same (clocks per round of the loop
+// at 64 rows, two multiplying wavefronts per SIMD): the activations through its vector memory path (64 KB at 21.6 clocks per
+// KB, 1400), the fragment reads from LDS (1024 + 512 for writing them), the dequantization (1280) and the products (1024).
+// Taken out one at a time they all shorten the loop, none by much (4096 x 4096 at 256 rows, bfloat16: 17.0 us, without
+// activations 13.3, without dequantization 16.5, without products 15.4, loads of weights and barriers alone 8.9).  Hence
+//   * a workgroup owns 64 channels (128 where that still fills the chip: half the activation bytes per product) and a slice of
+//     K (a few slices of K fill the chip where N / 64 workgroups do not; their fp32 sums meet in a second kernel, added in
+//     slice order);
+//   * its eight multiplying wavefronts are CW channel positions x KW steps of 128 k: a round of the loop covers KW steps, whose
+//     activations two more wavefronts fetch by direct global -> LDS loads (whole lines, one copy per workgroup, double
+//     buffered, the swizzle of the fragment reads applied on the global side) while the round before is multiplied.  A direct
+//     load blocks the wavefront that issues it until the memory path accepts it, and vector loads return in order, so in a
+//     multiplying wavefront it would stand in front of the products and tie the weights' prefetch to the activations';
+//   * packed weights and parameters are loaded two rounds ahead, into registers (four rounds: the same times, 40 registers
+//     more, and the tall tiles spill);
+//   * a lane (i, q) dequantizes the 32 codes of channel i at k = 128 s + 32 q: codes are brought under an fp16 exponent in place
+//     and one v_fma_mix per code applies scale and zero point in fp32, rounded once to the operand type (float16: the mix
+//     instruction's own rounding; bfloat16: v_cvt_pk_bf16_f32; float32: no rounding).  They are the A operand of
+//     v_mfma_f32_16x16x32_{f16,bf16} (float32: v_mfma_f32_16x16x4_f32), the activations as they lie in memory the B operand;
+//   * the KW partial sums of a tile meet in LDS at the end.
+// Measured (us, weights from HBM, this kernel / what ran before): int4, bfloat16, 11008 -> 4096 in groups of 64: 24 / 48 / 128 / 256
+// rows 12.4 / 22.8, 14.8 / 39, 24 / 43, 36 / 71; 4096 x 4096 in groups of 128: 33 / 64 / 256 rows 9.8 / 12.5, 11.2 / 20, 15.8 / 34;
+// 4768 -> 13544 in groups of 32 (K % 128 != 0): 3 / 33 rows 14.5 / 94, 24 / 871.  float32 4096 x 4096: 3 / 19 / 64 rows 11.7 / 21, 16 / 39,
+// 25 / 44 (bound by its MFMAs, 32 clocks for 16 x 16 x 4).  2 bits, bfloat16: 4096 -> 11008 at 32 / 56 / 203 rows 13.7 / 21, 16.7 / 42,
+// 52 / 68; 4096 x 4096 in groups of 32: 1 / 16 / 80 rows 8.0 / 26, 8.3 / 45, 12.5 / 168.
+// Rows >= M repeat row M - 1, steps of k behind the end of the slice are loaded (from the last step) and not multiplied, the
+// chunks of a last partial step behind K are cleared in LDS.
+#pragma once
+
+#include <atomic>
+#include <type_traits>
+
+#include "int4_lane.h"
+
+namespace tpq {
+namespace {
+
+typedef __attribute__((address_space(3))) void* pr_lds_ptr;
+typedef uint32_t pr_word4 __attribute__((ext_vector_type(4)));
+typedef _Float16 pr_half8 __attribute__((ext_vector_type(8)));
+typedef __bf16 pr_bf8 __attribute__((ext_vector_type(8)));
+
+constexpr int pr_vmcnt(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }  // s_waitcnt immediate, vmcnt only
+
+// a workgroup's eight multiplying wavefronts: CW (2 or 4) positions of two blocks of 16 channels x 8 / CW steps of k,
+constexpr int kRowsNB = 2;
+// and two more that only request activations
+constexpr int kRowsProducers = 2, kRowsThreads = (8 + kRowsProducers) * kWave;
+constexpr int kRowsAhead = 2;  // rounds of packed weights in registers
+
+#define TPQ_GLOBAL const __attribute__((address_space(1)))
+typedef uint32_t pr_word2 __attribute__((ext_vector_type(2)));
+
+struct PackedRowsArgs {
+    const void* x;         // [M][K]
+    const void* w;         // packed
+    const void* sz;        // int4: [K / group][N][2] of the activation type; n-bit: the same in float32
+    const float* bias;     // added in fp32 before the rounding (n-bit modules), or null
+    void* y;               // [M][N]
+    float* partial;        // [slices][M][N], or null: y
+    int M, N, K, tiles_per_group, steps_per_slice;
+    float inv_tiles_per_group;
+};
+
+// ---- the two weight sources ------------------------------------------------------------------------------
+// codes(): the lane's 32 codes as 16 pairs under fp16 exponents, pair p = codes 2 p, 2 p + 1 in k order
+// offset(p, half): what the exponent adds to the code (and to its bias) in that half
+
+// int4 device layout, [N / 8][K / 32] tiles of 8 rows x 16 bytes: word r of a row holds k = 2 r + 8 j, + 1 in nibbles j, 4 + j
+struct SourceInt4 {
+    static constexpr int kLoads = 1, kStepBytes = 512;  // (bytes from a step to the next)
+    static constexpr bool kTypedParams = true;          // (scale, zero) in the activation type; value = (code - 8) scale + zero
+    struct Words { uint4 v[1]; };
+    // byte offset of the lane's codes in step 0, and how far the last step's lie behind K (a partial last step)
+    static __device__ __forceinline__ uint32_t lane_offset(const PackedRowsArgs& a, int n, int q) {
+        const int tiles = a.N / 8, tile = n >> 3;
+        return static_cast<uint32_t>(tile < tiles ? tile : tiles - 1) * static_cast<uint32_t>(a.K / 32) * 128u + static_cast<uint32_t>(q * 128 + (n & 7) * 16);
+    }
+    static __device__ __forceinline__ uint32_t edge_back(int tiles_behind) { return static_cast<uint32_t>(tiles_behind) * 128u; }
+    static __device__ __forceinline__ void load(TPQ_GLOBAL char* step_base, uint32_t off, Words& d) {
+        const pr_word4 t = __builtin_nontemporal_load((TPQ_GLOBAL pr_word4*)(step_base + off));
+        d.v[0] = make_uint4(t.x, t.y, t.z, t.w);
+    }
+    static constexpr float offset(int p, int) { return ((p >> 2) & 1) ? 72.0f : 1032.0f; }  // exponent + 8
+    static __device__ __forceinline__ uint32_t pair(const Words& d, int p, const uint32_t (&magic)[2]) {
+        const int j = p >> 2, r = p & 3;  // k = 8 j + 2 r, + 1
+        const uint32_t w = r == 0 ? d.v[0].x : r == 1 ? d.v[0].y : r == 2 ? d.v[0].z : d.v[0].w;
+        const uint32_t t = j & 2 ? w >> 8 : w;
+        return (j & 1) ? (t & 0x00F000F0u) | magic[1] : (t & 0x000F000Fu) | magic[0];
+    }
+    static constexpr uint32_t kMagic0 = 0x64006400u, kMagic1 = 0x54005400u;
+};
+
+// rows of n-bit codes, 8 / BITS per byte (one for 5 .. 8 bits), the first in the most significant bits or (LSB) the least
+template <int BITS, bool LSB>
+struct SourceBits {
+    static constexpr int kPerByte = 8 / BITS, kBytes = 32 / kPerByte;  // bytes of a lane's 32 codes: 4, 8, 16 or 32
+    static constexpr int kLoads = kBytes == 32 ? 2 : 1, kStepBytes = 4 * kBytes;
+    static constexpr bool kTypedParams = false;  // float32 (scale, zero); value = (code - zero) scale
+    static constexpr uint32_t kField = (1u << BITS) - 1u;
+    struct Words { uint32_t v[kBytes / 4]; };
+    static __device__ __forceinline__ uint32_t lane_offset(const PackedRowsArgs& a, int n, int q) {
+        return static_cast<uint32_t>(n < a.N ? n : a.N - 1) * static_cast<uint32_t>(a.K / kPerByte) + static_cast<uint32_t>(q * kBytes);
+    }
+    static __device__ __forceinline__ uint32_t edge_back(int tiles_behind) { return static_cast<uint32_t>(tiles_behind * kBytes); }
+    static __device__ __forceinline__ void load(TPQ_GLOBAL char* step_base, uint32_t off, Words& d) {
+        TPQ_GLOBAL char* const p = step_base + off;
+        if constexpr (kBytes == 4) {
+            d.v[0] = __builtin_nontemporal_load((TPQ_GLOBAL uint32_t*)p);
+        } else if constexpr (kBytes == 8) {
+            const pr_word2 t = __builtin_nontemporal_load((TPQ_GLOBAL pr_word2*)p);
+            d.v[0] = t.x; d.v[1] = t.y;
+        } else {
+#pragma unroll
+            for (int e = 0; e < kBytes / 16; ++e) {
+                const pr_word4 t = __builtin_nontemporal_load((TPQ_GLOBAL pr_word4*)p + e);
+                d.v[4 * e] = t.x; d.v[4 * e + 1] = t.y; d.v[4 * e + 2] = t.z; d.v[4 * e + 3] = t.w;
+            }
+        }
+    }
+    static constexpr int pos(int c) { return LSB ? (c % kPerByte) * BITS : 8 - (c % kPerByte + 1) * BITS; }  // bit position of code c in its byte
+    static constexpr uint32_t exponent(int p) { return static_cast<uint32_t>(25 - p) << 10; }               // fp16 bits of 2^(10 - p)
+    // 8-bit codes are signed (the reference's unpack ends in int8): byte ^ 0x80 = value + 128
+    static constexpr float offset(int p, int half) { return static_cast<float>(1 << (10 - pos(2 * p + half))) + (BITS == 8 ? 128.0f : 0.0f); }
+    static __device__ __forceinline__ uint32_t pair(const Words& d, int p, const uint32_t (&)[2]) {
+        const int lo = 2 * p, hi = 2 * p + 1, byte_lo = lo / kPerByte, byte_hi = hi / kPerByte;
+        uint32_t w = d.v[byte_lo >> 2];
+        if constexpr (BITS == 8) w ^= 0x80808080u;
+        const uint32_t both = __builtin_amdgcn_perm(0u, w, 0x0C000C00u | (byte_lo & 3) | ((byte_hi & 3) << 16));
+        return (both & ((kField << pos(lo)) | (kField << (pos(hi) + 16)))) | (exponent(pos(lo)) | (exponent(pos(hi)) << 16));
+    }
+    static constexpr uint32_t kMagic0 = 0, kMagic1 = 0;
+};
+
+template <int FIRST, int LAST, class F>
+__device__ __forceinline__ void pr_static_for(F&& f) {
+    if constexpr (FIRST < LAST) {
+        f(std::integral_constant<int, FIRST>{});
+        pr_static_for<FIRST + 1, LAST>(f);
+    }
+}
+
+// step(0), step(1), .. for all but the last of `left` rounds, last() for that one, as nested straight-line code
+template <int R, int MOST, class F, class G>
+__device__ __forceinline__ void pr_last_rounds(int left, F&& step, G&& last) {
+    if constexpr (R + 1 < MOST) {
+        if (R + 1 < left) {
+            step(std::integral_constant<int, R>{});
+            pr_last_rounds<R + 1, MOST>(left, step, last);
+            return;
+        }
+    }
+    last(std::integral_constant<int, R>{});
+}
+
+// ---- operand types -----------------------------------------------------------------------------------
+template <int DT>
+struct RowsArith {  // 16-bit
+    static constexpr int kElem = 2, kChunks = 16;  // 16-byte chunks of a row and step
+    // four words = the eight dequantized weights of a 16-byte chunk
+    static __device__ __forceinline__ uint32_t pack(float lo, float hi) {
+        typedef float f2_t __attribute__((ext_vector_type(2)));
+        const f2_t v = {lo, hi};
+        if constexpr (DT == TPQ_DTYPE_BF16) {
+            typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+            return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf2_t));
+        } else {
+            return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, half2_t));
+        }
+    }
+    static __device__ __forceinline__ float4_t mfma(const pr_word4& a, const pr_word4& b, float4_t c) {
+        if constexpr (DT == TPQ_DTYPE_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pr_bf8, a), __builtin_bit_cast(pr_bf8, b), c, 0, 0, 0);
+        else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(pr_half8, a), __builtin_bit_cast(pr_half8, b), c, 0, 0, 0);
+    }
+};
+template <>
+struct RowsArith<TPQ_DTYPE_F32> {
+    static constexpr int kElem = 4, kChunks = 32;
+};
+
+// (scale, zero) of one channel and group
+template <int DT, bool TYPED>
+struct RowsParams {
+    using raw_t = typename std::conditional<TYPED && DT != TPQ_DTYPE_F32, uint32_t, uint2>::type;
+    static __device__ __forceinline__ float scale(raw_t p) {
+        if constexpr (TYPED && DT != TPQ_DTYPE_F32) return Elem<DT>::load(static_cast<uint16_t>(p & 0xFFFFu));
+        else return __builtin_bit_cast(float, p.x);
+    }
+    static __device__ __forceinline__ float zero(raw_t p) {
+        if constexpr (TYPED && DT != TPQ_DTYPE_F32) return Elem<DT>::load(static_cast<uint16_t>(p >> 16));
+        else return __builtin_bit_cast(float, p.y);
+    }
+};
+
+template <int DT, class Source, int MB, int CW, bool EDGE>
+__global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedRowsArgs a) {
+    using A = RowsArith<DT>;
+    using P = RowsParams<DT, Source::kTypedParams>;
+    using storage = typename Elem<DT>::storage;
+    constexpr int KW = 8 / CW, NB = kRowsNB, kRows = 16 * MB, kStepBytes = A::kChunks * 16;
+    constexpr int kRoundLoads = KW * kRows * kStepBytes / 1024, kMine = kRoundLoads / kRowsProducers;  // 1 KB loads of a round, a requesting wavefront's
+    constexpr int kLoadsPerStep = kRows * kStepBytes / 1024, kRowsPerLoad = 64 / A::kChunks;
+    constexpr int kBuffer = kRoundLoads * 1024;
+    static_assert(kRoundLoads % kRowsProducers == 0, "every wavefront loads the same number of pieces");
+    extern __shared__ uint4 pr_lds[];  // [2][KW][kRows][kStepBytes], later the partial sums [CW][NB][MB][KW][64 lanes]
+    char* const lds = reinterpret_cast<char*>(pr_lds);
+
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cw = wave % CW, kk = wave / CW;
+    const int i = lane & 15, q = lane >> 4;
+    const int m0 = blockIdx.y * kRows;
+    const int steps_all = (a.K + 127) / 128, s_begin = blockIdx.z * a.steps_per_slice;
+    const int s_end = steps_all < s_begin + a.steps_per_slice ? steps_all : s_begin + a.steps_per_slice;
+    const int rounds = (s_end - s_begin + KW - 1) / KW;
+    const int edge_chunks = EDGE ? (a.K % 128) * A::kElem / 16 : A::kChunks;  // 16-byte chunks of a row in the last step of K
+    auto step_of = [&](int round, int k) __attribute__((always_inline)) {     // clamped: a step behind the slice repeats its last one
+        const int s = s_begin + round * KW + k;
+        return s < s_end ? s : s_end - 1;
+    };
+
+    // LDS traffic only: the loads of weights stay in flight
+    auto lds_barrier = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    // ---- the requesting wavefronts: pieces of 1 KB, kRowsPerLoad rows of a step each; one barrier per round
+    if (wave >= 8) {
+        const uint32_t row_bytes = static_cast<uint32_t>(a.K) * A::kElem;
+        const char* const x_base = static_cast<const char*>(a.x) + static_cast<size_t>(m0) * row_bytes;
+        const uint32_t ring_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((pr_lds_ptr)pr_lds));
+        const int first = (wave - 8) * kMine;
+        uint32_t x_off[kMine];  // byte offset of the lane's chunk in step 0
+#pragma unroll
+        for (int j = 0; j < kMine; ++j) {
+            const int row = (first + j) % kLoadsPerStep * kRowsPerLoad + lane / A::kChunks;
+            x_off[j] = static_cast<uint32_t>(m0 + row < a.M ? row : a.M - 1 - m0) * row_bytes + static_cast<uint32_t>((lane % A::kChunks) ^ (row & 15)) * 16;
+        }
+        for (int round = 0; round < rounds; ++round) {
+            const uint32_t buffer_addr = ring_addr + (round & 1) * kBuffer;
+#pragma unroll
+            for (int j = 0; j < kMine; ++j) {
+                const int step = step_of(round, (first + j) / kLoadsPerStep);
+                uint32_t off = x_off[j];
+                if constexpr (EDGE) {  // the last chunk of the row in place of the ones behind it
+                    const int chunk = (lane % A::kChunks) ^ (((first + j) % kLoadsPerStep * kRowsPerLoad + lane / A::kChunks) & 15);
+                    const int behind = chunk - ((step == steps_all - 1 ? edge_chunks : A::kChunks) - 1);
+                    off -= static_cast<uint32_t>(behind > 0 ? behind : 0) * 16;
+                }
+                const char* const from = x_base + static_cast<size_t>(step) * kStepBytes;
+                const uint32_t to = buffer_addr + (first + j) * 1024;
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(from) : "memory", "m0");
+            }
+            __builtin_amdgcn_s_waitcnt(pr_vmcnt(0));
+            if constexpr (EDGE) {  // zeros over what was fetched in place of chunks behind K
+#pragma unroll
+                for (int j = 0; j < kMine; ++j) {
+                    const int chunk = (lane % A::kChunks) ^ (((first + j) % kLoadsPerStep * kRowsPerLoad + lane / A::kChunks) & 15);
+                    if (step_of(round, (first + j) / kLoadsPerStep) == steps_all - 1 && chunk >= edge_chunks)
+                        *reinterpret_cast<uint4*>(lds + (round & 1) * kBuffer + (first + j) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+                }
+            }
+            lds_barrier();  // round `round` is there, and everybody is done with the round before it
+        }
+        __syncthreads();  // the products of the last round are done
+        __syncthreads();  // the sums are in LDS
+        return;
+    }
+
+    // ---- weights
+    struct Loaded {
+        typename Source::Words w[NB];
+        typename P::raw_t p[NB];
+    };
+    uint32_t w_off[NB], p_off[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int n = blockIdx.x * (16 * NB * CW) + (cw * NB + b) * 16 + i;
+        w_off[b] = Source::lane_offset(a, n, q);
+        p_off[b] = static_cast<uint32_t>(n < a.N ? n : a.N - 1) * static_cast<uint32_t>(sizeof(typename P::raw_t));
+    }
+    const int last_tile = a.K / 32 - 1;
+    const uint32_t group_bytes = static_cast<uint32_t>(a.N) * static_cast<uint32_t>(sizeof(typename P::raw_t));
+    auto load_w = [&](int round, Loaded& d) __attribute__((always_inline)) {
+        const int step = step_of(round, kk);
+        int tile = 4 * step + q;
+        uint32_t back = 0;
+        if constexpr (EDGE) {
+            const int behind = tile - last_tile;
+            tile = behind > 0 ? last_tile : tile;
+            back = Source::edge_back(behind > 0 ? behind : 0);
+        }
+        // exact: tile < 2^20
+        const uint32_t group = static_cast<uint32_t>((static_cast<float>(tile) + 0.5f) * a.inv_tiles_per_group);
+        const uint32_t group_off = group * group_bytes;
+        auto from = (TPQ_GLOBAL char*)a.w + static_cast<size_t>(step) * Source::kStepBytes;
+        auto params = (TPQ_GLOBAL char*)a.sz;
+        asm volatile("" : "+s"(from), "+s"(params));  // the loads stay here (see pinned_global)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            Source::load(from, w_off[b] - back, d.w[b]);
+            if constexpr (sizeof(typename P::raw_t) == 4) {
+                d.p[b] = *(TPQ_GLOBAL uint32_t*)(params + (group_off + p_off[b]));
+            } else {
+                const pr_word2 t = *(TPQ_GLOBAL pr_word2*)(params + (group_off + p_off[b]));
+                d.p[b].x = t.x; d.p[b].y = t.y;
+            }
+        }
+    };
+    uint32_t magic[2];  // in VGPRs behind opaque moves: v_and_or_b32 takes one literal only
+    asm volatile("v_mov_b32 %0, %1" : "=v"(magic[0]) : "s"(Source::kMagic0));
+    asm volatile("v_mov_b32 %0, %1" : "=v"(magic[1]) : "s"(Source::kMagic1));
+    // pair p of a block's codes, dequantized
+    auto weight_pair = [&](const Loaded& d, int b, int p, float scale, float zero, float& lo, float& hi) __attribute__((always_inline)) {
+        half2_t h = __builtin_bit_cast(half2_t, Source::pair(d.w[b], p, magic));
+        if constexpr (DT == TPQ_DTYPE_F32) {  // the offset leaves exactly, in fp16
+            h = h - half2_t{static_cast<_Float16>(Source::offset(p, 0)), static_cast<_Float16>(Source::offset(p, 1))};
+            const float z = Source::kTypedParams ? zero : -zero * scale;
+            lo = __builtin_fmaf(static_cast<float>(h.x), scale, z);
+            hi = __builtin_fmaf(static_cast<float>(h.y), scale, z);
+        } else {  // the offset folded into the constant: an error of 2^-24 x 1032 scale at most, below the operand type's rounding
+            const float z_lo = Source::kTypedParams ? zero - Source::offset(p, 0) * scale : -(zero + Source::offset(p, 0)) * scale;
+            const float z_hi = Source::kTypedParams ? zero - Source::offset(p, 1) * scale : -(zero + Source::offset(p, 1)) * scale;
+            lo = __builtin_fmaf(static_cast<float>(h.x), scale, z_lo);
+            hi = __builtin_fmaf(static_cast<float>(h.y), scale, z_hi);
+        }
+    };
+    // Dequantized weights that go with one 16-byte chunk of the lane's activations, of two chunks in turn: four words (eight
+    // 16-bit values, four floats) per block
+    constexpr int kChunkPairs = DT == TPQ_DTYPE_F32 ? 2 : 4;
+    uint32_t wq[2][NB][4];
+    // pairs [first, last) of the NB kChunkPairs pairs of chunk u
+    auto dequantize = [&](const Loaded& d, auto u_c, auto first, auto last) __attribute__((always_inline)) {
+        constexpr int U = decltype(u_c)::value;
+#pragma unroll
+        for (int e = decltype(first)::value; e < decltype(last)::value; ++e) {
+            const int b = e % NB, p = e / NB;
+            float lo, hi;
+            weight_pair(d, b, U * kChunkPairs + p, P::scale(d.p[b]), P::zero(d.p[b]), lo, hi);
+            if constexpr (DT == TPQ_DTYPE_F32) {
+                wq[U & 1][b][2 * p] = __builtin_bit_cast(uint32_t, lo);
+                wq[U & 1][b][2 * p + 1] = __builtin_bit_cast(uint32_t, hi);
+            } else {
+                wq[U & 1][b][p] = A::pack(lo, hi);
+            }
+        }
+    };
+    // the values exist from here on (moved down to their use, the codes would have to live on beside the ones loaded next)
+    auto settle = [&](auto u_c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t& v = wq[decltype(u_c)::value & 1][b][e];
+                asm volatile("" : "+v"(v));
+            }
+    };
+
+    float4_t acc[NB][MB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < MB; ++r) acc[b][r] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // A step's products in pieces: piece c = u MB + r is chunk u of the lane's activations for row block r
+    constexpr int kU = A::kChunks / 4, kPieces = kU * MB, kFragments = kPieces < 3 ? kPieces : 3;
+    const char* const frag_base = lds + kk * (kLoadsPerStep * 1024) + i * kStepBytes;
+    pr_word4 frag[kFragments];
+    auto read_piece = [&](int buffer, auto c) __attribute__((always_inline)) {
+        constexpr int C = decltype(c)::value;
+        if constexpr (C < kPieces)
+            frag[C % kFragments] = *reinterpret_cast<const pr_word4*>(frag_base + buffer * kBuffer + (C % MB) * (16 * kStepBytes) + (((kU * q + C / MB)) ^ i) * 16);
+    };
+    auto multiply_piece = [&](auto c) __attribute__((always_inline)) {
+        constexpr int C = decltype(c)::value, U = C / MB, r = C % MB;
+        if constexpr (DT == TPQ_DTYPE_F32) {
+            const float4_t f = __builtin_bit_cast(float4_t, frag[C % kFragments]);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) acc[b][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, wq[U & 1][b][t]), f[t], acc[b][r], 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                acc[b][r] = A::mfma(pr_word4{wq[U & 1][b][0], wq[U & 1][b][1], wq[U & 1][b][2], wq[U & 1][b][3]}, frag[C % kFragments], acc[b][r]);
+        }
+    };
+    // The products of one step (weights d, in ring slot SLOT) and, dealt over their pieces, the dequantization of the following
+    // chunk's weights: the matrix cores and the vector ALU are separate pipes, and both multiplying wavefronts of a SIMD are in
+    // the same phase.  The order of the pieces is fixed: left to itself the compiler dequantizes first and multiplies
+    // afterwards.  The last chunk prepares the first one of the next step (next; NEXT), and the ring slot is asked for again
+    // as soon as its last codes are used.
+    constexpr int kShare = NB * kChunkPairs;
+    auto products = [&](Loaded& d, const Loaded& next, int buffer, int load_round, auto has_next, auto load_c) __attribute__((always_inline)) {
+        constexpr bool NEXT = decltype(has_next)::value, LOAD = decltype(load_c)::value;
+        pr_static_for<0, kFragments - 1>([&](auto c) __attribute__((always_inline)) { read_piece(buffer, c); });
+        pr_static_for<0, kPieces>([&](auto c) __attribute__((always_inline)) {
+            constexpr int C = decltype(c)::value, U = C / MB, r = C % MB;
+            constexpr std::integral_constant<int, r * kShare / MB> first{};
+            constexpr std::integral_constant<int, (r + 1) * kShare / MB> last{};
+            constexpr std::integral_constant<int, (U + 1) % kU> following{};
+            read_piece(buffer, std::integral_constant<int, C + kFragments - 1>{});
+            multiply_piece(c);
+            if constexpr (U + 1 < kU) dequantize(d, following, first, last);
+            else if constexpr (NEXT) dequantize(next, following, first, last);
+            if constexpr (r == MB - 1 && (U + 1 < kU || NEXT)) settle(following);
+            if constexpr (LOAD && r == MB - 1 && U + 2 == kU) load_w(load_round, d);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+
+    Loaded ring[kRowsAhead];
+    auto phase = [&](int round, auto slot_c, auto load_c) __attribute__((always_inline)) {  // a round that is not the last; slot_c = round % kRowsAhead
+        constexpr int SLOT = decltype(slot_c)::value;
+        products(ring[SLOT], ring[(SLOT + 1) % kRowsAhead], SLOT & 1, round + kRowsAhead, std::true_type{}, load_c);
+        lds_barrier();
+    };
+    pr_static_for<0, kRowsAhead>([&](auto r) __attribute__((always_inline)) { load_w(decltype(r)::value, ring[decltype(r)::value]); });
+    dequantize(ring[0], std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, kShare>{});
+    settle(std::integral_constant<int, 0>{});
+    lds_barrier();
+    int round = 0;
+    for (; round + kRowsAhead < rounds; round += kRowsAhead)
+        pr_static_for<0, kRowsAhead>([&](auto r) __attribute__((always_inline)) { phase(round + decltype(r)::value, r, std::true_type{}); });
+    // 1 .. kRowsAhead rounds left, their weights all asked for; in the last one a wavefront whose step lies behind the slice multiplies nothing
+    pr_last_rounds<0, kRowsAhead>(rounds - round, [&](auto r) __attribute__((always_inline)) { phase(round + decltype(r)::value, r, std::false_type{}); },
+                                  [&](auto r) __attribute__((always_inline)) {
+                                      constexpr int SLOT = decltype(r)::value;
+                                      if (s_begin + (round + SLOT) * KW + kk < s_end) products(ring[SLOT], ring[SLOT], SLOT & 1, 0, std::false_type{}, std::false_type{});
+                                  });
+    __syncthreads();
+
+    // ---- the KW sums of a tile meet in LDS; wavefront t finishes tiles t, t + 8, ...
+    float4_t* const sums = reinterpret_cast<float4_t*>(lds);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < MB; ++r) sums[(((cw * NB + b) * MB + r) * KW + kk) * kWave + lane] = acc[b][r];
+    __syncthreads();
+    for (int t = wave; t < CW * NB * MB; t += 8) {
+        float4_t s = sums[(t * KW) * kWave + lane];
+#pragma unroll
+        for (int k = 1; k < KW; ++k) {
+            const float4_t more = sums[(t * KW + k) * kWave + lane];
+            s = float4_t{s[0] + more[0], s[1] + more[1], s[2] + more[2], s[3] + more[3]};
+        }
+        const int block = t / MB, r = t % MB;
+        const int m = m0 + 16 * r + i, n = blockIdx.x * (16 * NB * CW) + block * 16 + 4 * q;
+        if (m >= a.M || n >= a.N) continue;  // N % 4 == 0: all four channels exist
+        const size_t at = static_cast<size_t>(m) * a.N + n;
+        if (a.partial != nullptr) {
+            *reinterpret_cast<float4_t*>(a.partial + static_cast<size_t>(blockIdx.z) * a.M * a.N + at) = s;
+            continue;
+        }
+        if (a.bias != nullptr) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += a.bias[n + e];
+        }
+        storage* const y = static_cast<storage*>(a.y) + at;
+        if constexpr (DT == TPQ_DTYPE_F32) *reinterpret_cast<float4_t*>(y) = s;
+        else
+            *reinterpret_cast<uint2*>(y) = make_uint2(Elem<DT>::store(s[0]) | (static_cast<uint32_t>(Elem<DT>::store(s[1])) << 16),
+                                                      Elem<DT>::store(s[2]) | (static_cast<uint32_t>(Elem<DT>::store(s[3])) << 16));
+    }
+}
+
+// y = round(sum over the slices, in slice order (+ bias)); a thread takes four consecutive elements (N % 4 == 0)
+template <int DT>
+__global__ __launch_bounds__(256) void packed_rows_finish_kernel(const float* __restrict__ partial, int slices, int64_t quads, const float* __restrict__ bias,
+                                                                 int quads_per_row, typename Elem<DT>::storage* __restrict__ y) {
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (e >= quads) return;
+    // four slices requested together; a batch past the last slice asks for the last one again and leaves it out of the sum
+    float4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int z0 = 0; z0 < slices; z0 += 4) {
+        float4_t more[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) more[j] = reinterpret_cast<const float4_t*>(partial)[static_cast<int64_t>(z0 + j < slices ? z0 + j : slices - 1) * quads + e];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (z0 + j < slices) sum = float4_t{sum[0] + more[j][0], sum[1] + more[j][1], sum[2] + more[j][2], sum[3] + more[j][3]};
+    }
+    if (bias != nullptr) {
+        const int n = static_cast<int>(static_cast<uint32_t>(e) % static_cast<uint32_t>(quads_per_row)) * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] += bias[n + j];
+    }
+    if constexpr (DT == TPQ_DTYPE_F32) reinterpret_cast<float4_t*>(y)[e] = sum;
+    else
+        reinterpret_cast<uint2*>(y)[e] = make_uint2(Elem<DT>::store(sum[0]) | (static_cast<uint32_t>(Elem<DT>::store(sum[1])) << 16),
+                                                    Elem<DT>::store(sum[2]) | (static_cast<uint32_t>(Elem<DT>::store(sum[3])) << 16));
+}
+
+// ---- launch ------------------------------------------------------------------------------------------
+struct PackedRowsPlan {
+    int mb;        // blocks of 16 rows per workgroup: 1 .. 4 (float32: 1, 2)
+    int cw;        // channel positions: 2 (64 channels per workgroup) or 4 (128; three or four blocks of rows and K % 128 == 0 only)
+    int slices, steps_per_slice;
+};
+
+// Tile height, channels per workgroup and slices of K by an estimate (us) fitted to a sweep of 1 .. 8 slices and both widths
+// over six shapes and 16 .. 256 rows: 4 for the launch, the first loads and the epilogue, per round what the comment on the
+// kernel says, per round of workgroups over the compute units, and 2 + the bytes of the slices' sums (written and read) at
+// 4 TB/s for the second kernel.  Within 5 % of the sweep's best nearly everywhere (11008 -> 4096 at 128 rows 24.8, best 22.7).
+inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, int units = 256) {
+    PackedRowsPlan p;
+    const bool wide = dtype == TPQ_DTYPE_F32;
+    const int64_t blocks = (M + 15) / 16;
+    const int64_t most = wide ? 2 : 4, row_tiles = (blocks + most - 1) / most;
+    p.mb = static_cast<int>((blocks + row_tiles - 1) / row_tiles);  // tiles of equal height
+    const int64_t steps = (K + 127) / 128;
+    int64_t best = 1;
+    double best_us = 1e30;
+    p.cw = 2;
+    for (int cw = 2; cw <= (p.mb >= 3 && K % 128 == 0 ? 4 : 2); cw += 2) {
+        const int kw = 8 / cw;
+        const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
+        for (int64_t z = 1; z <= 16 && z <= steps; ++z) {
+            if (z > 1 && z * M * N > room_floats) break;
+            const int64_t per = (steps + z - 1) / z, rounds = (per + kw - 1) / kw, real = (steps + per - 1) / per;
+            if (real != z) continue;
+            const double waves = static_cast<double>((tiles * z + units - 1) / units);
+            const double round_us = wide ? 0.2 + 2.1 * p.mb : cw == 2 ? 0.5 + 0.18 * p.mb : 0.45 + 0.13 * p.mb;
+            const double us = waves * (4.0 + round_us * static_cast<double>(rounds)) + (z == 1 ? 0.0 : 2.0 + static_cast<double>(z * M * N) * 8.0 / 4e6);
+            if (us < best_us) { best_us = us; best = z; p.cw = cw; }
+        }
+    }
+    if (const char* e = tuning_env("TPQ_ROWS_SLICES")) best = std::atoi(e);
+    if (const char* e = tuning_env("TPQ_ROWS_CW")) p.cw = std::atoi(e);
+    p.steps_per_slice = static_cast<int>((steps + best - 1) / best);
+    p.slices = static_cast<int>((steps + p.steps_per_slice - 1) / p.steps_per_slice);
+    return p;
+}
+
+template <int DT, class Source, int MB, int CW, bool EDGE>
+int launch_packed_rows_shape(const PackedRowsArgs& a, int slices, hipStream_t s) {
+    constexpr int KW = 8 / CW, NB = kRowsNB;
+    constexpr size_t stage = 2 * static_cast<size_t>(KW) * 16 * MB * RowsArith<DT>::kChunks * 16, sums = static_cast<size_t>(8) * NB * MB * 1024;
+    constexpr size_t smem = stage > sums ? stage : sums;
+    static_assert(smem <= 160 * 1024, "LDS of one compute unit");
+    auto kernel = packed_rows_kernel<DT, Source, MB, CW, EDGE>;
+    static std::atomic<uint64_t> configured{0};
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), smem, configured, "packed rows")) return rc;
+    const dim3 grid(static_cast<unsigned>((a.N + 16 * NB * CW - 1) / (16 * NB * CW)), static_cast<unsigned>((a.M + 16 * MB - 1) / (16 * MB)), static_cast<unsigned>(slices));
+    kernel<<<grid, kRowsThreads, smem, s>>>(a);
+    return check_launch("packed rows");
+}
+
+template <int DT, class Source, int MB, int CW>
+int launch_packed_rows_as(const PackedRowsArgs& a, int slices, hipStream_t s) {
+    if constexpr (CW == 2) {
+        if (a.K % 128 != 0) return launch_packed_rows_shape<DT, Source, MB, CW, true>(a, slices, s);
+    }
+    return launch_packed_rows_shape<DT, Source, MB, CW, false>(a, slices, s);
+}
+
+template <int DT, class Source>
+int launch_packed_rows(PackedRowsArgs a, const PackedRowsPlan& p, hipStream_t s) {
+    a.steps_per_slice = p.steps_per_slice;
+    a.inv_tiles_per_group = 1.0f / static_cast<float>(a.tiles_per_group);
+    if (p.slices == 1) a.partial = nullptr;
+    int rc;
+    const bool wide = p.cw == 4;
+    if (p.mb == 1) rc = launch_packed_rows_as<DT, Source, 1, 2>(a, p.slices, s);
+    else if (p.mb == 2) rc = launch_packed_rows_as<DT, Source, 2, 2>(a, p.slices, s);
+    else {
+        if constexpr (DT == TPQ_DTYPE_F32) rc = fail(TPQ_ERR_RUNTIME, "packed rows: no such tile");
+        else if (p.mb == 3) rc = wide ? launch_packed_rows_as<DT, Source, 3, 4>(a, p.slices, s) : launch_packed_rows_as<DT, Source, 3, 2>(a, p.slices, s);
+        else rc = wide ? launch_packed_rows_as<DT, Source, 4, 4>(a, p.slices, s) : launch_packed_rows_as<DT, Source, 4, 2>(a, p.slices, s);
+    }
+    if (rc != TPQ_OK || a.partial == nullptr) return rc;
+    const int64_t quads = static_cast<int64_t>(a.M) * a.N / 4;
+    packed_rows_finish_kernel<DT><<<static_cast<unsigned>((quads + 255) / 256), 256, 0, s>>>(
+        a.partial, p.slices, quads, a.bias, a.N / 4, static_cast<typename Elem<DT>::storage*>(a.y));
+    return check_launch("packed rows (sum of the slices)");
+}
+
+}  // namespace
+}  // namespace tpq

@@ -365,6 +365,74 @@ def _dense_mm(x: torch.Tensor, dense: torch.Tensor, out: torch.Tensor) -> torch.
     return torch.matmul(x, dense.t(), out=out)
 
 
+# ---- packed weights, a block of activation rows (tpq_int4_mm_rows, tpq_lowbit_mm_rows) -------------------------------
+#
+# Between the decode kernels and the dense route.  Upper limit, measured (us, this kernel / what runs above it): float16 and
+# bfloat16 alike, N < 16384: 384 rows of 4096 -> 11008 69 / 70, 8192 x 8192 78 / 104, 5120 -> 13824 84 / 97, 3072 -> 7088 33 / 39;
+# 512 rows of 8192 x 8192 90 / 103, 14336 -> 4096 71 / 110, 4096 x 4096 24 / 41, but 5120 -> 13824 111 / 99; 768 rows of
+# 4096 x 4096 42 / 43, 2048 x 2048 14 / 24, but 8192 x 8192 128 / 125.  Wider weights: bfloat16 4096 -> 32000 at 384 rows
+# 142 / 165, at 512 195 / 180; float16 (the tiled kernel of packed weights) at 256 rows 98 / 102, at 384 148 / 132.  float32: 192
+# rows of 4096 -> 11008 193 / 223, 4096 -> 16384 232 / 250, at 256 rows 309 / 305.  K that is no multiple of 128 has the narrow
+# tiles only: 4768 -> 13544 at 256 rows 120 / 106 (float32 at 96 rows 176 / 182, at 128 244 / 215).
+def _rows_limit(n: int, k: int, dtype: torch.dtype) -> int:
+    if dtype == torch.float32:
+        return 96 if k % 128 else 192
+    if k % 128:
+        return 192
+    if n >= 16384:
+        return 256 if dtype == torch.float16 else 384
+    return 768 if n * k <= (1 << 24) else 512 if n * k <= (1 << 26) else 384
+
+
+def _int4_rows_takes(m: int, n: int, k: int, group: int, dtype: torch.dtype) -> bool:
+    """Does the rows kernel take an int4 product (innerKTiles = 2, K % 32 == 0)?  Lower limit, measured (us, this kernel /
+    decode kernels): groups of 128, 24 rows: 4096 -> 16384 12.1 / 15.7, 14336 -> 4096 13.6 / 18.2, 4096 -> 11008 11.5 / 11.8, but
+    4096 x 4096 8.7 / 8.0, and 33 rows there 9.8 / 12.5; groups of 64, 17 rows: 11008 -> 4096 12.0 / 23.1, 16 rows 11.3 / 12.0.  K % 128 != 0
+    (slabs of four rows): 4768 -> 13544 at 1 / 3 / 33 rows 14.5 / 39, 14.5 / 94, 24 / 871.  float32: 4096 -> 11008 at 1, 2, 64 rows
+    24.4 / 24.2, 24.7 / 45, 68 / 110; 2048 x 2048 at 1 and 2 rows 8.1 / 7.2, 8.2 / 7.4.
+    bfloat16 stops at INT4_PREFILL_ROWS rows: beyond, results are held to within 1e-2, element by element, of the reference's
+    device formulation, whose dense weight is rounded to bfloat16 twice; a weight rounded once misses that on single elements
+    (it is the one that lies closer to the exact product)."""
+    if k % 32 or n * k >= (1 << 33) or k >= (1 << 24) or m > _rows_limit(n, k, dtype):
+        return False
+    if dtype == torch.bfloat16 and m > INT4_PREFILL_ROWS:
+        return False
+    if dtype == torch.float32:
+        return m >= 2 or (n * k >= (1 << 24) and k > 4096)
+    if k % 128:
+        return True
+    return m >= 33 or (m >= 17 and (group < 128 or n * k >= (1 << 25)))
+
+
+def _lowbit_rows_takes(m: int, n: int, k: int, bits: int, lsb_first: bool, group: int, dtype: torch.dtype) -> bool:
+    """The same for n-bit codes.  Lower limit, measured (us, this kernel / what ran below): bfloat16 and float16, groups of 128
+    (where the decode kernels are at home), 4096 -> 11008, 2 bits: 16 / 32 / 56 rows 11.7 / 11.2, 13.7 / 21.4, 16.7 / 41.8; other
+    groups, 4096 x 4096 in groups of 32, 2 bits: 1 / 16 / 80 rows 8.0 / 26, 8.3 / 45, 12.5 / 168; one row of 4 bits stays with the row
+    kernel (8.6 / 6.1).  float32 4096 -> 11008: 1 / 8 / 64 rows 27 / 35, 26 / 57, 70 / 112."""
+    if bits not in (1, 2, 4, 8) or (lsb_first and bits != 1) or k % 32 or group % 32 or n % 4:
+        return False
+    if n * k * bits >= (1 << 35) or k >= (1 << 24):
+        return False
+    limit = _rows_limit(n, k, dtype)
+    if bits == 8 and dtype != torch.float32:  # twice the bytes: 4096 -> 11008 at 300 rows 74 / 85, at 512 111 / 83; 4096 x 4096 at 512 33 / 42
+        limit = min(limit, 512 if n * k <= (1 << 24) else 300)
+    if m > limit:
+        return False
+    if dtype == torch.float32:
+        return True
+    step = 64 if bits == 8 else 128
+    at_home = k % step == 0 and group % step == 0 and ((group // step) & (group // step - 1)) == 0
+    if m == 1:
+        row_chunk = 16 if bits == 8 else 32 if bits == 4 else 64
+        row_kernel = k % row_chunk == 0 and group % row_chunk == 0 and k <= (32768 if bits == 8 else 65536) and (bits != 8 or dtype == torch.float16)
+        return not (at_home or row_kernel)
+    return m >= 17 or not at_home
+
+
+def _rows_workspace(dtype: torch.dtype, m: int, n: int, k: int, device: torch.device) -> torch.Tensor:
+    return torch.empty(int(_lib.load().tpq_packed_rows_workspace_bytes(_DT[dtype], m, n, k)), dtype=torch.uint8, device=device)
+
+
 def _int4_dequantize(packed: torch.Tensor, inner: int, n: int, k: int, group: int, sz: torch.Tensor) -> torch.Tensor:
     """Dense [N, K] weight in sz.dtype: T(code - 8) * scale + zero, product and sum each rounded to T."""
     dense = torch.empty((n, k), dtype=sz.dtype, device=packed.device)
@@ -404,6 +472,12 @@ def _weight_int4pack_mm(self: torch.Tensor, mat2: torch.Tensor, qGroupSize: int,
     x = self.contiguous()
     w = mat2.contiguous()
     sz = qScaleAndZeros.to(self.dtype).contiguous()
+    if inner == 2 and _int4_rows_takes(m, n, k, qGroupSize, self.dtype):
+        with torch.cuda.device(self.device):
+            ws = _rows_workspace(self.dtype, m, n, k, self.device)
+            _check(_lib.load().tpq_int4_mm_rows(_ptr(x), _DT[x.dtype], m, k, _ptr(w), n, qGroupSize, _ptr(sz), _ptr(out), _ptr(ws),
+                                                ws.numel(), _stream(self)))
+        return out
     if self.dtype == torch.float32:
         prefill_rows = INT4_PREFILL_ROWS_F32
     elif self.dtype == torch.bfloat16:
@@ -757,6 +831,13 @@ def _lowbit_mm(input: torch.Tensor, packed: torch.Tensor, bits: int, columns: in
     x = input.contiguous()
     m = x.shape[0]
     b = None if bias is None else bias.to(torch.float32).contiguous()
+    if m and _lowbit_rows_takes(m, n, columns, bits, lsb_first, group, x.dtype):
+        out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+        with torch.cuda.device(x.device):
+            ws = _rows_workspace(x.dtype, m, n, columns, x.device)
+            _check(_lib.load().tpq_lowbit_mm_rows(_ptr(x), _DT[x.dtype], m, columns, _ptr(w), bits, int(lsb_first), n, group, _ptr(sz), _ptr(b),
+                                                  _ptr(out), _ptr(ws), ws.numel(), _stream(x)))
+        return out
     if m > (LOWBIT_PREFILL_ROWS_F32 if x.dtype == torch.float32 else LOWBIT_PREFILL_ROWS_SMALL if n * columns <= (1 << 24) else LOWBIT_PREFILL_ROWS):
         dense = _lowbit_dequantize(w, bits, columns, sz, x.dtype, lsb_first)
         out = _dense_mm(x, dense, torch.empty((m, n), dtype=x.dtype, device=x.device))

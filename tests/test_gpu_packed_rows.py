@@ -1,0 +1,78 @@
+"""GPU: packed weights against a block of activation rows (tpq_int4_mm_rows, tpq_lowbit_mm_rows), every element within the
+bound that its roundings give, against float64 on the same quantized operands."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+UNIT = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+# (M, N, K, group): one and two rounds of four steps of 128 k, rounds of which the last is partial, several slices of k, rows at
+# and one past the edges of 16- and 64-row tiles, channels that leave a tile of 64 (128) partly empty, a last step of 32, 64, 96 k
+SHAPES = [(1, 64, 32, 32), (16, 72, 512, 128), (17, 136, 544, 32), (33, 264, 1024, 64), (48, 64, 2048, 128), (49, 200, 4032, 64),
+          (64, 520, 4096, 128), (65, 72, 1152, 128), (128, 1032, 8192, 128), (130, 4104, 608, 32), (200, 2056, 1280, 128)]
+
+
+def _check(got, x, w, bias, scale_max, dtype):
+    x64, w64 = x.double().cpu(), w.double().cpu()
+    exact = x64 @ w64.t()
+    if bias is not None:
+        exact = exact + bias.double().cpu()
+    size = x64.abs() @ w64.abs().t()
+    u, k = UNIT[dtype], x.shape[1]
+    # weights rounded once (not in float32), fp32 sums of k terms, the fp16 offset of a code (at most 1024 + 128) leaving
+    # through an fp32 constant of the size of offset x scale, the result rounded once
+    bound = ((0 if dtype == torch.float32 else u) + (k + 16) * 2.0 ** -24) * size + u * exact.abs()
+    bound = bound + 2 * 1160 * 2.0 ** -24 * scale_max * x64.abs().sum(1, keepdim=True) * (0 if dtype == torch.float32 else 1) + 1e-30
+    err = (got.double().cpu() - exact).abs()
+    assert torch.isfinite(got).all() and bool((err <= bound).all()), f"{float((err / bound).max()):.3f} times the bound"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,group", SHAPES)
+def test_int4_rows(dtype, M, N, K, group):
+    from tensorplay_amd import _lib, ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    codes = torch.randint(0, 16, (N, K), dtype=torch.int32, device=DEV, generator=gen)
+    packed = ops._convert_weight_to_int4pack(codes, 2)
+    sz = torch.stack([torch.rand(K // group, N, device=DEV, generator=gen) * 0.01 + 1e-3,
+                      torch.randn(K // group, N, device=DEV, generator=gen) * 0.01], -1).to(dtype).contiguous()
+    x = torch.randn(M, K, device=DEV, generator=gen).to(dtype)
+    w = (codes - 8).double() * sz[..., 0].double().t().repeat_interleave(group, 1) + sz[..., 1].double().t().repeat_interleave(group, 1)
+    lib = _lib.load()
+    need = int(lib.tpq_packed_rows_workspace_bytes(ops._DT[dtype], M, N, K))
+    for room in {need, 0}:  # with its slices, and without a workspace
+        out = torch.empty(M, N, dtype=dtype, device=DEV)
+        ws = torch.empty(max(room, 1), dtype=torch.uint8, device=DEV)
+        ops._check(lib.tpq_int4_mm_rows(x.data_ptr(), ops._DT[dtype], M, K, packed.data_ptr(), N, group, sz.data_ptr(), out.data_ptr(),
+                                        ws.data_ptr() if room else None, room, ops._stream(x)))
+        _check(out, x, w, None, 0.011, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bits,lsb_first", [(1, False), (1, True), (2, False), (4, False), (8, False)])
+@pytest.mark.parametrize("M,N,K,group", [(17, 68, 160, 32), (33, 264, 1056, 96), (64, 200, 4096, 512), (130, 1028, 640, 128)])
+def test_lowbit_rows(dtype, bits, lsb_first, M, N, K, group):
+    from tensorplay_amd import _lib, ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K + bits)
+    codes = torch.randint(0, 1 << bits, (N, K), dtype=torch.uint8, device=DEV, generator=gen)
+    packed = ops.pack_lowbit(codes, bits, lsb_first)
+    sz = torch.stack([torch.rand(K // group, N, device=DEV, generator=gen) * 0.01 + 1e-3,
+                      torch.rand(K // group, N, device=DEV, generator=gen) * (1 << bits)], -1).contiguous()
+    bias = torch.randn(N, device=DEV, generator=gen)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(dtype)
+    value = (codes.view(torch.int8) if bits == 8 else codes).double()  # 8-bit codes are signed
+    scale, zero = (sz[..., i].double().t().repeat_interleave(group, 1) for i in (0, 1))
+    w = (value - zero) * scale
+    out = torch.empty(M, N, dtype=dtype, device=DEV)
+    lib = _lib.load()
+    need = int(lib.tpq_packed_rows_workspace_bytes(ops._DT[dtype], M, N, K))
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
+    ops._check(lib.tpq_lowbit_mm_rows(x.data_ptr(), ops._DT[dtype], M, K, packed.data_ptr(), bits, int(lsb_first), N, group, sz.data_ptr(),
+                                      bias.data_ptr(), out.data_ptr(), ws.data_ptr(), need, ops._stream(x)))
+    # the zero point and the code meet after their products with the scale: |zero| scale on top of |w|
+    _check(out, x, w, bias, 0.011 * (1 + (1 << bits) / 8), dtype)
