@@ -224,6 +224,14 @@ int tpq_ternary_mm_ws(const int8_t* x, const float* row_scale, const uint8_t* pa
  * slices are added in a fixed order.
  */
 int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
+/*
+ * 1 where _weight_int4pack_mm (innerKTiles = 2) and the n-bit linear run the products below, 0 where another kernel is the
+ * faster one or these do not take the operands (type, sizes, alignment).  Host logic only.
+ */
+int tpq_int4_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int64_t group, const int32_t* packed,
+                           const void* scales_and_zeros);
+int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int bits, int lsb_first,
+                             int64_t group, const uint8_t* packed, const float* scales_and_zeros);
 int tpq_int4_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, int64_t N, int64_t group,
                      const void* scales_and_zeros, void* out, void* workspace, int64_t workspace_bytes, void* stream);
 int tpq_lowbit_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const uint8_t* packed, int bits, int lsb_first,

@@ -10,6 +10,7 @@ import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libtpq_gfx950.so")
+CALLS_PATH = os.path.join(HERE, "_calls.so")
 
 TPQ_OK, TPQ_ERR_INVALID_VALUE, TPQ_ERR_INVALID_TYPE, TPQ_ERR_RUNTIME, TPQ_ERR_UNSUPPORTED = range(5)
 F32, F16, BF16 = 0, 1, 2
@@ -36,6 +37,8 @@ SIGNATURES = {
     "tpq_int4_mm_workspace_bytes": [_i64],
     "tpq_int4_mm_rows_workspace_bytes": [_i64, _i64, _i64],
     "tpq_packed_rows_workspace_bytes": [_int, _i64, _i64, _i64],
+    "tpq_int4_mm_rows_takes": [_ptr, _int, _i64, _i64, _i64, _i64, _ptr, _ptr],
+    "tpq_lowbit_mm_rows_takes": [_ptr, _int, _i64, _i64, _i64, _int, _int, _i64, _ptr, _ptr],
     "tpq_int4_mm_rows": [_ptr, _int, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr],
     "tpq_lowbit_mm_rows": [_ptr, _int, _i64, _i64, _ptr, _int, _int, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr],
     "tpq_ternary_pack": [_ptr, _i64, _i64, _ptr, _ptr],
@@ -83,13 +86,26 @@ def load() -> ctypes.CDLL:
     # process, so that device pointers and streams are shared with the tensors we are handed.
     import torch  # noqa: F401
 
-    _lib = bind(LIB_PATH)
+    lib = bind(LIB_PATH)
+    lib.calls = _bind_calls(lib)
+    _lib = lib
     return _lib
+
+
+def _bind_calls(lib: ctypes.CDLL):
+    """The native form of the operators' host path (csrc/calls.cpp), on the entry points of this library."""
+    if not os.path.exists(CALLS_PATH):
+        raise RuntimeError(f"{CALLS_PATH} is missing: build it with `python -m tensorplay_amd.build`")
+    from . import _calls
+
+    _calls.bind(lib._handle)
+    return _calls
 
 
 def bind(path: str) -> ctypes.CDLL:
     """Opens a build of the kernel library and declares the operators' signatures on it."""
     lib = ctypes.CDLL(path)
+    lib.calls = None  # only the shipped library has native calls bound to it
     for name, args in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.argtypes = args

@@ -43,12 +43,7 @@ def bitnet_linear_packed(input: torch.Tensor, packed: torch.Tensor, scale: Union
     """BitNet linear from pre-packed ternary weights (reference :215-241): float32 output
     ``(float(x_i8 . codes) * row_scale) * scale (+ bias)``.  A tensor ``scale`` is read back to the
     host once per call; modules keep it as a Python float instead."""
-    batch_dims = input.shape[:-1]
-    x = input.reshape(-1, in_features)
-    x_i8, row_scale = ops._quantize_int8_rowwise(x, eps)
-    w_scale = float(scale)
-    out = ops.ternary_mm(x_i8, row_scale, packed, w_scale, in_features, bias=bias, out_dtype=torch.float32)
-    return out.reshape(*batch_dims, packed.shape[0])
+    return ops._ternary_linear(input, packed, float(scale), in_features, bias, eps)
 
 
 class BitNetPacked2bitLinear(nn.Module):

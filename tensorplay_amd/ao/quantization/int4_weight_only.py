@@ -53,10 +53,7 @@ def _pack_int4_weight(weight: torch.Tensor, groupsize: int) -> Tuple[torch.Tenso
 
 
 def _int4_mm(input: torch.Tensor, packed: torch.Tensor, scale_zero: torch.Tensor, groupsize: int) -> torch.Tensor:
-    lead = input.shape[:-1]
-    x = input.reshape(-1, input.shape[-1])
-    out = ops._weight_int4pack_mm(x, packed, groupsize, scale_zero)
-    return out.reshape(*lead, out.shape[-1])
+    return ops._int4_linear(input, packed, groupsize, scale_zero)
 
 
 class WeightOnlyInt4Linear(nn.Module):

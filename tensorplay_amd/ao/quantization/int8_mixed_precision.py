@@ -74,10 +74,7 @@ class Int8DynamicLinear(nn.Module):
         return cls(codes, scale, None if linear.bias is None else linear.bias, out_dtype)
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
-        x = input.reshape(-1, self.in_features)
-        x_i8, x_scale = ops._quantize_int8_rowwise(x, 1e-5)
-        out = ops.int8_mm_dequant(x_i8, self.weight, x_scale, self.weight_scale, self.bias, self.out_dtype)
-        return out.reshape(*input.shape[:-1], self.out_features)
+        return ops._int8_dynamic_linear(input, self.weight, self.weight_scale, self.bias, self.out_dtype)
 
 
 @register_quantize_module_handler(Int8DynamicLinearConfig)

@@ -61,10 +61,7 @@ def _intx_mm(input: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, zer
 
 
 def _packed_linear(input, packed, bits, columns, scales_and_zeros, bias, lsb_first=False):
-    lead = input.shape[:-1]
-    x = input.reshape(-1, input.shape[-1])
-    out = ops._lowbit_mm(x, packed, bits, columns, scales_and_zeros, bias, lsb_first)
-    return out.reshape(*lead, out.shape[-1])
+    return ops._lowbit_linear(input, packed, bits, columns, scales_and_zeros, bias, lsb_first)
 
 
 class WeightOnlyIntxLinear(nn.Module):

@@ -3,9 +3,10 @@
 ``libtpq_gfx950.so``        the C-ABI kernel library: the operators of include/tpq.h and nothing else.
 ``libtpq_gfx950_hooks.so``  the same sources with -DTPQ_TEST_HOOKS: exports tpq_set_kernel_override as well, with which the
                             tests pin a route so that a kernel is checked on every shape it can take.  Only tests load it.
+``_calls.so``               CPython module with the hot operators' host path (csrc/calls.cpp); finds the library's entry points at run time.
 ``libtpq_probe.so``         the pure-read measurement probe (csrc/probe.hip).  Only bench.py loads it.
 
-Usage: ``python -m tensorplay_amd.build`` (all three) or ``tensorplay_amd.build.build_library()``.
+Usage: ``python -m tensorplay_amd.build`` (all of them) or ``tensorplay_amd.build.build_library()``.
 """
 from __future__ import annotations
 
@@ -13,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libtpq_gfx950.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+CALLS_PATH = os.path.join(HERE, "_calls.so")
 HOOKS_LIB_PATH = os.path.join(HERE, "libtpq_gfx950_hooks.so")
 PROBE_LIB_PATH = os.path.join(HERE, "libtpq_probe.so")
 QUANT_STAMPS_LIB_PATH = os.path.join(HERE, "libtpq_quant_stamps.so")  # the row quantizer with clock readings per phase (quant_stamps.py)
@@ -76,6 +79,26 @@ def _link(cc: str, objs: list, path: str) -> str:
     return path
 
 
+def _build_calls(verbose: bool) -> str:
+    from torch.utils import cpp_extension
+
+    import torch
+
+    includes = [flag for path in cpp_extension.include_paths() for flag in ("-isystem", path)]
+    tmp = CALLS_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + os.path.join(os.path.dirname(HERE), "include"), *includes,
+           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "calls.cpp"), "-o", tmp,
+           *[f"-L{path}" for path in cpp_extension.library_paths()], "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python", "-ldl"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on calls.cpp:\n{proc.stderr}")
+    os.replace(tmp, CALLS_PATH)
+    return CALLS_PATH
+
+
 def build_library(verbose: bool = False, jobs: int = 6, tuning: bool = False, hooks: bool = True, probe: bool = True) -> str:
     """Compiles every source and links the kernel library; with hooks / probe also the test-hook library and the
     measurement probe.  tuning=True compiles the sweep knobs in (-DTPQ_TUNING: TPQ_* environment variables pick kernels
@@ -91,7 +114,9 @@ def build_library(verbose: bool = False, jobs: int = 6, tuning: bool = False, ho
         work.append(("probe.hip", os.path.join(obj_dir, "probe.o"), []))
         work.append(("quantize_rowwise.hip", os.path.join(obj_dir, "quantize_rowwise.stamps.o"), ["-DTPQ_QUANT_STAMPS"]))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        calls = pool.submit(_build_calls, verbose)
         list(pool.map(lambda w: _compile(cc, w[0], w[1], w[2], verbose), work))
+        calls.result()
     plain = [os.path.join(obj_dir, src.replace(".hip", ".o")) for src in SOURCES]
     _link(cc, plain, LIB_PATH)
     if hooks:

@@ -8,10 +8,69 @@ namespace {
 template <int DT>
 int run_int4(const PackedRowsArgs& a, const PackedRowsPlan& p, hipStream_t s) { return launch_packed_rows<DT, SourceInt4>(a, p, s); }
 
+// Between the decode kernels and the dense route.  Upper limit, measured (us, this kernel / what runs above it): float16 and
+// bfloat16 alike, N < 16384: 384 rows of 4096 -> 11008 69 / 70, 8192 x 8192 78 / 104, 5120 -> 13824 84 / 97, 3072 -> 7088 33 / 39;
+// 512 rows of 8192 x 8192 90 / 103, 14336 -> 4096 71 / 110, 4096 x 4096 24 / 41, but 5120 -> 13824 111 / 99; 768 rows of
+// 4096 x 4096 42 / 43, 2048 x 2048 14 / 24, but 8192 x 8192 128 / 125.  Wider weights: bfloat16 4096 -> 32000 at 384 rows
+// 142 / 165, at 512 195 / 180; float16 (the tiled kernel of packed weights) at 256 rows 98 / 102, at 384 148 / 132.  float32: 192
+// rows of 4096 -> 11008 193 / 223, 4096 -> 16384 232 / 250, at 256 rows 309 / 305.  K that is no multiple of 128 has the narrow
+// tiles only: 4768 -> 13544 at 256 rows 120 / 106 (float32 at 96 rows 176 / 182, at 128 244 / 215).
+int64_t rows_limit(int64_t N, int64_t K, int dtype) {
+    if (dtype == TPQ_DTYPE_F32) return K % 128 ? 96 : 192;
+    if (K % 128) return 192;
+    if (N >= 16384) return dtype == TPQ_DTYPE_F16 ? 256 : 384;
+    return N * K <= (int64_t{1} << 24) ? 768 : N * K <= (int64_t{1} << 26) ? 512 : 384;
+}
+
 }  // namespace
 }  // namespace tpq
 
 using namespace tpq;
+
+// Lower limit, measured (us, this kernel / decode kernels): groups of 128, 24 rows: 4096 -> 16384 12.1 / 15.7, 14336 -> 4096
+// 13.6 / 18.2, 4096 -> 11008 11.5 / 11.8, but 4096 x 4096 8.7 / 8.0, and 33 rows there 9.8 / 12.5; groups of 64, 17 rows:
+// 11008 -> 4096 12.0 / 23.1, 16 rows 11.3 / 12.0.  K % 128 != 0 (slabs of four rows): 4768 -> 13544 at 1 / 3 / 33 rows 14.5 / 39,
+// 14.5 / 94, 24 / 871.  float32: 4096 -> 11008 at 1, 2, 64 rows 24.4 / 24.2, 24.7 / 45, 68 / 110; 2048 x 2048 at 1 and 2 rows
+// 8.1 / 7.2, 8.2 / 7.4.  bfloat16 stops at 256 rows: beyond, results are held to within 1e-2, element by element, of the
+// reference's device formulation, whose dense weight is rounded to bfloat16 twice; a weight rounded once misses that on
+// single elements (it is the one that lies closer to the exact product).
+// Operands off the alignment that the kernel wants stay with the kernels that take any address.
+TPQ_EXPORT int tpq_int4_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int64_t group, const int32_t* packed,
+                                      const void* scales_and_zeros) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 32 || N % 8 || N * K >= (int64_t{1} << 33) || K >= (1 << 24) || M > rows_limit(N, K, dtype)) return 0;
+    if (!aligned(x, 16) || !aligned(packed, 16) || !aligned(scales_and_zeros, dtype == TPQ_DTYPE_F32 ? 8 : 4)) return 0;
+    if (dtype == TPQ_DTYPE_BF16 && M > 256) return 0;
+    if (dtype == TPQ_DTYPE_F32) return M >= 2 || (N * K >= (1 << 24) && K > 4096);
+    if (K % 128) return 1;
+    return M >= 33 || (M >= 17 && (group < 128 || N * K >= (1 << 25)));
+}
+
+// Lower limit, measured (us, this kernel / what ran below): bfloat16 and float16, groups of 128 (where the decode kernels are
+// at home), 4096 -> 11008, 2 bits: 16 / 32 / 56 rows 11.7 / 11.2, 13.7 / 21.4, 16.7 / 41.8; other groups, 4096 x 4096 in groups of
+// 32, 2 bits: 1 / 16 / 80 rows 8.0 / 26, 8.3 / 45, 12.5 / 168; one row of 4 bits stays with the row kernel (8.6 / 6.1).  float32
+// 4096 -> 11008: 1 / 8 / 64 rows 27 / 35, 26 / 57, 70 / 112.  8 bits are twice the bytes: 4096 -> 11008 at 300 rows 74 / 85, at
+// 512 111 / 83; 4096 x 4096 at 512 33 / 42.
+TPQ_EXPORT int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int bits, int lsb_first, int64_t group,
+                                        const uint8_t* packed, const float* scales_and_zeros) {
+    if (M <= 0 || N <= 0 || K <= 0 || group <= 0 || (bits != 1 && bits != 2 && bits != 4 && bits != 8) || (lsb_first && bits != 1)) return 0;
+    if (K % 32 || group % 32 || N % 4 || N * K * bits >= (int64_t{1} << 35) || K >= (1 << 24)) return 0;
+    if (!aligned(x, 16) || !aligned(packed, 16) || !aligned(scales_and_zeros, 8)) return 0;
+    int64_t limit = rows_limit(N, K, dtype);
+    if (bits == 8 && dtype != TPQ_DTYPE_F32) {
+        const int64_t wide = N * K <= (int64_t{1} << 24) ? 512 : 300;
+        limit = limit < wide ? limit : wide;
+    }
+    if (M > limit) return 0;
+    if (dtype == TPQ_DTYPE_F32) return 1;
+    const int64_t step = bits == 8 ? 64 : 128, steps = group / step;
+    const bool at_home = K % step == 0 && group % step == 0 && (steps & (steps - 1)) == 0;
+    if (M == 1) {
+        const int64_t chunk = bits == 8 ? 16 : bits == 4 ? 32 : 64;
+        const bool row_kernel = K % chunk == 0 && group % chunk == 0 && K <= (bits == 8 ? 32768 : 65536) && (bits != 8 || dtype == TPQ_DTYPE_F16);
+        return !(at_home || row_kernel);
+    }
+    return M >= 17 || !at_home;
+}
 
 TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;

@@ -43,6 +43,9 @@ def _require_device(t: torch.Tensor, what: str) -> None:
 
 
 def _quantize_rowwise(self, eps, divisor, qmin, qmax, sign_mode, name):
+    calls = _lib.load().calls
+    if calls is not None and (pair := calls.quantize_rowwise(self, eps, divisor, qmin, qmax, int(sign_mode))) is not None:
+        return pair
     if self.dim() != 2:
         raise ValueError(f"{name}(): expected a 2-D tensor")
     if self.dtype not in _DT:
@@ -224,6 +227,9 @@ def int8_mm_dequant(A_i8: torch.Tensor, B_t_i8: torch.Tensor, row_scale: torch.T
     ``cast((float(acc) * row_scale[m]) * col_scale[n] (+ bias[n]))``: the fp32 value the two
     reference ops produce, rounded once when ``out_dtype`` is a 16-bit float.
     """
+    calls = _lib.load().calls
+    if calls is not None and (out := calls.int8_mm_dequant(A_i8, B_t_i8, row_scale, col_scale, bias, out_dtype, INT8_RAGGED_ROWS)) is not None:
+        return out
     if A_i8.dim() != 2 or B_t_i8.dim() != 2 or A_i8.size(1) != B_t_i8.size(1):
         raise ValueError("int8_mm_dequant: expected A [M,K] and B_t [N,K]")
     if A_i8.dtype != torch.int8 or B_t_i8.dtype != torch.int8:
@@ -260,6 +266,18 @@ def int8_mm_dequant(A_i8: torch.Tensor, B_t_i8: torch.Tensor, row_scale: torch.T
             _check(lib.tpq_int8_mm_dequant(_ptr(a), _ptr(w), _ptr(rs), _ptr(cs), _ptr(b), _ptr(out),
                                            _DT[out_dtype], M, N, K, _stream(a)))
     return out
+
+
+def _int8_dynamic_linear(input: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor, bias: Optional[torch.Tensor],
+                         out_dtype: torch.dtype, eps: float = 1e-5) -> torch.Tensor:
+    """``_quantize_int8_rowwise`` of the rows of input [..., K], then ``int8_mm_dequant`` with the weight [N, K]."""
+    calls = _lib.load().calls
+    if calls is not None and (out := calls.int8_linear(input, weight, weight_scale, bias, eps, out_dtype, INT8_RAGGED_ROWS)) is not None:
+        return out
+    n, k = weight.shape
+    x_i8, x_scale = _quantize_int8_rowwise(input.reshape(-1, k), eps)
+    out = int8_mm_dequant(x_i8, weight, x_scale, weight_scale, bias, out_dtype)
+    return out.reshape(*input.shape[:-1], n)
 
 
 _int4_workspaces = {}
@@ -365,69 +383,7 @@ def _dense_mm(x: torch.Tensor, dense: torch.Tensor, out: torch.Tensor) -> torch.
     return torch.matmul(x, dense.t(), out=out)
 
 
-# ---- packed weights, a block of activation rows (tpq_int4_mm_rows, tpq_lowbit_mm_rows) -------------------------------
-#
-# Between the decode kernels and the dense route.  Upper limit, measured (us, this kernel / what runs above it): float16 and
-# bfloat16 alike, N < 16384: 384 rows of 4096 -> 11008 69 / 70, 8192 x 8192 78 / 104, 5120 -> 13824 84 / 97, 3072 -> 7088 33 / 39;
-# 512 rows of 8192 x 8192 90 / 103, 14336 -> 4096 71 / 110, 4096 x 4096 24 / 41, but 5120 -> 13824 111 / 99; 768 rows of
-# 4096 x 4096 42 / 43, 2048 x 2048 14 / 24, but 8192 x 8192 128 / 125.  Wider weights: bfloat16 4096 -> 32000 at 384 rows
-# 142 / 165, at 512 195 / 180; float16 (the tiled kernel of packed weights) at 256 rows 98 / 102, at 384 148 / 132.  float32: 192
-# rows of 4096 -> 11008 193 / 223, 4096 -> 16384 232 / 250, at 256 rows 309 / 305.  K that is no multiple of 128 has the narrow
-# tiles only: 4768 -> 13544 at 256 rows 120 / 106 (float32 at 96 rows 176 / 182, at 128 244 / 215).
-def _rows_limit(n: int, k: int, dtype: torch.dtype) -> int:
-    if dtype == torch.float32:
-        return 96 if k % 128 else 192
-    if k % 128:
-        return 192
-    if n >= 16384:
-        return 256 if dtype == torch.float16 else 384
-    return 768 if n * k <= (1 << 24) else 512 if n * k <= (1 << 26) else 384
-
-
-def _int4_rows_takes(m: int, n: int, k: int, group: int, dtype: torch.dtype) -> bool:
-    """Does the rows kernel take an int4 product (innerKTiles = 2, K % 32 == 0)?  Lower limit, measured (us, this kernel /
-    decode kernels): groups of 128, 24 rows: 4096 -> 16384 12.1 / 15.7, 14336 -> 4096 13.6 / 18.2, 4096 -> 11008 11.5 / 11.8, but
-    4096 x 4096 8.7 / 8.0, and 33 rows there 9.8 / 12.5; groups of 64, 17 rows: 11008 -> 4096 12.0 / 23.1, 16 rows 11.3 / 12.0.  K % 128 != 0
-    (slabs of four rows): 4768 -> 13544 at 1 / 3 / 33 rows 14.5 / 39, 14.5 / 94, 24 / 871.  float32: 4096 -> 11008 at 1, 2, 64 rows
-    24.4 / 24.2, 24.7 / 45, 68 / 110; 2048 x 2048 at 1 and 2 rows 8.1 / 7.2, 8.2 / 7.4.
-    bfloat16 stops at INT4_PREFILL_ROWS rows: beyond, results are held to within 1e-2, element by element, of the reference's
-    device formulation, whose dense weight is rounded to bfloat16 twice; a weight rounded once misses that on single elements
-    (it is the one that lies closer to the exact product)."""
-    if k % 32 or n * k >= (1 << 33) or k >= (1 << 24) or m > _rows_limit(n, k, dtype):
-        return False
-    if dtype == torch.bfloat16 and m > INT4_PREFILL_ROWS:
-        return False
-    if dtype == torch.float32:
-        return m >= 2 or (n * k >= (1 << 24) and k > 4096)
-    if k % 128:
-        return True
-    return m >= 33 or (m >= 17 and (group < 128 or n * k >= (1 << 25)))
-
-
-def _lowbit_rows_takes(m: int, n: int, k: int, bits: int, lsb_first: bool, group: int, dtype: torch.dtype) -> bool:
-    """The same for n-bit codes.  Lower limit, measured (us, this kernel / what ran below): bfloat16 and float16, groups of 128
-    (where the decode kernels are at home), 4096 -> 11008, 2 bits: 16 / 32 / 56 rows 11.7 / 11.2, 13.7 / 21.4, 16.7 / 41.8; other
-    groups, 4096 x 4096 in groups of 32, 2 bits: 1 / 16 / 80 rows 8.0 / 26, 8.3 / 45, 12.5 / 168; one row of 4 bits stays with the row
-    kernel (8.6 / 6.1).  float32 4096 -> 11008: 1 / 8 / 64 rows 27 / 35, 26 / 57, 70 / 112."""
-    if bits not in (1, 2, 4, 8) or (lsb_first and bits != 1) or k % 32 or group % 32 or n % 4:
-        return False
-    if n * k * bits >= (1 << 35) or k >= (1 << 24):
-        return False
-    limit = _rows_limit(n, k, dtype)
-    if bits == 8 and dtype != torch.float32:  # twice the bytes: 4096 -> 11008 at 300 rows 74 / 85, at 512 111 / 83; 4096 x 4096 at 512 33 / 42
-        limit = min(limit, 512 if n * k <= (1 << 24) else 300)
-    if m > limit:
-        return False
-    if dtype == torch.float32:
-        return True
-    step = 64 if bits == 8 else 128
-    at_home = k % step == 0 and group % step == 0 and ((group // step) & (group // step - 1)) == 0
-    if m == 1:
-        row_chunk = 16 if bits == 8 else 32 if bits == 4 else 64
-        row_kernel = k % row_chunk == 0 and group % row_chunk == 0 and k <= (32768 if bits == 8 else 65536) and (bits != 8 or dtype == torch.float16)
-        return not (at_home or row_kernel)
-    return m >= 17 or not at_home
-
+# ---- packed weights, a block of activation rows (tpq_int4_mm_rows, tpq_lowbit_mm_rows): the library says for which
 
 def _rows_workspace(dtype: torch.dtype, m: int, n: int, k: int, device: torch.device) -> torch.Tensor:
     return torch.empty(int(_lib.load().tpq_packed_rows_workspace_bytes(_DT[dtype], m, n, k)), dtype=torch.uint8, device=device)
@@ -445,6 +401,9 @@ def _int4_dequantize(packed: torch.Tensor, inner: int, n: int, k: int, group: in
 def _weight_int4pack_mm(self: torch.Tensor, mat2: torch.Tensor, qGroupSize: int,
                         qScaleAndZeros: torch.Tensor) -> torch.Tensor:
     """``self @ W.T`` with W dequantised per group: (code - 8) * scale + zero; result in self.dtype."""
+    calls = _lib.load().calls
+    if calls is not None and self.dim() == 2 and (out := calls.int4_mm(self, mat2, qGroupSize, qScaleAndZeros, _int4_workspaces)) is not None:
+        return out
     if mat2.dtype != torch.int32 or mat2.dim() != 4:
         raise TypeError("_weight_int4pack_mm(): packed weight must be 4-D int32 in the tensor-core B layout")
     if self.dim() != 2:
@@ -472,7 +431,7 @@ def _weight_int4pack_mm(self: torch.Tensor, mat2: torch.Tensor, qGroupSize: int,
     x = self.contiguous()
     w = mat2.contiguous()
     sz = qScaleAndZeros.to(self.dtype).contiguous()
-    if inner == 2 and _int4_rows_takes(m, n, k, qGroupSize, self.dtype):
+    if inner == 2 and _lib.load().tpq_int4_mm_rows_takes(_ptr(x), _DT[x.dtype], m, n, k, qGroupSize, _ptr(w), _ptr(sz)):
         with torch.cuda.device(self.device):
             ws = _rows_workspace(self.dtype, m, n, k, self.device)
             _check(_lib.load().tpq_int4_mm_rows(_ptr(x), _DT[x.dtype], m, k, _ptr(w), n, qGroupSize, _ptr(sz), _ptr(out), _ptr(ws),
@@ -497,6 +456,15 @@ def _weight_int4pack_mm(self: torch.Tensor, mat2: torch.Tensor, qGroupSize: int,
         _check(_lib.load().tpq_int4_mm_ws(_ptr(x), _DT[x.dtype], m, k, _ptr(w), inner, n, qGroupSize, _ptr(sz),
                                           _ptr(out), _ptr(ws), ws.numel(), _stream(self)))
     return out
+
+
+def _int4_linear(input: torch.Tensor, packed: torch.Tensor, group: int, scales_and_zeros: torch.Tensor) -> torch.Tensor:
+    """``_weight_int4pack_mm`` of the rows of input [..., K]."""
+    calls = _lib.load().calls
+    if calls is not None and (out := calls.int4_mm(input, packed, group, scales_and_zeros, _int4_workspaces)) is not None:
+        return out
+    out = _weight_int4pack_mm(input.reshape(-1, input.shape[-1]), packed, group, scales_and_zeros)
+    return out.reshape(*input.shape[:-1], out.shape[-1])
 
 
 def pack_ternary(codes: torch.Tensor) -> torch.Tensor:
@@ -558,6 +526,17 @@ def ternary_mm(x_i8: torch.Tensor, row_scale: torch.Tensor, packed: torch.Tensor
             _check(lib.tpq_ternary_mm_ws(_ptr(x), _ptr(rs), _ptr(p), float(w_scale), _ptr(b), M, N, K,
                                          _ptr(out), _DT[out_dtype], _ptr(acc), _ptr(scratch), scratch_bytes, _stream(x)))
     return (out, acc) if return_acc else out
+
+
+def _ternary_linear(input: torch.Tensor, packed: torch.Tensor, w_scale: float, in_features: int, bias: Optional[torch.Tensor],
+                    eps: float) -> torch.Tensor:
+    """``_quantize_int8_rowwise`` of the rows of input [..., K], then ``ternary_mm`` in float32."""
+    calls = _lib.load().calls
+    if calls is not None and (out := calls.ternary_linear(input, packed, w_scale, in_features, bias, eps)) is not None:
+        return out
+    x_i8, row_scale = _quantize_int8_rowwise(input.reshape(-1, in_features), eps)
+    out = ternary_mm(x_i8, row_scale, packed, w_scale, in_features, bias=bias, out_dtype=torch.float32)
+    return out.reshape(*input.shape[:-1], packed.shape[0])
 
 
 # Above this many activation rows _weight_int8pack_mm dequantises and multiplies with the dense 16-bit tile kernel.
@@ -703,6 +682,9 @@ def quantize_affine(input: torch.Tensor, block_size, scales: torch.Tensor, zero_
     import ctypes
     name = _affine_dtype_name(dtype, "quantize_affine")
     tag, code_dtype, pack = _AFFINE_STORAGE[name]
+    calls = _lib.load().calls
+    if calls is not None and (out := calls.quantize_affine(input, block_size, scales, zero_points, tag, pack, code_dtype, quant_min, quant_max)) is not None:
+        return out if pack == 1 else PackedCodes(out, input.shape, name)
     _require_device(input, "quantize_affine")
     if input.dtype not in _DT:
         input = input.to(torch.float32)
@@ -736,6 +718,9 @@ def dequantize_affine(input, block_size, scales: torch.Tensor, zero_points: Opti
             raise TypeError(f"dequantize_affine(): expected a quantized tensor, got {getattr(input, 'dtype', type(input))}")
         name, codes, shape = by_dtype[input.dtype], input.contiguous(), tuple(input.shape)
     tag = _AFFINE_STORAGE[name][0]
+    calls = _lib.load().calls
+    if calls is not None and (out := calls.dequantize_affine(codes, shape, block_size, scales, zero_points, tag)) is not None:
+        return out
     _require_device(codes, "dequantize_affine")
     sizes, blocks, sc, zp = _affine_args("dequantize_affine", shape, block_size, scales, zero_points, codes.device)
     out = torch.empty(shape, dtype=torch.float32, device=codes.device)
@@ -822,6 +807,9 @@ def _lowbit_mm(input: torch.Tensor, packed: torch.Tensor, bits: int, columns: in
                bias: Optional[torch.Tensor] = None, lsb_first: bool = False) -> torch.Tensor:
     """``input @ dequantize(packed).T (+ bias)`` for a packed n-bit weight, without the dense weight
     (``_intx_mm`` / ``_int2_mm`` / ``_binary_mm`` of the reference).  input [M, K] f32 / f16 / bf16."""
+    calls = _lib.load().calls
+    if calls is not None and input.dim() == 2 and (out := calls.lowbit_mm(input, packed, bits, columns, scales_and_zeros, bias, lsb_first)) is not None:
+        return out
     if input.dim() != 2 or input.shape[1] != columns:
         raise ValueError(f"_lowbit_mm: expected activations [M, {columns}]")
     if input.dtype not in _DT:
@@ -831,7 +819,7 @@ def _lowbit_mm(input: torch.Tensor, packed: torch.Tensor, bits: int, columns: in
     x = input.contiguous()
     m = x.shape[0]
     b = None if bias is None else bias.to(torch.float32).contiguous()
-    if m and _lowbit_rows_takes(m, n, columns, bits, lsb_first, group, x.dtype):
+    if m and _lib.load().tpq_lowbit_mm_rows_takes(_ptr(x), _DT[x.dtype], m, n, columns, bits, int(lsb_first), group, _ptr(w), _ptr(sz)):
         out = torch.empty((m, n), dtype=x.dtype, device=x.device)
         with torch.cuda.device(x.device):
             ws = _rows_workspace(x.dtype, m, n, columns, x.device)
@@ -847,6 +835,16 @@ def _lowbit_mm(input: torch.Tensor, packed: torch.Tensor, bits: int, columns: in
         _check(_lib.load().tpq_lowbit_mm(_ptr(x), _DT[x.dtype], m, columns, _ptr(w), bits, int(lsb_first), n, group,
                                          _ptr(sz), _ptr(b), _ptr(out), _stream(x)))
     return out
+
+
+def _lowbit_linear(input: torch.Tensor, packed: torch.Tensor, bits: int, columns: int, scales_and_zeros: torch.Tensor,
+                   bias: Optional[torch.Tensor], lsb_first: bool) -> torch.Tensor:
+    """``_lowbit_mm`` of the rows of input [..., K]."""
+    calls = _lib.load().calls
+    if calls is not None and (out := calls.lowbit_mm(input, packed, bits, columns, scales_and_zeros, bias, lsb_first)) is not None:
+        return out
+    out = _lowbit_mm(input.reshape(-1, input.shape[-1]), packed, bits, columns, scales_and_zeros, bias, lsb_first)
+    return out.reshape(*input.shape[:-1], out.shape[-1])
 
 
 # ---- fusions around the int4 decode matmul (MLP of a decoder layer) -------------------------------
