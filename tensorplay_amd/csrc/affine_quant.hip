@@ -14,9 +14,9 @@
 // along the last dimension, per leading channel) collapses to "rows of K contiguous elements
 // cut into groups of g".  When K and g are multiples of four, a thread works on pieces of four
 // consecutive elements and consecutive lanes on consecutive pieces, so every wavefront load or
-// store of the float side is whole cache lines (measured 4.6 TB/s quantizing and 5.1 TB/s
-// dequantizing 4096 x 4096 to packed 4-bit; 16 contiguous elements per thread instead gave 4.2 and
-// 2.4 TB/s).  Other K / g: a thread takes 16 consecutive elements and walks (row, group) with
+// store of the float side is whole cache lines (4096 x 4096, packed 4-bit: 4.8 TB/s quantizing float32 and 5.4 TB/s
+// dequantizing; 16 contiguous elements per thread instead gave 4.2 and
+// 2.4 TB/s; 16-bit inputs go by eights where K and g allow).  Other K / g: a thread takes 16 consecutive elements and walks (row, group) with
 // counters.  Any other grid (blocks that tile two dimensions at once) takes the general kernel, one
 // thread per output byte with the full index arithmetic.
 #include "tpq_common.h"
@@ -328,26 +328,29 @@ __global__ __launch_bounds__(256) void dequantize_runs_kernel(const void* __rest
     }
 }
 
-// Rows and groups that are multiples of four: a thread takes pieces of four consecutive elements
+// Rows and groups that are multiples of four: a thread takes pieces of a few consecutive elements
 // (one block each), consecutive lanes take consecutive pieces, so the float side moves as whole
 // cache lines per wavefront instruction.  Four pieces per thread are in flight at once.
 struct Pieces {
-    int64_t K, g, G;
+    int64_t K, g, G;       // whole groups per row (the usual case): K = g, G = 1, and a block is a row of this
     int k_shift, g_shift;  // log2 when a power of two, else -1
     int small;             // numel < 2^31: 32-bit index arithmetic
     int need_block;        // some parameter differs between blocks
 };
 
+// block of the piece that starts at element c0
 __device__ __forceinline__ int64_t piece_block(const Pieces& ps, int64_t c0) {
     if (!ps.need_block) return 0;
     if (ps.small) {
         const uint32_t c = static_cast<uint32_t>(c0), K = static_cast<uint32_t>(ps.K), g = static_cast<uint32_t>(ps.g);
         const uint32_t row = ps.k_shift >= 0 ? c >> ps.k_shift : c / K;
+        if (ps.G == 1) return row;
         const uint32_t col = c - row * K;
         const uint32_t grp = ps.g_shift >= 0 ? col >> ps.g_shift : col / g;
         return static_cast<int64_t>(row) * ps.G + grp;
     }
     const int64_t row = ps.k_shift >= 0 ? c0 >> ps.k_shift : c0 / ps.K;
+    if (ps.G == 1) return row;
     const int64_t col = c0 - row * ps.K;
     const int64_t grp = ps.g_shift >= 0 ? col >> ps.g_shift : col / ps.g;
     return row * ps.G + grp;
@@ -405,37 +408,59 @@ __global__ __launch_bounds__(256) void dequantize_pieces_kernel(const void* __re
     }
 }
 
-template <int DT>
-__device__ __forceinline__ void load_piece_floats(const void* x, int64_t p, float v[4]) {
+// P elements, a piece of the float side: 16 bytes, or 8 (P = 4 of a 16-bit type)
+template <int DT, int P>
+__device__ __forceinline__ void load_piece_floats(const void* x, int64_t p, float v[P]) {
     if constexpr (DT == TPQ_DTYPE_F32) {
+        static_assert(P == 4, "16 bytes");
         const uint4 t = nt_load(static_cast<const uint4*>(x) + p);
         v[0] = __builtin_bit_cast(float, t.x); v[1] = __builtin_bit_cast(float, t.y);
         v[2] = __builtin_bit_cast(float, t.z); v[3] = __builtin_bit_cast(float, t.w);
     } else {
-        const uint2 t = nt_load(static_cast<const uint2*>(x) + p);
-        v[0] = Elem<DT>::load(static_cast<uint16_t>(t.x)); v[1] = Elem<DT>::load(static_cast<uint16_t>(t.x >> 16));
-        v[2] = Elem<DT>::load(static_cast<uint16_t>(t.y)); v[3] = Elem<DT>::load(static_cast<uint16_t>(t.y >> 16));
+        uint32_t w[P / 2];
+        if constexpr (P == 8) {
+            const uint4 t = nt_load(static_cast<const uint4*>(x) + p);
+            w[0] = t.x; w[1] = t.y; w[2] = t.z; w[3] = t.w;
+        } else {
+            const uint2 t = nt_load(static_cast<const uint2*>(x) + p);
+            w[0] = t.x; w[1] = t.y;
+        }
+#pragma unroll
+        for (int i = 0; i < P / 2; ++i) {
+            v[2 * i] = Elem<DT>::load(static_cast<uint16_t>(w[i]));
+            v[2 * i + 1] = Elem<DT>::load(static_cast<uint16_t>(w[i] >> 16));
+        }
     }
 }
 
-// Every lane of a wavefront must call this together (the 1-bit storage pairs neighbouring lanes);
+// Every lane of a wavefront must call this together (pieces of half a byte pair neighbouring lanes);
 // `live` says whether piece p exists.
-template <int BITS>
-__device__ __forceinline__ void store_piece(void* out, int64_t p, bool live, const int32_t q[4]) {
+template <int BITS, int P>
+__device__ __forceinline__ void store_piece(void* out, int64_t p, bool live, const int32_t q[P]) {
     if constexpr (BITS == 32) {
-        if (live) static_cast<int4*>(out)[p] = make_int4(q[0], q[1], q[2], q[3]);
+        if (live) {
+#pragma unroll
+            for (int i = 0; i < P / 4; ++i) static_cast<int4*>(out)[p * (P / 4) + i] = make_int4(q[4 * i], q[4 * i + 1], q[4 * i + 2], q[4 * i + 3]);
+        }
     } else if constexpr (BITS == 8) {
-        const uint32_t w = (static_cast<uint32_t>(q[0]) & 0xFFu) | ((static_cast<uint32_t>(q[1]) & 0xFFu) << 8) |
-                           ((static_cast<uint32_t>(q[2]) & 0xFFu) << 16) | (static_cast<uint32_t>(q[3]) << 24);
-        if (live) static_cast<uint32_t*>(out)[p] = w;
+        uint32_t w[P / 4];
+#pragma unroll
+        for (int i = 0; i < P / 4; ++i)
+            w[i] = (static_cast<uint32_t>(q[4 * i]) & 0xFFu) | ((static_cast<uint32_t>(q[4 * i + 1]) & 0xFFu) << 8) |
+                   ((static_cast<uint32_t>(q[4 * i + 2]) & 0xFFu) << 16) | (static_cast<uint32_t>(q[4 * i + 3]) << 24);
+        if (live) {
+            if constexpr (P == 8) static_cast<uint2*>(out)[p] = make_uint2(w[0], w[1]);
+            else static_cast<uint32_t*>(out)[p] = w[0];
+        }
     } else {
         // the clamp keeps every code inside its field, as in the reference nothing is masked
         uint32_t w = 0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w |= static_cast<uint32_t>(q[e]) << (e * BITS);
-        if constexpr (BITS == 4) { if (live) static_cast<uint16_t*>(out)[p] = static_cast<uint16_t>(w); }
-        if constexpr (BITS == 2) { if (live) static_cast<uint8_t*>(out)[p] = static_cast<uint8_t>(w); }
-        if constexpr (BITS == 1) {
+        for (int e = 0; e < P; ++e) w |= static_cast<uint32_t>(q[e]) << (e * BITS);
+        if constexpr (P * BITS == 32) { if (live) static_cast<uint32_t*>(out)[p] = w; }
+        if constexpr (P * BITS == 16) { if (live) static_cast<uint16_t*>(out)[p] = static_cast<uint16_t>(w); }
+        if constexpr (P * BITS == 8) { if (live) static_cast<uint8_t*>(out)[p] = static_cast<uint8_t>(w); }
+        if constexpr (P * BITS == 4) {
             // pieces 2i and 2i+1 share a byte and sit in neighbouring lanes (the thread index and the
             // piece index have the same parity): the even lane stores both nibbles
             const uint32_t mine = live ? w : 0u;
@@ -445,7 +470,39 @@ __device__ __forceinline__ void store_piece(void* out, int64_t p, bool live, con
     }
 }
 
-template <int DT, int BITS>
+// The codes of a piece.  Up to 8 bits both ends of the range are whole numbers that a float holds, so the clamp commutes
+// with the truncation and is one v_med3_f32 ahead of the conversion; a position beyond 2^31, infinite or NaN (never in a
+// sane weight) sends the whole wavefront through the general form, behind a branch that the compiler cannot turn into a
+// select (the divisor-like 64-bit conversions were computed for every element that way).
+template <int BITS, int P>
+__device__ __forceinline__ void quantize_piece(const float v[P], float inv, float zero, bool has_zero, const Params& pr, int32_t q[P]) {
+    if constexpr (BITS == 32) {
+#pragma unroll
+        for (int e = 0; e < P; ++e) q[e] = quantize_one<false>(v[e], inv, zero, has_zero, pr.qmin, pr.qmax);
+    } else {
+        const float lo = static_cast<float>(pr.qmin), hi = static_cast<float>(pr.qmax);
+        bool wild = false;
+#pragma unroll
+        for (int e = 0; e < P; ++e) {
+            const float r = __builtin_rintf(v[e] * inv);
+            const float position = has_zero ? r + zero : r;
+            wild |= !(__builtin_fabsf(position) < 0x1p31f);
+            q[e] = static_cast<int32_t>(__builtin_amdgcn_fmed3f(position, lo, hi));
+        }
+        if (__builtin_amdgcn_ballot_w64(wild) != 0) {
+            float factor = inv;
+            asm volatile("; piece redone in general form" : "+v"(factor));
+#pragma unroll
+            for (int e = 0; e < P; ++e) q[e] = quantize_one<(BITS < 8)>(v[e], factor, zero, has_zero, pr.qmin, pr.qmax);
+        }
+    }
+}
+
+// What bounds it: the bytes.  Pieces of 16 bytes on the float side where rows and groups allow (8 elements of a 16-bit type
+// share a division, a block index and a store), about 11 vector instructions per element.  4096 x 4096 bfloat16 to 4 bits in
+// groups of 128: 18.2 -> 11.1 us (pieces of four, each code through the general form: 37 instructions per element); float32
+// 17.4 -> 15.7.
+template <int DT, int BITS, int P>
 __global__ __launch_bounds__(256) void quantize_pieces_kernel(const void* __restrict__ x, void* __restrict__ out, int64_t pieces,
                                                               Pieces ps, Params pr) {
     constexpr int kFlight = 4;
@@ -454,29 +511,22 @@ __global__ __launch_bounds__(256) void quantize_pieces_kernel(const void* __rest
     // whole wavefronts stay in the loop together: the bound is rounded up to the wavefront
     const int64_t first = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     for (int64_t p0 = first; (p0 & ~int64_t{kWave - 1}) < pieces; p0 += kFlight * stride) {
-        float v[kFlight][4], inv[kFlight], zero[kFlight];
+        float v[kFlight][P], scale[kFlight], zero[kFlight];
+        // no branch around the loads (each would wait for its own): a piece behind the end reads the last one again
 #pragma unroll
         for (int j = 0; j < kFlight; ++j) {
-            const int64_t p = p0 + j * stride;
-            if (p < pieces) {
-                load_piece_floats<DT>(x, p, v[j]);
-                const int64_t b = piece_block(ps, 4 * p);
-                inv[j] = pr.scales[pr.scale_is_scalar ? 0 : b];
-                zero[j] = has_zero ? pr.zeros[pr.zero_is_scalar ? 0 : b] : 0.0f;
-            } else {
-                v[j][0] = v[j][1] = v[j][2] = v[j][3] = 0.0f;
-                inv[j] = 1.0f;
-                zero[j] = 0.0f;
-            }
+            const int64_t at = p0 + j * stride, p = at < pieces ? at : pieces - 1;
+            load_piece_floats<DT, P>(x, p, v[j]);
+            const int64_t b = piece_block(ps, P * p);
+            scale[j] = pr.scales[pr.scale_is_scalar ? 0 : b];
+            zero[j] = has_zero ? pr.zeros[pr.zero_is_scalar ? 0 : b] : 0.0f;
         }
 #pragma unroll
         for (int j = 0; j < kFlight; ++j) {
             const int64_t p = p0 + j * stride;
-            const float r = inverse_of(inv[j]);
-            int32_t q[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) q[e] = quantize_one<(BITS < 8)>(v[j][e], r, zero[j], has_zero, pr.qmin, pr.qmax);
-            store_piece<BITS>(out, p, p < pieces, q);
+            int32_t q[P];
+            quantize_piece<BITS, P>(v[j], inverse_of(scale[j]), zero[j], has_zero, pr, q);
+            store_piece<BITS, P>(out, p, p < pieces, q);
         }
     }
 }
@@ -547,7 +597,8 @@ int log2_if_power_of_two(int64_t v) {
 }
 
 Pieces pieces_of(const Plan& plan, const Params& pr) {
-    const Runs& r = plan.runs;
+    Runs r = plan.runs;
+    if (r.K % r.g == 0) r = {r.g, r.g, 1};  // whole groups in every row: blocks follow each other in memory
     return {r.K, r.g, r.G, log2_if_power_of_two(r.K), log2_if_power_of_two(r.g), plan.numel < (int64_t{1} << 31),
             !(pr.scale_is_scalar && (pr.zeros == nullptr || pr.zero_is_scalar)) && plan.num_blocks > 1};
 }
@@ -557,9 +608,12 @@ int launch_quantize(int bits, bool runs_ok, const void* x, void* out, const Plan
     const int64_t n = plan.numel;
     const Pieces ps = pieces_of(plan, pr);
     const bool pieces_ok = runs_ok && plan.runs.K % 4 == 0 && plan.runs.g % 4 == 0;
+    constexpr int kWide = DT == TPQ_DTYPE_F32 ? 4 : 8;  // elements in 16 bytes
+    const bool wide_ok = pieces_ok && plan.runs.K % kWide == 0 && plan.runs.g % kWide == 0;
 #define TPQ_AQ_CASE(BITS)                                                                                         \
     case BITS:                                                                                                    \
-        if (pieces_ok) quantize_pieces_kernel<DT, BITS><<<grid_for((n / 4 + 3) / 4), 256, 0, s>>>(x, out, n / 4, ps, pr); \
+        if (wide_ok) quantize_pieces_kernel<DT, BITS, kWide><<<grid_for((n / kWide + 3) / 4), 256, 0, s>>>(x, out, n / kWide, ps, pr); \
+        else if (pieces_ok) quantize_pieces_kernel<DT, BITS, 4><<<grid_for((n / 4 + 3) / 4), 256, 0, s>>>(x, out, n / 4, ps, pr); \
         else if (runs_ok) quantize_runs_kernel<DT, BITS><<<grid_for((n + kChunk - 1) / kChunk), 256, 0, s>>>(x, out, n, plan.runs, pr); \
         else quantize_grid_kernel<DT, BITS><<<grid_for(n), 256, 0, s>>>(x, out, n, plan.grid, pr);                \
         break;

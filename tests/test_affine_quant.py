@@ -233,6 +233,33 @@ def test_gpu_sixteen_bit_inputs(tdtype, name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tdtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,block", [((5, 40), (1, 24)), ((5, 24), (1, 24)), ((3, 36), (1, 12)), ((1, 8), (1, 8)), ((67, 264), (1, 88)),
+                                         ((9, 1032), (9, 1032)), ((3, 20), (1, 8)), ((513, 64), (1, 32))])
+@pytest.mark.parametrize("dtype", list(BOUNDS))
+def test_gpu_sixteen_bit_pieces(tdtype, shape, block, dtype):
+    """Pieces of eight and of four elements, whole and cut groups, one piece to several passes of the grid; values beyond
+    2^31, infinite and NaN among ordinary ones."""
+    rng = np.random.default_rng(zlib.crc32(repr((shape, block, dtype)).encode()))
+    lo, hi = BOUNDS[dtype]
+    span = min(hi - lo, 255)
+    x = torch.from_numpy(rng.uniform(-1.2 * span, 1.2 * span, shape).astype(np.float32)).to(tdtype)
+    _, n = blocks_of(shape, block)
+    scales = rng.uniform(0.2, 2.0, n).astype(np.float32)
+    for wild in (False, True):
+        if wild:
+            flat = x.view(-1)
+            for at, v in ((0, float("nan")), (3, float("inf")), (x.numel() // 2, float("-inf")), (x.numel() - 1, 6e4)):
+                flat[at] = v
+            scales[-1] = 1e-9
+        for zeros in (None, rng.integers(0, 3, n).astype(np.float32) + np.float32(0.25)):
+            want = oracle.quantize_affine(x.float().numpy(), block, scales, zeros, dtype)
+            got, back = _run_gpu(x, block, scales, zeros, dtype)
+            np.testing.assert_array_equal(got, want)
+            np.testing.assert_array_equal(back, oracle.dequantize_affine(want, shape, block, scales, zeros, dtype))
+
+
+@pytest.mark.gpu
 def test_gpu_full_size_rowwise_codes_and_round_trip():
     """2048 x 4096 activations, one block per row: the step before the int8 GEMM
     (tensorplay/ao/quantization/bitnet.py:127-135 takes this route for large inputs)."""
