@@ -40,6 +40,22 @@ def test_int8_rowwise_bit_exact(ops, dtype, shape):
     np.testing.assert_array_equal(host(codes), want_codes)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("k", [4, 12, 20, 60, 68, 132, 260, 516, 1020, 1028, 2044, 2052, 5284, 16388, 65532])
+def test_rows_of_fours_bit_exact(ops, dtype, k):
+    """K % 8 == 4: the last eight elements of a row overlap the chunk before them, and rows start on 8 bytes; the row maximum in
+    the last four, in the overlap and in the first element."""
+    rng = np.random.default_rng(k)
+    x = rng.normal(size=(5, k)).astype(np.float32)
+    for row, at in ((0, k - 1), (1, max(k - 8, 0)), (2, 0), (3, k // 2)):
+        x[row, at] = -9.0
+    xb = cast_bits(x, dtype)
+    want_codes, want_scales = oracle.quantize_int8_rowwise(xb, dtype, 1e-5)
+    codes, scales = ops._quantize_int8_rowwise(dev(xb, dtype), 1e-5)
+    np.testing.assert_array_equal(host(scales), want_scales)
+    np.testing.assert_array_equal(host(codes), want_codes)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_lowbit_variants_bit_exact(ops, dtype):
     rng = np.random.default_rng(5)
