@@ -234,6 +234,10 @@ int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int
                              int64_t group, const uint8_t* packed, const float* scales_and_zeros);
 int tpq_int4_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, int64_t N, int64_t group,
                      const void* scales_and_zeros, void* out, void* workspace, int64_t workspace_bytes, void* stream);
+/* the same + bias [N] of the activation type (or NULL): added to the rounded product and rounded again, as a separate add does */
+int tpq_int4_mm_rows_bias(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, int64_t N, int64_t group,
+                          const void* scales_and_zeros, const void* bias, void* out, void* workspace, int64_t workspace_bytes,
+                          void* stream);
 int tpq_lowbit_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const uint8_t* packed, int bits, int lsb_first,
                        int64_t N, int64_t group, const float* scales_and_zeros, const float* bias, void* out,
                        void* workspace, int64_t workspace_bytes, void* stream);

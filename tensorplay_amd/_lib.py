@@ -40,6 +40,7 @@ SIGNATURES = {
     "tpq_int4_mm_rows_takes": [_ptr, _int, _i64, _i64, _i64, _i64, _ptr, _ptr],
     "tpq_lowbit_mm_rows_takes": [_ptr, _int, _i64, _i64, _i64, _int, _int, _i64, _ptr, _ptr],
     "tpq_int4_mm_rows": [_ptr, _int, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr],
+    "tpq_int4_mm_rows_bias": [_ptr, _int, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr],
     "tpq_lowbit_mm_rows": [_ptr, _int, _i64, _i64, _ptr, _int, _int, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr],
     "tpq_ternary_pack": [_ptr, _i64, _i64, _ptr, _ptr],
     "tpq_ternary_unpack": [_ptr, _i64, _i64, _ptr, _ptr],

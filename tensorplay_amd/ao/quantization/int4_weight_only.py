@@ -81,10 +81,7 @@ class WeightOnlyInt4Linear(nn.Module):
         act_pre_scale = getattr(self, "act_pre_scale", None)
         if act_pre_scale is not None:
             input = input * act_pre_scale
-        out = _int4_mm(input, self.weight, self.scales_and_zeros, self.groupsize)
-        if self.bias is not None:
-            out = out + self.bias
-        return out
+        return ops._int4_linear(input, self.weight, self.groupsize, self.scales_and_zeros, self.bias)
 
     # Layout of a CPU-packed ``weight`` met in a state_dict: (columns per block, half-split nibbles).  The reference's
     # CPU pack depends on the ISA tier it was compiled for (p10/src/backend/cpu/QuantizedElementwiseKernels.cpp:19,

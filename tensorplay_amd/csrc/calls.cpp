@@ -7,7 +7,7 @@
 // What it answers: a decode step calls these at 5 to 10 us of kernel time, and the same steps in Python took 20 us (int4
 // product) to 30 us (row quantizer + int8 product) of host time a call, so the card waited.
 // Measured (us a pass with the modules' own Python, host time, before / with this): int8 dynamic linear 30.6 / 10.0, int4 at one
-// row 21.2 / 6.6, int4 with bias at 48 rows 27.5 / 14.6, 2-bit linear 20.2 / 6.3, ternary MLP (two linears and a relu) 59.9 / 21.7,
+// row 21.2 / 6.6, int4 with bias at 48 rows 27.5 / 12.4, 2-bit linear 20.2 / 6.3, ternary MLP (two linears and a relu) 59.9 / 21.7,
 // affine quantize + dequantize 28.3 / 9.4.  Above 16 rows only the routes that the library picks itself are taken here: from there
 // on the kernels are longer than either form.
 #include <Python.h>
@@ -17,6 +17,7 @@
 #include <cstdint>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
@@ -37,7 +38,7 @@ struct Library {
 #define TPQ_ENTRIES                                                                                                       \
     TPQ_ENTRY(tpq_quantize_rowwise) TPQ_ENTRY(tpq_int8_mm_workspace_bytes) TPQ_ENTRY(tpq_int8_mm_dequant_ws)                \
     TPQ_ENTRY(tpq_ternary_mm_workspace_bytes) TPQ_ENTRY(tpq_ternary_mm_ws) TPQ_ENTRY(tpq_int4_mm_ws)                        \
-    TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows)      \
+    TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
     TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
     TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine)
     TPQ_ENTRIES
@@ -273,19 +274,21 @@ TPQ_CALL(ternary_linear, 6)
     return THPVariable_Wrap(std::move(out));
 TPQ_CALL_END
 
-// int4_mm(x [..., K], packed int32 [N / 8, K / 32, 32, 1], group, scales_and_zeros [K / group, N, 2] of x's type, workspaces):
-// the rows kernel and, up to 16 rows, the decode kernels.  workspaces: {(device, stream): zero-filled buffer} of
+// int4_mm(x [..., K], packed int32 [N / 8, K / 32, 32, 1], group, scales_and_zeros [K / group, N, 2] of x's type, bias or None,
+// workspaces): the rows kernel, which adds the bias as a separate add would, and, up to 16 rows, the decode kernels and an add.  workspaces: {(device, stream): zero-filled buffer} of
 // ops._int4_workspace; a stream that has none yet, or too small a one, gets it in the Python form.
-TPQ_CALL(int4_mm, 5)
-    const at::Tensor *x = plain(args[0]), *packed = plain(args[1]), *sz = plain(args[3]);
+TPQ_CALL(int4_mm, 6)
+    const at::Tensor *x = plain(args[0]), *packed = plain(args[1]), *sz = plain(args[3]), *bias;
     int64_t group;
-    if (!x || !packed || !sz || !as_int(args[2], &group) || !PyDict_CheckExact(args[4]) || (group != 32 && group != 64 && group != 128) || x->dim() < 1 ||
+    if (!x || !packed || !sz || !as_int(args[2], &group) || !PyDict_CheckExact(args[5]) || (group != 32 && group != 64 && group != 128) || x->dim() < 1 ||
         x->numel() == 0 || packed->dim() != 4 || packed->scalar_type() != at::kInt || packed->size(0) == 0 || packed->size(2) != 32 || packed->size(3) != 1 ||
         sz->dim() != 3 || sz->scalar_type() != x->scalar_type() || !same_device(*x, *packed) || !same_device(*x, *sz))
         Py_RETURN_NONE;
     const int tag = float_tag(x->scalar_type());
     const int64_t K = x->size(-1), N = packed->size(0) * 8;
     if (tag < 0 || packed->size(1) != (K + 31) / 32 || sz->size(0) != (K + group - 1) / group || sz->size(1) != N || sz->size(2) != 2) Py_RETURN_NONE;
+    // a bias that something differentiates is added where that is seen
+    if (!optional_vector(args[4], x->scalar_type(), N, *x, &bias) || (bias && (bias->dim() != 1 || bias->requires_grad() || bias->_fw_grad(0).defined()))) Py_RETURN_NONE;
     int64_t M;
     const auto sizes = product_sizes(*x, N, &M);
     const bool rows = lib.tpq_int4_mm_rows_takes(x->const_data_ptr(), tag, M, N, K, group, ptr<int32_t>(packed), sz->const_data_ptr()) != 0;
@@ -298,7 +301,7 @@ TPQ_CALL(int4_mm, 5)
         const int64_t stream = static_cast<int64_t>(reinterpret_cast<intptr_t>(c10::hip::getCurrentHIPStream(x->device().index()).stream()));
         PyObject* key = Py_BuildValue("(iL)", static_cast<int>(x->device().index()), static_cast<long long>(stream));
         if (!key) return nullptr;
-        PyObject* held = PyDict_GetItemWithError(args[4], key);
+        PyObject* held = PyDict_GetItemWithError(args[5], key);
         Py_DECREF(key);
         if (!held) {
             if (PyErr_Occurred()) return nullptr;
@@ -316,11 +319,15 @@ TPQ_CALL(int4_mm, 5)
         out = allocate(sizes, x->scalar_type(), *x);
         if (rows) {
             const at::Tensor part = workspace_bytes ? allocate({workspace_bytes}, at::kByte, *x) : at::Tensor();
-            status = lib.tpq_int4_mm_rows(x->const_data_ptr(), tag, M, K, ptr<int32_t>(packed), N, group, sz->const_data_ptr(), out.data_ptr(),
+            status = lib.tpq_int4_mm_rows_bias(x->const_data_ptr(), tag, M, K, ptr<int32_t>(packed), N, group, sz->const_data_ptr(), ptr<void>(bias), out.data_ptr(),
                                           workspace_bytes ? part.data_ptr() : nullptr, workspace_bytes, q.stream);
         } else {
             status = lib.tpq_int4_mm_ws(x->const_data_ptr(), tag, M, K, ptr<int32_t>(packed), 2, N, group, sz->const_data_ptr(), out.data_ptr(), workspace->data_ptr(),
                                         static_cast<size_t>(workspace_bytes), q.stream);
+            if (status == TPQ_OK && bias) {
+                const at::AutoDispatchBelowADInplaceOrView raw;
+                out.add_(*bias);
+            }
         }
     }
     if (status != TPQ_OK) Py_RETURN_NONE;

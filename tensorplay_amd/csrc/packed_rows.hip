@@ -80,6 +80,12 @@ TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t
 
 TPQ_EXPORT int tpq_int4_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, int64_t N, int64_t group,
                                 const void* scales_and_zeros, void* out, void* workspace, int64_t workspace_bytes, void* stream) {
+    return tpq_int4_mm_rows_bias(x, dtype, M, K, packed, N, group, scales_and_zeros, nullptr, out, workspace, workspace_bytes, stream);
+}
+
+TPQ_EXPORT int tpq_int4_mm_rows_bias(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, int64_t N, int64_t group,
+                                     const void* scales_and_zeros, const void* bias, void* out, void* workspace, int64_t workspace_bytes,
+                                     void* stream) {
     TPQ_REQUIRE(dtype == TPQ_DTYPE_F32 || dtype == TPQ_DTYPE_F16 || dtype == TPQ_DTYPE_BF16, TPQ_ERR_INVALID_TYPE, "int4_mm_rows: unsupported activation dtype");
     TPQ_REQUIRE(M >= 0 && N >= 0 && K >= 0 && N % 8 == 0, TPQ_ERR_INVALID_VALUE, "int4_mm_rows: bad shape");
     TPQ_REQUIRE(group == 32 || group == 64 || group == 128, TPQ_ERR_INVALID_VALUE, "int4_mm_rows: qGroupSize must be 32, 64 or 128");
@@ -87,12 +93,12 @@ TPQ_EXPORT int tpq_int4_mm_rows(const void* x, int dtype, int64_t M, int64_t K, 
     TPQ_REQUIRE(K > 0 && K % 32 == 0 && K < (1 << 24) && M < (1 << 22) && N * K / 2 < (int64_t{1} << 32), TPQ_ERR_UNSUPPORTED, "int4_mm_rows: K must be a positive multiple of 32, the weight below 4 GB");
     TPQ_REQUIRE(x && packed && scales_and_zeros && out, TPQ_ERR_INVALID_VALUE, "int4_mm_rows: null pointer");
     const bool wide = dtype == TPQ_DTYPE_F32;
-    TPQ_REQUIRE(aligned(x, 16) && aligned(packed, 16) && aligned(scales_and_zeros, wide ? 8 : 4) && aligned(out, wide ? 16 : 8), TPQ_ERR_UNSUPPORTED,
+    TPQ_REQUIRE(aligned(x, 16) && aligned(packed, 16) && aligned(scales_and_zeros, wide ? 8 : 4) && aligned(out, wide ? 16 : 8) && aligned(bias, wide ? 4 : 2), TPQ_ERR_UNSUPPORTED,
                 "int4_mm_rows: unaligned operand");
     const bool room = workspace != nullptr && aligned(workspace, 16);
     const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, room ? workspace_bytes / 4 : 0);
     PackedRowsArgs a{};
-    a.x = x; a.w = packed; a.sz = scales_and_zeros; a.y = out; a.partial = static_cast<float*>(workspace);
+    a.x = x; a.w = packed; a.sz = scales_and_zeros; a.y = out; a.after = bias; a.partial = static_cast<float*>(workspace);
     a.M = static_cast<int>(M); a.N = static_cast<int>(N); a.K = static_cast<int>(K); a.tiles_per_group = static_cast<int>(group / 32);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == TPQ_DTYPE_F32) return run_int4<TPQ_DTYPE_F32>(a, p, s);

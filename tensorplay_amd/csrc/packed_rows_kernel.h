@@ -62,6 +62,7 @@ struct PackedRowsArgs {
     const void* w;         // packed
     const void* sz;        // int4: [K / group][N][2] of the activation type; n-bit: the same in float32
     const float* bias;     // added in fp32 before the rounding (n-bit modules), or null
+    const void* after;     // of the activation type, added to the rounded product, which is rounded again (int4 modules), or null
     void* y;               // [M][N]
     float* partial;        // [slices][M][N], or null: y
     int M, N, K, tiles_per_group, steps_per_slice;
@@ -197,6 +198,20 @@ struct RowsParams {
         else return __builtin_bit_cast(float, p.y);
     }
 };
+
+// four sums of the channels n .. n + 3 rounded (+ after[n ..], rounded again)
+template <int DT>
+__device__ __forceinline__ void store_rows_result(const float4_t& s, typename Elem<DT>::storage* y, const typename Elem<DT>::storage* after, int n) {
+    typename Elem<DT>::storage o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = Elem<DT>::store(s[e]);
+    if (after != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = Elem<DT>::store(Elem<DT>::load(o[e]) + Elem<DT>::load(after[n + e]));
+    }
+    if constexpr (DT == TPQ_DTYPE_F32) *reinterpret_cast<float4_t*>(y) = float4_t{o[0], o[1], o[2], o[3]};
+    else *reinterpret_cast<uint2*>(y) = make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16));
+}
 
 template <int DT, class Source, int MB, int CW, bool EDGE>
 __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedRowsArgs a) {
@@ -460,18 +475,15 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
 #pragma unroll
             for (int e = 0; e < 4; ++e) s[e] += a.bias[n + e];
         }
-        storage* const y = static_cast<storage*>(a.y) + at;
-        if constexpr (DT == TPQ_DTYPE_F32) *reinterpret_cast<float4_t*>(y) = s;
-        else
-            *reinterpret_cast<uint2*>(y) = make_uint2(Elem<DT>::store(s[0]) | (static_cast<uint32_t>(Elem<DT>::store(s[1])) << 16),
-                                                      Elem<DT>::store(s[2]) | (static_cast<uint32_t>(Elem<DT>::store(s[3])) << 16));
+        store_rows_result<DT>(s, static_cast<storage*>(a.y) + at, static_cast<const storage*>(a.after), n);
     }
 }
 
 // y = round(sum over the slices, in slice order (+ bias)); a thread takes four consecutive elements (N % 4 == 0)
 template <int DT>
 __global__ __launch_bounds__(256) void packed_rows_finish_kernel(const float* __restrict__ partial, int slices, int64_t quads, const float* __restrict__ bias,
-                                                                 int quads_per_row, typename Elem<DT>::storage* __restrict__ y) {
+                                                                 const typename Elem<DT>::storage* __restrict__ after, int quads_per_row,
+                                                                 typename Elem<DT>::storage* __restrict__ y) {
     const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (e >= quads) return;
     // four slices requested together; a batch past the last slice asks for the last one again and leaves it out of the sum
@@ -484,15 +496,12 @@ __global__ __launch_bounds__(256) void packed_rows_finish_kernel(const float* __
         for (int j = 0; j < 4; ++j)
             if (z0 + j < slices) sum = float4_t{sum[0] + more[j][0], sum[1] + more[j][1], sum[2] + more[j][2], sum[3] + more[j][3]};
     }
+    const int n = bias != nullptr || after != nullptr ? static_cast<int>(static_cast<uint32_t>(e) % static_cast<uint32_t>(quads_per_row)) * 4 : 0;
     if (bias != nullptr) {
-        const int n = static_cast<int>(static_cast<uint32_t>(e) % static_cast<uint32_t>(quads_per_row)) * 4;
 #pragma unroll
         for (int j = 0; j < 4; ++j) sum[j] += bias[n + j];
     }
-    if constexpr (DT == TPQ_DTYPE_F32) reinterpret_cast<float4_t*>(y)[e] = sum;
-    else
-        reinterpret_cast<uint2*>(y)[e] = make_uint2(Elem<DT>::store(sum[0]) | (static_cast<uint32_t>(Elem<DT>::store(sum[1])) << 16),
-                                                    Elem<DT>::store(sum[2]) | (static_cast<uint32_t>(Elem<DT>::store(sum[3])) << 16));
+    store_rows_result<DT>(sum, y + e * 4, after, n);
 }
 
 // ---- launch ------------------------------------------------------------------------------------------
@@ -575,7 +584,7 @@ int launch_packed_rows(PackedRowsArgs a, const PackedRowsPlan& p, hipStream_t s)
     if (rc != TPQ_OK || a.partial == nullptr) return rc;
     const int64_t quads = static_cast<int64_t>(a.M) * a.N / 4;
     packed_rows_finish_kernel<DT><<<static_cast<unsigned>((quads + 255) / 256), 256, 0, s>>>(
-        a.partial, p.slices, quads, a.bias, a.N / 4, static_cast<typename Elem<DT>::storage*>(a.y));
+        a.partial, p.slices, quads, a.bias, static_cast<const typename Elem<DT>::storage*>(a.after), a.N / 4, static_cast<typename Elem<DT>::storage*>(a.y));
     return check_launch("packed rows (sum of the slices)");
 }
 

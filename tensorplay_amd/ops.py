@@ -402,7 +402,7 @@ def _weight_int4pack_mm(self: torch.Tensor, mat2: torch.Tensor, qGroupSize: int,
                         qScaleAndZeros: torch.Tensor) -> torch.Tensor:
     """``self @ W.T`` with W dequantised per group: (code - 8) * scale + zero; result in self.dtype."""
     calls = _lib.load().calls
-    if calls is not None and self.dim() == 2 and (out := calls.int4_mm(self, mat2, qGroupSize, qScaleAndZeros, _int4_workspaces)) is not None:
+    if calls is not None and self.dim() == 2 and (out := calls.int4_mm(self, mat2, qGroupSize, qScaleAndZeros, None, _int4_workspaces)) is not None:
         return out
     if mat2.dtype != torch.int32 or mat2.dim() != 4:
         raise TypeError("_weight_int4pack_mm(): packed weight must be 4-D int32 in the tensor-core B layout")
@@ -458,13 +458,15 @@ def _weight_int4pack_mm(self: torch.Tensor, mat2: torch.Tensor, qGroupSize: int,
     return out
 
 
-def _int4_linear(input: torch.Tensor, packed: torch.Tensor, group: int, scales_and_zeros: torch.Tensor) -> torch.Tensor:
-    """``_weight_int4pack_mm`` of the rows of input [..., K]."""
+def _int4_linear(input: torch.Tensor, packed: torch.Tensor, group: int, scales_and_zeros: torch.Tensor,
+                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``_weight_int4pack_mm`` of the rows of input [..., K] (+ bias, added to the rounded product)."""
     calls = _lib.load().calls
-    if calls is not None and (out := calls.int4_mm(input, packed, group, scales_and_zeros, _int4_workspaces)) is not None:
+    if calls is not None and (out := calls.int4_mm(input, packed, group, scales_and_zeros, bias, _int4_workspaces)) is not None:
         return out
     out = _weight_int4pack_mm(input.reshape(-1, input.shape[-1]), packed, group, scales_and_zeros)
-    return out.reshape(*input.shape[:-1], out.shape[-1])
+    out = out.reshape(*input.shape[:-1], out.shape[-1])
+    return out if bias is None else out + bias
 
 
 def pack_ternary(codes: torch.Tensor) -> torch.Tensor:

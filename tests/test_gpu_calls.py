@@ -64,7 +64,8 @@ def _module(kind, k, n, dtype, bias):
 def test_modules(monkeypatch, kind, dtype, rows):
     gen = torch.Generator(device="cuda").manual_seed(rows)
     # 192: a K that no 128-wide kernel takes whole; 4 more for the kernels that want nothing of K
-    for k, n, bias in ((512, 200, True), (192, 72, False), *(((196, 72, False),) if kind in ("int8", "bitnet") else ())):
+    # 4096 against few channels: slices of K, whose second kernel adds the bias
+    for k, n, bias in ((512, 200, True), (4096, 72, True), (192, 72, False), *(((196, 72, False),) if kind in ("int8", "bitnet") else ())):
         module = _module(kind, k, n, DTYPES[dtype], bias)
         x = torch.randn(rows, k, device="cuda", generator=gen).to(DTYPES[dtype])
         for form in _forms(x):
