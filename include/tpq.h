@@ -215,6 +215,14 @@ int tpq_ternary_mm_ws(const int8_t* x, const float* row_scale, const uint8_t* pa
                       int32_t* acc_out, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * tpq_quantize_rowwise (divisor 127, codes -127 .. 127) of ONE activation row x [K] and tpq_ternary_mm of its codes, in one
+ * launch with the same result bits: bitnet_linear_packed of a decode step (tensorplay/ao/quantization/bitnet.py:215-241).
+ * K % 64 == 0, K <= 8192, x and packed 16-byte aligned; else TPQ_ERR_UNSUPPORTED.  out [N] float32, bias f32 [N] or NULL.
+ */
+int tpq_ternary_linear_row(const void* x, int x_dtype, const uint8_t* packed, float w_scale, const float* bias, int64_t N,
+                           int64_t K, float eps, float* out, void* stream);
+
+/*
  * The int4 and n-bit weight-only products for a block of activation rows (about 17 .. 500; any count is taken), float32 /
  * float16 / bfloat16, groups of any multiple of 32 (int4: 32, 64 or 128, innerKTiles = 2), K % 32 == 0; anything else
  * returns TPQ_ERR_UNSUPPORTED.  Same operations and reference lines as tpq_int4_mm and tpq_lowbit_mm (1, 2, 4, 8 bits); the

@@ -37,7 +37,8 @@ struct Library {
 #define TPQ_ENTRY(NAME) decltype(&::NAME) NAME = nullptr;
 #define TPQ_ENTRIES                                                                                                       \
     TPQ_ENTRY(tpq_quantize_rowwise) TPQ_ENTRY(tpq_int8_mm_workspace_bytes) TPQ_ENTRY(tpq_int8_mm_dequant_ws)                \
-    TPQ_ENTRY(tpq_ternary_mm_workspace_bytes) TPQ_ENTRY(tpq_ternary_mm_ws) TPQ_ENTRY(tpq_int4_mm_ws)                        \
+    TPQ_ENTRY(tpq_ternary_mm_workspace_bytes) TPQ_ENTRY(tpq_ternary_mm_ws) TPQ_ENTRY(tpq_ternary_linear_row)                \
+    TPQ_ENTRY(tpq_int4_mm_ws)                                                                                             \
     TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
     TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
     TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine)
@@ -260,15 +261,20 @@ TPQ_CALL(ternary_linear, 6)
     {
         Enqueue q(*x);
         out = allocate(sizes, at::kFloat, *x);
-        const int64_t scratch_bytes = lib.tpq_ternary_mm_workspace_bytes(M, N, K), scales_at = padded(M * K), scratch_at = scales_at + padded(4 * M);
-        const at::Tensor part = allocate({scratch_at + scratch_bytes}, at::kByte, *x);
-        char* base = out_ptr<char>(part);
-        status = lib.tpq_quantize_rowwise(x->const_data_ptr(), float_tag(x->scalar_type()), M, K, static_cast<float>(eps), 127.0f, -127, 127, 0,
-                                          reinterpret_cast<int8_t*>(base), reinterpret_cast<float*>(base + scales_at), q.stream);
-        if (status == TPQ_OK)
-            status = lib.tpq_ternary_mm_ws(reinterpret_cast<int8_t*>(base), reinterpret_cast<float*>(base + scales_at), ptr<uint8_t>(packed), static_cast<float>(w_scale),
-                                           ptr<float>(bias), M, N, K, out_ptr<float>(out), TPQ_DTYPE_F32, nullptr, scratch_bytes ? base + scratch_at : nullptr, scratch_bytes,
-                                           q.stream);
+        status = M == 1 ? lib.tpq_ternary_linear_row(x->const_data_ptr(), float_tag(x->scalar_type()), ptr<uint8_t>(packed), static_cast<float>(w_scale), ptr<float>(bias), N, K,
+                                                     static_cast<float>(eps), out_ptr<float>(out), q.stream)
+                        : TPQ_ERR_UNSUPPORTED;
+        if (status != TPQ_OK) {
+            const int64_t scratch_bytes = lib.tpq_ternary_mm_workspace_bytes(M, N, K), scales_at = padded(M * K), scratch_at = scales_at + padded(4 * M);
+            const at::Tensor part = allocate({scratch_at + scratch_bytes}, at::kByte, *x);
+            char* base = out_ptr<char>(part);
+            status = lib.tpq_quantize_rowwise(x->const_data_ptr(), float_tag(x->scalar_type()), M, K, static_cast<float>(eps), 127.0f, -127, 127, 0,
+                                              reinterpret_cast<int8_t*>(base), reinterpret_cast<float*>(base + scales_at), q.stream);
+            if (status == TPQ_OK)
+                status = lib.tpq_ternary_mm_ws(reinterpret_cast<int8_t*>(base), reinterpret_cast<float*>(base + scales_at), ptr<uint8_t>(packed),
+                                               static_cast<float>(w_scale), ptr<float>(bias), M, N, K, out_ptr<float>(out), TPQ_DTYPE_F32, nullptr,
+                                               scratch_bytes ? base + scratch_at : nullptr, scratch_bytes, q.stream);
+        }
     }
     if (status != TPQ_OK) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(out));

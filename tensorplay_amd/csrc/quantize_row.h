@@ -1,0 +1,182 @@
+// The arithmetic of the row-wise int8 quantizer, shared by its own kernels and by those that quantize an activation row on its
+// way into a product: the same codes and scales wherever a row is quantized.
+#pragma once
+
+#include "tpq_common.h"
+
+namespace tpq {
+namespace {
+
+constexpr int kVec = 8;  // elements per lane per chunk
+
+struct QParams {
+    float eps, divisor;
+    int qmin, qmax, sign_mode;
+    int no_clamp;  // no quotient |v| / scale, |v| <= absmax, can round outside [qmin, qmax]
+};
+
+__device__ __forceinline__ int quantize_one(float v, float scale, const QParams& p) {
+    if (p.sign_mode) return v >= 0.0f ? p.qmax : p.qmin;
+    // __fdiv_rn: correctly rounded division regardless of compiler flags
+    float q = rintf(__fdiv_rn(v, scale));
+    q = fminf(fmaxf(q, static_cast<float>(p.qmin)), static_cast<float>(p.qmax));
+    return static_cast<int>(q);
+}
+
+// Eight codes with one reciprocal instead of eight divisions, same bits as quantize_one.
+// q = v * (1/scale) is within 2^-21 relative of the true quotient, |quotient| <= 128 here, so its
+// absolute error is below 2^-14.  If q lies at least 2^-13 inside (c - 1/2, c + 1/2), so does the
+// correctly rounded quotient, and both round to c.  Otherwise (about one element in a few thousand;
+// also NaN and infinities) the element is redone with the IEEE division.
+// The codes leave as two packed words.  v_cvt_pk_u8_f32 converts a float to an unsigned byte (saturating at 0 and
+// 255) and drops it into one byte of a register: the rounded quotient c is an integer already, so c + 128 converts
+// exactly, the upper clamp is the saturation when qmax = 127, and one xor takes the 128 off the four bytes again.
+// Four instructions per code less than clamp, convert, mask, shift, or.
+__device__ __forceinline__ void quantize_eight_packed(const float (&v)[kVec], float scale, float inv_scale, const QParams& p,
+                                                      uint32_t& lo, uint32_t& hi) {
+    bool redo = false;
+    uint32_t word[2] = {0u, 0u};
+    const float qmin = static_cast<float>(p.qmin), qmax = static_cast<float>(p.qmax);
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) {
+        const float q = v[i] * inv_scale;
+        const float c = rintf(q);
+        redo |= !(fabsf(q - c) <= 0.5f - 0x1p-13f);
+        const float biased = fminf(fmaxf(c, qmin), qmax) + 128.0f;  // 0 .. 255, an integer
+        word[i >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(biased, i & 3, word[i >> 2]);
+    }
+    lo = word[0] ^ 0x80808080u;
+    hi = word[1] ^ 0x80808080u;
+    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, with a statement the
+    // compiler may not move: left as a plain "if", the eight divisions were computed for every chunk and selected away.
+    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, and with the divisor
+    // passed through a statement the compiler may not move: as a plain "if", the eight divisions were hoisted above the
+    // branch, computed for every chunk and selected away.
+    if (__builtin_amdgcn_ballot_w64(redo) != 0) {
+        float divisor = scale;
+        asm volatile("; elements redone with the division" : "+v"(divisor));
+        if (redo) {
+            lo = hi = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                lo |= (static_cast<uint32_t>(quantize_one(v[i], divisor, p)) & 0xFFu) << (8 * i);
+                hi |= (static_cast<uint32_t>(quantize_one(v[i + 4], divisor, p)) & 0xFFu) << (8 * i);
+            }
+        }
+    }
+}
+
+// The same codes with fewer instructions, for parameters under which no quotient can leave the code range
+// (rint(divisor (1 + 2^-20)) <= qmax and >= -qmin, true for the usual divisor = qmax = -qmin = 127): no clamp is
+// needed, and the code is read off the mantissa.  t = fma(v, 1/scale, 1.5 * 2^23) rounds the exact product to the
+// nearest integer (ties to even) and leaves it in two's complement in the low mantissa bits; c = t - 1.5 * 2^23 is that
+// integer, r = fma(v, 1/scale, -c) its distance from the product.  The product is within 2^-16 of the correctly rounded
+// quotient the reference rounds, so |r| <= 1/2 - 2^-13 proves both round to c; anything else (also NaN) is redone with
+// the division.  Five instructions per code and three byte permutes per four codes.
+__device__ __forceinline__ void quantize_eight_lean(const float (&v)[kVec], float scale, float inv_scale, const QParams& p,
+                                                    uint32_t& lo, uint32_t& hi) {
+    constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
+    bool redo = false;
+    uint32_t t[kVec];
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) {
+        const float tf = __builtin_fmaf(v[i], inv_scale, kMagic);
+        const float c = tf - kMagic;
+        const float r = __builtin_fmaf(v[i], inv_scale, -c);
+        redo |= !(fabsf(r) <= 0.5f - 0x1p-13f);
+        t[i] = __builtin_bit_cast(uint32_t, tf);
+    }
+    // v_perm_b32(a, b, sel): selector bytes 0..3 take bytes of b, 4..7 of a, 0x0c a zero byte
+    lo = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0400u) | __builtin_amdgcn_perm(t[3], t[2], 0x04000c0cu);
+    hi = __builtin_amdgcn_perm(t[5], t[4], 0x0c0c0400u) | __builtin_amdgcn_perm(t[7], t[6], 0x04000c0cu);
+    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, with a statement the
+    // compiler may not move: left as a plain "if", the eight divisions were computed for every chunk and selected away.
+    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, and with the divisor
+    // passed through a statement the compiler may not move: as a plain "if", the eight divisions were hoisted above the
+    // branch, computed for every chunk and selected away.
+    if (__builtin_amdgcn_ballot_w64(redo) != 0) {
+        float divisor = scale;
+        asm volatile("; elements redone with the division" : "+v"(divisor));
+        if (redo) {
+            lo = hi = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                lo |= (static_cast<uint32_t>(quantize_one(v[i], divisor, p)) & 0xFFu) << (8 * i);
+                hi |= (static_cast<uint32_t>(quantize_one(v[i + 4], divisor, p)) & 0xFFu) << (8 * i);
+            }
+        }
+    }
+}
+
+// What a row's maximum makes of its parameters
+struct RowScale {
+    float scale, inverse;
+    bool shortcut, lean;
+};
+__device__ __forceinline__ RowScale scale_of_row(float absmax, const QParams& p) {
+    RowScale r;
+    r.scale = __fdiv_rn(fmaxf(absmax, p.eps), p.divisor);
+    // the shortcut needs |quotient| <= 128 and a finite reciprocal: true for every scale the formula
+    // above produces from finite inputs with divisor <= 128; anything else takes the divisions
+    r.inverse = __fdiv_rn(1.0f, r.scale);
+    r.shortcut = !p.sign_mode && p.divisor <= 128.0f && r.inverse < 3.0e38f && absmax <= 3.0e38f;
+    r.lean = r.shortcut && p.no_clamp;
+    return r;
+}
+__device__ __forceinline__ void quantize_eight(const float (&v)[kVec], const RowScale& r, const QParams& p, uint32_t& lo, uint32_t& hi) {
+    lo = hi = 0;
+    if (r.lean) {
+        quantize_eight_lean(v, r.scale, r.inverse, p, lo, hi);
+    } else if (r.shortcut) {
+        quantize_eight_packed(v, r.scale, r.inverse, p, lo, hi);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            lo |= (static_cast<uint32_t>(quantize_one(v[i], r.scale, p)) & 0xFFu) << (8 * i);
+            hi |= (static_cast<uint32_t>(quantize_one(v[i + 4], r.scale, p)) & 0xFFu) << (8 * i);
+        }
+    }
+}
+
+// Where a row's chunk of eight that would start at k0 starts: the last eight elements in place of a chunk that reaches past the
+// end.  With K % 8 == 4 the last one overlaps the one before it (the same codes are stored twice).
+__device__ __forceinline__ int chunk_start(int k0, int K) { return k0 + kVec <= K ? k0 : K - kVec; }
+
+// 16 bytes from a dword-aligned address, non-temporal
+__device__ __forceinline__ uint4 nt_load_dword_aligned(const void* p) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(4)));
+    const u4 v = __builtin_nontemporal_load(static_cast<const u4*>(p));
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// NT: non-temporal, for rows that one workgroup reads once
+template <int DT, bool NT = true>
+__device__ __forceinline__ void load_chunk(const typename Elem<DT>::storage* p, float (&v)[kVec]) {
+    if constexpr (DT == TPQ_DTYPE_F32) {
+        const uint4* const q = reinterpret_cast<const uint4*>(p);
+        const uint4 a = NT ? nt_load(q) : q[0], b = NT ? nt_load(q + 1) : q[1];
+        v[0] = __builtin_bit_cast(float, a.x); v[1] = __builtin_bit_cast(float, a.y);
+        v[2] = __builtin_bit_cast(float, a.z); v[3] = __builtin_bit_cast(float, a.w);
+        v[4] = __builtin_bit_cast(float, b.x); v[5] = __builtin_bit_cast(float, b.y);
+        v[6] = __builtin_bit_cast(float, b.z); v[7] = __builtin_bit_cast(float, b.w);
+    } else {
+        const uint4 raw = NT ? nt_load_dword_aligned(p) : *reinterpret_cast<const uint4*>(p);  // NT: rows of K % 8 == 4 start on 8 bytes
+        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[2 * i] = Elem<DT>::load(static_cast<uint16_t>(w[i] & 0xFFFFu));
+            v[2 * i + 1] = Elem<DT>::load(static_cast<uint16_t>(w[i] >> 16));
+        }
+    }
+}
+
+// the parameters of a quantizer: divisor 127, codes -127 .. 127 and its lower-bit relatives
+inline QParams row_quantizer(float eps, float divisor, int qmin, int qmax, int sign_mode) {
+    // |v| / scale <= divisor (1 + 2^-22) for every element of the row, whatever the rounding of scale and of the quotient
+    const float reach = rintf(divisor * (1.0f + 0x1p-20f));
+    const int no_clamp = divisor <= 127.0f && reach <= static_cast<float>(qmax) && -reach >= static_cast<float>(qmin);
+    return QParams{eps, divisor, qmin, qmax, sign_mode ? 1 : 0, no_clamp};
+}
+
+}  // namespace
+}  // namespace tpq

@@ -15,13 +15,12 @@
 // p10/src/backend/cpu/LowBitGemmKernels.cpp:19-52):
 //   absmax = max |float(x)|;  scale = fmaxf(absmax, eps) / divisor  (IEEE divide)
 //   code   = clamp(rintf(float(x) / scale), qmin, qmax)              (IEEE divide, RNE)
-#include "tpq_common.h"
+#include "quantize_row.h"
 
 namespace tpq {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kVec = 8;  // elements per lane per chunk
 // Rows up to this length: one wavefront (or a part of one) per row.  Longer rows on one wavefront were measured
 // (2048 x 4096 bfloat16: 7.0 us against 6.6 with four wavefronts per row, 8.9 against 7.1 from HBM; two wavefronts per
 // row: 8.3 against 7.9): a quarter of the wavefronts to launch, but too few loads in flight per compute unit.
@@ -44,105 +43,6 @@ __device__ unsigned long long g_quant_stamps[kStampRows * kStampSlots];
 #define TPQ_QUANT_STAMP(I) do { } while (0)
 #endif
 
-struct QParams {
-    float eps, divisor;
-    int qmin, qmax, sign_mode;
-    int no_clamp;  // no quotient |v| / scale, |v| <= absmax, can round outside [qmin, qmax]
-};
-
-__device__ __forceinline__ int quantize_one(float v, float scale, const QParams& p) {
-    if (p.sign_mode) return v >= 0.0f ? p.qmax : p.qmin;
-    // __fdiv_rn: correctly rounded division regardless of compiler flags
-    float q = rintf(__fdiv_rn(v, scale));
-    q = fminf(fmaxf(q, static_cast<float>(p.qmin)), static_cast<float>(p.qmax));
-    return static_cast<int>(q);
-}
-
-// Eight codes with one reciprocal instead of eight divisions, same bits as quantize_one.
-// q = v * (1/scale) is within 2^-21 relative of the true quotient, |quotient| <= 128 here, so its
-// absolute error is below 2^-14.  If q lies at least 2^-13 inside (c - 1/2, c + 1/2), so does the
-// correctly rounded quotient, and both round to c.  Otherwise (about one element in a few thousand;
-// also NaN and infinities) the element is redone with the IEEE division.
-// The codes leave as two packed words.  v_cvt_pk_u8_f32 converts a float to an unsigned byte (saturating at 0 and
-// 255) and drops it into one byte of a register: the rounded quotient c is an integer already, so c + 128 converts
-// exactly, the upper clamp is the saturation when qmax = 127, and one xor takes the 128 off the four bytes again.
-// Four instructions per code less than clamp, convert, mask, shift, or.
-__device__ __forceinline__ void quantize_eight_packed(const float (&v)[kVec], float scale, float inv_scale, const QParams& p,
-                                                      uint32_t& lo, uint32_t& hi) {
-    bool redo = false;
-    uint32_t word[2] = {0u, 0u};
-    const float qmin = static_cast<float>(p.qmin), qmax = static_cast<float>(p.qmax);
-#pragma unroll
-    for (int i = 0; i < kVec; ++i) {
-        const float q = v[i] * inv_scale;
-        const float c = rintf(q);
-        redo |= !(fabsf(q - c) <= 0.5f - 0x1p-13f);
-        const float biased = fminf(fmaxf(c, qmin), qmax) + 128.0f;  // 0 .. 255, an integer
-        word[i >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(biased, i & 3, word[i >> 2]);
-    }
-    lo = word[0] ^ 0x80808080u;
-    hi = word[1] ^ 0x80808080u;
-    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, with a statement the
-    // compiler may not move: left as a plain "if", the eight divisions were computed for every chunk and selected away.
-    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, and with the divisor
-    // passed through a statement the compiler may not move: as a plain "if", the eight divisions were hoisted above the
-    // branch, computed for every chunk and selected away.
-    if (__builtin_amdgcn_ballot_w64(redo) != 0) {
-        float divisor = scale;
-        asm volatile("; elements redone with the division" : "+v"(divisor));
-        if (redo) {
-            lo = hi = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                lo |= (static_cast<uint32_t>(quantize_one(v[i], divisor, p)) & 0xFFu) << (8 * i);
-                hi |= (static_cast<uint32_t>(quantize_one(v[i + 4], divisor, p)) & 0xFFu) << (8 * i);
-            }
-        }
-    }
-}
-
-// The same codes with fewer instructions, for parameters under which no quotient can leave the code range
-// (rint(divisor (1 + 2^-20)) <= qmax and >= -qmin, true for the usual divisor = qmax = -qmin = 127): no clamp is
-// needed, and the code is read off the mantissa.  t = fma(v, 1/scale, 1.5 * 2^23) rounds the exact product to the
-// nearest integer (ties to even) and leaves it in two's complement in the low mantissa bits; c = t - 1.5 * 2^23 is that
-// integer, r = fma(v, 1/scale, -c) its distance from the product.  The product is within 2^-16 of the correctly rounded
-// quotient the reference rounds, so |r| <= 1/2 - 2^-13 proves both round to c; anything else (also NaN) is redone with
-// the division.  Five instructions per code and three byte permutes per four codes.
-__device__ __forceinline__ void quantize_eight_lean(const float (&v)[kVec], float scale, float inv_scale, const QParams& p,
-                                                    uint32_t& lo, uint32_t& hi) {
-    constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
-    bool redo = false;
-    uint32_t t[kVec];
-#pragma unroll
-    for (int i = 0; i < kVec; ++i) {
-        const float tf = __builtin_fmaf(v[i], inv_scale, kMagic);
-        const float c = tf - kMagic;
-        const float r = __builtin_fmaf(v[i], inv_scale, -c);
-        redo |= !(fabsf(r) <= 0.5f - 0x1p-13f);
-        t[i] = __builtin_bit_cast(uint32_t, tf);
-    }
-    // v_perm_b32(a, b, sel): selector bytes 0..3 take bytes of b, 4..7 of a, 0x0c a zero byte
-    lo = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0400u) | __builtin_amdgcn_perm(t[3], t[2], 0x04000c0cu);
-    hi = __builtin_amdgcn_perm(t[5], t[4], 0x0c0c0400u) | __builtin_amdgcn_perm(t[7], t[6], 0x04000c0cu);
-    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, with a statement the
-    // compiler may not move: left as a plain "if", the eight divisions were computed for every chunk and selected away.
-    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, and with the divisor
-    // passed through a statement the compiler may not move: as a plain "if", the eight divisions were hoisted above the
-    // branch, computed for every chunk and selected away.
-    if (__builtin_amdgcn_ballot_w64(redo) != 0) {
-        float divisor = scale;
-        asm volatile("; elements redone with the division" : "+v"(divisor));
-        if (redo) {
-            lo = hi = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                lo |= (static_cast<uint32_t>(quantize_one(v[i], divisor, p)) & 0xFFu) << (8 * i);
-                hi |= (static_cast<uint32_t>(quantize_one(v[i + 4], divisor, p)) & 0xFFu) << (8 * i);
-            }
-        }
-    }
-}
-
 // Block-wide max over THREADS threads; every thread gets the result.
 template <int THREADS = kThreads>
 __device__ __forceinline__ float block_max(float v, float* smem) {
@@ -154,36 +54,6 @@ __device__ __forceinline__ float block_max(float v, float* smem) {
 #pragma unroll
     for (int w = 1; w < THREADS / kWave; ++w) r = fmaxf(r, smem[w]);
     return r;
-}
-
-// Where a row's chunk of eight that would start at k0 starts: the last eight elements in place of a chunk that reaches past the
-// end.  With K % 8 == 4 the last one overlaps the one before it (the same codes are stored twice).
-__device__ __forceinline__ int chunk_start(int k0, int K) { return k0 + kVec <= K ? k0 : K - kVec; }
-
-// 16 bytes from a dword-aligned address, non-temporal
-__device__ __forceinline__ uint4 nt_load_dword_aligned(const void* p) {
-    typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(4)));
-    const u4 v = __builtin_nontemporal_load(static_cast<const u4*>(p));
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-
-template <int DT>
-__device__ __forceinline__ void load_chunk(const typename Elem<DT>::storage* p, float (&v)[kVec]) {
-    if constexpr (DT == TPQ_DTYPE_F32) {
-        const uint4 a = nt_load(reinterpret_cast<const uint4*>(p)), b = nt_load(reinterpret_cast<const uint4*>(p) + 1);
-        v[0] = __builtin_bit_cast(float, a.x); v[1] = __builtin_bit_cast(float, a.y);
-        v[2] = __builtin_bit_cast(float, a.z); v[3] = __builtin_bit_cast(float, a.w);
-        v[4] = __builtin_bit_cast(float, b.x); v[5] = __builtin_bit_cast(float, b.y);
-        v[6] = __builtin_bit_cast(float, b.z); v[7] = __builtin_bit_cast(float, b.w);
-    } else {
-        const uint4 raw = nt_load_dword_aligned(p);  // rows of K % 8 == 4 start on 8 bytes
-        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[2 * i] = Elem<DT>::load(static_cast<uint16_t>(w[i] & 0xFFFFu));
-            v[2 * i + 1] = Elem<DT>::load(static_cast<uint16_t>(w[i] >> 16));
-        }
-    }
 }
 
 // eight codes to a dword-aligned address
@@ -225,30 +95,15 @@ __global__ __launch_bounds__(THREADS) void quantize_rows_cached(
     TPQ_QUANT_STAMP(2);
     absmax = block_max<THREADS>(absmax, smem);
     TPQ_QUANT_STAMP(3);
-    const float scale = __fdiv_rn(fmaxf(absmax, p.eps), p.divisor);
-    if (threadIdx.x == 0) scales[row] = scale;
-    // the shortcut needs |quotient| <= 128 and a finite reciprocal: true for every scale the formula
-    // above produces from finite inputs with divisor <= 128; anything else takes the divisions
-    const float inv_scale = __fdiv_rn(1.0f, scale);
-    const bool shortcut = !p.sign_mode && p.divisor <= 128.0f && inv_scale < 3.0e38f && absmax <= 3.0e38f;
-    const bool lean = shortcut && p.no_clamp;
+    const RowScale r = scale_of_row(absmax, p);
+    if (threadIdx.x == 0) scales[row] = r.scale;
 
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
         const int k0 = (c * THREADS + threadIdx.x) * kVec;
         if (k0 < K) {
-            uint32_t lo = 0, hi = 0;
-            if (lean) {
-                quantize_eight_lean(v[c], scale, inv_scale, p, lo, hi);
-            } else if (shortcut) {
-                quantize_eight_packed(v[c], scale, inv_scale, p, lo, hi);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    lo |= (static_cast<uint32_t>(quantize_one(v[c][i], scale, p)) & 0xFFu) << (8 * i);
-                    hi |= (static_cast<uint32_t>(quantize_one(v[c][i + 4], scale, p)) & 0xFFu) << (8 * i);
-                }
-            }
+            uint32_t lo, hi;
+            quantize_eight(v[c], r, p, lo, hi);
             store_codes(cr + chunk_start(k0, K), lo, hi);
         }
     }
@@ -288,28 +143,15 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_subwave(
     }
 #pragma unroll
     for (int off = LANES / 2; off >= 1; off >>= 1) absmax = fmaxf(absmax, __shfl_xor(absmax, off));
-    const float scale = __fdiv_rn(fmaxf(absmax, p.eps), p.divisor);
-    if (live && sub == 0) scales[row] = scale;
-    const float inv_scale = __fdiv_rn(1.0f, scale);
-    const bool shortcut = !p.sign_mode && p.divisor <= 128.0f && inv_scale < 3.0e38f && absmax <= 3.0e38f;  // as above
-    const bool lean = shortcut && p.no_clamp;
+    const RowScale r = scale_of_row(absmax, p);
+    if (live && sub == 0) scales[row] = r.scale;
 
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
         const int k0 = (c * LANES + sub) * kVec;
         if (live && k0 < K) {
-            uint32_t lo = 0, hi = 0;
-            if (lean) {
-                quantize_eight_lean(v[c], scale, inv_scale, p, lo, hi);
-            } else if (shortcut) {
-                quantize_eight_packed(v[c], scale, inv_scale, p, lo, hi);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    lo |= (static_cast<uint32_t>(quantize_one(v[c][i], scale, p)) & 0xFFu) << (8 * i);
-                    hi |= (static_cast<uint32_t>(quantize_one(v[c][i + 4], scale, p)) & 0xFFu) << (8 * i);
-                }
-            }
+            uint32_t lo, hi;
+            quantize_eight(v[c], r, p, lo, hi);
             store_codes(cr + chunk_start(k0, K), lo, hi);
         }
     }
@@ -396,10 +238,7 @@ TPQ_EXPORT int tpq_quantize_rowwise(const void* x, int x_dtype, int64_t M, int64
     if (M == 0 || K == 0) return TPQ_OK;
     TPQ_REQUIRE(x && codes && scales, TPQ_ERR_INVALID_VALUE, "quantize_rowwise: null pointer");
     TPQ_REQUIRE(M <= 0x7FFFFFFF, TPQ_ERR_INVALID_VALUE, "quantize_rowwise: more than 2^31-1 rows");
-    // |v| / scale <= divisor (1 + 2^-22) for every element of the row, whatever the rounding of scale and of the quotient
-    const float reach = rintf(divisor * (1.0f + 0x1p-20f));
-    const int no_clamp = divisor <= 127.0f && reach <= static_cast<float>(qmax) && -reach >= static_cast<float>(qmin);
-    const QParams p{eps, divisor, qmin, qmax, sign_mode ? 1 : 0, no_clamp};
+    const QParams p = row_quantizer(eps, divisor, qmin, qmax, sign_mode);
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (x_dtype) {
         case TPQ_DTYPE_F32: return launch<TPQ_DTYPE_F32>(x, M, K, p, codes, scales, s);

@@ -16,9 +16,14 @@
 //   * chunk t of the workgroup belongs to channel t / (K / 64): the lanes add their sums to the channel's word in LDS
 //     (ds_add_u32), the first rows_wg threads scale, round and store.
 // Exact int32 sums, the same as every other ternary kernel here.
+//
+// The row comes as int8 codes with a scale, or (XDT a float type) as the floats themselves, which every workgroup quantizes for
+// itself, sixteen to a thread, while its weights travel: K elements again in each workgroup, from L2, cost less than the quantizer's
+// launch and the trip of its codes through memory.  2560 -> 6912 and back, one row: TNEW.
 #pragma once
 
 #include "int8_gemm_kernel.h"
+#include "quantize_row.h"
 #include "ternary_decode_mfma.h"
 
 namespace tpq {
@@ -29,9 +34,11 @@ constexpr int kTernaryRowMaxThreads = 1024;
 __host__ __device__ constexpr int ternary_row_x_slots(int K) { return (K >> 4) + (K >> 8) + 1; }  // 16-byte slots of the parked activations
 
 // grid: ceil(N / rows_wg); block: 64 * ceil(rows_wg * K / 64 / 64) threads >= K / 16; LDS: 16 ternary_row_x_slots(K) + 4 rows_wg bytes
-template <class Epilogue>
-__global__ __launch_bounds__(kTernaryRowMaxThreads) void ternary_row_kernel(const int8_t* __restrict__ x, const uint8_t* __restrict__ packed, int N,
-                                                                           int K, int rows_wg, float inv_chunks_per_row, Epilogue ep) {
+// XDT: TPQ_DTYPE_* of the floats at x, or kTernaryRowCodes
+constexpr int kTernaryRowCodes = -1;
+template <class Epilogue, int XDT>
+__global__ __launch_bounds__(kTernaryRowMaxThreads) void ternary_row_kernel(const void* __restrict__ x, const uint8_t* __restrict__ packed, int N,
+                                                                           int K, int rows_wg, float inv_chunks_per_row, QParams quantizer, Epilogue ep) {
     // [K / 16 + K / 256]: slot 4 c + d + c / 4 holds the transposed piece d of chunk c (one slot of padding per four
     // chunks: the sixteen lanes a 16-byte read serves together, chunks c .. c + 15, then hit sixteen different groups of
     // four banks; without it chunks four apart met in the same banks and most of the kernel's LDS cycles were conflicts)
@@ -45,14 +52,42 @@ __global__ __launch_bounds__(kTernaryRowMaxThreads) void ternary_row_kernel(cons
     const int pieces = K >> 4;
 
     // requests in the order they are needed (loads come back in the order they were made): activations, weights, bias
-    const uint4 xr = reinterpret_cast<const uint4*>(x)[t < pieces ? t : 0];
+    constexpr bool kFloats = XDT != kTernaryRowCodes;
+    uint4 xr;
+    [[maybe_unused]] float xv[2][kVec];
+    if constexpr (kFloats) {
+        using S = typename Elem<XDT>::storage;
+        const S* const from = static_cast<const S*>(x) + (t < pieces ? t : 0) * 16;
+        load_chunk<XDT, false>(from, xv[0]);
+        load_chunk<XDT, false>(from + kVec, xv[1]);
+    } else {
+        xr = static_cast<const uint4*>(x)[t < pieces ? t : 0];
+    }
     const uint4 w = nt_load(reinterpret_cast<const uint4*>(packed + static_cast<size_t>(row0) * (static_cast<size_t>(K) >> 2)) + (live ? t : 0));
-    const float row_scale = ep.row_scale_of(0);
+    float row_scale = 0.0f;
+    if constexpr (!kFloats) row_scale = ep.row_scale_of(0);
     const int n = row0 + (t < rows_here ? t : 0);
     const bool with_bias = ep.out && ep.bias;
     const float bias_raw = *(with_bias ? ep.bias + n : reinterpret_cast<const float*>(x));  // no branch around a load: some readable word instead
 
     if (t < rows_wg) sums[t] = 0;
+    if constexpr (kFloats) {
+        __shared__ float most[kTernaryRowMaxThreads / kWave];
+        float absmax = 0.0f;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < kVec; ++e) absmax = fmaxf(absmax, fabsf(xv[h][e]));
+        absmax = wave_max(absmax);
+        if ((t & (kWave - 1)) == 0) most[t >> 6] = absmax;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        absmax = most[0];
+        for (int i = 1; i < static_cast<int>(blockDim.x) / kWave; ++i) absmax = fmaxf(absmax, most[i]);
+        const RowScale r = scale_of_row(absmax, quantizer);
+        row_scale = r.scale;
+        quantize_eight(xv[0], r, quantizer, xr.x, xr.y);
+        quantize_eight(xv[1], r, quantizer, xr.z, xr.w);
+    }
     if (t < pieces) {
         const v4i f = transpose_4x4_bytes(xr);
         const int c = t >> 2, d = t & 3;
@@ -117,14 +152,14 @@ inline int ternary_row_rows_per_workgroup(int64_t M, int64_t N, int64_t K, int c
     return static_cast<int>(most);
 }
 
-template <class Epilogue>
-int launch_ternary_row(const int8_t* x, const uint8_t* packed, int64_t N, int64_t K, int rows_wg, Epilogue ep, hipStream_t s) {
+template <int XDT = kTernaryRowCodes, class Epilogue>
+int launch_ternary_row(const void* x, const uint8_t* packed, int64_t N, int64_t K, int rows_wg, Epilogue ep, hipStream_t s, const QParams& quantizer = {}) {
     const int64_t cpr = K / 64, threads = (rows_wg * cpr + 63) / 64 * 64;
     TPQ_REQUIRE(K % 64 == 0 && K <= kTernaryRowMaxK && rows_wg >= 4 && threads <= kTernaryRowMaxThreads && threads >= K / 16 && threads >= rows_wg,
                 TPQ_ERR_INVALID_VALUE, "ternary row kernel: workgroup shape");
     const size_t smem = 16 * static_cast<size_t>(ternary_row_x_slots(static_cast<int>(K))) + 4 * static_cast<size_t>(rows_wg);
-    ternary_row_kernel<Epilogue><<<static_cast<unsigned>((N + rows_wg - 1) / rows_wg), static_cast<unsigned>(threads), smem, s>>>(
-        x, packed, static_cast<int>(N), static_cast<int>(K), rows_wg, 1.0f / static_cast<float>(cpr), ep);
+    ternary_row_kernel<Epilogue, XDT><<<static_cast<unsigned>((N + rows_wg - 1) / rows_wg), static_cast<unsigned>(threads), smem, s>>>(
+        x, packed, static_cast<int>(N), static_cast<int>(K), rows_wg, 1.0f / static_cast<float>(cpr), quantizer, ep);
     return check_launch("tpq_ternary_mm (one row)");
 }
 

@@ -175,3 +175,36 @@ def test_ternary_expanded(ops, M, K, N):
         want, _ = oracle.ternary_mm(x, rs, packed, 0.03, K, bias=bias, out_dtype=name)
         got = ops.ternary_mm(dev(x), dev(rs), dev(packed), 0.03, K, bias=dev(bias), out_dtype=TORCH_DT[name])
         np.testing.assert_array_equal(host(got), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("k,n", [(64, 1), (64, 300), (1088, 72), (2560, 2561), (6912, 260), (8192, 36), (4160, 5)])
+def test_one_row_quantized_in_the_product(dtype, k, n):
+    """tpq_ternary_linear_row: the bits of the row quantizer followed by the product, for ordinary rows and for ones whose maximum
+    is below eps, infinite, NaN or in the last element."""
+    from tensorplay_amd import _lib, ops
+
+    gen = torch.Generator(device="cuda").manual_seed(k + n)
+    packed = ops.pack_ternary(torch.randint(-1, 2, (n, k), device="cuda", generator=gen, dtype=torch.int8))
+    bias = torch.randn(n, device="cuda", generator=gen)
+    lib = _lib.load()
+    for case in range(6):
+        x = torch.randn(1, k, device="cuda", generator=gen)
+        if case == 1:
+            x *= 0.0
+        if case == 2:
+            x[0, k // 2] = float("inf")
+        if case == 3:
+            x[0, 0] = float("nan")
+        if case == 4:
+            x[0, k - 1] = -300.0
+        if case == 5:
+            x *= 1e-7
+        x = x.to(dtype)
+        codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
+        for b in (None, bias):
+            want = ops.ternary_mm(codes, scale, packed, 0.037, k, bias=b)
+            got = torch.empty(1, n, device="cuda")
+            ops._check(lib.tpq_ternary_linear_row(x.data_ptr(), ops._DT[dtype], packed.data_ptr(), 0.037, ops._ptr(b), n, k, 1e-5, got.data_ptr(),
+                                                  ops._stream(x)))
+            assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (case, b is not None)
