@@ -8,7 +8,7 @@
 // product) to 30 us (row quantizer + int8 product) of host time a call, so the card waited.
 // Measured (us a pass with the modules' own Python, host time, before / with this): int8 dynamic linear 30.6 / 10.0, int4 at one
 // row 21.2 / 6.6, int4 with bias at 48 rows 27.5 / 12.4, 2-bit linear 20.2 / 6.3, ternary MLP (two linears and a relu) 59.9 / 21.7,
-// affine quantize + dequantize 28.3 / 9.4.  Above 16 rows only the routes that the library picks itself are taken here: from there
+// affine quantize + dequantize 28.3 / 9.4.  Above 32 rows only the routes that the library picks itself are taken here: from there
 // on the kernels are longer than either form.
 #include <Python.h>
 
@@ -311,7 +311,7 @@ TPQ_CALL(ternary_linear, 6)
 TPQ_CALL_END
 
 // int4_mm(x [..., K], packed int32 [N / 8, K / 32, 32, 1], group, scales_and_zeros [K / group, N, 2] of x's type, bias or None,
-// workspaces): the rows kernel, which adds the bias as a separate add would, and, up to 16 rows, the decode kernels and an add.  workspaces: {(device, stream): zero-filled buffer} of
+// workspaces): the rows kernel, which adds the bias as a separate add would, and, up to 32 rows, the decode kernels and an add.  workspaces: {(device, stream): zero-filled buffer} of
 // ops._int4_workspace; a stream that has none yet, or too small a one, gets it in the Python form.
 TPQ_CALL(int4_mm, 6)
     const at::Tensor *x = plain(args[0]), *packed = plain(args[1]), *sz = plain(args[3]), *bias;
@@ -328,7 +328,7 @@ TPQ_CALL(int4_mm, 6)
     int64_t M;
     const auto sizes = product_sizes(*x, N, &M);
     const bool rows = lib.tpq_int4_mm_rows_takes(x->const_data_ptr(), tag, M, N, K, group, ptr<int32_t>(packed), sz->const_data_ptr()) != 0;
-    if (!rows && M > (tag == TPQ_DTYPE_F32 ? 1 : 16)) Py_RETURN_NONE;
+    if (!rows && M > (tag == TPQ_DTYPE_F32 ? 1 : 32)) Py_RETURN_NONE;
     const at::Tensor* workspace = nullptr;
     int64_t workspace_bytes = 0;
     if (rows) {
@@ -371,7 +371,7 @@ TPQ_CALL(int4_mm, 6)
 TPQ_CALL_END
 
 // lowbit_mm(x [..., K], packed uint8 [N, ceil(K / per_byte)], bits, K, scales_and_zeros float32 [groups, N, 2], bias or None, lsb_first):
-// the rows kernel and, up to 16 rows, the decode kernels
+// the rows kernel and, up to 32 rows, the decode kernels
 TPQ_CALL(lowbit_mm, 7)
     const at::Tensor *x = plain(args[0]), *packed = plain(args[1]), *sz = plain(args[4]), *bias;
     int64_t bits, K;
@@ -385,7 +385,7 @@ TPQ_CALL(lowbit_mm, 7)
     const auto sizes = product_sizes(*x, N, &M);
     if (tag < 0 || packed->size(1) != (K + per_byte - 1) / per_byte || !optional_vector(args[5], at::kFloat, N, *x, &bias)) Py_RETURN_NONE;
     const bool rows = lib.tpq_lowbit_mm_rows_takes(x->const_data_ptr(), tag, M, N, K, static_cast<int>(bits), lsb_first, group, ptr<uint8_t>(packed), ptr<float>(sz)) != 0;
-    if (!rows && M > 16) Py_RETURN_NONE;
+    if (!rows && M > 32) Py_RETURN_NONE;
     at::Tensor out;
     int status;
     {

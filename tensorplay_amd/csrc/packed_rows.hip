@@ -1,4 +1,5 @@
 // Entry points of the packed-weight products for a block of activation rows (packed_rows_kernel.h).
+#include "int4_gemm_kernel.h"
 #include "packed_rows_bits.h"
 
 namespace tpq {
@@ -22,15 +23,24 @@ int64_t rows_limit(int64_t N, int64_t K, int dtype) {
     return N * K <= (int64_t{1} << 24) ? 768 : N * K <= (int64_t{1} << 26) ? 512 : 384;
 }
 
+// Where the kernels that take any K or (groups of 128) the decode kernels on the matrix cores ran: they keep the weight in float32
+// or apply the scales to sums of whole codes.  With groups of 32 and 64 the latter dequantize to 16 bits, as the tiled kernel and
+// the dense route above those rows do.
+bool int4_weights_unrounded(int dtype, int64_t M, int64_t N, int64_t K, int64_t group) {
+    if (dtype == TPQ_DTYPE_F32) return false;
+    if (K % 128) return dtype == TPQ_DTYPE_F16 || M <= 112 || N >= 16384;
+    return group == 128 && !int4_gemm_takes(M, N, K, ~size_t{0});
+}
+
 }  // namespace
 }  // namespace tpq
 
 using namespace tpq;
 
-// Lower limit, measured (us, this kernel / decode kernels): groups of 128, 24 rows: 4096 -> 16384 12.1 / 15.7, 14336 -> 4096
-// 13.6 / 18.2, 4096 -> 11008 11.5 / 11.8, but 4096 x 4096 8.7 / 8.0, and 33 rows there 9.8 / 12.5; groups of 64, 17 rows:
-// 11008 -> 4096 12.0 / 23.1, 16 rows 11.3 / 12.0.  K % 128 != 0 (slabs of four rows): 4768 -> 13544 at 1 / 3 / 33 rows 14.5 / 39,
-// 14.5 / 94, 24 / 871.  float32: 4096 -> 11008 at 1, 2, 64 rows 24.4 / 24.2, 24.7 / 45, 68 / 110; 2048 x 2048 at 1 and 2 rows
+// Lower limit, measured (us, this kernel / decode kernels): groups of 128 (weights unrounded): 24 rows of 4096 -> 16384 17.5 / 15.4,
+// 33 of 4096 x 4096 10.8 / 15.1, 48 of 4096 -> 11008 18.5 / 20.2; groups of 64, 17 rows:
+// 11008 -> 4096 12.0 / 23.1, 16 rows 11.3 / 12.0.  K % 128 != 0 (slabs of four rows): 4768 -> 13544 at 3 / 33 rows 19.4 /
+// 92, 31 / 868.  float32: 4096 -> 11008 at 1, 2, 64 rows 24.4 / 24.2, 24.7 / 45, 68 / 110; 2048 x 2048 at 1 and 2 rows
 // 8.1 / 7.2, 8.2 / 7.4.  bfloat16 stops at 256 rows: beyond, results are held to within 1e-2, element by element, of the
 // reference's device formulation, whose dense weight is rounded to bfloat16 twice; a weight rounded once misses that on
 // single elements (it is the one that lies closer to the exact product).
@@ -42,13 +52,14 @@ TPQ_EXPORT int tpq_int4_mm_rows_takes(const void* x, int dtype, int64_t M, int64
     if (dtype == TPQ_DTYPE_BF16 && M > 256) return 0;
     if (dtype == TPQ_DTYPE_F32) return M >= 2 || (N * K >= (1 << 24) && K > 4096);
     if (K % 128) return 1;
-    return M >= 33 || (M >= 17 && (group < 128 || N * K >= (1 << 25)));
+    return M >= (group < 128 ? 17 : 33);
 }
 
-// Lower limit, measured (us, this kernel / what ran below): bfloat16 and float16, groups of 128 (where the decode kernels are
-// at home), 4096 -> 11008, 2 bits: 16 / 32 / 56 rows 11.7 / 11.2, 13.7 / 21.4, 16.7 / 41.8; other groups, 4096 x 4096 in groups of
-// 32, 2 bits: 1 / 16 / 80 rows 8.0 / 26, 8.3 / 45, 12.5 / 168; one row of 4 bits stays with the row kernel (8.6 / 6.1).  float32
-// 4096 -> 11008: 1 / 8 / 64 rows 27 / 35, 26 / 57, 70 / 112.  8 bits are twice the bytes: 4096 -> 11008 at 300 rows 74 / 85, at
+// Lower limit, measured (us, this kernel with unrounded weights / what ran below): groups of 128, where the decode kernels are at
+// home: 4096 x 4096 at 19 rows, 1 / 2 / 4 / 8 bits 10.7 / 10.0, 10.8 / 10.5, 11.4 / 11.9, 13.1 / 16.9; 4096 -> 11008, 2 bits, 24 / 32 /
+// 40 rows 21.7 / 20.6, 21.6 / 21.5, 20 / 31; 1024 -> 512 at 18 rows 7.3 / 6.0.  Other groups, 4096 x 4096 in groups of 32, 2 bits:
+// 1 / 16 / 80 rows 10.1 / 25, 10.4 / 46, 17.6 / 175; one row of 4 bits stays with the row kernel (8.6 / 6.1).  float32
+// 4096 -> 11008: 1 / 8 / 64 rows 33 / 35, 33 / 57, 84 / 99.  8 bits are twice the bytes: 4096 -> 11008 at 300 rows 74 / 85, at
 // 512 111 / 83; 4096 x 4096 at 512 33 / 42.
 TPQ_EXPORT int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int bits, int lsb_first, int64_t group,
                                         const uint8_t* packed, const float* scales_and_zeros) {
@@ -69,7 +80,7 @@ TPQ_EXPORT int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int
         const bool row_kernel = K % chunk == 0 && group % chunk == 0 && K <= (bits == 8 ? 32768 : 65536) && (bits != 8 || dtype == TPQ_DTYPE_F16);
         return !(at_home || row_kernel);
     }
-    return M >= 17 || !at_home;
+    return M >= (bits == 8 ? 17 : 33) || !at_home;
 }
 
 TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
@@ -96,7 +107,7 @@ TPQ_EXPORT int tpq_int4_mm_rows_bias(const void* x, int dtype, int64_t M, int64_
     TPQ_REQUIRE(aligned(x, 16) && aligned(packed, 16) && aligned(scales_and_zeros, wide ? 8 : 4) && aligned(out, wide ? 16 : 8) && aligned(bias, wide ? 4 : 2), TPQ_ERR_UNSUPPORTED,
                 "int4_mm_rows: unaligned operand");
     const bool room = workspace != nullptr && aligned(workspace, 16);
-    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, room ? workspace_bytes / 4 : 0);
+    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, room ? workspace_bytes / 4 : 0, int4_weights_unrounded(dtype, M, N, K, group));
     PackedRowsArgs a{};
     a.x = x; a.w = packed; a.sz = scales_and_zeros; a.y = out; a.after = bias; a.partial = static_cast<float*>(workspace);
     a.M = static_cast<int>(M); a.N = static_cast<int>(N); a.K = static_cast<int>(K); a.tiles_per_group = static_cast<int>(group / 32);

@@ -23,7 +23,10 @@ namespace {
 
 template <int DT>
 int run_packed_rows_bits(const PackedRowsBits& c) {
-    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats);
+    // up to these rows the decode kernels ran, which apply the scales to sums of whole codes: no weight is rounded to 16 bits; above, the
+    // dense route's 16-bit weight
+    const bool split = c.M <= (c.N * c.K <= (int64_t{1} << 24) ? 80 : 56);
+    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats, split);
     PackedRowsArgs a{};
     a.x = c.x; a.w = c.packed; a.sz = c.sz; a.bias = c.bias; a.y = c.out; a.partial = static_cast<float*>(c.workspace);
     a.M = static_cast<int>(c.M); a.N = static_cast<int>(c.N); a.K = static_cast<int>(c.K); a.tiles_per_group = static_cast<int>(c.group / 32);

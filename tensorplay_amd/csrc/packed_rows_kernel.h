@@ -23,12 +23,18 @@
 //     and one v_fma_mix per code applies scale and zero point in fp32, rounded once to the operand type (float16: the mix
 //     instruction's own rounding; bfloat16: v_cvt_pk_bf16_f32; float32: no rounding).  They are the A operand of
 //     v_mfma_f32_16x16x32_{f16,bf16} (float32: v_mfma_f32_16x16x4_f32), the activations as they lie in memory the B operand;
+//   * where the kernels for fewer rows keep the weight in float32 (scales applied to sums), a 16-bit weight is not rounded here
+//     either: SPLIT, the rounding's remainder goes through the matrix cores as a second operand.  The groups of 32 lie across a
+//     lane group's k range, so scales cannot be applied to sums instead;
+//   * float32 sums are formed over 16 k, these added up over a step and the steps over the slice: in one chain over the slice
+//     the roundings of the long sum weigh twice as much as all others together (error against float64 with 8 bits, 4096 x 4096 at
+//     19 rows: one chain 3.3e-7, so 1.3e-7; the one-row kernels 1.9e-7);
 //   * the KW partial sums of a tile meet in LDS at the end.
 // Measured (us, weights from HBM, this kernel / what ran before): int4, bfloat16, 11008 -> 4096 in groups of 64: 24 / 48 / 128 / 256
-// rows 12.4 / 22.8, 14.8 / 39, 24 / 43, 36 / 71; 4096 x 4096 in groups of 128: 33 / 64 / 256 rows 9.8 / 12.5, 11.2 / 20, 15.8 / 34;
-// 4768 -> 13544 in groups of 32 (K % 128 != 0): 3 / 33 rows 14.5 / 94, 24 / 871.  float32 4096 x 4096: 3 / 19 / 64 rows 11.7 / 21, 16 / 39,
-// 25 / 44 (bound by its MFMAs, 32 clocks for 16 x 16 x 4).  2 bits, bfloat16: 4096 -> 11008 at 32 / 56 / 203 rows 13.7 / 21, 16.7 / 42,
-// 52 / 68; 4096 x 4096 in groups of 32: 1 / 16 / 80 rows 8.0 / 26, 8.3 / 45, 12.5 / 168.
+// rows 12.4 / 22.8, 14.8 / 39, 24 / 43, 36 / 71; 4096 x 4096 in groups of 128: 33 rows (SPLIT) 10.8 / 12.5, 64 / 256 rows 11.2 / 20, 15.8 / 34;
+// 4768 -> 13544 in groups of 32 (K % 128 != 0): 3 / 33 rows (SPLIT) 19.4 / 92, 31 / 868.  float32 4096 x 4096: 3 / 19 / 64 rows 12.4 / 22, 18 / 38,
+// 29 / 47 (bound by its MFMAs, 32 clocks for 16 x 16 x 4).  2 bits: 4096 -> 11008 at 203 rows 50 /
+// 67, (SPLIT) at 40 rows 20 / 31; 4096 x 4096 in groups of 32 (SPLIT): 1 / 16 / 80 rows 10.1 / 25, 10.4 / 46, 17.6 / 175.
 // Rows >= M repeat row M - 1, steps of k behind the end of the slice are loaded (from the last step) and not multiplied, the
 // chunks of a last partial step behind K are cleared in LDS.
 #pragma once
@@ -213,7 +219,7 @@ __device__ __forceinline__ void store_rows_result(const float4_t& s, typename El
     else *reinterpret_cast<uint2*>(y) = make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16));
 }
 
-template <int DT, class Source, int MB, int CW, bool EDGE>
+template <int DT, class Source, int MB, int CW, bool EDGE, bool SPLIT>
 __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedRowsArgs a) {
     using A = RowsArith<DT>;
     using P = RowsParams<DT, Source::kTypedParams>;
@@ -222,6 +228,7 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     constexpr int kRoundLoads = KW * kRows * kStepBytes / 1024, kMine = kRoundLoads / kRowsProducers;  // 1 KB loads of a round, a requesting wavefront's
     constexpr int kLoadsPerStep = kRows * kStepBytes / 1024, kRowsPerLoad = 64 / A::kChunks;
     constexpr int kBuffer = kRoundLoads * 1024;
+    static_assert(!SPLIT || DT != TPQ_DTYPE_F32, "float32 weights are not rounded");
     static_assert(kRoundLoads % kRowsProducers == 0, "every wavefront loads the same number of pieces");
     extern __shared__ uint4 pr_lds[];  // [2][KW][kRows][kStepBytes], later the partial sums [CW][NB][MB][KW][64 lanes]
     char* const lds = reinterpret_cast<char*>(pr_lds);
@@ -332,11 +339,15 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     // pair p of a block's codes, dequantized
     auto weight_pair = [&](const Loaded& d, int b, int p, float scale, float zero, float& lo, float& hi) __attribute__((always_inline)) {
         half2_t h = __builtin_bit_cast(half2_t, Source::pair(d.w[b], p, magic));
-        if constexpr (DT == TPQ_DTYPE_F32) {  // the offset leaves exactly, in fp16
+        if constexpr (DT == TPQ_DTYPE_F32 || SPLIT) {  // the offset leaves exactly, in fp16
             h = h - half2_t{static_cast<_Float16>(Source::offset(p, 0)), static_cast<_Float16>(Source::offset(p, 1))};
-            const float z = Source::kTypedParams ? zero : -zero * scale;
-            lo = __builtin_fmaf(static_cast<float>(h.x), scale, z);
-            hi = __builtin_fmaf(static_cast<float>(h.y), scale, z);
+            if constexpr (Source::kTypedParams) {
+                lo = __builtin_fmaf(static_cast<float>(h.x), scale, zero);
+                hi = __builtin_fmaf(static_cast<float>(h.y), scale, zero);
+            } else {  // zero points are whole numbers as a rule: one rounding
+                lo = (static_cast<float>(h.x) - zero) * scale;
+                hi = (static_cast<float>(h.y) - zero) * scale;
+            }
         } else {  // the offset folded into the constant: an error of 2^-24 x 1032 scale at most, below the operand type's rounding
             const float z_lo = Source::kTypedParams ? zero - Source::offset(p, 0) * scale : -(zero + Source::offset(p, 0)) * scale;
             const float z_hi = Source::kTypedParams ? zero - Source::offset(p, 1) * scale : -(zero + Source::offset(p, 1)) * scale;
@@ -348,6 +359,7 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     // 16-bit values, four floats) per block
     constexpr int kChunkPairs = DT == TPQ_DTYPE_F32 ? 2 : 4;
     uint32_t wq[2][NB][4];
+    uint32_t wr[SPLIT ? 2 : 1][NB][4];  // SPLIT: what their rounding left
     // pairs [first, last) of the NB kChunkPairs pairs of chunk u
     auto dequantize = [&](const Loaded& d, auto u_c, auto first, auto last) __attribute__((always_inline)) {
         constexpr int U = decltype(u_c)::value;
@@ -360,7 +372,10 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
                 wq[U & 1][b][2 * p] = __builtin_bit_cast(uint32_t, lo);
                 wq[U & 1][b][2 * p + 1] = __builtin_bit_cast(uint32_t, hi);
             } else {
-                wq[U & 1][b][p] = A::pack(lo, hi);
+                const uint32_t rounded = A::pack(lo, hi);
+                wq[U & 1][b][p] = rounded;
+                if constexpr (SPLIT)
+                    wr[U & 1][b][p] = A::pack(lo - Elem<DT>::load(static_cast<uint16_t>(rounded & 0xFFFFu)), hi - Elem<DT>::load(static_cast<uint16_t>(rounded >> 16)));
             }
         }
     };
@@ -372,6 +387,10 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
             for (int e = 0; e < 4; ++e) {
                 uint32_t& v = wq[decltype(u_c)::value & 1][b][e];
                 asm volatile("" : "+v"(v));
+                if constexpr (SPLIT) {
+                    uint32_t& rest = wr[decltype(u_c)::value & 1][b][e];
+                    asm volatile("" : "+v"(rest));
+                }
             }
     };
 
@@ -390,6 +409,22 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
         if constexpr (C < kPieces)
             frag[C % kFragments] = *reinterpret_cast<const pr_word4*>(frag_base + buffer * kBuffer + (C % MB) * (16 * kStepBytes) + (((kU * q + C / MB)) ^ i) * 16);
     };
+    // float32: a piece's own sum, added to its step's while the next piece multiplies
+    float4_t piece[DT == TPQ_DTYPE_F32 ? 2 : 1][NB], step_sum[NB][DT == TPQ_DTYPE_F32 ? MB : 1];
+    auto add_piece = [&](auto c) __attribute__((always_inline)) {
+        if constexpr (DT == TPQ_DTYPE_F32) {
+            constexpr int C = decltype(c)::value, U = C / MB, r = C % MB;
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float more = piece[C & 1][b][e];
+                    if constexpr (U == 0) step_sum[b][r][e] = more;
+                    else if constexpr (U + 1 < kU) step_sum[b][r][e] += more;
+                    else acc[b][r][e] += step_sum[b][r][e] + more;
+                }
+        }
+    };
     auto multiply_piece = [&](auto c) __attribute__((always_inline)) {
         constexpr int C = decltype(c)::value, U = C / MB, r = C % MB;
         if constexpr (DT == TPQ_DTYPE_F32) {
@@ -397,8 +432,17 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int b = 0; b < NB; ++b) acc[b][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, wq[U & 1][b][t]), f[t], acc[b][r], 0, 0, 0);
+                for (int b = 0; b < NB; ++b)
+                    piece[C & 1][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, wq[U & 1][b][t]), f[t],
+                                                                           t == 0 ? float4_t{0.0f, 0.0f, 0.0f, 0.0f} : piece[C & 1][b], 0, 0, 0);
+            if constexpr (C > 0) add_piece(std::integral_constant<int, C - 1>{});
+            if constexpr (C == kPieces - 1) add_piece(c);
         } else {
+            if constexpr (SPLIT) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[b][r] = A::mfma(pr_word4{wr[U & 1][b][0], wr[U & 1][b][1], wr[U & 1][b][2], wr[U & 1][b][3]}, frag[C % kFragments], acc[b][r]);
+            }
 #pragma unroll
             for (int b = 0; b < NB; ++b)
                 acc[b][r] = A::mfma(pr_word4{wq[U & 1][b][0], wq[U & 1][b][1], wq[U & 1][b][2], wq[U & 1][b][3]}, frag[C % kFragments], acc[b][r]);
@@ -509,14 +553,16 @@ struct PackedRowsPlan {
     int mb;        // blocks of 16 rows per workgroup: 1 .. 4 (float32: 1, 2)
     int cw;        // channel positions: 2 (64 channels per workgroup) or 4 (128; three or four blocks of rows and K % 128 == 0 only)
     int slices, steps_per_slice;
+    bool split;    // the weights' remainders multiplied too (64 channels per workgroup)
 };
 
 // Tile height, channels per workgroup and slices of K by an estimate (us) fitted to a sweep of 1 .. 8 slices and both widths
 // over six shapes and 16 .. 256 rows: 4 for the launch, the first loads and the epilogue, per round what the comment on the
 // kernel says, per round of workgroups over the compute units, and 2 + the bytes of the slices' sums (written and read) at
 // 4 TB/s for the second kernel.  Within 5 % of the sweep's best nearly everywhere (11008 -> 4096 at 128 rows 24.8, best 22.7).
-inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, int units = 256) {
+inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, bool split = false, int units = 256) {
     PackedRowsPlan p;
+    p.split = split && dtype != TPQ_DTYPE_F32;
     const bool wide = dtype == TPQ_DTYPE_F32;
     const int64_t blocks = (M + 15) / 16;
     const int64_t most = wide ? 2 : 4, row_tiles = (blocks + most - 1) / most;
@@ -525,7 +571,7 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
     int64_t best = 1;
     double best_us = 1e30;
     p.cw = 2;
-    for (int cw = 2; cw <= (p.mb >= 3 && K % 128 == 0 ? 4 : 2); cw += 2) {
+    for (int cw = 2; cw <= (p.mb >= 3 && K % 128 == 0 && !p.split ? 4 : 2); cw += 2) {
         const int kw = 8 / cw;
         const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
         for (int64_t z = 1; z <= 16 && z <= steps; ++z) {
@@ -545,13 +591,13 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
     return p;
 }
 
-template <int DT, class Source, int MB, int CW, bool EDGE>
+template <int DT, class Source, int MB, int CW, bool EDGE, bool SPLIT>
 int launch_packed_rows_shape(const PackedRowsArgs& a, int slices, hipStream_t s) {
     constexpr int KW = 8 / CW, NB = kRowsNB;
     constexpr size_t stage = 2 * static_cast<size_t>(KW) * 16 * MB * RowsArith<DT>::kChunks * 16, sums = static_cast<size_t>(8) * NB * MB * 1024;
     constexpr size_t smem = stage > sums ? stage : sums;
     static_assert(smem <= 160 * 1024, "LDS of one compute unit");
-    auto kernel = packed_rows_kernel<DT, Source, MB, CW, EDGE>;
+    auto kernel = packed_rows_kernel<DT, Source, MB, CW, EDGE, SPLIT>;
     static std::atomic<uint64_t> configured{0};
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), smem, configured, "packed rows")) return rc;
     const dim3 grid(static_cast<unsigned>((a.N + 16 * NB * CW - 1) / (16 * NB * CW)), static_cast<unsigned>((a.M + 16 * MB - 1) / (16 * MB)), static_cast<unsigned>(slices));
@@ -560,11 +606,15 @@ int launch_packed_rows_shape(const PackedRowsArgs& a, int slices, hipStream_t s)
 }
 
 template <int DT, class Source, int MB, int CW>
-int launch_packed_rows_as(const PackedRowsArgs& a, int slices, hipStream_t s) {
+int launch_packed_rows_as(const PackedRowsArgs& a, const PackedRowsPlan& p, hipStream_t s) {
     if constexpr (CW == 2) {
-        if (a.K % 128 != 0) return launch_packed_rows_shape<DT, Source, MB, CW, true>(a, slices, s);
+        if constexpr (DT != TPQ_DTYPE_F32) {
+            if (p.split) return a.K % 128 != 0 ? launch_packed_rows_shape<DT, Source, MB, CW, true, true>(a, p.slices, s)
+                                               : launch_packed_rows_shape<DT, Source, MB, CW, false, true>(a, p.slices, s);
+        }
+        if (a.K % 128 != 0) return launch_packed_rows_shape<DT, Source, MB, CW, true, false>(a, p.slices, s);
     }
-    return launch_packed_rows_shape<DT, Source, MB, CW, false>(a, slices, s);
+    return launch_packed_rows_shape<DT, Source, MB, CW, false, false>(a, p.slices, s);
 }
 
 template <int DT, class Source>
@@ -574,12 +624,12 @@ int launch_packed_rows(PackedRowsArgs a, const PackedRowsPlan& p, hipStream_t s)
     if (p.slices == 1) a.partial = nullptr;
     int rc;
     const bool wide = p.cw == 4;
-    if (p.mb == 1) rc = launch_packed_rows_as<DT, Source, 1, 2>(a, p.slices, s);
-    else if (p.mb == 2) rc = launch_packed_rows_as<DT, Source, 2, 2>(a, p.slices, s);
+    if (p.mb == 1) rc = launch_packed_rows_as<DT, Source, 1, 2>(a, p, s);
+    else if (p.mb == 2) rc = launch_packed_rows_as<DT, Source, 2, 2>(a, p, s);
     else {
         if constexpr (DT == TPQ_DTYPE_F32) rc = fail(TPQ_ERR_RUNTIME, "packed rows: no such tile");
-        else if (p.mb == 3) rc = wide ? launch_packed_rows_as<DT, Source, 3, 4>(a, p.slices, s) : launch_packed_rows_as<DT, Source, 3, 2>(a, p.slices, s);
-        else rc = wide ? launch_packed_rows_as<DT, Source, 4, 4>(a, p.slices, s) : launch_packed_rows_as<DT, Source, 4, 2>(a, p.slices, s);
+        else if (p.mb == 3) rc = wide ? launch_packed_rows_as<DT, Source, 3, 4>(a, p, s) : launch_packed_rows_as<DT, Source, 3, 2>(a, p, s);
+        else rc = wide ? launch_packed_rows_as<DT, Source, 4, 4>(a, p, s) : launch_packed_rows_as<DT, Source, 4, 2>(a, p, s);
     }
     if (rc != TPQ_OK || a.partial == nullptr) return rc;
     const int64_t quads = static_cast<int64_t>(a.M) * a.N / 4;

@@ -76,3 +76,50 @@ def test_lowbit_rows(dtype, bits, lsb_first, M, N, K, group):
                                       bias.data_ptr(), out.data_ptr(), ws.data_ptr(), need, ops._stream(x)))
     # the zero point and the code meet after their products with the scale: |zero| scale on top of |w|
     _check(out, x, w, bias, 0.011 * (1 + (1 << bits) / 8), dtype)
+
+
+def _fragment(kind, M, N, K, group, bits, dtype):
+    """(result, exact float64 result) on weights whose (scale, zero) have no short form in 16 bits."""
+    from tensorplay_amd import ops
+
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K + bits)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(dtype)
+    sz = torch.rand(K // group, N, 2, device=DEV, generator=gen) * 0.01 + 0.001
+    if kind == "int4":
+        codes = torch.randint(0, 16, (N, K), dtype=torch.int32, device=DEV, generator=gen)
+        packed, sz = ops._convert_weight_to_int4pack(codes, 2), sz.to(dtype)
+        w = (codes.double() - 8).view(N, -1, group) * sz[..., 0].double().t()[..., None] + sz[..., 1].double().t()[..., None]
+        got = ops._weight_int4pack_mm(x, packed, group, sz)
+    else:
+        sz[..., 1] *= 100
+        per_byte = 8 // bits
+        packed = torch.randint(0, 256, (N, K // per_byte), dtype=torch.uint8, device=DEV, generator=gen)
+        shifts = torch.arange(8 - bits, -1, -bits, device=DEV)
+        codes = ((packed.int()[..., None] >> shifts) & ((1 << bits) - 1)).reshape(N, K)
+        if bits == 8:
+            codes = codes.to(torch.int8)
+        w = (codes.double().view(N, -1, group) - sz[..., 1].double().t()[..., None]) * sz[..., 0].double().t()[..., None]
+        got = ops._lowbit_mm(x, packed, bits, K, sz)
+    return got, x.double().cpu() @ w.view(N, K).cpu().t().contiguous()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind,M,N,K,group,bits", [("int4", 3, 72, 544, 32, 4), ("int4", 33, 520, 608, 32, 4), ("int4", 48, 11008, 1024, 128, 4),
+                                                   ("intx", 5, 72, 544, 32, 2), ("intx", 33, 264, 1024, 128, 1), ("intx", 40, 200, 4032, 64, 4),
+                                                   ("intx", 49, 520, 1024, 128, 8), ("intx", 80, 136, 2048, 32, 4)])
+def test_weights_are_not_rounded_where_the_kernels_before_kept_them(dtype, kind, M, N, K, group, bits):
+    """The result is the exact sum rounded once.  Per term the weight is off by 2^-18 (bfloat16: two parts of 8 bits) or, beside the
+    result's rounding, by nothing (float16), so with sums of random signs at most about one result in 2^9 lands on the other side
+    of a rounding boundary; cancellation moves some more.  A weight rounded to the type moves about four in ten."""
+    got, exact = _fragment(kind, M, N, K, group, bits, dtype)
+    moved = (got.cpu() != exact.to(dtype)).float().mean().item()
+    assert moved < 0.05, moved
+
+
+@pytest.mark.parametrize("bits", [1, 4, 8])
+def test_float32_sums_are_not_one_chain(bits):
+    """A rounding is off by 0.41 x 2^-24 of the partial sum (root mean square); chains of 16, 8 and 8 terms whose partial sums grow
+    like a random walk give 0.41 x 2^-24 sqrt(32 / 2) = 1e-7 of the result, the offset and the parts' sums a little more; one chain
+    of 1024 terms gives five times that."""
+    got, exact = _fragment("intx", 19, 4096, 4096, 128, bits, torch.float32)
+    assert ((got.cpu().double() - exact).norm() / exact.norm()).item() < 2e-7
