@@ -329,7 +329,8 @@ TPQ_CALL(int4_mm, 6)
     const auto sizes = product_sizes(*x, N, &M);
     const bool rows = lib.tpq_int4_mm_rows_takes(x->const_data_ptr(), tag, M, N, K, group, ptr<int32_t>(packed), sz->const_data_ptr()) != 0;
     if (!rows && M > (tag == TPQ_DTYPE_F32 ? 1 : 32)) Py_RETURN_NONE;
-    const at::Tensor* workspace = nullptr;
+    // owned by this call: without the GIL, another thread may put a larger buffer in its place in the dict
+    at::Tensor workspace;
     int64_t workspace_bytes = 0;
     if (rows) {
         workspace_bytes = lib.tpq_packed_rows_workspace_bytes(tag, M, N, K);
@@ -343,10 +344,10 @@ TPQ_CALL(int4_mm, 6)
             if (PyErr_Occurred()) return nullptr;
             Py_RETURN_NONE;
         }
-        workspace = plain(held);
-        workspace_bytes = static_cast<int64_t>(lib.tpq_int4_mm_rows_workspace_bytes(M, N, K));
-        if (!workspace || workspace->numel() < workspace_bytes) Py_RETURN_NONE;
-        workspace_bytes = workspace->numel();
+        const at::Tensor* const found = plain(held);
+        if (!found || found->numel() < static_cast<int64_t>(lib.tpq_int4_mm_rows_workspace_bytes(M, N, K))) Py_RETURN_NONE;
+        workspace = *found;
+        workspace_bytes = workspace.numel();
     }
     at::Tensor out;
     int status;
@@ -358,7 +359,7 @@ TPQ_CALL(int4_mm, 6)
             status = lib.tpq_int4_mm_rows_bias(x->const_data_ptr(), tag, M, K, ptr<int32_t>(packed), N, group, sz->const_data_ptr(), ptr<void>(bias), out.data_ptr(),
                                           workspace_bytes ? part.data_ptr() : nullptr, workspace_bytes, q.stream);
         } else {
-            status = lib.tpq_int4_mm_ws(x->const_data_ptr(), tag, M, K, ptr<int32_t>(packed), 2, N, group, sz->const_data_ptr(), out.data_ptr(), workspace->data_ptr(),
+            status = lib.tpq_int4_mm_ws(x->const_data_ptr(), tag, M, K, ptr<int32_t>(packed), 2, N, group, sz->const_data_ptr(), out.data_ptr(), workspace.data_ptr(),
                                         static_cast<size_t>(workspace_bytes), q.stream);
             if (status == TPQ_OK && bias) {
                 const at::AutoDispatchBelowADInplaceOrView raw;

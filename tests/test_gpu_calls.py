@@ -164,3 +164,38 @@ def test_streams_and_graph():
         assert torch.equal(outs[0], want[0]) and torch.equal(outs[1], want[1])
         if not step:
             assert torch.equal(first[0], want[0]) and torch.equal(first[1], want[1])
+
+
+def test_int4_workspace_lives_until_the_launch():
+    """Another thread may replace the stream's workspace while a call is without the GIL: the call's own stays alive until its
+    kernel is enqueued.  The replacement happens where the call allocates its result (the allocator reports every allocation)."""
+    import weakref
+
+    from torch.cuda import _gpu_trace
+
+    module = q.WeightOnlyInt4Linear.from_float(torch.nn.Linear(4096, 264, bias=False, device="cuda", dtype=torch.float16), 128)
+    x = torch.randn(8, 4096, device="cuda", dtype=torch.float16)
+    with torch.no_grad():
+        want = module(x)
+    key = (torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream)
+    held = weakref.ref(ops._int4_workspaces[key])
+    larger = torch.zeros(ops._int4_workspaces[key].numel() + 4096, dtype=torch.uint8, device="cuda")
+    seen = []
+
+    def replace(_):
+        if not seen:
+            ops._int4_workspaces[key] = larger
+            seen.append(held() is not None)
+
+    callbacks = _gpu_trace.MemoryAllocationCallbacks
+    torch._C._activate_gpu_trace()
+    callbacks.add_callback(replace)
+    try:
+        with torch.no_grad():
+            got = module(x)
+    finally:
+        callbacks.callback_list.remove(replace)
+    assert seen == [True] and torch.equal(got, want)
+    with torch.no_grad():
+        assert torch.equal(module(x), want)
+    assert held() is None  # and no longer
