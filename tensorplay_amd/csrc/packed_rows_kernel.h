@@ -26,6 +26,10 @@
 //   * where the kernels for fewer rows keep the weight in float32 (scales applied to sums), a 16-bit weight is not rounded here
 //     either: SPLIT, the rounding's remainder goes through the matrix cores as a second operand.  The groups of 32 lie across a
 //     lane group's k range, so scales cannot be applied to sums instead;
+//   * a sum that comes out NaN there (SPLIT, or a last step that is partial) is formed again term by term, by the lane that stores
+//     it: an infinite activation meets the weight's remainder, which is zero or of the other sign, an infinite weight meets the zeros
+//     behind K, and a weight beyond the 16-bit range becomes two infinities of opposite signs; the sum itself is infinite or finite.
+//     Finite results pay one comparison;
 //   * float32 sums are formed over 16 k, these added up over a step and the steps over the slice: in one chain over the slice
 //     the roundings of the long sum weigh twice as much as all others together (error against float64 with 8 bits, 4096 x 4096 at
 //     19 rows: one chain 3.3e-7, so 1.3e-7; the one-row kernels 1.9e-7);
@@ -102,6 +106,12 @@ struct SourceInt4 {
         return (j & 1) ? (t & 0x00F000F0u) | magic[1] : (t & 0x000F000Fu) | magic[0];
     }
     static constexpr uint32_t kMagic0 = 0x64006400u, kMagic1 = 0x54005400u;
+    // one code less its bias, for the rare sums that are formed again
+    static __device__ __forceinline__ float code(const PackedRowsArgs& a, int n, int k) {
+        const size_t tile = static_cast<size_t>(n >> 3) * (a.K / 32) + (k >> 5);
+        const uint32_t w = static_cast<const uint32_t*>(a.w)[tile * 32 + (n & 7) * 4 + ((k >> 1) & 3)];
+        return static_cast<float>(static_cast<int>((w >> (4 * ((k >> 3) & 3) + 16 * (k & 1))) & 15u) - 8);
+    }
 };
 
 // rows of n-bit codes, 8 / BITS per byte (one for 5 .. 8 bits), the first in the most significant bits or (LSB) the least
@@ -143,6 +153,11 @@ struct SourceBits {
         return (both & ((kField << pos(lo)) | (kField << (pos(hi) + 16)))) | (exponent(pos(lo)) | (exponent(pos(hi)) << 16));
     }
     static constexpr uint32_t kMagic0 = 0, kMagic1 = 0;
+    static __device__ __forceinline__ float code(const PackedRowsArgs& a, int n, int k) {
+        const uint32_t byte = static_cast<const uint8_t*>(a.w)[static_cast<size_t>(n) * (a.K / kPerByte) + k / kPerByte];
+        if constexpr (BITS == 8) return static_cast<float>(static_cast<int>(byte ^ 0x80u) - 128);
+        else return static_cast<float>((byte >> (LSB ? (k % kPerByte) * BITS : 8 - (k % kPerByte + 1) * BITS)) & kField);
+    }
 };
 
 template <int FIRST, int LAST, class F>
@@ -217,6 +232,23 @@ __device__ __forceinline__ void store_rows_result(const float4_t& s, typename El
     }
     if constexpr (DT == TPQ_DTYPE_F32) *reinterpret_cast<float4_t*>(y) = float4_t{o[0], o[1], o[2], o[3]};
     else *reinterpret_cast<uint2*>(y) = make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16));
+}
+
+// One row's sum over k in [k0, k1) term by term, the weight as the kernel's dequantization defines it (SPLIT: not rounded); ends at
+// the first NaN.
+template <int DT, class Source, bool SPLIT>
+__device__ float one_sum(const PackedRowsArgs& a, int m, int n, int k0, int k1) {
+    using P = RowsParams<DT, Source::kTypedParams>;
+    const auto* const x = static_cast<const typename Elem<DT>::storage*>(a.x) + static_cast<size_t>(m) * a.K;
+    float sum = 0.0f;
+    for (int k = k0; k < k1 && sum == sum; ++k) {
+        const auto params = static_cast<const typename P::raw_t*>(a.sz)[static_cast<size_t>((k >> 5) / a.tiles_per_group) * a.N + n];
+        const float code = Source::code(a, n, k), scale = P::scale(params), zero = P::zero(params);
+        float w = Source::kTypedParams ? __builtin_fmaf(code, scale, zero) : (code - zero) * scale;
+        if constexpr (!SPLIT) w = Elem<DT>::load(Elem<DT>::store(w));
+        sum = __builtin_fmaf(Elem<DT>::load(x[k]), w, sum);
+    }
+    return sum;
 }
 
 template <int DT, class Source, int MB, int CW, bool EDGE, bool SPLIT>
@@ -510,6 +542,18 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
         const int block = t / MB, r = t % MB;
         const int m = m0 + 16 * r + i, n = blockIdx.x * (16 * NB * CW) + block * 16 + 4 * q;
         if (m >= a.M || n >= a.N) continue;  // N % 4 == 0: all four channels exist
+        if constexpr (SPLIT || EDGE) {
+            const int k0 = s_begin * 128, k1 = s_end * 128 < a.K ? s_end * 128 : a.K;
+            const float all = (s[0] + s[1]) + (s[2] + s[3]);
+            if (all != all) {  // one copy of the loop: four of them cost every call 0.2 us
+#pragma unroll 1
+                for (int e = 0; e < 4; ++e) {
+                    float v = e == 0 ? s[0] : e == 1 ? s[1] : e == 2 ? s[2] : s[3];
+                    if (v != v) v = one_sum<DT, Source, SPLIT>(a, m, n + e, k0, k1);
+                    s = float4_t{e == 0 ? v : s[0], e == 1 ? v : s[1], e == 2 ? v : s[2], e == 3 ? v : s[3]};
+                }
+            }
+        }
         const size_t at = static_cast<size_t>(m) * a.N + n;
         if (a.partial != nullptr) {
             *reinterpret_cast<float4_t*>(a.partial + static_cast<size_t>(blockIdx.z) * a.M * a.N + at) = s;

@@ -78,8 +78,9 @@ def test_lowbit_rows(dtype, bits, lsb_first, M, N, K, group):
     _check(out, x, w, bias, 0.011 * (1 + (1 << bits) / 8), dtype)
 
 
-def _fragment(kind, M, N, K, group, bits, dtype):
-    """(result, exact float64 result) on weights whose (scale, zero) have no short form in 16 bits."""
+def _fragment(kind, M, N, K, group, bits, dtype, change=lambda x, sz: None):
+    """(result, exact float64 result) on weights whose (scale, zero) have no short form in 16 bits.  change: of x and the pairs, in
+    place, before the call (sz [K / group, N, 2], of the type that the call takes)."""
     from tensorplay_amd import ops
 
     gen = torch.Generator(device=DEV).manual_seed(M + N + K + bits)
@@ -88,10 +89,12 @@ def _fragment(kind, M, N, K, group, bits, dtype):
     if kind == "int4":
         codes = torch.randint(0, 16, (N, K), dtype=torch.int32, device=DEV, generator=gen)
         packed, sz = ops._convert_weight_to_int4pack(codes, 2), sz.to(dtype)
+        change(x, sz)
         w = (codes.double() - 8).view(N, -1, group) * sz[..., 0].double().t()[..., None] + sz[..., 1].double().t()[..., None]
         got = ops._weight_int4pack_mm(x, packed, group, sz)
     else:
         sz[..., 1] *= 100
+        change(x, sz)
         per_byte = 8 // bits
         packed = torch.randint(0, 256, (N, K // per_byte), dtype=torch.uint8, device=DEV, generator=gen)
         shifts = torch.arange(8 - bits, -1, -bits, device=DEV)
@@ -123,3 +126,56 @@ def test_float32_sums_are_not_one_chain(bits):
     of 1024 terms gives five times that."""
     got, exact = _fragment("intx", 19, 4096, 4096, 128, bits, torch.float32)
     assert ((got.cpu().double() - exact).norm() / exact.norm()).item() < 2e-7
+
+
+# (kind, M, N, K, group, bits): where a 16-bit weight's remainder is multiplied too; a last step that is partial, whole steps, slices of k
+SPLIT_SHAPES = [("int4", 5, 72, 544, 32, 4), ("int4", 48, 11008, 1024, 128, 4), ("intx", 33, 264, 1056, 32, 2), ("intx", 40, 72, 8192, 128, 4),
+                ("intx", 35, 72, 1024, 128, 8)]
+
+
+def _assert_same_classes(got, exact):
+    """NaN, +inf and -inf where the exact sums are, anything finite elsewhere."""
+    got = got.double().cpu()
+    assert torch.equal(got.isnan(), exact.isnan())
+    assert torch.equal(got.isposinf(), exact.isposinf()) and torch.equal(got.isneginf(), exact.isneginf())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind,M,N,K,group,bits", SPLIT_SHAPES)
+def test_non_finite_activations(dtype, kind, M, N, K, group, bits):
+    """An infinite activation gives +-inf with the sign of its product, NaN only where infinities of both signs or a NaN meet."""
+    def change(x, sz):
+        x[0, 5], x[1, K - 1], x[2, 3], x[2, K // 2] = float("inf"), float("-inf"), float("inf"), float("inf")
+        if M > 4:
+            x[4, K - 2], x[M - 1, 40] = float("nan"), float("inf")
+
+    got, exact = _fragment(kind, M, N, K, group, bits, dtype, change)
+    _assert_same_classes(got, exact)
+    fine = exact.isfinite()
+    assert ((got.double().cpu() - exact)[fine].norm() / exact[fine].norm()).item() < max(UNIT[dtype], 3e-7)  # float32: as the sums of ordinary operands
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_infinite_weights_beside_a_partial_step(dtype):
+    """A zero point that is infinite in the last group of a K that ends inside a step: positive activations give +inf."""
+    def change(x, sz):
+        x.abs_().add_(0.1)
+        sz[-1, 7, 1] = float("inf")
+
+    got, exact = _fragment("int4", 19, 72, 544, 32, 4, dtype, change)
+    assert bool(exact[:, 7].isposinf().all())
+    _assert_same_classes(got, exact)
+
+
+@pytest.mark.parametrize("kind,M,N,K,group,bits", SPLIT_SHAPES)
+def test_weights_beyond_float16(kind, M, N, K, group, bits):
+    """Weights of 10^5, beyond float16, with activations that bring the sums back into its range."""
+    def change(x, sz):
+        sz[..., 0] *= 2.0 ** (16 if bits == 8 else 21 if kind == "int4" else 23)
+        if kind == "int4":
+            sz[..., 1] *= 2.0 ** 21
+        x *= 2.0 ** -14
+
+    got, exact = _fragment(kind, M, N, K, group, bits, torch.float16, change)
+    assert bool(got.isfinite().all())
+    assert ((got.double().cpu() - exact).norm() / exact.norm()).item() < UNIT[torch.float16]
