@@ -153,6 +153,7 @@ struct SourceBits {
         return (both & ((kField << pos(lo)) | (kField << (pos(hi) + 16)))) | (exponent(pos(lo)) | (exponent(pos(hi)) << 16));
     }
     static constexpr uint32_t kMagic0 = 0, kMagic1 = 0;
+    static constexpr float kMostCode = BITS == 8 ? 128.0f : static_cast<float>((1 << BITS) - 1);
     static __device__ __forceinline__ float code(const PackedRowsArgs& a, int n, int k) {
         const uint32_t byte = static_cast<const uint8_t*>(a.w)[static_cast<size_t>(n) * (a.K / kPerByte) + k / kPerByte];
         if constexpr (BITS == 8) return static_cast<float>(static_cast<int>(byte ^ 0x80u) - 128);
@@ -368,6 +369,13 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     uint32_t magic[2];  // in VGPRs behind opaque moves: v_and_or_b32 takes one literal only
     asm volatile("v_mov_b32 %0, %1" : "=v"(magic[0]) : "s"(Source::kMagic0));
     asm volatile("v_mov_b32 %0, %1" : "=v"(magic[1]) : "s"(Source::kMagic1));
+    // float16 and n-bit rows, whose scales are float32: remainders of small weights would lie on the grid of float16's subnormals, large
+    // weights beyond its range.  NORMALIZE multiplies a channel's scales by a power of two (exact) that brings the bound of its
+    // first group to 64 .. 128, and the float32 sums by its inverse.  A group may then be 2^9 times as large as the first, or
+    // 2^14 times smaller and still be held to 2^-18.  At most 2^16, for a first group that is nearly zero and says nothing about
+    // the others: below weights of 1e-7 the grid shows (at 1e-8 3e-5 of a weight).  (int4: scale and zero point are float16, so every weight and remainder is a whole multiple of 2^-24 already.)
+    constexpr bool NORMALIZE = SPLIT && DT == TPQ_DTYPE_F16 && !Source::kTypedParams;
+    int power[NB] = {};
     // pair p of a block's codes, dequantized
     auto weight_pair = [&](const Loaded& d, int b, int p, float scale, float zero, float& lo, float& hi) __attribute__((always_inline)) {
         half2_t h = __builtin_bit_cast(half2_t, Source::pair(d.w[b], p, magic));
@@ -399,7 +407,8 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
         for (int e = decltype(first)::value; e < decltype(last)::value; ++e) {
             const int b = e % NB, p = e / NB;
             float lo, hi;
-            weight_pair(d, b, U * kChunkPairs + p, P::scale(d.p[b]), P::zero(d.p[b]), lo, hi);
+            const float scale = NORMALIZE ? __builtin_amdgcn_ldexpf(P::scale(d.p[b]), power[b]) : P::scale(d.p[b]);
+            weight_pair(d, b, U * kChunkPairs + p, scale, P::zero(d.p[b]), lo, hi);
             if constexpr (DT == TPQ_DTYPE_F32) {
                 wq[U & 1][b][2 * p] = __builtin_bit_cast(uint32_t, lo);
                 wq[U & 1][b][2 * p + 1] = __builtin_bit_cast(uint32_t, hi);
@@ -511,6 +520,16 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
         lds_barrier();
     };
     pr_static_for<0, kRowsAhead>([&](auto r) __attribute__((always_inline)) { load_w(decltype(r)::value, ring[decltype(r)::value]); });
+    if constexpr (NORMALIZE) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            float most = (Source::kMostCode + fabsf(P::zero(ring[0].p[b]))) * fabsf(P::scale(ring[0].p[b]));
+            most = fmaxf(most, __shfl_xor(most, 16));  // the four lanes of a channel: up to four groups of 32
+            most = fmaxf(most, __shfl_xor(most, 32));
+            const int up = 7 - __builtin_amdgcn_frexp_expf(most);
+            power[b] = up < 16 ? up : 16;
+        }
+    }
     dequantize(ring[0], std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, kShare>{});
     settle(std::integral_constant<int, 0>{});
     lds_barrier();
@@ -527,6 +546,16 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
 
     // ---- the KW sums of a tile meet in LDS; wavefront t finishes tiles t, t + 8, ...
     float4_t* const sums = reinterpret_cast<float4_t*>(lds);
+    if constexpr (NORMALIZE) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int down = -__shfl(power[b], 4 * q + e);  // element e: channel 4 q + e
+#pragma unroll
+                for (int r = 0; r < MB; ++r) acc[b][r][e] = __builtin_amdgcn_ldexpf(acc[b][r][e], down);
+            }
+    }
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll

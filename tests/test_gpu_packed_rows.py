@@ -179,3 +179,25 @@ def test_weights_beyond_float16(kind, M, N, K, group, bits):
     got, exact = _fragment(kind, M, N, K, group, bits, torch.float16, change)
     assert bool(got.isfinite().all())
     assert ((got.double().cpu() - exact).norm() / exact.norm()).item() < UNIT[torch.float16]
+
+
+@pytest.mark.parametrize("first", [0, -14, 8])
+@pytest.mark.parametrize("power", [0, -10, -16])
+@pytest.mark.parametrize("kind,M,N,K,group,bits", SPLIT_SHAPES)
+def test_float16_weights_of_any_size_are_not_rounded(kind, M, N, K, group, bits, power, first):
+    """(scale, zero) 2^power times the ordinary ones, those of a channel's first group 2^first times the others (where that is the
+    larger one, its activations are zero, so that the others count): the exact sum rounded once, as with ordinary weights."""
+    def change(x, sz):
+        factor = torch.full((K // group, 1), 2.0 ** (max(power, -10) if kind == "int4" else power), device=DEV)
+        factor[0] *= 2.0 ** first
+        sz[..., 0] *= factor
+        if kind == "int4":
+            sz[..., 1] *= factor
+        x *= 2.0 ** min(-power, 12)
+        if first > 0:
+            x[:, :group] = 0.0
+
+    got, exact = _fragment(kind, M, N, K, group, bits, torch.float16, change)
+    assert bool((exact.abs() > 2.0 ** -14).float().mean() > 0.9)  # the result's own rounding is a normal one
+    moved = (got.cpu() != exact.to(torch.float16)).float().mean().item()
+    assert moved < 0.05, moved
