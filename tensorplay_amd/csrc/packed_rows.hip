@@ -32,6 +32,12 @@ bool int4_weights_unrounded(int dtype, int64_t M, int64_t N, int64_t K, int64_t 
     return group == 128 && !int4_gemm_takes(M, N, K, ~size_t{0});
 }
 
+// n-bit rows: the kernel's offsets into the weight and into the (scale, zero) pairs are 32-bit.  The pairs are the larger tensor with
+// few bits and short groups (1 bit in groups of 32: twice the weight).
+bool lowbit_offsets_fit(int64_t N, int64_t K, int bits, int64_t group) {
+    return N * K / (8 / bits) < (int64_t{1} << 32) && K / group * N * 8 <= (int64_t{1} << 32);
+}
+
 }  // namespace
 }  // namespace tpq
 
@@ -64,7 +70,7 @@ TPQ_EXPORT int tpq_int4_mm_rows_takes(const void* x, int dtype, int64_t M, int64
 TPQ_EXPORT int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int bits, int lsb_first, int64_t group,
                                         const uint8_t* packed, const float* scales_and_zeros) {
     if (M <= 0 || N <= 0 || K <= 0 || group <= 0 || (bits != 1 && bits != 2 && bits != 4 && bits != 8) || (lsb_first && bits != 1)) return 0;
-    if (K % 32 || group % 32 || N % 4 || N * K * bits >= (int64_t{1} << 35) || K >= (1 << 24)) return 0;
+    if (K % 32 || group % 32 || N % 4 || !lowbit_offsets_fit(N, K, bits, group) || K >= (1 << 24)) return 0;
     if (!aligned(x, 16) || !aligned(packed, 16) || !aligned(scales_and_zeros, 8)) return 0;
     int64_t limit = rows_limit(N, K, dtype);
     if (bits == 8 && dtype != TPQ_DTYPE_F32) {
@@ -126,8 +132,8 @@ TPQ_EXPORT int tpq_lowbit_mm_rows(const void* x, int dtype, int64_t M, int64_t K
     if (M == 0 || N == 0) return TPQ_OK;
     TPQ_REQUIRE((bits == 1 || bits == 2 || bits == 4 || bits == 8) && (!lsb_first || bits == 1 || bits == 8), TPQ_ERR_UNSUPPORTED,
                 "lowbit_mm_rows: 1, 2, 4 or 8 bits, first code in the most significant bits (1 bit: either order)");
-    TPQ_REQUIRE(K > 0 && K % 32 == 0 && group % 32 == 0 && N % 4 == 0 && K < (1 << 24) && M < (1 << 22) && N * K / (8 / bits) < (int64_t{1} << 32), TPQ_ERR_UNSUPPORTED,
-                "lowbit_mm_rows: K and the group must be multiples of 32, N of 4");
+    TPQ_REQUIRE(K > 0 && K % 32 == 0 && group % 32 == 0 && N % 4 == 0 && K < (1 << 24) && M < (1 << 22) && lowbit_offsets_fit(N, K, bits, group), TPQ_ERR_UNSUPPORTED,
+                "lowbit_mm_rows: K and the group must be multiples of 32, N of 4, the weight below 4 GB and the (scale, zero) pairs within it");
     TPQ_REQUIRE(x && packed && scales_and_zeros && out, TPQ_ERR_INVALID_VALUE, "lowbit_mm_rows: null pointer");
     TPQ_REQUIRE(aligned(x, 16) && aligned(packed, 16) && aligned(scales_and_zeros, 8) && aligned(out, dtype == TPQ_DTYPE_F32 ? 16 : 8), TPQ_ERR_UNSUPPORTED,
                 "lowbit_mm_rows: unaligned operand");

@@ -137,3 +137,17 @@ def test_dispatch_does_not_depend_on_the_environment():
     assert probe.tpq_probe_read(16, 1024, 1, 8, 8, 32, 16, None) == _lib.TPQ_ERR_INVALID_VALUE   # fewer bytes than one tile row
     assert probe.tpq_probe_read(16, 1 << 30, 1, 8, 8, 5000, 16, None) == _lib.TPQ_ERR_INVALID_VALUE
     assert probe.tpq_probe_read(16, 16384 * 8, 1, 8, 7, 32, 16, None) == _lib.TPQ_ERR_INVALID_VALUE
+
+
+def test_block_kernel_refuses_parameters_beyond_its_offsets():
+    """1 bit in groups of 32: the (scale, zero) pairs are twice the weight and pass 4 GB, where the kernel's 32-bit offsets end, first.
+    Host logic only: no operand is read."""
+    from tensorplay_amd import _lib
+
+    lib = _lib.load()
+    n = 1 << 17
+    for k, fits in ((1 << 17, True), ((1 << 17) + 32, False)):
+        assert bool(lib.tpq_lowbit_mm_rows_takes(256, _lib.F16, 40, n, k, 1, 0, 32, 256, 256)) is fits
+    k = (1 << 17) + 32
+    status = lib.tpq_lowbit_mm_rows(256, _lib.F16, 40, k, 256, 1, 0, n, 32, 256, None, 256, None, 0, None)
+    assert status == _lib.TPQ_ERR_UNSUPPORTED
