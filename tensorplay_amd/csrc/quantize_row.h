@@ -47,8 +47,6 @@ __device__ __forceinline__ void quantize_eight_packed(const float (&v)[kVec], fl
     }
     lo = word[0] ^ 0x80808080u;
     hi = word[1] ^ 0x80808080u;
-    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, with a statement the
-    // compiler may not move: left as a plain "if", the eight divisions were computed for every chunk and selected away.
     // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, and with the divisor
     // passed through a statement the compiler may not move: as a plain "if", the eight divisions were hoisted above the
     // branch, computed for every chunk and selected away.
@@ -89,8 +87,6 @@ __device__ __forceinline__ void quantize_eight_lean(const float (&v)[kVec], floa
     // v_perm_b32(a, b, sel): selector bytes 0..3 take bytes of b, 4..7 of a, 0x0c a zero byte
     lo = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0400u) | __builtin_amdgcn_perm(t[3], t[2], 0x04000c0cu);
     hi = __builtin_amdgcn_perm(t[5], t[4], 0x0c0c0400u) | __builtin_amdgcn_perm(t[7], t[6], 0x04000c0cu);
-    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, with a statement the
-    // compiler may not move: left as a plain "if", the eight divisions were computed for every chunk and selected away.
     // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, and with the divisor
     // passed through a statement the compiler may not move: as a plain "if", the eight divisions were hoisted above the
     // branch, computed for every chunk and selected away.
@@ -149,25 +145,34 @@ __device__ __forceinline__ uint4 nt_load_dword_aligned(const void* p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// NT: non-temporal, for rows that one workgroup reads once
+// eight elements as they lie; NT: non-temporal, for rows that one workgroup reads once
+template <int DT>
+struct RawChunk { uint4 w[DT == TPQ_DTYPE_F32 ? 2 : 1]; };
 template <int DT, bool NT = true>
-__device__ __forceinline__ void load_chunk(const typename Elem<DT>::storage* p, float (&v)[kVec]) {
-    if constexpr (DT == TPQ_DTYPE_F32) {
-        const uint4* const q = reinterpret_cast<const uint4*>(p);
-        const uint4 a = NT ? nt_load(q) : q[0], b = NT ? nt_load(q + 1) : q[1];
-        v[0] = __builtin_bit_cast(float, a.x); v[1] = __builtin_bit_cast(float, a.y);
-        v[2] = __builtin_bit_cast(float, a.z); v[3] = __builtin_bit_cast(float, a.w);
-        v[4] = __builtin_bit_cast(float, b.x); v[5] = __builtin_bit_cast(float, b.y);
-        v[6] = __builtin_bit_cast(float, b.z); v[7] = __builtin_bit_cast(float, b.w);
-    } else {
-        const uint4 raw = NT ? nt_load_dword_aligned(p) : *reinterpret_cast<const uint4*>(p);  // NT: rows of K % 8 == 4 start on 8 bytes
-        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+__device__ __forceinline__ RawChunk<DT> load_raw(const typename Elem<DT>::storage* p) {
+    const uint4* const q = reinterpret_cast<const uint4*>(p);
+    if constexpr (DT == TPQ_DTYPE_F32) return {{NT ? nt_load(q) : q[0], NT ? nt_load(q + 1) : q[1]}};
+    else return {{NT ? nt_load_dword_aligned(p) : q[0]}};  // NT: rows of K % 8 == 4 start on 8 bytes
+}
+template <int DT>
+__device__ __forceinline__ void unpack_chunk(const RawChunk<DT>& raw, float (&v)[kVec]) {
+#pragma unroll
+    for (int h = 0; h < (DT == TPQ_DTYPE_F32 ? 2 : 1); ++h) {
+        const uint32_t w[4] = {raw.w[h].x, raw.w[h].y, raw.w[h].z, raw.w[h].w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            v[2 * i] = Elem<DT>::load(static_cast<uint16_t>(w[i] & 0xFFFFu));
-            v[2 * i + 1] = Elem<DT>::load(static_cast<uint16_t>(w[i] >> 16));
+            if constexpr (DT == TPQ_DTYPE_F32) {
+                v[4 * h + i] = __builtin_bit_cast(float, w[i]);
+            } else {
+                v[2 * i] = Elem<DT>::load(static_cast<uint16_t>(w[i] & 0xFFFFu));
+                v[2 * i + 1] = Elem<DT>::load(static_cast<uint16_t>(w[i] >> 16));
+            }
         }
     }
+}
+template <int DT, bool NT = true>
+__device__ __forceinline__ void load_chunk(const typename Elem<DT>::storage* p, float (&v)[kVec]) {
+    unpack_chunk<DT>(load_raw<DT, NT>(p), v);
 }
 
 // the parameters of a quantizer: divisor 127, codes -127 .. 127 and its lower-bit relatives

@@ -81,11 +81,14 @@ __global__ __launch_bounds__(THREADS) void quantize_rows_cached(
     // No branch around the loads: at the join of a branch the compiler waits for every outstanding load, which made
     // the chunks one round trip to memory each.  A chunk past the end re-reads the last chunk of the row: the same
     // elements again do not change the maximum, and nothing is stored for it.
+    RawChunk<DT> raw[CHUNKS];
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-        const int k0 = (c * THREADS + threadIdx.x) * kVec;
-        load_chunk<DT>(xr + chunk_start(k0, K), v[c]);
-    }
+    for (int c = 0; c < CHUNKS; ++c) raw[c] = load_raw<DT>(xr + chunk_start((c * THREADS + threadIdx.x) * kVec, K));
+    // The first use stays behind the last request: left to itself the compiler converted a chunk, and waited for it, between two
+    // requests (2048 x 4096 bfloat16 9.4 -> 10.9 us).
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) unpack_chunk<DT>(raw[c], v[c]);
     TPQ_QUANT_STAMP(1);
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c)
@@ -130,11 +133,12 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_subwave(
 
     float v[CHUNKS][kVec];
     float absmax = 0.0f;
+    RawChunk<DT> raw[CHUNKS];
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-        const int k0 = (c * LANES + sub) * kVec;
-        load_chunk<DT>(xr + chunk_start(k0, K), v[c]);  // branch-free: see quantize_rows_cached; dead rows read row 0
-    }
+    for (int c = 0; c < CHUNKS; ++c) raw[c] = load_raw<DT>(xr + chunk_start((c * LANES + sub) * kVec, K));  // as in quantize_rows_cached; dead rows read row 0
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) unpack_chunk<DT>(raw[c], v[c]);
     if (live) {
 #pragma unroll
         for (int c = 0; c < CHUNKS; ++c)
