@@ -274,6 +274,13 @@ TPQ_CALL(int8_linear, 7)
     return THPVariable_Wrap(std::move(out));
 TPQ_CALL_END
 
+// One row of a weight of up to this many codes: the product quantizes the row itself.  Each of its workgroups reads and quantizes
+// the whole row, so beyond, the quantizer's launch and codes in memory are the cheaper way.  Measured (us, weights from HBM,
+// float16, one launch / two): 2560 -> 6912 5.49 / 6.06, 4096 x 4096 5.34 / 6.02, 2560 -> 9216 5.67 / 5.91, 4096 -> 6144 6.01 / 5.98,
+// 5120 x 5120 6.23 / 6.41 (float32 7.30 / 6.62), 2560 -> 10240 6.39 / 6.16, 4096 -> 8192 7.23 / 6.75, 4096 -> 14336 10.2 / 7.6,
+// 8192 -> 28672 35.7 / 17.3.
+constexpr int64_t kRowQuantizedInProduct = int64_t{3} << 23;
+
 // ternary_linear(x [..., K] float, packed uint8 [N, ceil(K / 4)], w_scale, K, bias or None, eps) -> float32
 TPQ_CALL(ternary_linear, 6)
     const at::Tensor *x = plain(args[0]), *packed = plain(args[1]), *bias;
@@ -291,14 +298,15 @@ TPQ_CALL(ternary_linear, 6)
     int status = TPQ_ERR_UNSUPPORTED;
     {
         Enqueue q(*x);
-        if (M == 1) {
+        const bool one_launch = M == 1 && N * K <= kRowQuantizedInProduct;
+        if (one_launch) {
             out = allocate(sizes, at::kFloat, *x);
             status = lib.tpq_ternary_linear_row(x->const_data_ptr(), float_tag(x->scalar_type()), ptr<uint8_t>(packed), static_cast<float>(w_scale), ptr<float>(bias), N, K,
                                                 static_cast<float>(eps), out_ptr<float>(out), q.stream);
         }
-        if (M != 1 || status != TPQ_OK) {
+        if (!one_launch || status != TPQ_OK) {
             const Quantized room = room_for_codes(*x, M, K, lib.tpq_ternary_mm_workspace_bytes(M, N, K));
-            if (M != 1) out = allocate(sizes, at::kFloat, *x);
+            if (!one_launch) out = allocate(sizes, at::kFloat, *x);
             status = lib.tpq_quantize_rowwise(x->const_data_ptr(), float_tag(x->scalar_type()), M, K, static_cast<float>(eps), 127.0f, -127, 127, 0, room.codes, room.scales,
                                               q.stream);
             if (status == TPQ_OK)

@@ -208,3 +208,15 @@ def test_one_row_quantized_in_the_product(dtype, k, n):
             ops._check(lib.tpq_ternary_linear_row(x.data_ptr(), ops._DT[dtype], packed.data_ptr(), 0.037, ops._ptr(b), n, k, 1e-5, got.data_ptr(),
                                                   ops._stream(x)))
             assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (case, b is not None)
+
+
+@pytest.mark.parametrize("k,n", [(4096, 6144), (4096, 6145)])
+def test_one_row_linear_on_both_sides_of_the_rule(k, n):
+    """Up to 3 x 2^23 weights the product quantizes the row itself, beyond the row quantizer runs first: the same bits."""
+    from tensorplay_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    packed = torch.randint(0, 256, (n, k // 4), device="cuda", generator=gen, dtype=torch.uint8) & 0xAA
+    x = torch.randn(1, k, device="cuda", generator=gen).half()
+    codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
+    assert torch.equal(ops._ternary_linear(x, packed, 0.037, k, None, 1e-5), ops.ternary_mm(codes, scale, packed, 0.037, k))
