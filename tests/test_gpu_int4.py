@@ -68,7 +68,8 @@ CASES = [  # M, N, K, group
     (2, 64, 4096, 128), (5, 24, 96, 32), (1, 16, 70, 32), (7, 136, 1024, 64),
     # matrix-core decode kernel: 5..16 rows (64-channel workgroups, partial last one), slabs of 16 plus a last row
     (16, 72, 256, 128), (9, 136, 1024, 128), (17, 64, 256, 128), (33, 40, 384, 128), (8, 200, 2048, 128),
-    # slabs of 32 rows (two row blocks per workgroup), partial last block, every width of workgroup
+    # slabs of 32 rows (two row blocks per workgroup), partial last block, every width of workgroup; above 32 rows both routes,
+    # the slabs and the kernel for a block of rows
     (24, 136, 512, 128), (64, 72, 1024, 128), (50, 200, 256, 128), (130, 64, 384, 128), (81, 40, 1152, 128),
     (32, 6152, 256, 128), (31, 10248, 128, 128), (19, 5128, 256, 128), (128, 8200, 128, 128),
     # groups of 32 / 64: dequantized in registers (fp16, bf16), every shape of workgroup (by N and rows), one row too
@@ -78,6 +79,20 @@ CASES = [  # M, N, K, group
     # (K = 2048, 4096, 6144), every group size, a partial last column block
     (1, 10248, 2048, 128), (1, 10264, 4096, 32), (1, 10240, 4096, 64), (1, 10300 // 8 * 8, 6144, 128),
 ]
+
+
+def _slab_route(ops, x, packed, group, sz):
+    """tpq_int4_mm_ws: the decode kernels, above 32 rows in slabs (what operands off 16 bytes and the C entry point take where
+    _weight_int4pack_mm runs the kernel for a block of rows)."""
+    from tensorplay_amd import _lib
+
+    m, k, n = x.shape[0], x.shape[1], packed.shape[0] * 8
+    lib = _lib.load()
+    out = torch.empty(m, n, dtype=x.dtype, device=DEV)
+    ws = torch.zeros(int(lib.tpq_int4_mm_rows_workspace_bytes(m, n, k)), dtype=torch.uint8, device=DEV)
+    ops._check(lib.tpq_int4_mm_ws(x.data_ptr(), ops._DT[x.dtype], m, k, packed.data_ptr(), 2, n, group, sz.data_ptr(), out.data_ptr(),
+                                  ws.data_ptr(), ws.numel(), ops._stream(x)))
+    return out
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
@@ -91,20 +106,21 @@ def test_mm_matches_oracle(ops, dtype, M, N, K, group):
     x = rng.normal(0, 1, (M, K)).astype(np.float32)
     xb, szb = cast_bits(x, dtype), cast_bits(sz, dtype)
     packed = oracle.int4_pack_tc(codes, 2)
-    got = ops._weight_int4pack_mm(dev(xb, dtype), dev(packed), group, dev(szb, dtype))
-    assert got.dtype == TORCH_DT[dtype] and got.shape == (M, packed.shape[0] * 8)
-    got32 = got.float().cpu().numpy()
+    operands = dev(xb, dtype), dev(packed), group, dev(szb, dtype)
     ref_dev = oracle.to_f32(oracle.int4_mm_tc(xb, dtype, packed, szb, group, round_w=True), dtype)
     _, y64 = oracle.int4_mm_tc(xb, dtype, packed, szb, group, round_w=False, want_f64=True)
-    # the stated tolerance, 1e-2 normwise and elementwise, against the reference's CPU kernel
-    assert_close_to_cpu_formulation(got32, xb, dtype, codes, szb, group)
-    # secondary: the reference's device formulation, which rounds every weight to the activation dtype twice; for bf16
-    # (2^-8 per rounding) two correct evaluations of it differ by more than 1e-2 on a few of ~10^5 outputs, so the widest
-    # bf16 cases (and long sums, K >= 4096) get 1.5e-2 in this check only
-    assert_close_norm(got32, ref_dev, 1.5e-2 if dtype == "bf16" and (M * N > 50000 or K >= 4096) else 1e-2, "vs the device formulation (secondary)")
-    # fp32-accumulate comparison against the exact sums
-    tol = {"f16": 1e-3, "bf16": 1e-2, "f32": 1e-5}[dtype]
-    assert rel_err(got32, y64) < tol
+    for got in [ops._weight_int4pack_mm(*operands)] + ([_slab_route(ops, *operands)] if M > 32 else []):
+        assert got.dtype == TORCH_DT[dtype] and got.shape == (M, packed.shape[0] * 8)
+        got32 = got.float().cpu().numpy()
+        # the stated tolerance, 1e-2 normwise and elementwise, against the reference's CPU kernel
+        assert_close_to_cpu_formulation(got32, xb, dtype, codes, szb, group)
+        # secondary: the reference's device formulation, which rounds every weight to the activation dtype twice; for bf16
+        # (2^-8 per rounding) two correct evaluations of it differ by more than 1e-2 on a few of ~10^5 outputs, so the widest
+        # bf16 cases (and long sums, K >= 4096) get 1.5e-2 in this check only
+        assert_close_norm(got32, ref_dev, 1.5e-2 if dtype == "bf16" and (M * N > 50000 or K >= 4096) else 1e-2, "vs the device formulation (secondary)")
+        # fp32-accumulate comparison against the exact sums
+        tol = {"f16": 1e-3, "bf16": 1e-2, "f32": 1e-5}[dtype]
+        assert rel_err(got32, y64) < tol
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
@@ -271,8 +287,12 @@ def test_dequantize_bf16_non_finite_scale(ops):
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
 def test_mm_many_rows_takes_the_dense_route(ops, dtype):
-    """More than INT4_PREFILL_ROWS rows: dequantise + one dense GEMM (tpq_dense_mm where K allows), the reference's device formulation."""
-    M, N, K, group = ops.INT4_PREFILL_ROWS + 37, 136, 512, 128
+    """More rows than the kernel for a block of rows takes (768 for a weight this small; bfloat16 256, float32 192): dequantise + one dense
+    GEMM (tpq_dense_mm where K allows), the reference's device formulation."""
+    from tensorplay_amd import _lib
+
+    M, N, K, group = 768 + 37, 136, 512, 128
+    assert M > ops.INT4_PREFILL_ROWS and not _lib.load().tpq_int4_mm_rows_takes(16, ops._DT[TORCH_DT[dtype]], M, N, K, group, 16, 16)
     rng = np.random.default_rng(77)
     codes, sz = asym_quant(rng.normal(0, 0.02, (N, K)).astype(np.float32), group)
     x = rng.normal(0, 1, (M, K)).astype(np.float32)
@@ -360,7 +380,9 @@ def test_mm_all_in_flight_kernel_matches_oracle(ops, dtype, M, N, K, group):
     x = rng.normal(0, 1, (M, K)).astype(np.float32)
     xb, szb = cast_bits(x, dtype), cast_bits(sz, dtype)
     packed = ops._convert_weight_to_int4pack(torch.from_numpy(codes).to(DEV), 2)
-    got32 = ops._weight_int4pack_mm(dev(xb, dtype), packed, group, dev(szb, dtype)).float().cpu().numpy()
+    # above 32 rows the slabs: _weight_int4pack_mm runs the kernel for a block of rows there
+    product = ops._weight_int4pack_mm if M <= 32 else lambda *operands: _slab_route(ops, *operands)
+    got32 = product(dev(xb, dtype), packed, group, dev(szb, dtype)).float().cpu().numpy()
     assert got32.shape == (M, N)
     # the oracle on whole packed tiles of eight channels, first and last included
     tiles = _tile_subset(rng, N // 8, 40)

@@ -242,8 +242,12 @@ def test_packed_linear_general_form_bit_exact(ops, shape, unsigned, relu):
 @pytest.mark.parametrize("shape", [
     # rows of k read from any address: one step short of / at / past a step's edge, one and two blocks of rows, ragged N
     (1, 127, 17), (2, 129, 40), (16, 1001, 33), (17, 5284, 50), (32, 255, 16), (3, 16, 5), (9, 648, 70),
-    # more rows, K % 16 == 0: the staggered kernel's edge stage (first, second, late; both tile heights; more stages than the ring)
-    (33, 16, 40), (40, 112, 136), (70, 144, 72), (129, 400, 200), (300, 1328, 113), (33, 2064, 10248), (600, 976, 4104),
+    # 33 .. 64 rows, K % 16 == 0: the register-staged kernel
+    (33, 16, 40), (40, 112, 136), (33, 2064, 10248),
+    # more rows, K % 16 == 0: the staggered kernel's edge stage on tiles of 128 rows (the only stage, twice; second; late, more stages than
+    # the ring) and, where those would not fit the chip at once, on tiles of 256 rows (late, twice; the only stage)
+    (70, 16, 72), (100, 112, 136), (70, 144, 72), (129, 400, 200), (300, 1328, 113), (600, 976, 4104),
+    (2048, 1328, 4096), (2048, 976, 4104), (2056, 80, 8200),
     # more rows, any other K: both operands copied to padded rows (one short of and one past a stage, slices of the padded k)
     (33, 127, 40), (64, 129, 65), (130, 1001, 200), (300, 4100, 130)])
 def test_ragged_k(ops, shape):
@@ -251,7 +255,7 @@ def test_ragged_k(ops, shape):
     M, K, N = shape
     rng = np.random.default_rng(M * 3 + K + N)
     a, w = _rand_i8(rng, (M, K)), _rand_i8(rng, (N, K))
-    want = a.astype(np.int32) @ w.astype(np.int32).T
+    want = (a.astype(np.float64) @ w.astype(np.float64).T).astype(np.int32)  # whole numbers below 2^53: exact
     np.testing.assert_array_equal(host(ops._int_mm(dev(a), dev(w).t())), want)
     rs, cs = rng.uniform(1e-3, 1e-1, M).astype(np.float32), rng.uniform(1e-4, 1e-2, N).astype(np.float32)
     bias = rng.normal(0, 0.01, N).astype(np.float32)
