@@ -226,7 +226,9 @@ int tpq_ternary_linear_row(const void* x, int x_dtype, const uint8_t* packed, fl
  * The int4 and n-bit weight-only products for a block of activation rows (about 17 .. 500; any count is taken), float32 /
  * float16 / bfloat16, groups of any multiple of 32 (int4: 32, 64 or 128, innerKTiles = 2), K % 32 == 0; anything else
  * returns TPQ_ERR_UNSUPPORTED.  Same operations and reference lines as tpq_int4_mm and tpq_lowbit_mm (1, 2, 4, 8 bits); the
- * dequantized weight is rounded to the activation type once.  x, packed: 16-byte aligned; out: 8 bytes (float32: 16);
+ * dequantized weight is rounded to the activation type once, or, where the decode kernels keep it in float32 (int4: K % 128 != 0 and
+ * groups of 128 on the slab kernels; n-bit: up to 56 rows, 80 for small weights), multiplied in two parts of that type that hold it
+ * to 2^-22 (bfloat16: 2^-17).  The bytes of the weight and of scales_and_zeros: up to 4 GB.  x, packed: 16-byte aligned; out: 8 bytes (float32: 16);
  * lowbit: N % 4 == 0.  workspace (16-byte aligned, contents undefined, may be NULL): with
  * tpq_packed_rows_workspace_bytes bytes the k range can be cut into slices where the channels do not fill the chip; the
  * slices are added in a fixed order.

@@ -47,9 +47,11 @@ using namespace tpq;
 // 33 of 4096 x 4096 10.8 / 15.1, 48 of 4096 -> 11008 18.5 / 20.2; groups of 64, 17 rows:
 // 11008 -> 4096 12.0 / 23.1, 16 rows 11.3 / 12.0.  K % 128 != 0 (slabs of four rows): 4768 -> 13544 at 3 / 33 rows 19.4 /
 // 92, 31 / 868.  float32: 4096 -> 11008 at 1, 2, 64 rows 24.4 / 24.2, 24.7 / 45, 68 / 110; 2048 x 2048 at 1 and 2 rows
-// 8.1 / 7.2, 8.2 / 7.4.  bfloat16 stops at 256 rows: beyond, results are held to within 1e-2, element by element, of the
-// reference's device formulation, whose dense weight is rounded to bfloat16 twice; a weight rounded once misses that on
-// single elements (it is the one that lies closer to the exact product).
+// 8.1 / 7.2, 8.2 / 7.4.  bfloat16 stops at 256 rows although this kernel is the faster one beyond (384 rows of 8192 x 8192 78 / 104, 512 of
+// 4096 x 4096 24 / 41): from 257 rows on the results are those of the dense route, the reference's device formulation with a weight
+// rounded to bfloat16 twice, and are held to it within 1e-2, element by element, by tests.  A weight rounded once lies closer to
+// the exact product and misses that on single elements; below 257 rows, where the tiled kernel and the slabs ran, the comparison
+// is with the exact product.
 // Operands off the alignment that the kernel wants stay with the kernels that take any address.
 TPQ_EXPORT int tpq_int4_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int64_t group, const int32_t* packed,
                                       const void* scales_and_zeros) {

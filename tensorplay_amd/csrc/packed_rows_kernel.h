@@ -30,7 +30,8 @@
 //     it: an infinite activation meets the weight's remainder, which is zero or of the other sign, an infinite weight meets the zeros
 //     behind K, and a weight beyond the 16-bit range becomes two infinities of opposite signs; the sum itself is infinite or finite.
 //     Finite results pay one comparison;
-//   * float32 sums are formed over 16 k, these added up over a step and the steps over the slice: in one chain over the slice
+//   * with float32 activations sums are formed over 16 k, these added up over a step and the steps over the slice (16-bit operands
+//     keep one chain, their products' own roundings are larger): in one chain over the slice
 //     the roundings of the long sum weigh twice as much as all others together (error against float64 with 8 bits, 4096 x 4096 at
 //     19 rows: one chain 3.3e-7, so 1.3e-7; the one-row kernels 1.9e-7);
 //   * the KW partial sums of a tile meet in LDS at the end.

@@ -330,6 +330,8 @@ INT4_PREFILL_ROWS = 256
 INT4_PREFILL_ROWS_VERY_WIDE = 1024  # N >= 16384
 INT4_PREFILL_ROWS_BF16 = 112
 INT4_PREFILL_ROWS_BF16_VERY_WIDE = 768
+# (What tpq_int4_mm_rows_takes accepts never comes here.  With K % 128 == 0 it is all of bfloat16 up to 256 rows on 16-byte
+# aligned operands: the estimates below serve operands off that alignment.)
 # Between INT4_PREFILL_ROWS_BF16 and INT4_PREFILL_ROWS rows bfloat16 takes the tiled kernel where its estimate (1.4 times
 # float16's, which is int4_gemm_plan of int4_gemm_kernel.h restated below: with a workspace that kernel deals K to
 # slices when its tiles are few) is below the dense route's: 0.55 us per million weights for the dequantize pass and one
