@@ -88,7 +88,6 @@ __device__ __forceinline__ void int4_mfma_body(
     const uint32_t* __restrict__ sz_b, const uint16_t* __restrict__ residual, int block) {
     static_assert(!PAIR || NB == 2, "a pair is two blocks");
     static_assert(GKT == 4 || !PAIR, "in-register dequantization is not built for the pair");
-    static_assert(MB == 1 || !PAIR, "the pair takes 16 rows");
     constexpr bool DEQ = GKT < 4;
     using L = Lane16<DT>;
     using ML = MfmaLane<DT>;
@@ -123,9 +122,6 @@ __device__ __forceinline__ void int4_mfma_body(
         sz_base[b] = (PAIR && b == 1 ? sz_b : sz) + n4;
         if constexpr (DEQ) sz_base[b] = sz + ((nb0 + i) < N ? nb0 + i : N - 1);  // (scale, zero) of this lane's weight row
     }
-    bool row_live[MB];
-#pragma unroll
-    for (int r = 0; r < MB; ++r) row_live[r] = 16 * r + i < M;
     // load j of a step: row 4 j + lane / 16, piece lane % 16 of the step's 256 bytes (rows past M: row 0, dropped)
     const uint4* x_base[4 * MB];
 #pragma unroll
@@ -306,7 +302,9 @@ __device__ __forceinline__ void int4_mfma_body(
             for (int v = 0; v < 4; ++v) red[wave][b * MB + r][v][lane] = yacc[b][r][v];
     __syncthreads();
     if constexpr (PAIR) {
-        if (wave == 0) {  // lane (m, q): channels n0 + 4 q + v of both weights
+        // wavefront r finishes row block r; lane (m, q): row 16 r + m, channels n0 + 4 q + v of both weights
+        static_assert(MB <= WAVES, "a wavefront per row block");
+        if (wave < MB) {
             float sum[2][4];
 #pragma unroll
             for (int b = 0; b < 2; ++b)
@@ -314,13 +312,13 @@ __device__ __forceinline__ void int4_mfma_body(
                 for (int v = 0; v < 4; ++v) {
                     sum[b][v] = 0.0f;
 #pragma unroll
-                    for (int w = 0; w < WAVES; ++w) sum[b][v] += red[w][b][v][lane];
+                    for (int w = 0; w < WAVES; ++w) sum[b][v] += red[w][b * MB + wave][v][lane];
                 }
-            const int n = n0 + 4 * q;
-            if (row_live[0] && n < N) {
+            const int n = n0 + 4 * q, row = 16 * wave + i;
+            if (row < M && n < N) {
                 const uint32_t lo = swiglu_of<DT>(sum[0][0], sum[1][0]) | (static_cast<uint32_t>(swiglu_of<DT>(sum[0][1], sum[1][1])) << 16);
                 const uint32_t hi = swiglu_of<DT>(sum[0][2], sum[1][2]) | (static_cast<uint32_t>(swiglu_of<DT>(sum[0][3], sum[1][3])) << 16);
-                *reinterpret_cast<uint2*>(y + static_cast<size_t>(i) * N + n) = make_uint2(lo, hi);
+                *reinterpret_cast<uint2*>(y + static_cast<size_t>(row) * N + n) = make_uint2(lo, hi);
             }
         }
         return;
@@ -378,7 +376,7 @@ struct Int4MultiSet {
     int count;
 };
 
-template <int DT, int NB, int WAVES>
+template <int DT, int NB, int WAVES, int MB = 1>
 __global__ __launch_bounds__(WAVES * kWave) void int4_mfma_multi_kernel(const uint16_t* __restrict__ x, Int4MultiSet set, int M,
                                                                        int K, int group_shift) {
     const int block = static_cast<int>(blockIdx.x);
@@ -394,7 +392,7 @@ __global__ __launch_bounds__(WAVES * kWave) void int4_mfma_multi_kernel(const ui
 #pragma unroll
     for (int i = 1; i < kMultiMax; ++i)
         if (w == i) { packed = set.packed[i]; sz = set.sz[i]; y = set.y[i]; N = set.N[i]; first = set.first[i]; }
-    int4_mfma_body<DT, NB, WAVES>(x, packed, sz, y, M, N, K, group_shift, nullptr, nullptr, nullptr, block - first);
+    int4_mfma_body<DT, NB, WAVES, false, 4, MB>(x, packed, sz, y, M, N, K, group_shift, nullptr, nullptr, nullptr, block - first);
 }
 
 }  // namespace

@@ -934,6 +934,13 @@ def _norm_operand(x: torch.Tensor, norm_weight: torch.Tensor, what: str) -> torc
     return norm_weight.contiguous()
 
 
+# Up to this many rows a norm that the kernels do not fold into the products is a launch of its own in front of the fused products:
+# beyond, those run one launch per 32 rows, and the separate products have kernels for more rows.  Measured (us a layer's linears
+# in a graph, separate products and torch's float32 gate / norm and fused products): hidden 1024, MLP 2304: 37 / 20 at one row, 50 /
+# 26 at 32; hidden 4096, MLP 11008: 63 / 52 at 16 rows, 99 / 69 at 32; hidden 5120, MLP 13824: 72 / 62 at one row, 147 / 101 at 32.
+_INT4_FUSED_ROWS = 32
+
+
 def int4pack_mm_multi(input: torch.Tensor, mats, qGroupSize: int, scales_and_zeros, norm_weight: Optional[torch.Tensor] = None,
                       eps: float = 1e-5) -> list:
     """``[_weight_int4pack_mm(input, w, qGroupSize, sz) for w, sz in zip(mats, scales_and_zeros)]`` with one launch
@@ -953,9 +960,13 @@ def int4pack_mm_multi(input: torch.Tensor, mats, qGroupSize: int, scales_and_zer
 
     def separate():
         xn = x if g is None else rms_norm(x, g, eps)
+        if g is not None and 0 < m <= _INT4_FUSED_ROWS:
+            return int4pack_mm_multi(xn, mats, qGroupSize, scales_and_zeros)
         return [_weight_int4pack_mm(xn, w, qGroupSize, sz) for _, w, sz, _, _ in ops]
 
     if len(ops) > 4 or len({inner for _, _, _, inner, _ in ops}) != 1 or x.dtype == torch.float32:
+        return separate()
+    if g is not None and 16 < m <= _INT4_FUSED_ROWS:  # one launch for all rows behind the norm's, two with the norm folded in
         return separate()
     outs = [torch.empty((m, n), dtype=x.dtype, device=x.device) for _, _, _, _, n in ops]
     if m == 0:
@@ -1008,6 +1019,8 @@ def int4pack_mm_swiglu(input: torch.Tensor, gate: torch.Tensor, up: torch.Tensor
                                                          qGroupSize, _ptr(szg), _ptr(szu), _ptr(out), _stream(x))
     if status == _lib.TPQ_ERR_UNSUPPORTED:
         xn = x if nw is None else rms_norm(x, nw, eps)
+        if nw is not None and m <= _INT4_FUSED_ROWS:
+            return int4pack_mm_swiglu(xn, gate, up, qGroupSize, gate_scale_and_zeros, up_scale_and_zeros)
         g = _weight_int4pack_mm(xn, wg, qGroupSize, szg).float()
         u = _weight_int4pack_mm(xn, wu, qGroupSize, szu).float()
         return (g * torch.sigmoid(g) * u).to(x.dtype)

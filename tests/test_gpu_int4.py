@@ -592,6 +592,40 @@ def test_mm_swiglu_with_rms_norm_against_oracle(ops, tdt, tol, M, N, K):
     assert_close_norm(got.float().cpu().numpy()[:, cols], want, 2 * tol)
 
 
+@pytest.mark.parametrize("tdt,tol", [(torch.float16, 2e-3), (torch.bfloat16, 1.6e-2)])
+@pytest.mark.parametrize("M,K,widths", [(17, 384, (136, 8, 72)), (32, 1024, (4104, 72, 72)), (33, 1920, (48, 200, 200)), (31, 640, (8192, 1024, 1024)),
+                                        (24, 512, (12288, 72, 72)), (20, 2048, (136, 72, 72)), (30, 4096, (72, 136, 136))])
+def test_layer_products_of_two_row_blocks(ops, tdt, tol, M, K, widths):
+    """add, swiglu and multi at 17..32 rows (two blocks of 16 against one unpacking of the weight) equal the same calls on 16 rows at a time
+    bit for bit where those run the same loop kernel (K below 2048), and the norm in front of them the two-step formulation."""
+    rng = np.random.default_rng(M * 13 + K)
+    cases = [_fused_case(rng, M, n, K, tdt) for n in widths]
+    x = cases[0][2].to(DEV)
+    packed = [ops._convert_weight_to_int4pack(torch.from_numpy(c).to(DEV), 2) for c, _, _ in cases]
+    szs = [sz.to(DEV) for _, sz, _ in cases]
+    res = torch.from_numpy(rng.standard_normal((M, widths[0])).astype(np.float32)).to(tdt).to(DEV)
+    g = torch.from_numpy(rng.uniform(0.5, 1.5, K).astype(np.float32)).to(tdt).to(DEV)
+
+    def layer(rows, norm):
+        xs = x[rows]
+        return [ops.int4pack_mm_add(xs, packed[0], 128, szs[0], res[rows]),
+                ops.int4pack_mm_swiglu(xs, packed[1], packed[1], 128, szs[1], szs[1], norm_weight=norm),
+                *ops.int4pack_mm_multi(xs, packed, 128, szs, norm_weight=norm)]
+
+    whole = layer(slice(0, M), None)
+    if K < 2048:
+        parts = [layer(slice(m, min(m + 16, M)), None) for m in range(0, M, 16)]
+        for k, y in enumerate(whole):
+            assert torch.equal(y, torch.cat([p[k] for p in parts])), k
+    for p, sz, y in zip(packed, szs, whole[2:]):
+        assert_close_norm(y.float().cpu().numpy(), ops._weight_int4pack_mm(x, p, 128, sz).float().cpu().numpy(), tol)
+    xn = ops.rms_norm(x, g, 1e-5)
+    normed = layer(slice(0, M), g)
+    for p, sz, y in zip(packed, szs, normed[2:]):
+        assert_close_norm(y.float().cpu().numpy(), ops._weight_int4pack_mm(xn, p, 128, sz).float().cpu().numpy(), tol)
+    assert_close_norm(normed[1].float().cpu().numpy(), ops.int4pack_mm_swiglu(xn, packed[1], packed[1], 128, szs[1], szs[1]).float().cpu().numpy(), 2 * tol)
+
+
 def test_mm_multi_other_shapes_and_errors(ops):
     rng = np.random.default_rng(6)
     codes = rng.integers(0, 16, (32, 128)).astype(np.int32)
