@@ -356,6 +356,20 @@ int tpq_packed_linear_float(const void* x, int x_unsigned, double x_scale, int64
 int tpq_dense_mm(const void* x, int dtype, int64_t M, int64_t K, const void* w, int64_t N, void* out, void* stream);
 
 /*
+ * Gradients of out = x w^T in float32 (the straight-through backward of the quantized training linears: reference
+ * tensorplay/ao/quantization/int8_dyn_act_int4_weight.py:86-95, two plain products):
+ *   grad_x[M][K] = grad[M][N] w[N][K]       (grad_x null: not formed, w unused)
+ *   grad_w[N][K] = grad[M][N]^T x[M][K]     (grad_w null: not formed, x unused)
+ * float32 products and sums (each value in three bfloat16 parts, exactly; six part products, float32 accumulation).  Everything
+ * contiguous and 16-byte aligned, K and N multiples of 4; TPQ_ERR_UNSUPPORTED otherwise, nothing written then.  workspace: at least
+ * tpq_f32_linear_grads_workspace_bytes(M, K, N, grad_x wanted, grad_w wanted) bytes, no initial contents, free again when the
+ * work enqueued here is done.
+ */
+size_t tpq_f32_linear_grads_workspace_bytes(int64_t M, int64_t K, int64_t N, int want_x, int want_w);
+int tpq_f32_linear_grads(const float* grad, const float* x, const float* w, int64_t M, int64_t K, int64_t N, float* grad_x, float* grad_w,
+                         void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Dense weight [N, K] of `dtype` from the packed device layout: W = T(code - 8) * scale + zero, the
  * product and the sum each rounded to T.  The reference runs this before its library GEMM
  * (int4_tc_dequantize_kernel, p10/src/backend/cuda/QuantGemmKernels.cu:1170-1202, 1296-1341); the

@@ -5,7 +5,7 @@ int8_dyn_act_int1_weight.py).
 Forward, as in the reference: the activations are quantized per token to int8, the full-precision weight
 per row to signed 4 / 2 / 1-bit codes by the fused native quantizers, the product runs on the int8
 matrix cores and is rescaled by both scales.  Backward is the reference's straight-through estimator
-(plain matmuls on the full-precision weight), so the modules stay trainable.
+(float32 products with the full-precision weight), so the modules stay trainable.
 """
 from __future__ import annotations
 
@@ -50,9 +50,7 @@ class _Int8DynActLowBitLinear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         input, weight = ctx.saved_tensors
-        grad_weight = grad_output.reshape(-1, weight.shape[0]).T @ input.reshape(-1, weight.shape[1])
-        grad_input = grad_output @ weight.to(grad_output.dtype)
-        return grad_input, grad_weight, None
+        return *ops.linear_grads(grad_output, input, weight, *ctx.needs_input_grad[:2]), None
 
 
 class Int8DynActInt4WeightLinear(nn.Linear):

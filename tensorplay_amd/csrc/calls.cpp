@@ -17,10 +17,12 @@
 #include <cstdint>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -41,7 +43,8 @@ struct Library {
     TPQ_ENTRY(tpq_int4_mm_ws)                                                                                             \
     TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
     TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
-    TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine)
+    TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine) \
+    TPQ_ENTRY(tpq_f32_linear_grads_workspace_bytes) TPQ_ENTRY(tpq_f32_linear_grads)
     TPQ_ENTRIES
 #undef TPQ_ENTRY
 };
@@ -170,6 +173,19 @@ Quantized room_for_codes(const at::Tensor& x, int64_t M, int64_t K, int64_t scra
     return q;
 }
 
+// a tuple of two references, which it takes over; null (an error is set) where one of them is
+PyObject* pair_of(PyObject* first, PyObject* second) {
+    PyObject* pair = first && second ? PyTuple_New(2) : nullptr;
+    if (!pair) {
+        Py_XDECREF(first);
+        Py_XDECREF(second);
+        return nullptr;
+    }
+    PyTuple_SET_ITEM(pair, 0, first);
+    PyTuple_SET_ITEM(pair, 1, second);
+    return pair;
+}
+
 #define TPQ_CALL(NAME, COUNT)                                              \
     PyObject* NAME(PyObject*, PyObject* const* args, Py_ssize_t count) {   \
         HANDLE_TH_ERRORS                                                   \
@@ -202,20 +218,7 @@ TPQ_CALL(quantize_rowwise, 6)
     }
     if (status != TPQ_OK) Py_RETURN_NONE;
     PyObject* first = THPVariable_Wrap(std::move(codes));
-    PyObject* second = first ? THPVariable_Wrap(std::move(scales)) : nullptr;
-    if (!second) {
-        Py_XDECREF(first);
-        return nullptr;
-    }
-    PyObject* pair = PyTuple_New(2);
-    if (!pair) {
-        Py_DECREF(first);
-        Py_DECREF(second);
-        return nullptr;
-    }
-    PyTuple_SET_ITEM(pair, 0, first);
-    PyTuple_SET_ITEM(pair, 1, second);
-    return pair;
+    return pair_of(first, first ? THPVariable_Wrap(std::move(scales)) : nullptr);
 TPQ_CALL_END
 
 // int8_mm_dequant(a int8 [M, K], w int8 [N, K], row_scale, col_scale, bias or None, out_dtype, ragged_rows)
@@ -478,6 +481,34 @@ TPQ_CALL(dequantize_affine, 6)
     return THPVariable_Wrap(std::move(out));
 TPQ_CALL_END
 
+// linear_grads(grad [..., N], x [..., K], w [N, K], want_x, want_w), float32 -> (grad_x like x or None, grad_w or None).  Not while
+// gradients are recorded (a second derivative) or products are cast: those need the products as torch operations.
+TPQ_CALL(linear_grads, 5)
+    const at::Tensor *g = plain(args[0]), *x = plain(args[1]), *w = plain(args[2]);
+    if (!g || !x || !w || c10::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || g->scalar_type() != at::kFloat ||
+        x->scalar_type() != at::kFloat || w->scalar_type() != at::kFloat || g->dim() < 1 || x->dim() < 1 || w->dim() != 2 || g->numel() == 0 ||
+        x->numel() == 0 || g->size(-1) != w->size(0) || x->size(-1) != w->size(1) || g->numel() / w->size(0) != x->numel() / w->size(1) ||
+        !same_device(*g, *x) || !same_device(*g, *w))
+        Py_RETURN_NONE;
+    const int64_t N = w->size(0), K = w->size(1), M = g->numel() / N;
+    const bool want_x = args[3] == Py_True, want_w = args[4] == Py_True;
+    at::Tensor grad_x, grad_w;
+    int status;
+    {
+        Enqueue q(*g);
+        const size_t bytes = lib.tpq_f32_linear_grads_workspace_bytes(M, K, N, want_x, want_w);
+        const at::Tensor scratch = bytes ? allocate({static_cast<int64_t>(bytes)}, at::kByte, *g) : at::Tensor();
+        if (want_x) grad_x = allocate(x->sizes(), at::kFloat, *g);
+        if (want_w) grad_w = allocate({N, K}, at::kFloat, *g);
+        status = lib.tpq_f32_linear_grads(ptr<float>(g), ptr<float>(x), ptr<float>(w), M, K, N, want_x ? out_ptr<float>(grad_x) : nullptr,
+                                          want_w ? out_ptr<float>(grad_w) : nullptr, bytes ? scratch.data_ptr() : nullptr, bytes, q.stream);
+    }
+    if (status != TPQ_OK) Py_RETURN_NONE;
+    PyObject* first = want_x ? THPVariable_Wrap(std::move(grad_x)) : Py_NewRef(Py_None);
+    PyObject* second = !first ? nullptr : want_w ? THPVariable_Wrap(std::move(grad_w)) : Py_NewRef(Py_None);
+    return pair_of(first, second);
+TPQ_CALL_END
+
 // bind(handle): the entry points of the loaded library (a dlopen handle)
 PyObject* bind(PyObject*, PyObject* handle_obj) {
     void* handle = PyLong_AsVoidPtr(handle_obj);
@@ -498,6 +529,7 @@ PyObject* bind(PyObject*, PyObject* handle_obj) {
 #define TPQ_METHOD(NAME) {#NAME, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(NAME)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {TPQ_METHOD(quantize_rowwise), TPQ_METHOD(int8_mm_dequant),  TPQ_METHOD(int8_linear),       TPQ_METHOD(ternary_linear),
                          TPQ_METHOD(int4_mm),          TPQ_METHOD(lowbit_mm),        TPQ_METHOD(quantize_affine),   TPQ_METHOD(dequantize_affine),
+                         TPQ_METHOD(linear_grads),
                          {"bind", bind, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef definition = {PyModuleDef_HEAD_INIT, "_calls", "The hot operators' host path as native calls.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

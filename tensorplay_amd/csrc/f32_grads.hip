@@ -1,0 +1,347 @@
+// The two gradients of a linear layer in float32, one launch (and one that adds slices, where there are any):
+//   grad_x[M][K] = g[M][N] w[N][K]          grad_w[N][K] = g[M][N]^T x[M][K]
+// the straight-through backward of the quantized training linears (reference tensorplay/ao/quantization/int8_dyn_act_int4_weight.py:
+// 86-95, two plain float32 products).
+//
+// What bounds it: the matrix cores.  v_mfma_f32_16x16x4_f32 takes 32 clocks for 2048 flops, a sixteenth of what bfloat16 does, so every
+// float32 value is taken apart into three bfloat16 parts on its way into LDS (8 + 8 + 8 bits: exact, x = h + m + l) and a product
+// is the six part products down to 2^-18 of it (hh, hm, mh, mm, hl, lh; what is left out is below 2^-24): six bfloat16 instructions for
+// the work of sixteen.  No scaling, no range below float32's: the parts keep its exponent.  Two float16 parts would need three
+// products instead of six, but a scale for each row and column, whose maxima are a pass of their own, and lose what lies 2^17 below a
+// row's largest value.
+//   * tile 128 x 128, 32 k a stage; 4 wavefronts of 64 x 64, v_mfma_f32_32x32x16_bf16: 12 fragments of 16 bytes from LDS for 24
+//     instructions (384 of 768 clocks per 16 k); up to three workgroups a compute unit, so that one takes values apart (6.5 vector
+//     instructions each, 832 clocks a stage) while another multiplies (1536 clocks a stage);
+//   * the next stage's float32 values travel to registers while a stage is multiplied: half of the wavefronts fetch one operand,
+//     half the other.  An operand whose k is its slow index (both of grad_w, the weight of grad_x) is read as quads of rows x 8 k
+//     and transposed by the choice of registers;
+//   * LDS: [part][chunk of 8 k][slot] of 16 bytes, a slot per row: fragment reads are 512 consecutive bytes, and so are the
+//     writes, row 4 i + e of a transposed operand having the slot 32 e + i.  A wavefront's two column fragments then lie at
+//     columns 4 i + 0, 1 (or 2, 3): a lane stores two neighbours;
+//   * the k range is cut into slices where tiles are few, so that workgroups of both products are about equally long; float32
+//     sums of slices meet in a second kernel, in slice order;
+//   * a sum that comes out NaN is formed again term by term: an infinite value has h = inf and m = NaN.
+// Measured (us, both gradients with the adding launch, float32 library products before): 512 rows, 2048 -> 4096 140 -> 103 (matrix cores
+// busy for 41 of them; the write-back of 32 MB at the end of the launch takes 7, the rest is stages in which the workgroups of a unit
+// wait for each other's phases), 295 rows, 808 -> 3840 49 -> 41, 128 rows, 2048 -> 2048 38 -> 27, 72 rows, 1280 -> 712 39 -> 15.  Error against
+// float64 at the first: 3.5e-7 (grad_x) and 3.4e-7, the products before 1.15e-6 and 4.05e-7.  float32 values kept in LDS and taken apart
+// by the wavefronts that multiply them (no barrier between the two, each value twice): 113 - 130.
+// Rows behind the operand's end repeat its last ones and are not stored; k behind the end is cleared in both operands.
+#include "tpq_common.h"
+
+namespace tpq {
+namespace {
+
+typedef __bf16 fg_bf8 __attribute__((ext_vector_type(8)));
+typedef float fg_f2 __attribute__((ext_vector_type(2)));
+typedef float fg_f4 __attribute__((ext_vector_type(4)));
+typedef float fg_f16 __attribute__((ext_vector_type(16)));
+
+constexpr int kTile = 128, kStageK = 32, kThreads = 256, kParts = 3;
+constexpr int kChunkBytes = kTile * 16 + 64;  // (64: the four chunks of a row read along k fall into different banks)
+constexpr int kPartBytes = (kStageK / 8) * kChunkBytes, kOperandBytes = kParts * kPartBytes;
+
+// c[m][n] = sum over k of a(m, k) b(n, k); b lies as [k][n], a as [m][k] (ALONG) or [k][m]
+struct Product {
+    const float *a, *b;
+    float* c;        // [M][N], or [slices][M][N] in the workspace
+    int M, N, K;
+    int tiles_m, tiles_n, slices, stages_per_slice;
+};
+
+struct GradArgs {
+    Product p[2];    // grad_x, grad_w
+    int first;       // workgroups of p[0]
+};
+
+// the float32 values of one operand and stage that a thread carries: ALONG rows t / 4 + 32 j, k 8 (t % 4) .. + 7;
+// else rows 4 (t % 32) .. + 3 at k 8 (t / 32) + j
+template <bool ALONG>
+__device__ __forceinline__ void fetch(const float* __restrict__ base, int rows, int row0, int K, int k0, int t, fg_f4 (&v)[8]) {
+    if constexpr (ALONG) {
+        const int k = k0 + 8 * (t & 3);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int row = row0 + (t >> 2) + 32 * j;
+            const float* const p = base + static_cast<size_t>(row < rows ? row : rows - 1) * K;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[2 * j + h] = *reinterpret_cast<const fg_f4*>(p + (k + 4 * h < K ? k + 4 * h : K - 4));
+        }
+    } else {
+        const int row = row0 + 4 * (t & 31), k = k0 + 8 * (t >> 5);
+        const float* const p = base + (row < rows ? row : rows - 4);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const fg_f4*>(p + static_cast<size_t>(k + j < K ? k + j : K - 1) * rows);
+    }
+}
+
+// zeros for k >= K
+template <bool ALONG>
+__device__ __forceinline__ void clear_behind(int K, int k0, int t, fg_f4 (&v)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int k = ALONG ? k0 + 8 * (t & 3) + 4 * (j & 1) : k0 + 8 * (t >> 5) + j;
+        if (k >= K) v[j] = fg_f4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+}
+
+// Eight values as three chunks of bfloat16 parts: h is the upper half of the value after half a unit was added (to nearest; beyond the
+// largest bfloat16 it is infinite, m NaN and the sum is formed again), m the upper half of x - h, l what is left, 8 bits at most.
+// v_cvt_pk_bf16_f32 and v_dot2_f32_bf16, half as many instructions, take 8 - 10 % longer.
+__device__ __forceinline__ void store_parts(const float (&x)[8], char* lds) {
+    uint32_t h[4], m[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t upper[2], middle[2], lower[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float v = x[2 * i + e];
+            upper[e] = __builtin_bit_cast(uint32_t, v) + 0x8000u;
+            const float r = v - __builtin_bit_cast(float, upper[e] & 0xFFFF0000u);
+            middle[e] = __builtin_bit_cast(uint32_t, r);
+            lower[e] = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, middle[e] & 0xFFFF0000u));
+        }
+        h[i] = __builtin_amdgcn_perm(upper[1], upper[0], 0x07060302u);
+        m[i] = __builtin_amdgcn_perm(middle[1], middle[0], 0x07060302u);
+        l[i] = __builtin_amdgcn_perm(lower[1], lower[0], 0x07060302u);
+    }
+    *reinterpret_cast<uint4*>(lds) = make_uint4(h[0], h[1], h[2], h[3]);
+    *reinterpret_cast<uint4*>(lds + kPartBytes) = make_uint4(m[0], m[1], m[2], m[3]);
+    *reinterpret_cast<uint4*>(lds + 2 * kPartBytes) = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+template <bool ALONG>
+__device__ __forceinline__ void put(const fg_f4 (&v)[8], char* lds, int t) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = ALONG ? v[2 * e + (j >> 2)][j & 3] : v[j][e];
+        const int chunk = ALONG ? t & 3 : t >> 5, slot = 32 * e + (ALONG ? t >> 2 : t & 31);
+        store_parts(x, lds + chunk * kChunkBytes + slot * 16);
+    }
+}
+
+__device__ __forceinline__ fg_bf8 fragment(const char* lds) { return __builtin_bit_cast(fg_bf8, *reinterpret_cast<const uint4*>(lds)); }
+
+// one sum of a slice term by term; ends at the first NaN
+template <bool ALONG>
+__device__ __attribute__((noinline)) float one_sum(const float* a, const float* b, int M, int N, int K, int m, int n, int k0, int k1) {
+    float sum = 0.0f;
+    for (int k = k0; k < k1 && sum == sum; ++k) {
+        const float av = ALONG ? a[static_cast<size_t>(m) * K + k] : a[static_cast<size_t>(k) * M + m];
+        sum = __builtin_fmaf(av, b[static_cast<size_t>(k) * N + n], sum);
+    }
+    return sum;
+}
+
+template <bool ALONG>
+__device__ __forceinline__ void product(const Product& p, int block, int blocks, char* lds) {
+    // consecutive workgroups go round the eight dies: each die gets one run of neighbouring tiles, whose operands its L2 holds
+    const int die = block & 7, each = blocks >> 3, more = blocks & 7;
+    const int id = die * each + (die < more ? die : more) + (block >> 3);
+    const int tiles = p.tiles_m * p.tiles_n, slice = id / tiles, at = id - slice * tiles;
+    // groups of eight tile rows, down each group's columns
+    const int group = at / (8 * p.tiles_n), in_group = at - group * 8 * p.tiles_n;
+    const int high = p.tiles_m - 8 * group < 8 ? p.tiles_m - 8 * group : 8;
+    const int tile_n = in_group / high, tile_m = 8 * group + in_group - tile_n * high;
+    const int m0 = tile_m * kTile, n0 = tile_n * kTile;
+    const int begin = slice * p.stages_per_slice * kStageK;
+    const int end = begin + p.stages_per_slice * kStageK < p.K ? begin + p.stages_per_slice * kStageK : p.K;
+
+    const int t = threadIdx.x & 127, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 31, half = lane >> 5, wm = wave >> 1, wn = wave & 1;
+    const bool first_operand = wave < 2;
+    char* const lds_b = lds + kOperandBytes;
+    fg_f4 v[8];
+    const auto load = [&](int k0) {
+        if (first_operand) fetch<ALONG>(p.a, p.M, m0, p.K, k0, t, v);
+        else fetch<false>(p.b, p.N, n0, p.K, k0, t, v);
+    };
+    const auto store = [&](int k0) {
+        if (k0 + kStageK > p.K) {
+            if (first_operand) clear_behind<ALONG>(p.K, k0, t, v);
+            else clear_behind<false>(p.K, k0, t, v);
+        }
+        if (first_operand) put<ALONG>(v, lds, t);
+        else put<false>(v, lds_b, t);
+    };
+
+    fg_f16 acc[2][2];
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[f >> 1][f & 1][e] = 0.0f;
+
+    load(begin);
+    store(begin);
+    __syncthreads();
+    for (int k0 = begin; k0 < end; k0 += kStageK) {
+        const bool more_stages = k0 + kStageK < end;
+        if (more_stages) load(k0 + kStageK);
+#pragma unroll
+        for (int s = 0; s < kStageK / 16; ++s) {
+            const char* const la = lds + (2 * s + half) * kChunkBytes + (64 * wm + i) * 16;
+            const char* const lb = lds_b + (2 * s + half) * kChunkBytes + (64 * wn + i) * 16;
+            fg_bf8 a[kParts][2], b[kParts][2];
+#pragma unroll
+            for (int part = 0; part < kParts; ++part)
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    a[part][f] = fragment(la + part * kPartBytes + f * 32 * 16);
+                    b[part][f] = fragment(lb + part * kPartBytes + f * 32 * 16);
+                }
+            constexpr int kA[6] = {2, 0, 1, 1, 0, 0}, kB[6] = {0, 2, 1, 0, 1, 0};  // small products first
+#pragma unroll
+            for (int e = 0; e < 6; ++e)
+#pragma unroll
+                for (int f = 0; f < 4; ++f)
+                    acc[f >> 1][f & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kA[e]][f >> 1], b[kB[e]][f & 1], acc[f >> 1][f & 1], 0, 0, 0);
+        }
+        __syncthreads();
+        if (more_stages) {
+            store(k0 + kStageK);
+            __syncthreads();
+        }
+    }
+
+    // register e of a lane: slot 8 (e / 4) + 4 half + e % 4 of a fragment; row slot 32 f + s is row s of 32 rows (ALONG) or row 4 s + f,
+    // column slot 32 f + s column 4 s + f: the two column fragments are neighbours
+    const int n = n0 + 4 * i + 2 * wn;
+    float* const c = p.c + static_cast<size_t>(slice) * p.M * p.N;
+    if (n >= p.N) return;
+    const auto row_of = [&](int f, int e) {
+        const int in = 8 * (e >> 2) + 4 * half + (e & 3);
+        return m0 + (ALONG ? 32 * (2 * wm + f) + in : 4 * in + 2 * wm + f);
+    };
+    bool nan = false;
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const fg_f2 sum = {acc[f][0][e], acc[f][1][e]};
+            const int m = row_of(f, e);
+            nan |= sum.x != sum.x || sum.y != sum.y;
+            if (m < p.M) *reinterpret_cast<fg_f2*>(c + static_cast<size_t>(m) * p.N + n) = sum;
+        }
+    // (apart from the stores: a call between them makes each wait for the one before it)
+    if (!nan) return;
+    for (int e = 0; e < 64; ++e) {
+        const int m = row_of(e >> 5, (e >> 1) & 15);
+        float* const at = c + static_cast<size_t>(m) * p.N + n + (e & 1);
+        if (m < p.M && *at != *at) *at = one_sum<ALONG>(p.a, p.b, p.M, p.N, p.K, m, n + (e & 1), begin, end);
+    }
+}
+
+__global__ __launch_bounds__(kThreads, 3) void f32_grads_kernel(const GradArgs args) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * kOperandBytes];
+    const int block = static_cast<int>(blockIdx.x);
+    if (block < args.first) product<true>(args.p[0], block, args.first, lds);
+    else product<false>(args.p[1], block - args.first, static_cast<int>(gridDim.x) - args.first, lds);
+}
+
+struct Finish {
+    const fg_f4* partial;
+    fg_f4* out;
+    int64_t quads;
+    int slices, blocks;
+};
+
+// the slices' sums, added in slice order; blocks of both products in one launch
+__global__ __launch_bounds__(256) void f32_grads_finish_kernel(const Finish x, const Finish w) {
+    const bool second = static_cast<int>(blockIdx.x) >= x.blocks;
+    const Finish f = second ? w : x;
+    const int64_t q = static_cast<int64_t>(static_cast<int>(blockIdx.x) - (second ? x.blocks : 0)) * 256 + threadIdx.x;
+    if (q >= f.quads) return;
+    fg_f4 sum = f.partial[q];
+    for (int s = 1; s < f.slices; ++s) sum += f.partial[s * f.quads + q];
+    f.out[q] = sum;
+}
+
+constexpr int64_t kPlaces = 512;  // two workgroups on each of 256 compute units
+constexpr int kLeastStages = 4, kMostSlices = 8;
+
+struct Plan {
+    int64_t tiles_m, tiles_n, slices, stages;
+};
+
+Plan plan_of(int64_t M, int64_t N, int64_t K, int64_t stages_each) {
+    Plan p{(M + kTile - 1) / kTile, (N + kTile - 1) / kTile, 1, 0};
+    const int64_t stages = (K + kStageK - 1) / kStageK;
+    int64_t slices = (stages + stages_each / 2) / stages_each;
+    slices = slices < 1 ? 1 : slices > kMostSlices ? kMostSlices : slices;
+    p.stages = (stages + slices - 1) / slices;
+    p.slices = (stages + p.stages - 1) / p.stages;
+    return p;
+}
+
+// plans of grad_x and grad_w: about the stages that each place gets if all are shared out evenly
+void plans(int64_t M, int64_t K, int64_t N, bool want_x, bool want_w, Plan (&plan)[2]) {
+    const auto tiles = [](int64_t a, int64_t b) { return ((a + kTile - 1) / kTile) * ((b + kTile - 1) / kTile); };
+    const int64_t all = (want_x ? tiles(M, K) * ((N + kStageK - 1) / kStageK) : 0) + (want_w ? tiles(N, K) * ((M + kStageK - 1) / kStageK) : 0);
+    int64_t each = (all + kPlaces - 1) / kPlaces;
+    if (each < kLeastStages) each = kLeastStages;
+    plan[0] = plan_of(M, K, N, each);
+    plan[1] = plan_of(N, K, M, each);
+}
+
+}  // namespace
+}  // namespace tpq
+
+using namespace tpq;
+
+TPQ_EXPORT size_t tpq_f32_linear_grads_workspace_bytes(int64_t M, int64_t K, int64_t N, int want_x, int want_w) {
+    if (M <= 0 || K <= 0 || N <= 0) return 0;
+    Plan plan[2];
+    plans(M, K, N, want_x != 0, want_w != 0, plan);
+    size_t bytes = 0;
+    if (want_x && plan[0].slices > 1) bytes += static_cast<size_t>(plan[0].slices * M * K) * 4;
+    if (want_w && plan[1].slices > 1) bytes += static_cast<size_t>(plan[1].slices * N * K) * 4;
+    return bytes;
+}
+
+TPQ_EXPORT int tpq_f32_linear_grads(const float* grad, const float* x, const float* w, int64_t M, int64_t K, int64_t N, float* grad_x,
+                                    float* grad_w, void* workspace, size_t workspace_bytes, void* stream) {
+    TPQ_REQUIRE(M >= 0 && K >= 0 && N >= 0, TPQ_ERR_INVALID_VALUE, "tpq_f32_linear_grads: negative dimension");
+    TPQ_REQUIRE(M > 0 && K > 0 && N > 0 && K % 4 == 0 && N % 4 == 0 && M <= (1 << 24) && K <= (1 << 24) && N <= (1 << 24), TPQ_ERR_UNSUPPORTED,
+                "tpq_f32_linear_grads: sizes of 1 to 2^24, K and N multiples of 4");
+    if (grad_x == nullptr && grad_w == nullptr) return TPQ_OK;
+    TPQ_REQUIRE(grad && (grad_x == nullptr || w) && (grad_w == nullptr || x), TPQ_ERR_INVALID_VALUE, "tpq_f32_linear_grads: null pointer");
+    TPQ_REQUIRE(aligned(grad, 16) && aligned(x, 16) && aligned(w, 16) && aligned(grad_x, 16) && aligned(grad_w, 16) && aligned(workspace, 16),
+                TPQ_ERR_UNSUPPORTED, "tpq_f32_linear_grads: operands must be 16-byte aligned");
+    TPQ_REQUIRE(workspace_bytes >= tpq_f32_linear_grads_workspace_bytes(M, K, N, grad_x != nullptr, grad_w != nullptr) &&
+                    (workspace != nullptr || workspace_bytes == 0),
+                TPQ_ERR_INVALID_VALUE, "tpq_f32_linear_grads: workspace too small");
+    Plan plan[2];
+    plans(M, K, N, grad_x != nullptr, grad_w != nullptr, plan);
+    GradArgs args{};
+    Finish finish[2] = {};
+    int64_t blocks[2] = {0, 0};
+    float* space = static_cast<float*>(workspace);
+    const int m = static_cast<int>(M), k = static_cast<int>(K), n = static_cast<int>(N);
+    args.p[0] = Product{grad, w, grad_x, m, k, n, 0, 0, 0, 0};
+    args.p[1] = Product{grad, x, grad_w, n, k, m, 0, 0, 0, 0};
+    for (int e = 0; e < 2; ++e) {
+        Product& p = args.p[e];
+        if (p.c == nullptr) continue;
+        p.tiles_m = static_cast<int>(plan[e].tiles_m);
+        p.tiles_n = static_cast<int>(plan[e].tiles_n);
+        p.slices = static_cast<int>(plan[e].slices);
+        p.stages_per_slice = static_cast<int>(plan[e].stages);
+        blocks[e] = plan[e].tiles_m * plan[e].tiles_n * plan[e].slices;
+        if (p.slices > 1) {
+            const int64_t quads = static_cast<int64_t>(p.M) * p.N / 4;
+            finish[e] = Finish{reinterpret_cast<const fg_f4*>(space), reinterpret_cast<fg_f4*>(p.c), quads, p.slices, static_cast<int>((quads + 255) / 256)};
+            p.c = space;
+            space += p.slices * quads * 4;
+        }
+    }
+    TPQ_REQUIRE(blocks[0] + blocks[1] <= (1 << 24), TPQ_ERR_UNSUPPORTED, "tpq_f32_linear_grads: too many tiles");
+    args.first = static_cast<int>(blocks[0]);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    f32_grads_kernel<<<dim3(static_cast<unsigned>(blocks[0] + blocks[1])), dim3(kThreads), 0, s>>>(args);
+    if (int rc = check_launch("tpq_f32_linear_grads")) return rc;
+    const int adding = finish[0].blocks + finish[1].blocks;
+    if (adding == 0) return TPQ_OK;
+    f32_grads_finish_kernel<<<dim3(adding), dim3(256), 0, s>>>(finish[0], finish[1]);
+    return check_launch("tpq_f32_linear_grads (finish)");
+}

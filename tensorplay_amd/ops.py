@@ -941,6 +941,17 @@ def _norm_operand(x: torch.Tensor, norm_weight: torch.Tensor, what: str) -> torc
 _INT4_FUSED_ROWS = 32
 
 
+def linear_grads(grad: torch.Tensor, input: torch.Tensor, weight: torch.Tensor, want_input: bool = True, want_weight: bool = True):
+    """Gradients of ``input @ weight.T`` for ``grad`` [..., N], input [..., K] and weight [N, K]: (grad @ weight like input, grad.T @ input
+    over all leading dims), None for one that is not wanted.  Contiguous float32 GPU tensors with N and K multiples of 4 run in
+    one kernel for both; anything else, and any call whose own gradient is recorded, as the two products."""
+    calls = _lib.load().calls if grad.is_cuda else None
+    if calls is not None and (pair := calls.linear_grads(grad, input, weight, bool(want_input), bool(want_weight))) is not None:
+        return pair
+    grad_weight = grad.reshape(-1, weight.shape[0]).T @ input.reshape(-1, weight.shape[1]) if want_weight else None
+    return (grad @ weight.to(grad.dtype) if want_input else None), grad_weight
+
+
 def int4pack_mm_multi(input: torch.Tensor, mats, qGroupSize: int, scales_and_zeros, norm_weight: Optional[torch.Tensor] = None,
                       eps: float = 1e-5) -> list:
     """``[_weight_int4pack_mm(input, w, qGroupSize, sz) for w, sz in zip(mats, scales_and_zeros)]`` with one launch

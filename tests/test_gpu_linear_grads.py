@@ -1,0 +1,114 @@
+"""The two float32 gradients of a linear layer in one kernel (tpq_f32_linear_grads) against float64."""
+import pytest
+import torch
+
+from tensorplay_amd import ops
+from tensorplay_amd.ao import quantization as q
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(m, k, n, seed=0):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    g = torch.randn(m, n, device="cuda", generator=gen) * 1e-3
+    x = torch.randn(m, k, device="cuda", generator=gen)
+    w = torch.randn(n, k, device="cuda", generator=gen) * 0.02
+    return g, x, w
+
+
+def _grads(g, x, w, **want):
+    with torch.no_grad():
+        return ops.linear_grads(g, x, w, **want)
+
+
+# one value, edges of the 128 x 128 tiles and of the 32 k stages, several slices of k on either product, many more rows than columns
+SIZES = [(1, 4, 4), (3, 132, 260), (31, 128, 124), (33, 1280, 712), (128, 512, 512), (129, 260, 132), (72, 1280, 4096), (295, 808, 3840), (2100, 96, 64)]
+
+
+@pytest.mark.parametrize("m,k,n", SIZES)
+def test_against_float64(m, k, n):
+    g, x, w = _case(m, k, n)
+    gx, gw = _grads(g, x, w)
+    for got, a, b in ((gx, g, w), (gw, g.T, x)):
+        want, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+        # six part products leave out 3 x 2^-24 of a term at most; the chain of float32 sums rounds each of its at most 6 K / 16 steps once
+        # (slices only shorten it): 2^-24 of the sum so far, taken as the sum of the magnitudes, with the steps' roundings in all
+        # directions (their square root, four times over)
+        steps = 6 * ((a.shape[1] + 15) // 16) + 8
+        bound = size * (3 * 2.0 ** -24 + 4 * steps ** 0.5 * 2.0 ** -24)
+        assert bool(((got.double() - want).abs() <= bound).all())
+    torch_err = ((g.T @ x).double() - g.T.double() @ x.double()).norm()
+    assert (gw.double() - g.T.double() @ x.double()).norm() <= 1.05 * torch_err + 1e-30  # as exact as the float32 product it replaces
+
+
+def test_wide_range_of_values_keeps_float32_precision():
+    """Rows whose values span 2^60: every term keeps its own 24 bits, nothing is scaled by the largest."""
+    g, x, w = _case(64, 256, 256)
+    g = g * torch.exp2(torch.randint(-30, 30, (1, 256), device="cuda").float())
+    w = w * torch.exp2(torch.randint(-30, 30, (256, 1), device="cuda").float())
+    w[g.abs().amax(0) > 1e3] = 0.0  # the largest values meet zeros
+    gx, _ = _grads(g, x, w, want_weight=False)
+    size = g.double().abs() @ w.double().abs()
+    assert bool(((gx.double() - g.double() @ w.double()).abs() <= size * 2.0 ** -20).all())
+
+
+def test_infinities_and_nan_as_in_float32():
+    g, x, w = _case(40, 132, 260)
+    g[3, 7], g[4, 8], g[5, 9], g[6, 1] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    w[8] = 0.0  # -inf x 0
+    w[1] = 1.0
+    gx, gw = _grads(g, x, w)
+    for got, want in ((gx, g.cpu().double() @ w.cpu().double()), (gw, g.cpu().double().T @ x.cpu().double())):
+        want = want.float().cpu()
+        got = got.cpu()
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())
+
+
+def test_one_gradient_and_leading_dims():
+    g, x, w = _case(24, 64, 128)
+    gx, gw = _grads(g.view(2, 3, 4, 128), x.view(2, 3, 4, 64), w)
+    only_x, none = _grads(g, x, w, want_weight=False)
+    nothing, only_w = _grads(g, x, w, want_input=False)
+    assert none is None and nothing is None and gx.shape == (2, 3, 4, 64)
+    assert torch.equal(gx.view(24, 64), only_x) and torch.allclose(gw, only_w, rtol=1e-5, atol=1e-9)
+
+
+def test_forms_that_stay_with_the_plain_products():
+    """Sizes that are no multiple of 4, other layouts and types, an address off 16 bytes, a recorded backward."""
+    for m, k, n in ((5, 6, 8), (5, 8, 6)):
+        g, x, w = _case(m, k, n)
+        gx, gw = _grads(g, x, w)
+        assert torch.allclose(gx, g @ w, rtol=1e-5, atol=1e-8) and torch.allclose(gw, g.T @ x, rtol=1e-5, atol=1e-8)
+    g, x, w = _case(16, 64, 32)
+    for other in (g.T.contiguous().T, torch.randn(16 * 32 + 1, device="cuda")[1:].view(16, 32), g[:1].expand(16, 32)):
+        gx, gw = _grads(other, x, w)
+        assert torch.allclose(gx, other @ w, rtol=1e-5, atol=1e-6) and torch.allclose(gw, other.T @ x, rtol=1e-5, atol=1e-5)
+    lin = q.Int8DynActInt4WeightLinear(64, 32, bias=False, device="cuda")
+    x = x.requires_grad_()
+    grad = g.clone().requires_grad_()
+    gx, = torch.autograd.grad(lin(x), x, grad, create_graph=True)
+    second, = torch.autograd.grad(gx.square().sum(), grad)
+    assert torch.allclose(second, 2 * (g @ lin.weight) @ lin.weight.T, rtol=1e-4, atol=1e-7)
+
+
+def test_module_gradients_replay_in_a_graph():
+    lin = q.Int8DynActInt4WeightLinear(512, 768, bias=False, device="cuda")
+    x = torch.randn(96, 512, device="cuda", requires_grad=True)
+    grad = torch.randn(96, 768, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.autograd.grad(lin(x), (x, lin.weight), grad)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = torch.autograd.grad(lin(x), (x, lin.weight), grad)
+    for seed in range(3):
+        with torch.no_grad():
+            grad.copy_(torch.randn(96, 768, device="cuda", generator=torch.Generator(device="cuda").manual_seed(seed)))
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = torch.autograd.grad(lin(x), (x, lin.weight), grad)
+        assert all(torch.equal(a, b) for a, b in zip(out, eager))
