@@ -12,6 +12,9 @@
 //   * a workgroup owns 64 channels (128 where that still fills the chip: half the activation bytes per product) and a slice of
 //     K (a few slices of K fill the chip where N / 64 workgroups do not; their fp32 sums meet in a second kernel, added in
 //     slice order);
+//   * up to 64 rows, with 128 channels up to 128 (whose two rounds of activations fill 128 KB of LDS): a taller tile dequantizes
+//     its channels once for more rows, and 203 rows of 4096 -> 11008 are 172 tiles of 112 rows in one round of workgroups instead of 344 of 64
+//     in two (2 bits 48.5 -> 32, int4 41 -> 28 us; int4 at 256 rows 43 -> 34, at 384 66 -> 53);
 //   * its eight multiplying wavefronts are CW channel positions x KW steps of 128 k: a round of the loop covers KW steps, whose
 //     activations two more wavefronts fetch by direct global -> LDS loads (whole lines, one copy per workgroup, double
 //     buffered, the swizzle of the fragment reads applied on the global side) while the round before is multiplied.  A direct
@@ -38,7 +41,7 @@
 // Measured (us, weights from HBM, this kernel / what ran before): int4, bfloat16, 11008 -> 4096 in groups of 64: 24 / 48 / 128 / 256
 // rows 12.4 / 22.8, 14.8 / 39, 24 / 43, 36 / 71; 4096 x 4096 in groups of 128: 33 rows (SPLIT) 10.8 / 12.5, 64 / 256 rows 11.2 / 20, 15.8 / 34;
 // 4768 -> 13544 in groups of 32 (K % 128 != 0): 3 / 33 rows (SPLIT) 19.4 / 92, 31 / 868.  float32 4096 x 4096: 3 / 19 / 64 rows 12.4 / 22, 18 / 38,
-// 29 / 47 (bound by its MFMAs, 32 clocks for 16 x 16 x 4).  2 bits: 4096 -> 11008 at 203 rows 50 /
+// 29 / 47 (bound by its MFMAs, 32 clocks for 16 x 16 x 4).  2 bits: 4096 -> 11008 at 203 rows 32 /
 // 67, (SPLIT) at 40 rows 20 / 31; 4096 x 4096 in groups of 32 (SPLIT): 1 / 16 / 80 rows 10.1 / 25, 10.4 / 46, 17.6 / 175.
 // Rows >= M repeat row M - 1, steps of k behind the end of the slice are loaded (from the last step) and not multiplied, the
 // chunks of a last partial step behind K are cleared in LDS.
@@ -624,38 +627,42 @@ __global__ __launch_bounds__(256) void packed_rows_finish_kernel(const float* __
 
 // ---- launch ------------------------------------------------------------------------------------------
 struct PackedRowsPlan {
-    int mb;        // blocks of 16 rows per workgroup: 1 .. 4 (float32: 1, 2)
-    int cw;        // channel positions: 2 (64 channels per workgroup) or 4 (128; three or four blocks of rows and K % 128 == 0 only)
+    int mb;        // blocks of 16 rows per workgroup: 1 .. 4, with 128 channels 3 .. 8 (float32: 1, 2)
+    int cw;        // channel positions: 2 (64 channels per workgroup) or 4 (128; 16-bit, three blocks of rows and more, K % 128 == 0)
     int slices, steps_per_slice;
     bool split;    // the weights' remainders multiplied too (64 channels per workgroup)
 };
 
 // Tile height, channels per workgroup and slices of K by an estimate (us) fitted to a sweep of 1 .. 8 slices and both widths
-// over six shapes and 16 .. 256 rows: 4 for the launch, the first loads and the epilogue, per round what the comment on the
+// over six shapes and 16 .. 256 rows (128 channels and 5 .. 8 blocks of rows, on the same line: 1.36 and 1.49 us a round at 7 and 8): 4 for the launch, the first loads and the epilogue, per round what the comment on the
 // kernel says, per round of workgroups over the compute units, and 2 + the bytes of the slices' sums (written and read) at
 // 4 TB/s for the second kernel.  Within 5 % of the sweep's best nearly everywhere (11008 -> 4096 at 128 rows 24.8, best 22.7).
 inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, bool split = false, int units = 256) {
     PackedRowsPlan p;
     p.split = split && dtype != TPQ_DTYPE_F32;
     const bool wide = dtype == TPQ_DTYPE_F32;
-    const int64_t blocks = (M + 15) / 16;
-    const int64_t most = wide ? 2 : 4, row_tiles = (blocks + most - 1) / most;
-    p.mb = static_cast<int>((blocks + row_tiles - 1) / row_tiles);  // tiles of equal height
-    const int64_t steps = (K + 127) / 128;
+    const int64_t blocks = (M + 15) / 16, steps = (K + 127) / 128;
     int64_t best = 1;
     double best_us = 1e30;
     p.cw = 2;
-    for (int cw = 2; cw <= (p.mb >= 3 && K % 128 == 0 && !p.split ? 4 : 2); cw += 2) {
-        const int kw = 8 / cw;
-        const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
-        for (int64_t z = 1; z <= 16 && z <= steps; ++z) {
-            if (z > 1 && z * M * N > room_floats) break;
-            const int64_t per = (steps + z - 1) / z, rounds = (per + kw - 1) / kw, real = (steps + per - 1) / per;
-            if (real != z) continue;
-            const double waves = static_cast<double>((tiles * z + units - 1) / units);
-            const double round_us = wide ? 0.2 + 2.1 * p.mb : cw == 2 ? 0.5 + 0.18 * p.mb : 0.45 + 0.13 * p.mb;
-            const double us = waves * (4.0 + round_us * static_cast<double>(rounds)) + (z == 1 ? 0.0 : 2.0 + static_cast<double>(z * M * N) * 8.0 / 4e6);
-            if (us < best_us) { best_us = us; best = z; p.cw = cw; }
+    for (int cw = 2; cw <= (K % 128 == 0 && !p.split && !wide ? 4 : 2); cw += 2) {
+        // 64 channels: tiles of equal height, as few as the tallest allows; 128 channels: any height that tiles of equal height can have
+        const int kw = 8 / cw, most = wide ? 2 : cw == 2 ? 4 : 8;
+        const int64_t fewest = (blocks + most - 1) / most;
+        const int tallest = static_cast<int>((blocks + fewest - 1) / fewest);
+        for (int mb = tallest; mb >= (cw == 2 ? tallest : 3); --mb) {
+            const int64_t row_tiles = (blocks + mb - 1) / mb;
+            if ((blocks + row_tiles - 1) / row_tiles != mb) continue;
+            const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
+            for (int64_t z = 1; z <= 16 && z <= steps; ++z) {
+                if (z > 1 && z * M * N > room_floats) break;
+                const int64_t per = (steps + z - 1) / z, rounds = (per + kw - 1) / kw, real = (steps + per - 1) / per;
+                if (real != z) continue;
+                const double waves = static_cast<double>((tiles * z + units - 1) / units);
+                const double round_us = wide ? 0.2 + 2.1 * mb : cw == 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb;
+                const double us = waves * (4.0 + round_us * static_cast<double>(rounds)) + (z == 1 ? 0.0 : 2.0 + static_cast<double>(z * M * N) * 8.0 / 4e6);
+                if (us < best_us) { best_us = us; best = z; p.cw = cw; p.mb = mb; }
+            }
         }
     }
     if (const char* e = tuning_env("TPQ_ROWS_SLICES")) best = std::atoi(e);
@@ -702,6 +709,10 @@ int launch_packed_rows(PackedRowsArgs a, const PackedRowsPlan& p, hipStream_t s)
     else if (p.mb == 2) rc = launch_packed_rows_as<DT, Source, 2, 2>(a, p, s);
     else {
         if constexpr (DT == TPQ_DTYPE_F32) rc = fail(TPQ_ERR_RUNTIME, "packed rows: no such tile");
+        else if (p.mb == 8) rc = launch_packed_rows_shape<DT, Source, 8, 4, false, false>(a, p.slices, s);
+        else if (p.mb == 7) rc = launch_packed_rows_shape<DT, Source, 7, 4, false, false>(a, p.slices, s);
+        else if (p.mb == 6) rc = launch_packed_rows_shape<DT, Source, 6, 4, false, false>(a, p.slices, s);
+        else if (p.mb == 5) rc = launch_packed_rows_shape<DT, Source, 5, 4, false, false>(a, p.slices, s);
         else if (p.mb == 3) rc = wide ? launch_packed_rows_as<DT, Source, 3, 4>(a, p, s) : launch_packed_rows_as<DT, Source, 3, 2>(a, p, s);
         else rc = wide ? launch_packed_rows_as<DT, Source, 4, 4>(a, p, s) : launch_packed_rows_as<DT, Source, 4, 2>(a, p, s);
     }

@@ -12,7 +12,9 @@ UNIT = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.
 # (M, N, K, group): one and two rounds of four steps of 128 k, rounds of which the last is partial, several slices of k, rows at
 # and one past the edges of 16- and 64-row tiles, channels that leave a tile of 64 (128) partly empty, a last step of 32, 64, 96 k
 SHAPES = [(1, 64, 32, 32), (16, 72, 512, 128), (17, 136, 544, 32), (33, 264, 1024, 64), (48, 64, 2048, 128), (49, 200, 4032, 64),
-          (64, 520, 4096, 128), (65, 72, 1152, 128), (128, 1032, 8192, 128), (130, 4104, 608, 32), (200, 2056, 1280, 128)]
+          (64, 520, 4096, 128), (65, 72, 1152, 128), (128, 1032, 8192, 128), (130, 4104, 608, 32), (200, 2056, 1280, 128),
+          # tiles of 80, 96, 112 and 128 rows (16-bit; taken where fewer tall tiles fit the compute units at once), one to four rounds
+          (75, 25608, 256, 64), (90, 25608, 640, 128), (112, 25608, 256, 32), (127, 25608, 896, 128)]
 
 
 def _check(got, x, w, bias, scale_max, dtype):
@@ -54,7 +56,7 @@ def test_int4_rows(dtype, M, N, K, group):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("bits,lsb_first", [(1, False), (1, True), (2, False), (4, False), (8, False)])
-@pytest.mark.parametrize("M,N,K,group", [(17, 68, 160, 32), (33, 264, 1056, 96), (64, 200, 4096, 512), (130, 1028, 640, 128)])
+@pytest.mark.parametrize("M,N,K,group", [(17, 68, 160, 32), (33, 264, 1056, 96), (64, 200, 4096, 512), (130, 1028, 640, 128), (90, 25604, 256, 32), (127, 25604, 640, 128)])
 def test_lowbit_rows(dtype, bits, lsb_first, M, N, K, group):
     from tensorplay_amd import _lib, ops
 
