@@ -223,6 +223,17 @@ int tpq_ternary_linear_row(const void* x, int x_dtype, const uint8_t* packed, fl
                            int64_t K, float eps, float* out, void* stream);
 
 /*
+ * The same of M > 0 activation rows x [M, K] with the codes (int8 [M, K], 16-byte aligned) and scales (f32 [M]) of the rows in the
+ * caller's memory: tpq_quantize_rowwise and tpq_ternary_mm_ws, with the same result bits.  Where the weight is written out as int8
+ * rows first (a workspace of tpq_ternary_linear_workspace_bytes, K % 4 == 0, 8 <= K <= 16384, x 16-byte aligned), one launch does
+ * that and quantizes the rows; what codes holds afterwards is unspecified then.
+ */
+int64_t tpq_ternary_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int tpq_ternary_linear(const void* x, int x_dtype, const uint8_t* packed, float w_scale, const float* bias, int64_t M, int64_t N,
+                       int64_t K, float eps, int8_t* codes, float* row_scales, float* out, void* workspace, int64_t workspace_bytes,
+                       void* stream);
+
+/*
  * The int4 and n-bit weight-only products for a block of activation rows (about 17 .. 500; any count is taken), float32 /
  * float16 / bfloat16, groups of any multiple of 32 (int4: 32, 64 or 128, innerKTiles = 2), K % 32 == 0; anything else
  * returns TPQ_ERR_UNSUPPORTED.  Same operations and reference lines as tpq_int4_mm and tpq_lowbit_mm (1, 2, 4, 8 bits); the

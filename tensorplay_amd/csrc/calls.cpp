@@ -39,7 +39,7 @@ struct Library {
 #define TPQ_ENTRY(NAME) decltype(&::NAME) NAME = nullptr;
 #define TPQ_ENTRIES                                                                                                       \
     TPQ_ENTRY(tpq_quantize_rowwise) TPQ_ENTRY(tpq_int8_mm_workspace_bytes) TPQ_ENTRY(tpq_int8_mm_dequant_ws)                \
-    TPQ_ENTRY(tpq_ternary_mm_workspace_bytes) TPQ_ENTRY(tpq_ternary_mm_ws) TPQ_ENTRY(tpq_ternary_linear_row)                \
+    TPQ_ENTRY(tpq_ternary_linear_workspace_bytes) TPQ_ENTRY(tpq_ternary_linear_row) TPQ_ENTRY(tpq_ternary_linear)                \
     TPQ_ENTRY(tpq_int4_mm_ws)                                                                                             \
     TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
     TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
@@ -309,13 +309,10 @@ TPQ_CALL(ternary_linear, 6)
                                                 static_cast<float>(eps), out_ptr<float>(out), q.stream);
         }
         if (!one_launch || status != TPQ_OK) {
-            const Quantized room = room_for_codes(*x, M, K, lib.tpq_ternary_mm_workspace_bytes(M, N, K));
+            const Quantized room = room_for_codes(*x, M, K, lib.tpq_ternary_linear_workspace_bytes(M, N, K));
             if (!one_launch) out = allocate(sizes, at::kFloat, *x);
-            status = lib.tpq_quantize_rowwise(x->const_data_ptr(), float_tag(x->scalar_type()), M, K, static_cast<float>(eps), 127.0f, -127, 127, 0, room.codes, room.scales,
-                                              q.stream);
-            if (status == TPQ_OK)
-                status = lib.tpq_ternary_mm_ws(room.codes, room.scales, ptr<uint8_t>(packed), static_cast<float>(w_scale), ptr<float>(bias), M, N, K, out_ptr<float>(out),
-                                               TPQ_DTYPE_F32, nullptr, room.scratch, room.scratch_bytes, q.stream);
+            status = lib.tpq_ternary_linear(x->const_data_ptr(), float_tag(x->scalar_type()), ptr<uint8_t>(packed), static_cast<float>(w_scale), ptr<float>(bias), M, N, K,
+                                            static_cast<float>(eps), room.codes, room.scales, out_ptr<float>(out), room.scratch, room.scratch_bytes, q.stream);
         }
     }
     if (status != TPQ_OK) Py_RETURN_NONE;

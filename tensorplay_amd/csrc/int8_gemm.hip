@@ -35,10 +35,12 @@ struct TiledPlan {
     TiledForm form;
     int slices;
 };
-inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, bool may_slice) {
+// weight_cached: the weight was written by the launch before (the ternary product's int8 rows) and comes out of the caches, so
+// "both" does not hold.
+inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, bool may_slice, bool weight_cached = false) {
     const double nk = static_cast<double>((K + kDmaRowBytes - 1) / kDmaRowBytes);
     const int64_t cols = (N + 127) / 128, t256 = ((M + 255) / 256) * cols, t128 = ((M + 127) / 128) * cols;
-    const double stream = 128.0 * static_cast<double>(K) / 12.5;  // a tile's weight bytes at what one compute unit pulls from HBM
+    const double stream = weight_cached ? 0.0 : 128.0 * static_cast<double>(K) / 12.5;  // a tile's weight bytes at what one compute unit pulls from HBM
     const double tall_tile = nk * 1080.0 + 9000.0, short_tile = nk * 690.0 + 8000.0;
     const double tall = static_cast<double>((t256 + 255) / 256) * (tall_tile > stream ? tall_tile : stream);
     const double shrt = static_cast<double>((t128 + 255) / 256) * (short_tile > stream ? short_tile : stream);
@@ -117,12 +119,12 @@ inline int int8_decode_rows(int64_t N) {
 // Slices of the k range the tiled kernel would be cut into for this shape (1: not cut); see dma_slices.
 // With a workspace at hand the decode kernel keeps only what it does in one pass (32 rows): two passes cost more
 // than the sliced kernel (K = N = 8192, 48 rows: 41 us against 28).
-inline int int8_slices(const void* a, const void* w, int64_t M, int64_t N, int64_t K) {
+inline int int8_slices(const void* a, const void* w, int64_t M, int64_t N, int64_t K, bool weight_cached = false) {
     const char* force = tuning_env("TPQ_INT8_KERNEL");
     if (K <= 0 || !mfma_path_ok(a, w, M, N, K) || (force && force[0] == 'r')) return 1;
     const int decode_rows = int8_decode_rows(N) < 32 ? int8_decode_rows(N) : 32;
     if (M <= decode_rows && int8_decode_ok(a, w, M, N, K)) return 1;
-    const TiledPlan plan = plan_tiled(M, N, K, true);
+    const TiledPlan plan = plan_tiled(M, N, K, true, weight_cached);
     return plan.form == kSliced ? plan.slices : 1;
 }
 
@@ -362,17 +364,18 @@ TPQ_EXPORT int tpq_int8_pad_rows(const int8_t* a, int64_t M, const int8_t* w, in
     return check_launch("int8_pad_rows");
 }
 
-TPQ_EXPORT int64_t tpq_int8_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+namespace tpq {
+
+int64_t int8_mm_workspace_bytes(int64_t M, int64_t N, int64_t K, bool weight_cached) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     // operand alignment is checked again at the call; a 16-byte aligned pair stands in for it here
-    const int slices = int8_slices(reinterpret_cast<const void*>(16), reinterpret_cast<const void*>(16), M, N, K);
+    const int slices = int8_slices(reinterpret_cast<const void*>(16), reinterpret_cast<const void*>(16), M, N, K, weight_cached);
     return slices >= 2 ? slices * M * N * 4 : 0;
 }
 
-TPQ_EXPORT int tpq_int8_mm_dequant_ws(const int8_t* a, const int8_t* w, const float* row_scale, const float* col_scale,
-                                      const float* bias, void* out, int out_dtype, int64_t M, int64_t N, int64_t K,
-                                      void* workspace, int64_t workspace_bytes, void* stream) {
-    const int slices = (M > 0 && N > 0 && K > 0 && a && w) ? int8_slices(a, w, M, N, K) : 1;
+int int8_mm_dequant_ws(const int8_t* a, const int8_t* w, const float* row_scale, const float* col_scale, const float* bias, void* out, int out_dtype,
+                       int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream, bool weight_cached) {
+    const int slices = (M > 0 && N > 0 && K > 0 && a && w) ? int8_slices(a, w, M, N, K, weight_cached) : 1;
     if (slices < 2 || workspace == nullptr || workspace_bytes < slices * M * N * 4 || !aligned(workspace, 16) || (M * N) % 4 != 0 ||
         !aligned(col_scale, 16) || !aligned(bias, 16))
         return tpq_int8_mm_dequant(a, w, row_scale, col_scale, bias, out, out_dtype, M, N, K, stream);
@@ -392,6 +395,16 @@ TPQ_EXPORT int tpq_int8_mm_dequant_ws(const int8_t* a, const int8_t* w, const fl
         default: int8_finish_kernel<TPQ_DTYPE_BF16><<<grid, 256, 0, s>>>(acc, slices, row_scale, col_scale, bias, static_cast<uint16_t*>(out), M, N); break;
     }
     return check_launch("int8_mm_dequant (finish)");
+}
+
+}  // namespace tpq
+
+TPQ_EXPORT int64_t tpq_int8_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) { return int8_mm_workspace_bytes(M, N, K, false); }
+
+TPQ_EXPORT int tpq_int8_mm_dequant_ws(const int8_t* a, const int8_t* w, const float* row_scale, const float* col_scale,
+                                      const float* bias, void* out, int out_dtype, int64_t M, int64_t N, int64_t K,
+                                      void* workspace, int64_t workspace_bytes, void* stream) {
+    return int8_mm_dequant_ws(a, w, row_scale, col_scale, bias, out, out_dtype, M, N, K, workspace, workspace_bytes, stream, false);
 }
 
 TPQ_EXPORT int tpq_int_mm_ws(const void* a, int a_unsigned, const int8_t* b, int64_t b_stride_k, int64_t b_stride_n, int32_t* c,

@@ -175,6 +175,79 @@ __device__ __forceinline__ void load_chunk(const typename Elem<DT>::storage* p, 
     unpack_chunk<DT>(load_raw<DT, NT>(p), v);
 }
 
+// Block-wide max over THREADS threads; every thread gets the result.
+template <int THREADS>
+__device__ __forceinline__ float block_max(float v, float* smem) {
+    v = wave_max(v);
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    if (lane == 0) smem[wave] = v;
+    __syncthreads();
+    float r = smem[0];
+#pragma unroll
+    for (int w = 1; w < THREADS / kWave; ++w) r = fmaxf(r, smem[w]);
+    return r;
+}
+
+// eight codes to a dword-aligned address
+__device__ __forceinline__ void store_codes(int8_t* p, uint32_t lo, uint32_t hi) {
+    typedef uint32_t u2 __attribute__((ext_vector_type(2), aligned(4)));
+    *reinterpret_cast<u2*>(p) = u2{lo, hi};
+}
+
+#ifndef TPQ_QUANT_STAMP  // readings of the clock, in a measuring build of the quantizer's own kernels
+#define TPQ_QUANT_STAMP(I) do { } while (0)
+#endif
+
+// One row by a workgroup of THREADS threads, kept in registers between the maximum and the codes: CHUNKS * THREADS * 8 >= K >= 8, K % 4 == 0.
+template <int DT, int CHUNKS, int THREADS>
+__device__ __forceinline__ void quantize_row_cached(const typename Elem<DT>::storage* __restrict__ xr, int8_t* __restrict__ cr,
+                                                    float* __restrict__ scale_out, int K, const QParams& p, float* smem) {
+#ifdef TPQ_QUANT_STAMPS
+    if (threadIdx.x == 0 && blockIdx.x < kStampRows) g_quant_stamps[blockIdx.x * kStampSlots + 6] = __builtin_amdgcn_s_memrealtime();
+#endif
+    TPQ_QUANT_STAMP(0);
+    float v[CHUNKS][kVec];
+    float absmax = 0.0f;
+    // No branch around the loads: at the join of a branch the compiler waits for every outstanding load, which made
+    // the chunks one round trip to memory each.  A chunk past the end re-reads the last chunk of the row: the same
+    // elements again do not change the maximum, and nothing is stored for it.
+    RawChunk<DT> raw[CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) raw[c] = load_raw<DT>(xr + chunk_start((c * THREADS + threadIdx.x) * kVec, K));
+    // The first use stays behind the last request: left to itself the compiler converted a chunk, and waited for it, between two
+    // requests (2048 x 4096 bfloat16 9.4 -> 10.9 us).
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) unpack_chunk<DT>(raw[c], v[c]);
+    TPQ_QUANT_STAMP(1);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+        for (int i = 0; i < kVec; ++i) absmax = fmaxf(absmax, fabsf(v[c][i]));
+    absmax = wave_max(absmax);
+    TPQ_QUANT_STAMP(2);
+    absmax = block_max<THREADS>(absmax, smem);
+    TPQ_QUANT_STAMP(3);
+    const RowScale r = scale_of_row(absmax, p);
+    if (threadIdx.x == 0) *scale_out = r.scale;
+
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const int k0 = (c * THREADS + threadIdx.x) * kVec;
+        if (k0 < K) {
+            uint32_t lo, hi;
+            quantize_eight(v[c], r, p, lo, hi);
+            store_codes(cr + chunk_start(k0, K), lo, hi);
+        }
+    }
+#ifdef TPQ_QUANT_STAMPS
+    TPQ_QUANT_STAMP(4);
+    __builtin_amdgcn_s_waitcnt(0);  // every store of this wavefront acknowledged
+    TPQ_QUANT_STAMP(5);
+    if (threadIdx.x == 0 && blockIdx.x < kStampRows) g_quant_stamps[blockIdx.x * kStampSlots + 7] = __builtin_amdgcn_s_memrealtime();
+#endif
+}
+
 // the parameters of a quantizer: divisor 127, codes -127 .. 127 and its lower-bit relatives
 inline QParams row_quantizer(float eps, float divisor, int qmin, int qmax, int sign_mode) {
     // |v| / scale <= divisor (1 + 2^-22) for every element of the row, whatever the rounding of scale and of the quotient

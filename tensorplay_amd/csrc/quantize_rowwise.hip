@@ -15,16 +15,10 @@
 // p10/src/backend/cpu/LowBitGemmKernels.cpp:19-52):
 //   absmax = max |float(x)|;  scale = fmaxf(absmax, eps) / divisor  (IEEE divide)
 //   code   = clamp(rintf(float(x) / scale), qmin, qmax)              (IEEE divide, RNE)
-#include "quantize_row.h"
+#include "tpq_common.h"
 
 namespace tpq {
 namespace {
-
-constexpr int kThreads = 256;
-// Rows up to this length: one wavefront (or a part of one) per row.  Longer rows on one wavefront were measured
-// (2048 x 4096 bfloat16: 7.0 us against 6.6 with four wavefronts per row, 8.9 against 7.1 from HBM; two wavefronts per
-// row: 8.3 against 7.9): a quarter of the wavefronts to launch, but too few loads in flight per compute unit.
-constexpr int kSubwaveMaxK = 1024;
 
 // -DTPQ_QUANT_STAMPS (a measuring build of its own, never the shipped library): every workgroup of the register-cached
 // kernel leaves six readings of the shader clock (entry, loads issued, own data arrived and reduced, row maximum known,
@@ -43,24 +37,19 @@ __device__ unsigned long long g_quant_stamps[kStampRows * kStampSlots];
 #define TPQ_QUANT_STAMP(I) do { } while (0)
 #endif
 
-// Block-wide max over THREADS threads; every thread gets the result.
-template <int THREADS = kThreads>
-__device__ __forceinline__ float block_max(float v, float* smem) {
-    v = wave_max(v);
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
-    if (lane == 0) smem[wave] = v;
-    __syncthreads();
-    float r = smem[0];
-#pragma unroll
-    for (int w = 1; w < THREADS / kWave; ++w) r = fmaxf(r, smem[w]);
-    return r;
-}
+}  // namespace
+}  // namespace tpq
 
-// eight codes to a dword-aligned address
-__device__ __forceinline__ void store_codes(int8_t* p, uint32_t lo, uint32_t hi) {
-    typedef uint32_t u2 __attribute__((ext_vector_type(2), aligned(4)));
-    *reinterpret_cast<u2*>(p) = u2{lo, hi};
-}
+#include "quantize_row.h"
+
+namespace tpq {
+namespace {
+
+constexpr int kThreads = 256;
+// Rows up to this length: one wavefront (or a part of one) per row.  Longer rows on one wavefront were measured
+// (2048 x 4096 bfloat16: 7.0 us against 6.6 with four wavefronts per row, 8.9 against 7.1 from HBM; two wavefronts per
+// row: 8.3 against 7.9): a quarter of the wavefronts to launch, but too few loads in flight per compute unit.
+constexpr int kSubwaveMaxK = 1024;
 
 // Row cached in registers: CHUNKS * THREADS * 8 >= K >= 8, K % 4 == 0.
 template <int DT, int CHUNKS, int THREADS = kThreads>
@@ -69,53 +58,7 @@ __global__ __launch_bounds__(THREADS) void quantize_rows_cached(
     float* __restrict__ scales, int K, QParams p) {
     __shared__ float smem[THREADS / kWave];
     const int64_t row = blockIdx.x;
-    const auto* xr = x + row * K;
-    int8_t* cr = codes + row * K;
-
-#ifdef TPQ_QUANT_STAMPS
-    if (threadIdx.x == 0 && blockIdx.x < kStampRows) g_quant_stamps[blockIdx.x * kStampSlots + 6] = __builtin_amdgcn_s_memrealtime();
-#endif
-    TPQ_QUANT_STAMP(0);
-    float v[CHUNKS][kVec];
-    float absmax = 0.0f;
-    // No branch around the loads: at the join of a branch the compiler waits for every outstanding load, which made
-    // the chunks one round trip to memory each.  A chunk past the end re-reads the last chunk of the row: the same
-    // elements again do not change the maximum, and nothing is stored for it.
-    RawChunk<DT> raw[CHUNKS];
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) raw[c] = load_raw<DT>(xr + chunk_start((c * THREADS + threadIdx.x) * kVec, K));
-    // The first use stays behind the last request: left to itself the compiler converted a chunk, and waited for it, between two
-    // requests (2048 x 4096 bfloat16 9.4 -> 10.9 us).
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) unpack_chunk<DT>(raw[c], v[c]);
-    TPQ_QUANT_STAMP(1);
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c)
-#pragma unroll
-        for (int i = 0; i < kVec; ++i) absmax = fmaxf(absmax, fabsf(v[c][i]));
-    absmax = wave_max(absmax);
-    TPQ_QUANT_STAMP(2);
-    absmax = block_max<THREADS>(absmax, smem);
-    TPQ_QUANT_STAMP(3);
-    const RowScale r = scale_of_row(absmax, p);
-    if (threadIdx.x == 0) scales[row] = r.scale;
-
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-        const int k0 = (c * THREADS + threadIdx.x) * kVec;
-        if (k0 < K) {
-            uint32_t lo, hi;
-            quantize_eight(v[c], r, p, lo, hi);
-            store_codes(cr + chunk_start(k0, K), lo, hi);
-        }
-    }
-#ifdef TPQ_QUANT_STAMPS
-    TPQ_QUANT_STAMP(4);
-    __builtin_amdgcn_s_waitcnt(0);  // every store of this wavefront acknowledged
-    TPQ_QUANT_STAMP(5);
-    if (threadIdx.x == 0 && blockIdx.x < kStampRows) g_quant_stamps[blockIdx.x * kStampSlots + 7] = __builtin_amdgcn_s_memrealtime();
-#endif
+    quantize_row_cached<DT, CHUNKS, THREADS>(x + row * K, codes + row * K, scales + row, K, p, smem);
 }
 
 // Short rows (8 <= K <= LANES * CHUNKS * 8, K % 4 == 0): LANES lanes of a wavefront per row, so a workgroup
@@ -172,7 +115,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_streaming(
     int8_t* cr = codes + row * K;
     float absmax = 0.0f;
     for (int64_t k = threadIdx.x; k < K; k += kThreads) absmax = fmaxf(absmax, fabsf(Elem<DT>::load(xr[k])));
-    absmax = block_max(absmax, smem);
+    absmax = block_max<kThreads>(absmax, smem);
     const float scale = __fdiv_rn(fmaxf(absmax, p.eps), p.divisor);
     if (threadIdx.x == 0) scales[row] = scale;
     for (int64_t k = threadIdx.x; k < K; k += kThreads)

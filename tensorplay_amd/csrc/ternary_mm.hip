@@ -32,6 +32,12 @@
 #include "ternary_slab_kernel.h"
 
 namespace tpq {
+
+// int8_gemm.hip: tpq_int8_mm_workspace_bytes and tpq_int8_mm_dequant_ws for a weight that the launch before wrote
+int64_t int8_mm_workspace_bytes(int64_t M, int64_t N, int64_t K, bool weight_cached);
+int int8_mm_dequant_ws(const int8_t* a, const int8_t* w, const float* row_scale, const float* col_scale, const float* bias, void* out, int out_dtype,
+                       int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream, bool weight_cached);
+
 namespace {
 
 constexpr int kRowsPerWave = 4;
@@ -128,6 +134,11 @@ __global__ __launch_bounds__(256) void ternary_generic_kernel(const int8_t* __re
 // 40 / 45, 45 / 81; 1024 -> 2048 11 / 6, 12.5 / 10.5, 13 / 19.  K that is no multiple of 256 (the tile kernel's stage):
 // 1920 -> 5504 at 256 rows 20 / 45; K % 64 != 0, where one thread computed an output: 3412 <-> 7872 at 759 rows (both
 // linears) 0.1 ms / 90 ms.
+// In the linear, whose row quantizer runs beside the expansion, that is 3 - 5 us less and pays earlier.  Measured with the quantizer (us,
+// expanded / packed kernels, weights from HBM, bfloat16; the packed kernels step up behind every 128 rows): 256 rows 2560 -> 6912 23.0 / 20.6,
+// 4096 -> 8192 30 / 28.4, 8192 -> 4096 41 / 32; 384 rows 23.6 / 27.7, 32.5 / 40, 38.6 / 46.4, 3072 -> 8192 27.8 / 33.4, but 6912 -> 2560 33 / 28.5,
+// 4096 x 4096 26.4 / 26.9; 512 rows 6912 -> 2560 33.7 / 39, 4096 x 4096 28.7 / 29.2, 1024 -> 4096 13.9 / 14.3, 1536 -> 2048 14.5 / 11.1; 640
+// rows 1024 -> 4096 15.9 / 19, 4096 x 4096 29.3 / 38.8, 1536 -> 2048 16.4 / 16.1; 1024 rows 2048 -> 1024 16.8 / 13.9.
 inline int64_t ternary_padded_k(int64_t K) { return (K + 127) / 128 * 128; }
 inline int64_t round_up_256(int64_t v) { return (v + 255) / 256 * 256; }
 
@@ -140,7 +151,7 @@ inline ExpandedPlan plan_expanded(int64_t M, int64_t N, int64_t K) {
     p.x_at = round_up_256(N * p.kp);
     p.scale_at = p.x_at + (p.kp == K ? 0 : round_up_256(M * p.kp));
     p.gemm_at = p.scale_at + round_up_256(N * 4);
-    p.gemm_bytes = tpq_int8_mm_workspace_bytes(M, N, p.kp);
+    p.gemm_bytes = int8_mm_workspace_bytes(M, N, p.kp, true);
     p.total = p.gemm_at + p.gemm_bytes;
     return p;
 }
@@ -152,30 +163,37 @@ inline bool ternary_packed_kernel_takes(int64_t M, int64_t N, int64_t K) {
     return ternary_slab_splits(M, N, K) >= 1 || K % kTgStage == 0;
 }
 
-inline bool ternary_wants_expanded(int64_t M, int64_t N, int64_t K) {
+inline bool ternary_wants_expanded(int64_t M, int64_t N, int64_t K, bool linear) {
     if (M < 1 || N < 1 || K < 1 || M > 0x7FFFFFFF || N > 0x7FFFFFF0 || K > 0x7FFFFF00) return false;
     if (!ternary_packed_kernel_takes(M, N, K)) return true;
     if (const char* e = tuning_env("TPQ_TERNARY_EXPAND")) return M >= std::atoll(e);
-    return M >= 1280 || (M > 640 && N * K >= (int64_t{1} << 23));
+    const int64_t weights = N * K;
+    if (M >= 1280 || (M > 640 && weights >= (int64_t{1} << 23))) return true;
+    return linear && ((M > 512 && weights >= (int64_t{1} << 22)) || (M > 384 && weights >= (int64_t{1} << 24)) ||
+                      (M > 256 && (weights >= (int64_t{3} << 23) || (weights >= (int64_t{1} << 24) && N >= 2 * K))));
 }
 
-// grid-stride over 16-byte chunks: first the weight's (a packed 32-bit word each), then the activations' (if x_out)
-__global__ __launch_bounds__(256) void ternary_expand_kernel(const uint8_t* __restrict__ packed, const int8_t* __restrict__ x, int64_t chunks_w,
-                                                             int64_t chunks, int N, int K, int chunks_per_row, float w_scale, uint4* __restrict__ w_out,
-                                                             uint4* __restrict__ x_out, float* __restrict__ scales) {
+// Chunks first, first + stride, ... of the weight's int8 rows (16 bytes, a packed 32-bit word each).  Rows without padding are one
+// flat run of words: no row to find, and four words are requested before the first is written out.
+__device__ __forceinline__ void expand_weight(const uint8_t* __restrict__ packed, int64_t chunks_w, int K, int chunks_per_row, int64_t first, int64_t stride,
+                                              uint4* __restrict__ w_out) {
     typedef uint32_t word_unaligned __attribute__((aligned(1)));
-    const int64_t bpr = (K + 3) >> 2;
-    const int64_t first = blockIdx.x * 256ll + threadIdx.x, stride = gridDim.x * 256ll;
-    for (int64_t i = first; i < N; i += stride) scales[i] = w_scale;
-    for (int64_t i = first; i < chunks; i += stride) {
-        const bool of_w = i < chunks_w;
-        const int64_t j = of_w ? i : i - chunks_w;
-        const int64_t row = j < 0x7FFFFFFF ? static_cast<uint32_t>(j) / static_cast<uint32_t>(chunks_per_row) : j / chunks_per_row;
-        const int k = static_cast<int>(j - row * chunks_per_row) * 16, left = K - k;
-        if (!of_w) {
-            x_out[j] = load_k16_ragged(x + row * K + k, left);
-            continue;
+    if (chunks_per_row * 16 == K) {
+        const word_unaligned* const words = reinterpret_cast<const word_unaligned*>(packed);
+        for (int64_t i = first; i < chunks_w; i += 4 * stride) {
+            uint32_t word[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) word[j] = words[i + j * stride < chunks_w ? i + j * stride : i];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (i + j * stride < chunks_w) w_out[i + j * stride] = ternary_word_to_i8x16(word[j]);
         }
+        return;
+    }
+    const int64_t bpr = (K + 3) >> 2;
+    for (int64_t i = first; i < chunks_w; i += stride) {
+        const int64_t row = i < 0x7FFFFFFF ? static_cast<uint32_t>(i) / static_cast<uint32_t>(chunks_per_row) : i / chunks_per_row;
+        const int k = static_cast<int>(i - row * chunks_per_row) * 16, left = K - k;
         uint4 codes = make_uint4(0, 0, 0, 0);
         if (left >= 16) {
             codes = ternary_word_to_i8x16(*reinterpret_cast<const word_unaligned*>(packed + row * bpr + (k >> 2)));
@@ -189,25 +207,88 @@ __global__ __launch_bounds__(256) void ternary_expand_kernel(const uint8_t* __re
             }
             codes = ternary_word_to_i8x16(word);
         }
-        w_out[j] = codes;
+        w_out[i] = codes;
     }
+}
+
+// the weight and its scales, then the activation codes in rows of chunks_per_row chunks (if x_out)
+__global__ __launch_bounds__(256) void ternary_expand_kernel(const uint8_t* __restrict__ packed, const int8_t* __restrict__ x, int64_t chunks_w,
+                                                             int64_t chunks_x, int N, int K, int chunks_per_row, float w_scale, uint4* __restrict__ w_out,
+                                                             uint4* __restrict__ x_out, float* __restrict__ scales) {
+    const int64_t first = blockIdx.x * 256ll + threadIdx.x, stride = gridDim.x * 256ll;
+    for (int64_t i = first; i < N; i += stride) scales[i] = w_scale;
+    expand_weight(packed, chunks_w, K, chunks_per_row, first, stride, w_out);
+    for (int64_t i = first; i < chunks_x; i += stride) {
+        const int64_t row = i < 0x7FFFFFFF ? static_cast<uint32_t>(i) / static_cast<uint32_t>(chunks_per_row) : i / chunks_per_row;
+        const int k = static_cast<int>(i - row * chunks_per_row) * 16;
+        x_out[i] = load_k16_ragged(x + row * K + k, K - k);
+    }
+}
+
+// workgroups that write the weight out: four chunks a thread
+inline unsigned expand_blocks(int64_t chunks) {
+    const int64_t blocks = (chunks + 1023) / 1024;
+    return static_cast<unsigned>(blocks > 16384 ? 16384 : blocks);
+}
+
+// The row quantizer and the expansion in one launch: neither needs the other, and each by itself leaves the chip waiting (a row is a
+// round trip, a reduction and a write; the expansion 7 us of stores).  Workgroups 0 .. M - 1 quantize a row each, straight into rows of
+// kp bytes (what lies behind K meets the weight's zeros), the others expand.  CHUNKS * 2048 >= K >= 8, K % 4 == 0.
+template <int DT, int CHUNKS>
+__global__ __launch_bounds__(256) void ternary_quantize_expand_kernel(const typename Elem<DT>::storage* __restrict__ x, int M, int K, int kp, QParams p,
+                                                                      int8_t* __restrict__ codes, float* __restrict__ row_scales,
+                                                                      const uint8_t* __restrict__ packed, int64_t chunks_w, int N, float w_scale,
+                                                                      uint4* __restrict__ w_out, float* __restrict__ scales) {
+    __shared__ float smem[4];
+    if (blockIdx.x < static_cast<unsigned>(M)) {
+        const int64_t row = blockIdx.x;
+        quantize_row_cached<DT, CHUNKS, 256>(x + row * K, codes + row * kp, row_scales + row, K, p, smem);
+        return;
+    }
+    const int64_t first = (blockIdx.x - static_cast<unsigned>(M)) * 256ll + threadIdx.x, stride = (gridDim.x - static_cast<unsigned>(M)) * 256ll;
+    for (int64_t i = first; i < N; i += stride) scales[i] = w_scale;
+    expand_weight(packed, chunks_w, K, kp / 16, first, stride, w_out);
+}
+
+constexpr int64_t kQuantizeExpandMaxK = 8 * 2048, kQuantizeExpandMaxRows = int64_t{1} << 30;
+
+template <int DT>
+int launch_quantize_expand(const void* x, int64_t M, int64_t N, int64_t K, const ExpandedPlan& p, const QParams& q, int8_t* codes, float* row_scales,
+                           const uint8_t* packed, float w_scale, int8_t* w8, float* scales, hipStream_t s) {
+    const int64_t chunks_w = N * (p.kp / 16);
+    const dim3 grid(static_cast<unsigned>(M) + expand_blocks(chunks_w));
+    auto run = [&](auto chunks) {
+        ternary_quantize_expand_kernel<DT, decltype(chunks)::value><<<grid, 256, 0, s>>>(
+            static_cast<const typename Elem<DT>::storage*>(x), static_cast<int>(M), static_cast<int>(K), static_cast<int>(p.kp), q, codes, row_scales, packed, chunks_w,
+            static_cast<int>(N), w_scale, reinterpret_cast<uint4*>(w8), scales);
+    };
+    if (K <= 2048) run(std::integral_constant<int, 1>{});
+    else if (K <= 2 * 2048) run(std::integral_constant<int, 2>{});
+    else if (K <= 4 * 2048) run(std::integral_constant<int, 4>{});
+    else run(std::integral_constant<int, 8>{});
+    return check_launch("tpq_ternary_linear (quantize, expand)");
+}
+
+// the int8 product of rows of kp codes with the weight written out in the workspace
+int multiply_expanded(const int8_t* x, const float* row_scale, const float* bias, int64_t M, int64_t N, void* out, int out_dtype, const ExpandedPlan& p,
+                      char* ws, hipStream_t s) {
+    return int8_mm_dequant_ws(x, reinterpret_cast<const int8_t*>(ws), row_scale, reinterpret_cast<const float*>(ws + p.scale_at), bias, out, out_dtype, M, N, p.kp,
+                              p.gemm_bytes ? ws + p.gemm_at : nullptr, p.gemm_bytes, s, true);
 }
 
 int launch_ternary_expanded(const int8_t* x, const float* row_scale, const uint8_t* packed, float w_scale, const float* bias, int64_t M, int64_t N,
                             int64_t K, void* out, int out_dtype, const ExpandedPlan& p, void* workspace, hipStream_t s) {
     char* const ws = static_cast<char*>(workspace);
     const bool copy_x = p.kp != K;
-    const int64_t chunks_w = N * (p.kp / 16), chunks = chunks_w + (copy_x ? M * (p.kp / 16) : 0);
+    const int64_t chunks_w = N * (p.kp / 16), chunks_x = copy_x ? M * (p.kp / 16) : 0;
     int8_t* const w8 = reinterpret_cast<int8_t*>(ws);
     int8_t* const x8 = reinterpret_cast<int8_t*>(ws + p.x_at);
     float* const scales = reinterpret_cast<float*>(ws + p.scale_at);
-    const int64_t blocks = (chunks + 255) / 256;
-    ternary_expand_kernel<<<static_cast<unsigned>(blocks > 16384 ? 16384 : blocks), 256, 0, s>>>(
-        packed, x, chunks_w, chunks, static_cast<int>(N), static_cast<int>(K), static_cast<int>(p.kp / 16), w_scale, reinterpret_cast<uint4*>(w8),
+    ternary_expand_kernel<<<expand_blocks(chunks_w + chunks_x), 256, 0, s>>>(
+        packed, x, chunks_w, chunks_x, static_cast<int>(N), static_cast<int>(K), static_cast<int>(p.kp / 16), w_scale, reinterpret_cast<uint4*>(w8),
         reinterpret_cast<uint4*>(x8), scales);
     if (int rc = check_launch("tpq_ternary_mm (expand)")) return rc;
-    return tpq_int8_mm_dequant_ws(copy_x ? x8 : x, w8, row_scale, scales, bias, out, out_dtype, M, N, p.kp, p.gemm_bytes ? ws + p.gemm_at : nullptr,
-                                  p.gemm_bytes, s);
+    return multiply_expanded(copy_x ? x8 : x, row_scale, bias, M, N, out, out_dtype, p, ws, s);
 }
 
 template <class Epilogue>
@@ -269,11 +350,22 @@ int launch_ternary(const int8_t* x, const uint8_t* packed, int64_t M, int64_t N,
 
 using namespace tpq;
 
-TPQ_EXPORT int64_t tpq_ternary_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (ternary_wants_expanded(M, N, K)) return plan_expanded(M, N, K).total;
+namespace tpq {
+namespace {
+// Does the row quantizer go with the expansion?  (its codes and x are aligned as allocations are)
+inline bool quantize_expand_takes(int64_t M, int64_t K) { return K % 4 == 0 && K >= kVec && K <= kQuantizeExpandMaxK && M <= kQuantizeExpandMaxRows; }
+
+inline int64_t ternary_workspace_bytes(int64_t M, int64_t N, int64_t K, bool linear) {
+    if (ternary_wants_expanded(M, N, K, linear)) return plan_expanded(M, N, K).total;
     const int splits = M > 0 && N > 0 && K > 0 ? ternary_slab_splits(M, N, K) : 0;
     return splits > 1 ? static_cast<int64_t>(splits) * M * N * 4 : 0;
 }
+}  // namespace
+}  // namespace tpq
+
+TPQ_EXPORT int64_t tpq_ternary_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) { return ternary_workspace_bytes(M, N, K, false); }
+
+TPQ_EXPORT int64_t tpq_ternary_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) { return ternary_workspace_bytes(M, N, K, quantize_expand_takes(M, K)); }
 
 TPQ_EXPORT int tpq_ternary_mm(const int8_t* x, const float* row_scale, const uint8_t* packed,
                               float w_scale, const float* bias, int64_t M, int64_t N, int64_t K,
@@ -294,7 +386,7 @@ TPQ_EXPORT int tpq_ternary_mm_ws(const int8_t* x, const float* row_scale, const 
                 "bitnet_linear_packed: null pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
     // (the raw sums are an output of the packed kernels only)
-    if (workspace != nullptr && !acc_out && K > 0 && aligned(workspace, 16) && aligned(x, 16) && ternary_wants_expanded(M, N, K)) {
+    if (workspace != nullptr && !acc_out && K > 0 && aligned(workspace, 16) && aligned(x, 16) && ternary_wants_expanded(M, N, K, false)) {
         const ExpandedPlan plan = plan_expanded(M, N, K);
         if (workspace_bytes >= plan.total)
             return launch_ternary_expanded(x, row_scale, packed, w_scale, bias, M, N, K, out, out_dtype, plan, workspace, s);
@@ -313,6 +405,30 @@ TPQ_EXPORT int tpq_ternary_mm_ws(const int8_t* x, const float* row_scale, const 
             return launch_ternary(x, packed, M, N, K, ep, s, workspace, workspace_bytes);
         }
     }
+}
+
+TPQ_EXPORT int tpq_ternary_linear(const void* x, int x_dtype, const uint8_t* packed, float w_scale, const float* bias, int64_t M, int64_t N,
+                                  int64_t K, float eps, int8_t* codes, float* row_scales, float* out, void* workspace, int64_t workspace_bytes,
+                                  void* stream) {
+    TPQ_REQUIRE(M > 0 && N > 0 && K > 0 && x && packed && codes && row_scales && out, TPQ_ERR_INVALID_VALUE, "ternary_linear: empty shape or null pointer");
+    TPQ_REQUIRE(x_dtype == TPQ_DTYPE_F32 || x_dtype == TPQ_DTYPE_F16 || x_dtype == TPQ_DTYPE_BF16, TPQ_ERR_INVALID_TYPE, "ternary_linear: unsupported input dtype");
+    if (workspace != nullptr && aligned(workspace, 16) && aligned(x, 16) && aligned(codes, 16) && quantize_expand_takes(M, K) &&
+        ternary_wants_expanded(M, N, K, true)) {
+        const ExpandedPlan plan = plan_expanded(M, N, K);
+        if (workspace_bytes >= plan.total) {
+            char* const ws = static_cast<char*>(workspace);
+            int8_t* const w8 = reinterpret_cast<int8_t*>(ws);
+            int8_t* const x8 = plan.kp == K ? codes : reinterpret_cast<int8_t*>(ws + plan.x_at);
+            float* const scales = reinterpret_cast<float*>(ws + plan.scale_at);
+            hipStream_t s = static_cast<hipStream_t>(stream);
+            const QParams quantizer = row_quantizer(eps, 127.0f, -127, 127, 0);
+            const auto launch = x_dtype == TPQ_DTYPE_F32 ? launch_quantize_expand<TPQ_DTYPE_F32> : x_dtype == TPQ_DTYPE_F16 ? launch_quantize_expand<TPQ_DTYPE_F16> : launch_quantize_expand<TPQ_DTYPE_BF16>;
+            if (int rc = launch(x, M, N, K, plan, quantizer, x8, row_scales, packed, w_scale, w8, scales, s)) return rc;
+            return multiply_expanded(x8, row_scales, bias, M, N, out, TPQ_DTYPE_F32, plan, ws, s);
+        }
+    }
+    if (int rc = tpq_quantize_rowwise(x, x_dtype, M, K, eps, 127.0f, -127, 127, 0, codes, row_scales, stream)) return rc;
+    return tpq_ternary_mm_ws(codes, row_scales, packed, w_scale, bias, M, N, K, out, TPQ_DTYPE_F32, nullptr, workspace, workspace_bytes, stream);
 }
 
 TPQ_EXPORT int tpq_ternary_linear_row(const void* x, int x_dtype, const uint8_t* packed, float w_scale, const float* bias, int64_t N, int64_t K,

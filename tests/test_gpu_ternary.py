@@ -220,3 +220,32 @@ def test_one_row_linear_on_both_sides_of_the_rule(k, n):
     x = torch.randn(1, k, device="cuda", generator=gen).half()
     codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
     assert torch.equal(ops._ternary_linear(x, packed, 0.037, k, None, 1e-5), ops.ternary_mm(codes, scale, packed, 0.037, k))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,k,n", [
+    # rows of whole and of padded stages; one, two, four and eight chunks of the row quantizer, each at an edge; the longest row and one beyond
+    (1300, 128, 40), (1281, 2048, 33), (33, 2052, 9), (700, 4096, 2049), (3, 4100, 70), (40, 8188, 17), (5, 16380, 3), (1280, 16384, 8), (2, 16388, 5),
+    # the shortest row, rows that are no multiple of four, one channel, words of the packed weight that do not start on a word
+    (5, 8, 6), (9, 4, 3), (7, 1023, 24), (1, 3788, 40), (1300, 60, 1), (40, 332, 5)])
+def test_rows_quantized_beside_the_expansion(m, k, n, dtype):
+    """The linear whose weight is written out as int8 rows: the bits of the row quantizer followed by the product, for ordinary rows and
+    for ones whose maximum is below eps, infinite, NaN or in the last element, several calls one after another."""
+    from tensorplay_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    packed = torch.randint(0, 256, (n, (k + 3) // 4), device="cuda", generator=gen, dtype=torch.uint8)
+    bias = torch.randn(n, device="cuda", generator=gen)
+    x = torch.randn(m, k, device="cuda", generator=gen)
+    if m > 4:
+        x[0] = 0.0
+        x[1, k // 2] = float("inf")
+        x[2, 0] = float("nan")
+        x[3, k - 1] = -300.0
+        x[4] *= 1e-7
+    x = x.to(dtype)
+    codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
+    for b in (None, bias, None):
+        want = ops.ternary_mm(codes, scale, packed, 0.037, k, bias=b)
+        got = ops._ternary_linear(x, packed, 0.037, k, b, 1e-5)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
