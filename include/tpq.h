@@ -62,6 +62,21 @@ int tpq_quantize_rowwise(const void* x, int x_dtype, int64_t M, int64_t K, float
                          float* scales, void* stream);
 
 /*
+ * The row quantizer and what the product behind it wants of the other operand, in one launch: the same codes and scales as
+ * tpq_quantize_rowwise, in rows of `pitch` bytes (a multiple of 16, K <= pitch < K + 1024) with zeros behind K.
+ *   both: x [M, K] to 8 bits (divisor 127, codes -127 .. 127) and w [N, K] of the same type by the parameters given, the two
+ *         quantizers of a training linear (tensorplay/ao/quantization/int8_dyn_act_int4_weight.py:72-84);
+ *   pad:  x as above and a copy of the int8 weight w [N, K] (any alignment).
+ * M, N > 0, K % 4 == 0, 8 <= K <= 16384, the other operands 16-byte aligned; else TPQ_ERR_UNSUPPORTED.
+ */
+int tpq_quantize_both_rowwise(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K, int64_t pitch, float x_eps,
+                              float w_eps, float w_divisor, int w_qmin, int w_qmax, int w_sign_mode, int8_t* x_codes,
+                              float* x_scales, int8_t* w_codes, float* w_scales, void* stream);
+int tpq_quantize_rowwise_pad(const void* x, int dtype, int64_t M, int64_t K, float eps, const int8_t* w, int64_t N, int64_t pitch,
+                             int8_t* codes, float* scales, int8_t* w_out, void* stream);
+
+
+/*
  * Integer matrix product C[M,N] (int32) = A[M,K] (int8, or uint8 when
  * a_unsigned) x B[K,N] (int8).  B is addressed as b[k*b_stride_k + n*b_stride_n]
  * so both a contiguous [K,N] operand (N,1) and the transposed view of a

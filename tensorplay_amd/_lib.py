@@ -48,6 +48,8 @@ SIGNATURES = {
     "tpq_ternary_mm_workspace_bytes": [_i64, _i64, _i64],
     "tpq_ternary_mm_ws": [_ptr, _ptr, _ptr, _f32, _ptr, _i64, _i64, _i64, _ptr, _int, _ptr, _ptr, _i64, _ptr],
     "tpq_ternary_linear_row": [_ptr, _int, _ptr, _f32, _ptr, _i64, _i64, _f32, _ptr, _ptr],
+    "tpq_quantize_both_rowwise": [_ptr, _ptr, _int, _i64, _i64, _i64, _i64, _f32, _f32, _f32, _int, _int, _int, _ptr, _ptr, _ptr, _ptr, _ptr],
+    "tpq_quantize_rowwise_pad": [_ptr, _int, _i64, _i64, _f32, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr],
     "tpq_ternary_linear_workspace_bytes": [_i64, _i64, _i64],
     "tpq_ternary_linear": [_ptr, _int, _ptr, _f32, _ptr, _i64, _i64, _i64, _f32, _ptr, _ptr, _ptr, _ptr, _i64, _ptr],
     "tpq_int4_mm_add": [_ptr, _int, _i64, _i64, _ptr, _int, _i64, _i64, _ptr, _ptr, _ptr, _ptr],

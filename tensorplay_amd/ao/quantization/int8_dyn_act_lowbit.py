@@ -35,11 +35,23 @@ def _quantize_binary_weight_signed(weight: torch.Tensor):
     return ops._quantize_binary_rowwise(weight, 1e-8)
 
 
+# (eps, divisor, least and largest code, sign mode) of these, for the call that quantizes both operands in one launch
+_ROW_QUANTIZERS = {
+    _quantize_int4_weight_signed: (1e-8, 7.0, -8, 7, False),
+    _quantize_int2_weight_signed: (1e-8, 2.0, -2, 1, False),
+    _quantize_binary_weight_signed: (1e-8, 1.0, -1, 1, True),
+}
+
+
 class _Int8DynActLowBitLinear(torch.autograd.Function):
     """Quantized forward, straight-through backward (reference int8_dyn_act_int4_weight.py:72-95)."""
 
     @staticmethod
     def forward(ctx, input, weight, quantize_weight):
+        row_quantizer = _ROW_QUANTIZERS.get(quantize_weight)
+        if row_quantizer is not None and (out := ops._dynamic_lowbit_linear(input, weight, *row_quantizer)) is not None:
+            ctx.save_for_backward(input, weight)
+            return out
         flat = input.reshape(-1, input.shape[-1])
         x_i8, x_scale = quantize_int8_rowwise(flat.detach())
         w_codes, w_scale = quantize_weight(weight.detach())

@@ -44,7 +44,8 @@ struct Library {
     TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
     TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
     TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine) \
-    TPQ_ENTRY(tpq_f32_linear_grads_workspace_bytes) TPQ_ENTRY(tpq_f32_linear_grads)
+    TPQ_ENTRY(tpq_f32_linear_grads_workspace_bytes) TPQ_ENTRY(tpq_f32_linear_grads) \
+    TPQ_ENTRY(tpq_quantize_both_rowwise) TPQ_ENTRY(tpq_quantize_rowwise_pad)
     TPQ_ENTRIES
 #undef TPQ_ENTRY
 };
@@ -248,7 +249,11 @@ TPQ_CALL(int8_mm_dequant, 7)
     return THPVariable_Wrap(std::move(out));
 TPQ_CALL_END
 
-// int8_linear(x [..., K] float, w int8 [N, K], col_scale, bias or None, eps, out_dtype, ragged_rows): quantize + product
+// Rows of codes that a product of more than ragged_rows rows reads: the next multiple of 128 where K is none of 16
+int64_t code_pitch(int64_t K) { return K % 16 ? (K + 127) / 128 * 128 : K; }
+
+// int8_linear(x [..., K] float, w int8 [N, K], col_scale, bias or None, eps, out_dtype, ragged_rows): quantize + product.  Above ragged_rows
+// rows with K % 16 != 0 the quantizer's launch copies the weight to padded rows as well.
 TPQ_CALL(int8_linear, 7)
     const at::Tensor *x = plain(args[0]), *w = plain(args[1]), *cs = plain(args[2]), *bias;
     double eps;
@@ -261,17 +266,55 @@ TPQ_CALL(int8_linear, 7)
     int64_t M;
     const auto sizes = product_sizes(*x, N, &M);
     const at::ScalarType type = reinterpret_cast<THPDtype*>(args[5])->scalar_type;
-    if (float_tag(type) < 0 || (K % 16 && M > ragged_rows) || !optional_vector(args[3], at::kFloat, N, *x, &bias)) Py_RETURN_NONE;
+    const bool pad = K % 16 != 0 && M > ragged_rows;
+    const int64_t pitch = pad ? code_pitch(K) : K;
+    if (float_tag(type) < 0 || !optional_vector(args[3], at::kFloat, N, *x, &bias)) Py_RETURN_NONE;
     at::Tensor out;
     int status;
     {
         Enqueue q(*x);
-        const Quantized room = room_for_codes(*x, M, K, lib.tpq_int8_mm_workspace_bytes(M, N, K));
+        const Quantized room = room_for_codes(*x, M, pitch, lib.tpq_int8_mm_workspace_bytes(M, N, pitch));
+        const at::Tensor padded_w = pad ? allocate({N, pitch}, at::kChar, *x) : at::Tensor();
         out = allocate(sizes, type, *x);
-        status = lib.tpq_quantize_rowwise(x->const_data_ptr(), float_tag(x->scalar_type()), M, K, static_cast<float>(eps), 127.0f, -127, 127, 0, room.codes, room.scales,
-                                          q.stream);
+        if (pad)
+            status = lib.tpq_quantize_rowwise_pad(x->const_data_ptr(), float_tag(x->scalar_type()), M, K, static_cast<float>(eps), ptr<int8_t>(w), N, pitch, room.codes,
+                                                  room.scales, out_ptr<int8_t>(padded_w), q.stream);
+        else
+            status = lib.tpq_quantize_rowwise(x->const_data_ptr(), float_tag(x->scalar_type()), M, K, static_cast<float>(eps), 127.0f, -127, 127, 0, room.codes, room.scales,
+                                              q.stream);
         if (status == TPQ_OK)
-            status = lib.tpq_int8_mm_dequant_ws(room.codes, ptr<int8_t>(w), room.scales, ptr<float>(cs), ptr<float>(bias), out.data_ptr(), float_tag(type), M, N, K, room.scratch,
+            status = lib.tpq_int8_mm_dequant_ws(room.codes, pad ? out_ptr<int8_t>(padded_w) : ptr<int8_t>(w), room.scales, ptr<float>(cs), ptr<float>(bias), out.data_ptr(),
+                                                float_tag(type), M, N, pitch, room.scratch, room.scratch_bytes, q.stream);
+    }
+    if (status != TPQ_OK) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+TPQ_CALL_END
+
+// lowbit_linear(x [..., K] float, w [N, K] of the same type, x_eps, w_eps, divisor, qmin, qmax, sign_mode) -> float32: rows of both
+// quantized in one launch (x to 8 bits, w by the parameters given) + product
+TPQ_CALL(lowbit_linear, 8)
+    const at::Tensor *x = plain(args[0]), *w = plain(args[1]);
+    double x_eps, w_eps, divisor;
+    int64_t qmin, qmax, sign_mode;
+    if (!x || !w || !as_float(args[2], &x_eps) || !as_float(args[3], &w_eps) || !as_float(args[4], &divisor) || !as_int(args[5], &qmin) || !as_int(args[6], &qmax) ||
+        !as_int(args[7], &sign_mode) || x->dim() < 1 || x->numel() == 0 || float_tag(x->scalar_type()) < 0 || w->scalar_type() != x->scalar_type() || w->dim() != 2 ||
+        w->numel() == 0 || x->size(-1) != w->size(1) || !same_device(*x, *w))
+        Py_RETURN_NONE;
+    const int64_t K = w->size(1), N = w->size(0), pitch = code_pitch(K);
+    int64_t M;
+    const auto sizes = product_sizes(*x, N, &M);
+    at::Tensor out;
+    int status;
+    {
+        Enqueue q(*x);
+        const Quantized room = room_for_codes(*x, M, pitch, lib.tpq_int8_mm_workspace_bytes(M, N, pitch));
+        const Quantized weight = room_for_codes(*x, N, pitch, 0);
+        out = allocate(sizes, at::kFloat, *x);
+        status = lib.tpq_quantize_both_rowwise(x->const_data_ptr(), w->const_data_ptr(), float_tag(x->scalar_type()), M, N, K, pitch, static_cast<float>(x_eps),
+                                               static_cast<float>(w_eps), static_cast<float>(divisor), static_cast<int>(qmin), static_cast<int>(qmax),
+                                               static_cast<int>(sign_mode), room.codes, room.scales, weight.codes, weight.scales, q.stream);
+        if (status == TPQ_OK)
+            status = lib.tpq_int8_mm_dequant_ws(room.codes, weight.codes, room.scales, weight.scales, nullptr, out.data_ptr(), TPQ_DTYPE_F32, M, N, pitch, room.scratch,
                                                 room.scratch_bytes, q.stream);
     }
     if (status != TPQ_OK) Py_RETURN_NONE;
@@ -525,6 +568,7 @@ PyObject* bind(PyObject*, PyObject* handle_obj) {
 
 #define TPQ_METHOD(NAME) {#NAME, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(NAME)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {TPQ_METHOD(quantize_rowwise), TPQ_METHOD(int8_mm_dequant),  TPQ_METHOD(int8_linear),       TPQ_METHOD(ternary_linear),
+                         TPQ_METHOD(lowbit_linear),
                          TPQ_METHOD(int4_mm),          TPQ_METHOD(lowbit_mm),        TPQ_METHOD(quantize_affine),   TPQ_METHOD(dequantize_affine),
                          TPQ_METHOD(linear_grads),
                          {"bind", bind, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};

@@ -40,6 +40,9 @@ __device__ unsigned long long g_quant_stamps[kStampRows * kStampSlots];
 }  // namespace
 }  // namespace tpq
 
+#include <type_traits>
+
+#include "int8_gemm_kernel.h"
 #include "quantize_row.h"
 
 namespace tpq {
@@ -102,6 +105,76 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_subwave(
             store_codes(cr + chunk_start(k0, K), lo, hi);
         }
     }
+}
+
+// The row quantizer with the preparation of the other operand of the product beside it, in one launch: workgroups 0 .. M - 1 take a row
+// of x each, the others the weight.  Codes go to rows of `pitch` bytes, zeros behind K, so that a product whose K is no multiple of
+// 16 reads both without a pass that copies them.  CHUNKS * 2048 >= K >= 8, K % 4 == 0.
+//
+// Two latency chains (load, reduce, store) that need nothing of each other: one after the other they take the sum of both and a gap.
+// Measured (us, a launch each / this): training step of 512 rows, 2048 -> 4096 (the two quantizers 4.8 and 9.1) 119.1 / 116.8; of 295 rows,
+// 808 -> 3840 (both operands copied to padded rows by a third launch before) 187 / 83, of 43 rows, 928 -> 2960 144 / 84 (host time,
+// as it is for 85 us in every small step); int8 linear, quantizer and copies in two launches / this: 142 rows, 3640 -> 1280 38 / 20,
+// 500 rows, 1060 -> 3000 33 / 15, 3000 rows, 2500 x 2500 49 / 44.
+template <int DT>
+struct SecondRows {  // a float matrix [N][K] quantized by rows
+    const typename Elem<DT>::storage* w;
+    int8_t* codes;
+    float* scales;
+    QParams p;
+};
+struct SecondCopy {  // an int8 matrix [N][K], 16-byte chunks of the copy
+    const int8_t* w;
+    uint4* out;
+    int64_t chunks;
+};
+
+template <int DT, int CHUNKS, class Second>
+__global__ __launch_bounds__(kThreads) void quantize_rows_beside(const typename Elem<DT>::storage* __restrict__ x, int8_t* __restrict__ codes,
+                                                                 float* __restrict__ scales, int M, int K, int pitch, QParams p, Second second) {
+    __shared__ float smem[kThreads / kWave];
+    const bool of_x = blockIdx.x < static_cast<unsigned>(M);
+    if constexpr (std::is_same_v<Second, SecondCopy>) {
+        if (!of_x) {
+            const int chunks_per_row = pitch >> 4;
+            const int64_t stride = (gridDim.x - static_cast<unsigned>(M)) * static_cast<int64_t>(kThreads);
+            for (int64_t j = (blockIdx.x - static_cast<unsigned>(M)) * static_cast<int64_t>(kThreads) + threadIdx.x; j < second.chunks; j += stride) {
+                const int64_t row = j < 0x7FFFFFFF ? static_cast<uint32_t>(j) / static_cast<uint32_t>(chunks_per_row) : j / chunks_per_row;
+                const int k = static_cast<int>(j - row * chunks_per_row) * 16;
+                second.out[j] = load_k16_ragged(second.w + row * K + k, K - k);
+            }
+            return;
+        }
+    }
+    const int64_t row = of_x ? blockIdx.x : blockIdx.x - static_cast<unsigned>(M);
+    const auto* from = x;
+    int8_t* to = codes;
+    float* scale_out = scales;
+    if constexpr (!std::is_same_v<Second, SecondCopy>) {
+        if (!of_x) { from = second.w; to = second.codes; scale_out = second.scales; p = second.p; }
+    }
+    if (static_cast<int>(threadIdx.x) * 4 < pitch - K) *reinterpret_cast<uint32_t*>(to + row * pitch + K + threadIdx.x * 4) = 0;
+    quantize_row_cached<DT, CHUNKS, kThreads>(from + row * K, to + row * pitch, scale_out + row, K, p, smem);
+}
+
+template <int DT, class Second>
+int launch_beside(const void* x, int64_t M, int64_t K, int64_t pitch, int64_t second_blocks, const QParams& p, const Second& second, int8_t* codes, float* scales,
+                  hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>(M + second_blocks));
+    auto run = [&](auto chunks) {
+        quantize_rows_beside<DT, decltype(chunks)::value, Second><<<grid, kThreads, 0, stream>>>(static_cast<const typename Elem<DT>::storage*>(x), codes, scales,
+                                                                                                 static_cast<int>(M), static_cast<int>(K), static_cast<int>(pitch), p, second);
+    };
+    if (K <= 2048) run(std::integral_constant<int, 1>{});
+    else if (K <= 4096) run(std::integral_constant<int, 2>{});
+    else if (K <= 8192) run(std::integral_constant<int, 4>{});
+    else run(std::integral_constant<int, 8>{});
+    return check_launch("tpq_quantize_rowwise (both operands)");
+}
+
+// (pitch - K: what 256 threads clear)
+inline bool beside_takes(int64_t M, int64_t N, int64_t K, int64_t pitch) {
+    return M > 0 && N > 0 && K % 4 == 0 && K >= kVec && K <= 8 * 2048 && pitch >= K && pitch - K < 4 * kThreads && pitch % 16 == 0 && M + N < (int64_t{1} << 31);
 }
 
 // Any K: two passes over the row with scalar accesses.
@@ -192,4 +265,40 @@ TPQ_EXPORT int tpq_quantize_rowwise(const void* x, int x_dtype, int64_t M, int64
         case TPQ_DTYPE_F16: return launch<TPQ_DTYPE_F16>(x, M, K, p, codes, scales, s);
         default: return launch<TPQ_DTYPE_BF16>(x, M, K, p, codes, scales, s);
     }
+}
+
+TPQ_EXPORT int tpq_quantize_both_rowwise(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K, int64_t pitch, float x_eps, float w_eps,
+                                         float w_divisor, int w_qmin, int w_qmax, int w_sign_mode, int8_t* x_codes, float* x_scales, int8_t* w_codes,
+                                         float* w_scales, void* stream) {
+    using namespace tpq;
+    TPQ_REQUIRE(dtype == TPQ_DTYPE_F32 || dtype == TPQ_DTYPE_F16 || dtype == TPQ_DTYPE_BF16, TPQ_ERR_INVALID_TYPE, "rowwise quantize: unsupported input dtype");
+    TPQ_REQUIRE(w_qmin >= -128 && w_qmax <= 127 && w_qmin <= w_qmax && w_divisor > 0.0f, TPQ_ERR_INVALID_VALUE, "quantize_both_rowwise: code range must fit int8 and divisor must be positive");
+    TPQ_REQUIRE(x && w && x_codes && x_scales && w_codes && w_scales, TPQ_ERR_INVALID_VALUE, "quantize_both_rowwise: null pointer");
+    TPQ_REQUIRE(beside_takes(M, N, K, pitch) && aligned(x, 16) && aligned(w, 16) && aligned(x_codes, 16) && aligned(w_codes, 16), TPQ_ERR_UNSUPPORTED,
+                "quantize_both_rowwise: K a multiple of 4, 8 .. 16384, operands 16-byte aligned");
+    const QParams px = row_quantizer(x_eps, 127.0f, -127, 127, 0), pw = row_quantizer(w_eps, w_divisor, w_qmin, w_qmax, w_sign_mode);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    auto run = [&](auto dt) {
+        constexpr int DT = decltype(dt)::value;
+        return launch_beside<DT>(x, M, K, pitch, N, px, SecondRows<DT>{static_cast<const typename Elem<DT>::storage*>(w), w_codes, w_scales, pw}, x_codes, x_scales, s);
+    };
+    if (dtype == TPQ_DTYPE_F32) return run(std::integral_constant<int, TPQ_DTYPE_F32>{});
+    if (dtype == TPQ_DTYPE_F16) return run(std::integral_constant<int, TPQ_DTYPE_F16>{});
+    return run(std::integral_constant<int, TPQ_DTYPE_BF16>{});
+}
+
+TPQ_EXPORT int tpq_quantize_rowwise_pad(const void* x, int dtype, int64_t M, int64_t K, float eps, const int8_t* w, int64_t N, int64_t pitch, int8_t* codes,
+                                        float* scales, int8_t* w_out, void* stream) {
+    using namespace tpq;
+    TPQ_REQUIRE(dtype == TPQ_DTYPE_F32 || dtype == TPQ_DTYPE_F16 || dtype == TPQ_DTYPE_BF16, TPQ_ERR_INVALID_TYPE, "rowwise quantize: unsupported input dtype");
+    TPQ_REQUIRE(x && w && codes && scales && w_out, TPQ_ERR_INVALID_VALUE, "quantize_rowwise_pad: null pointer");
+    TPQ_REQUIRE(beside_takes(M, N, K, pitch) && aligned(x, 16) && aligned(codes, 16) && aligned(w_out, 16), TPQ_ERR_UNSUPPORTED,
+                "quantize_rowwise_pad: K a multiple of 4, 8 .. 16384, operands 16-byte aligned");
+    const QParams p = row_quantizer(eps, 127.0f, -127, 127, 0);
+    const SecondCopy copy{w, reinterpret_cast<uint4*>(w_out), N * (pitch / 16)};
+    const int64_t wanted = (copy.chunks + kThreads - 1) / kThreads, blocks = wanted > 16384 ? 16384 : wanted;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == TPQ_DTYPE_F32) return launch_beside<TPQ_DTYPE_F32>(x, M, K, pitch, blocks, p, copy, codes, scales, s);
+    if (dtype == TPQ_DTYPE_F16) return launch_beside<TPQ_DTYPE_F16>(x, M, K, pitch, blocks, p, copy, codes, scales, s);
+    return launch_beside<TPQ_DTYPE_BF16>(x, M, K, pitch, blocks, p, copy, codes, scales, s);
 }

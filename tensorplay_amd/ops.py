@@ -83,6 +83,13 @@ def _quantize_binary_rowwise(self: torch.Tensor, eps: float) -> Tuple[torch.Tens
     return _quantize_rowwise(self, eps, 1.0, -1, 1, True, "_quantize_binary_rowwise")
 
 
+def _dynamic_lowbit_linear(input: torch.Tensor, weight: torch.Tensor, weight_eps: float, divisor: float, qmin: int, qmax: int, sign_mode: bool):
+    """``_quantize_int8_rowwise`` (eps 1e-5) of the rows of input [..., K], the row quantizer with these parameters of weight [N, K], and their
+    ``int8_mm_dequant`` in float32, where the native call takes them; None elsewhere."""
+    calls = _lib.load().calls if input.is_cuda else None
+    return None if calls is None else calls.lowbit_linear(input, weight, 1e-5, weight_eps, divisor, qmin, qmax, int(sign_mode))
+
+
 def _check_int_mm_operands(self, mat2):
     if self.dim() != 2 or mat2.dim() != 2:
         raise RuntimeError(f"_int_mm: expected two matrices but got {self.dim()}-D and {mat2.dim()}-D tensors")

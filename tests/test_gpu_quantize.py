@@ -92,3 +92,38 @@ def test_non_contiguous_and_empty_and_errors(ops):
         ops._quantize_int8_rowwise(torch.zeros(2, 2, 2, device=DEV), 1e-5)
     with pytest.raises(TypeError):
         ops._quantize_int8_rowwise(torch.zeros(2, 2, device=DEV, dtype=torch.float64), 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,k,n", [
+    # rows read as they are and padded to 128; one, two, four and eight chunks of the quantizer at their edges; the longest row and one beyond
+    (40, 16, 9), (33, 2048, 70), (5, 2052, 33), (129, 4096, 65), (36, 4100, 40), (3, 8188, 17), (2, 16384, 5), (34, 16388, 6),
+    # the shortest row, a row below it, rows that are no multiple of four
+    (40, 8, 5), (40, 4, 5), (35, 1023, 24), (300, 808, 256)])
+def test_both_operands_prepared_in_one_launch(m, k, n, dtype):
+    """The quantizer of the activations beside that of the weight (training linears) or the copy of an int8 weight to padded rows: the
+    bits of the separate operators, for ordinary rows and for ones that are zero, tiny, infinite or NaN, several calls one after another."""
+    from tensorplay_amd import ops
+    from tensorplay_amd.ao.quantization import int8_dyn_act_lowbit as low
+
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    x, w = (torch.randn(r, k, device="cuda", generator=gen) for r in (m, n))
+    for a in (x, w):
+        a[0] = 0.0
+        a[1] *= 1e-9
+        a[-1, k // 2] = -300.0
+    x[m // 2, k - 1] = float("inf")
+    w[n // 2, 0] = float("nan")
+    x, w = x.to(dtype), w.to(dtype)
+    codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
+    for quantize in (low._quantize_int4_weight_signed, low._quantize_int2_weight_signed, low._quantize_binary_weight_signed):
+        w_codes, w_scale = quantize(w)
+        want = ops.int8_mm_dequant(codes, w_codes, scale, w_scale)
+        got = low._Int8DynActLowBitLinear.apply(x, w, quantize)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+    w8, w_scale = ops._quantize_int8_rowwise(torch.randn(n, k, device="cuda", generator=gen), 1e-5)
+    bias = torch.randn(n, device="cuda", generator=gen)
+    for b in (None, bias, None):
+        want = ops.int8_mm_dequant(codes, w8, scale, w_scale, b, torch.float32)
+        got = ops._int8_dynamic_linear(x, w8, w_scale, b, torch.float32)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
