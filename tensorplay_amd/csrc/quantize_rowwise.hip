@@ -172,9 +172,9 @@ int launch_beside(const void* x, int64_t M, int64_t K, int64_t pitch, int64_t se
     return check_launch("tpq_quantize_rowwise (both operands)");
 }
 
-// (pitch - K: what 256 threads clear)
+// (pitch - K: what 256 threads clear; M + N: a workgroup of 256 threads per row, and a launch holds fewer than 2^32 threads)
 inline bool beside_takes(int64_t M, int64_t N, int64_t K, int64_t pitch) {
-    return M > 0 && N > 0 && K % 4 == 0 && K >= kVec && K <= 8 * 2048 && pitch >= K && pitch - K < 4 * kThreads && pitch % 16 == 0 && M + N < (int64_t{1} << 31);
+    return M > 0 && N > 0 && K % 4 == 0 && K >= kVec && K <= 8 * 2048 && pitch >= K && pitch - K < 4 * kThreads && pitch % 16 == 0 && M <= (int64_t{1} << 23) && N <= (int64_t{1} << 23) - 16384;
 }
 
 // Any K: two passes over the row with scalar accesses.

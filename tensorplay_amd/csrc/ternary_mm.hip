@@ -250,7 +250,8 @@ __global__ __launch_bounds__(256) void ternary_quantize_expand_kernel(const type
     expand_weight(packed, chunks_w, K, kp / 16, first, stride, w_out);
 }
 
-constexpr int64_t kQuantizeExpandMaxK = 8 * 2048, kQuantizeExpandMaxRows = int64_t{1} << 30;
+// (a workgroup of 256 threads per row: a launch holds fewer than 2^32 threads)
+constexpr int64_t kQuantizeExpandMaxK = 8 * 2048, kQuantizeExpandMaxRows = int64_t{1} << 23;
 
 template <int DT>
 int launch_quantize_expand(const void* x, int64_t M, int64_t N, int64_t K, const ExpandedPlan& p, const QParams& q, int8_t* codes, float* row_scales,

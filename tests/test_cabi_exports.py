@@ -151,3 +151,14 @@ def test_block_kernel_refuses_parameters_beyond_its_offsets():
     k = (1 << 17) + 32
     status = lib.tpq_lowbit_mm_rows(256, _lib.F16, 40, k, 256, 1, 0, n, 32, 256, None, 256, None, 0, None)
     assert status == _lib.TPQ_ERR_UNSUPPORTED
+
+
+def test_quantizer_beside_the_other_operand_refuses_more_rows_than_a_launch_holds():
+    """A workgroup of 256 threads per row, fewer than 2^32 threads in a launch: more rows go to the separate operators.  Host logic
+    only: no operand is read."""
+    from tensorplay_amd import _lib
+
+    lib = _lib.load()
+    for m, n in ((1 << 24, 16), (16, 1 << 24)):
+        assert lib.tpq_quantize_both_rowwise(256, 256, _lib.F32, m, n, 64, 64, 1e-5, 1e-8, 7.0, -8, 7, 0, 256, 256, 256, 256, None) == _lib.TPQ_ERR_UNSUPPORTED
+        assert lib.tpq_quantize_rowwise_pad(256, _lib.F32, m, 36, 1e-5, 256, n, 128, 256, 256, 256, None) == _lib.TPQ_ERR_UNSUPPORTED
