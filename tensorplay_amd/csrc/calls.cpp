@@ -522,10 +522,11 @@ TPQ_CALL(dequantize_affine, 6)
 TPQ_CALL_END
 
 // linear_grads(grad [..., N], x [..., K], w [N, K], want_x, want_w), float32 -> (grad_x like x or None, grad_w or None).  Not while
-// gradients are recorded (a second derivative) or products are cast: those need the products as torch operations.
+// gradients are recorded (a second derivative), an operand carries a tangent (a derivative of the gradient in forward mode) or products
+// are cast: those need the products as torch operations.
 TPQ_CALL(linear_grads, 5)
     const at::Tensor *g = plain(args[0]), *x = plain(args[1]), *w = plain(args[2]);
-    if (!g || !x || !w || c10::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || g->scalar_type() != at::kFloat ||
+    if (!g || !x || !w || g->_fw_grad(0).defined() || x->_fw_grad(0).defined() || w->_fw_grad(0).defined() || c10::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || g->scalar_type() != at::kFloat ||
         x->scalar_type() != at::kFloat || w->scalar_type() != at::kFloat || g->dim() < 1 || x->dim() < 1 || w->dim() != 2 || g->numel() == 0 ||
         x->numel() == 0 || g->size(-1) != w->size(0) || x->size(-1) != w->size(1) || g->numel() / w->size(0) != x->numel() / w->size(1) ||
         !same_device(*g, *x) || !same_device(*g, *w))

@@ -92,6 +92,22 @@ def test_forms_that_stay_with_the_plain_products():
     assert torch.allclose(second, 2 * (g @ lin.weight) @ lin.weight.T, rtol=1e-4, atol=1e-7)
 
 
+def test_tangents_pass_through_the_backward():
+    """The derivative of the gradients along a direction of the output's gradient, in forward mode."""
+    import torch.autograd.forward_ad as fwad
+
+    lin = q.Int8DynActInt4WeightLinear(64, 32, bias=False, device="cuda")
+    g, x, _ = _case(16, 64, 32)
+    along = torch.randn_like(g)
+    x = x.requires_grad_()
+    out = lin(x)
+    with fwad.dual_level():
+        gx, gw = torch.autograd.grad(out, (x, lin.weight), fwad.make_dual(g, along))
+        gx, gw = fwad.unpack_dual(gx), fwad.unpack_dual(gw)
+    for got, want in ((gx.tangent, along @ lin.weight), (gw.tangent, along.T @ x), (gx.primal, g @ lin.weight), (gw.primal, g.T @ x)):
+        assert got is not None and torch.allclose(got, want, rtol=1e-4, atol=1e-6)
+
+
 def test_module_gradients_replay_in_a_graph():
     lin = q.Int8DynActInt4WeightLinear(512, 768, bias=False, device="cuda")
     x = torch.randn(96, 512, device="cuda", requires_grad=True)
