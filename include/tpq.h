@@ -386,7 +386,9 @@ int tpq_dense_mm(const void* x, int dtype, int64_t M, int64_t K, const void* w, 
  * tensorplay/ao/quantization/int8_dyn_act_int4_weight.py:86-95, two plain products):
  *   grad_x[M][K] = grad[M][N] w[N][K]       (grad_x null: not formed, w unused)
  *   grad_w[N][K] = grad[M][N]^T x[M][K]     (grad_w null: not formed, x unused)
- * float32 products and sums (each value in three bfloat16 parts, exactly; six part products, float32 accumulation).  Everything
+ * float32 products and sums: each value in three bfloat16 parts, exactly, and six part products, which leave out less than 2^-23 of a
+ * term, added in float32; float32 instructions for tiles whose values the parts do not hold (below 2^-110), whose sums are not finite
+ * or have fewer than four terms.  Everything
  * contiguous and 16-byte aligned, K and N multiples of 4; TPQ_ERR_UNSUPPORTED otherwise, nothing written then.  workspace: at least
  * tpq_f32_linear_grads_workspace_bytes(M, K, N, grad_x wanted, grad_w wanted) bytes, no initial contents, free again when the
  * work enqueued here is done.

@@ -4,11 +4,11 @@
 // 86-95, two plain float32 products).
 //
 // What bounds it: the matrix cores.  v_mfma_f32_16x16x4_f32 takes 32 clocks for 2048 flops, a sixteenth of what bfloat16 does, so every
-// float32 value is taken apart into three bfloat16 parts on its way into LDS (8 + 8 + 8 bits: exact, x = h + m + l) and a product
-// is the six part products down to 2^-18 of it (hh, hm, mh, mm, hl, lh; what is left out is below 2^-24): six bfloat16 instructions for
-// the work of sixteen.  No scaling, no range below float32's: the parts keep its exponent.  Two float16 parts would need three
-// products instead of six, but a scale for each row and column, whose maxima are a pass of their own, and lose what lies 2^17 below a
-// row's largest value.
+// float32 value is taken apart into three bfloat16 parts on its way into LDS (8 + 8 + 8 bits: exact from 2^-110 on, x = h + m + l) and a
+// product is the six part products down to 2^-18 of it (hh, hm, mh, mm, hl, lh; what is left out is below 2^-23 of it): six bfloat16
+// instructions for the work of sixteen.  No scaling: the parts keep float32's exponent.  Two float16 parts would need three products
+// instead of six, but a scale for each row and column, whose maxima are a pass of their own, and lose what lies 2^17 below a row's
+// largest value.
 //   * tile 128 x 128, 32 k a stage; 4 wavefronts of 64 x 64, v_mfma_f32_32x32x16_bf16: 12 fragments of 16 bytes from LDS for 24
 //     instructions (384 of 768 clocks per 16 k); up to three workgroups a compute unit, so that one takes values apart (6.5 vector
 //     instructions each, 832 clocks a stage) while another multiplies (1536 clocks a stage);
@@ -20,7 +20,13 @@
 //     columns 4 i + 0, 1 (or 2, 3): a lane stores two neighbours;
 //   * the k range is cut into slices where tiles are few, so that workgroups of both products are about equally long; float32
 //     sums of slices meet in a second kernel, in slice order;
-//   * a sum that comes out NaN is formed again term by term: an infinite value has h = inf and m = NaN.
+//   * where that is not float32's result a tile's slice is formed again with float32 instructions: a value below 2^-110 whose lowest
+//     bits the parts lose (its l is a subnormal bfloat16; seen in the bits that l cuts off, half an instruction a value), a sum that is not
+//     finite (an infinite value has h = inf and m = NaN, one next to 2^64 can have h x h = inf), and sums of up to three terms, whose
+//     error is that of a term (against float64, one / two / three terms: six products 3.7e-8 / 3.7e-8 / 3.6e-8, float32 2.5e-8 / 3.1e-8 /
+//     3.5e-8; from four on the six products have the smaller one).  512 rows, 2048 -> 4096 with such a value in every stage 166 us (the
+//     library products 131),
+//     with a row of infinities, seen at the end only, 240; the test for them costs the others 2 of 98.
 // Measured (us, both gradients with the adding launch, float32 library products before): 512 rows, 2048 -> 4096 140 -> 103 (matrix cores
 // busy for 41 of them; the write-back of 32 MB at the end of the launch takes 7, the rest is stages in which the workgroups of a unit
 // wait for each other's phases), 295 rows, 808 -> 3840 49 -> 41, 128 rows, 2048 -> 2048 38 -> 27, 72 rows, 1280 -> 712 39 -> 15.  Error against
@@ -86,9 +92,10 @@ __device__ __forceinline__ void clear_behind(int K, int k0, int t, fg_f4 (&v)[8]
 }
 
 // Eight values as three chunks of bfloat16 parts: h is the upper half of the value after half a unit was added (to nearest; beyond the
-// largest bfloat16 it is infinite, m NaN and the sum is formed again), m the upper half of x - h, l what is left, 8 bits at most.
+// largest bfloat16 it is infinite, m NaN and the sum is formed again), m the upper half of x - h, l what is left, 8 bits at most.  cut
+// gathers what is left of l: nothing from 2^-110 on.
 // v_cvt_pk_bf16_f32 and v_dot2_f32_bf16, half as many instructions, take 8 - 10 % longer.
-__device__ __forceinline__ void store_parts(const float (&x)[8], char* lds) {
+__device__ __forceinline__ void store_parts(const float (&x)[8], char* lds, uint32_t& cut) {
     uint32_t h[4], m[4], l[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -104,6 +111,8 @@ __device__ __forceinline__ void store_parts(const float (&x)[8], char* lds) {
         h[i] = __builtin_amdgcn_perm(upper[1], upper[0], 0x07060302u);
         m[i] = __builtin_amdgcn_perm(middle[1], middle[0], 0x07060302u);
         l[i] = __builtin_amdgcn_perm(lower[1], lower[0], 0x07060302u);
+        cut |= lower[0] | lower[1];
+        asm volatile("" : "+v"(cut));
     }
     *reinterpret_cast<uint4*>(lds) = make_uint4(h[0], h[1], h[2], h[3]);
     *reinterpret_cast<uint4*>(lds + kPartBytes) = make_uint4(m[0], m[1], m[2], m[3]);
@@ -111,43 +120,117 @@ __device__ __forceinline__ void store_parts(const float (&x)[8], char* lds) {
 }
 
 template <bool ALONG>
-__device__ __forceinline__ void put(const fg_f4 (&v)[8], char* lds, int t) {
+__device__ __forceinline__ void put(const fg_f4 (&v)[8], char* lds, int t, uint32_t& cut) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         float x[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = ALONG ? v[2 * e + (j >> 2)][j & 3] : v[j][e];
         const int chunk = ALONG ? t & 3 : t >> 5, slot = 32 * e + (ALONG ? t >> 2 : t & 31);
-        store_parts(x, lds + chunk * kChunkBytes + slot * 16);
+        store_parts(x, lds + chunk * kChunkBytes + slot * 16, cut);
     }
+}
+
+// the same values as they are: part p holds k 4 p .. 4 p + 3 of each chunk
+template <bool ALONG>
+__device__ __forceinline__ void put_whole(const fg_f4 (&v)[8], char* lds, int t) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            fg_f4 x;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = ALONG ? v[2 * e + p][j] : v[4 * p + j][e];
+            const int chunk = ALONG ? t & 3 : t >> 5, slot = 32 * e + (ALONG ? t >> 2 : t & 31);
+            *reinterpret_cast<fg_f4*>(lds + p * kPartBytes + chunk * kChunkBytes + slot * 16) = x;
+        }
 }
 
 __device__ __forceinline__ fg_bf8 fragment(const char* lds) { return __builtin_bit_cast(fg_bf8, *reinterpret_cast<const uint4*>(lds)); }
 
-// one sum of a slice term by term; ends at the first NaN
+// a workgroup's tile and its slice of k
+struct Place {
+    int m0, n0, begin, end, slice;
+};
+
+// Sums of a lane to memory.  Register e: slot 8 (e / 4) + 4 half + e % 4 of a fragment; row slot 32 f + s is row s of 32 rows (ALONG) or
+// row 4 s + f, column slot 32 f + s column 4 s + f: the two column fragments are neighbours
 template <bool ALONG>
-__device__ __attribute__((noinline)) float one_sum(const float* a, const float* b, int M, int N, int K, int m, int n, int k0, int k1) {
-    float sum = 0.0f;
-    for (int k = k0; k < k1 && sum == sum; ++k) {
-        const float av = ALONG ? a[static_cast<size_t>(m) * K + k] : a[static_cast<size_t>(k) * M + m];
-        sum = __builtin_fmaf(av, b[static_cast<size_t>(k) * N + n], sum);
+__device__ __forceinline__ void write_sums(const Product& p, const Place& at, int wave, int lane, const fg_f16 (&acc)[2][2]) {
+    const int i = lane & 31, half = lane >> 5, wm = wave >> 1, wn = wave & 1;
+    const int n = at.n0 + 4 * i + 2 * wn;
+    float* const c = p.c + static_cast<size_t>(at.slice) * p.M * p.N;
+    if (n >= p.N) return;
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int in = 8 * (e >> 2) + 4 * half + (e & 3);
+            const int m = at.m0 + (ALONG ? 32 * (2 * wm + f) + in : 4 * in + 2 * wm + f);
+            if (m < p.M) *reinterpret_cast<fg_f2*>(c + static_cast<size_t>(m) * p.N + n) = fg_f2{acc[f][0][e], acc[f][1][e]};
+        }
+}
+
+// A tile's slice again, with float32 instructions
+template <bool ALONG>
+__device__ __forceinline__ void whole_product(const Product& p, const Place& at, char* lds) {
+    int thread = threadIdx.x;
+    asm volatile("" : "+v"(thread));  // (or what the two forms have in common is kept in registers from the first to the second)
+    const int t = thread & 127, lane = thread & 63, wave = thread >> 6, i = lane & 31, half = lane >> 5, wm = wave >> 1, wn = wave & 1;
+    const bool first_operand = wave < 2;
+    char* const lds_b = lds + kOperandBytes;
+    fg_f16 acc[2][2];
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[f >> 1][f & 1][e] = 0.0f;
+    for (int k0 = at.begin; k0 < at.end; k0 += kStageK) {
+        fg_f4 v[8];
+        if (first_operand) fetch<ALONG>(p.a, p.M, at.m0, p.K, k0, t, v);
+        else fetch<false>(p.b, p.N, at.n0, p.K, k0, t, v);
+        if (k0 + kStageK > p.K) {
+            if (first_operand) clear_behind<ALONG>(p.K, k0, t, v);
+            else clear_behind<false>(p.K, k0, t, v);
+        }
+        __syncthreads();
+        if (first_operand) put_whole<ALONG>(v, lds, t);
+        else put_whole<false>(v, lds_b, t);
+        __syncthreads();
+#pragma unroll 1
+        for (int chunk = 0; chunk < kStageK / 8; ++chunk) {
+            // a lane's half multiplies k 4 half .. + 3 of the chunk, in both operands
+            const char* const la = lds + half * kPartBytes + chunk * kChunkBytes + (64 * wm + i) * 16;
+            const char* const lb = lds_b + half * kPartBytes + chunk * kChunkBytes + (64 * wn + i) * 16;
+            fg_f4 a[2], b[2];
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                a[f] = *reinterpret_cast<const fg_f4*>(la + f * 32 * 16);
+                b[f] = *reinterpret_cast<const fg_f4*>(lb + f * 32 * 16);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int f = 0; f < 4; ++f)
+                    acc[f >> 1][f & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[f >> 1][e], b[f & 1][e], acc[f >> 1][f & 1], 0, 0, 0);
+        }
     }
-    return sum;
+    write_sums<ALONG>(p, at, wave, lane, acc);
 }
 
 template <bool ALONG>
-__device__ __forceinline__ void product(const Product& p, int block, int blocks, char* lds) {
+__device__ __forceinline__ void product(const Product& p, int block, int blocks, char* lds, uint32_t* inexact) {
     // consecutive workgroups go round the eight dies: each die gets one run of neighbouring tiles, whose operands its L2 holds
     const int die = block & 7, each = blocks >> 3, more = blocks & 7;
     const int id = die * each + (die < more ? die : more) + (block >> 3);
-    const int tiles = p.tiles_m * p.tiles_n, slice = id / tiles, at = id - slice * tiles;
+    const int tiles = p.tiles_m * p.tiles_n, slice = id / tiles, tile = id - slice * tiles;
     // groups of eight tile rows, down each group's columns
-    const int group = at / (8 * p.tiles_n), in_group = at - group * 8 * p.tiles_n;
+    const int group = tile / (8 * p.tiles_n), in_group = tile - group * 8 * p.tiles_n;
     const int high = p.tiles_m - 8 * group < 8 ? p.tiles_m - 8 * group : 8;
     const int tile_n = in_group / high, tile_m = 8 * group + in_group - tile_n * high;
     const int m0 = tile_m * kTile, n0 = tile_n * kTile;
     const int begin = slice * p.stages_per_slice * kStageK;
     const int end = begin + p.stages_per_slice * kStageK < p.K ? begin + p.stages_per_slice * kStageK : p.K;
+    const Place at{m0, n0, begin, end, slice};
 
     const int t = threadIdx.x & 127, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 31, half = lane >> 5, wm = wave >> 1, wn = wave & 1;
     const bool first_operand = wave < 2;
@@ -162,8 +245,10 @@ __device__ __forceinline__ void product(const Product& p, int block, int blocks,
             if (first_operand) clear_behind<ALONG>(p.K, k0, t, v);
             else clear_behind<false>(p.K, k0, t, v);
         }
-        if (first_operand) put<ALONG>(v, lds, t);
-        else put<false>(v, lds_b, t);
+        uint32_t cut = 0;
+        if (first_operand) put<ALONG>(v, lds, t, cut);
+        else put<false>(v, lds_b, t, cut);
+        if (cut & 0xFFFFu) *inexact = 1;
     };
 
     fg_f16 acc[2][2];
@@ -173,10 +258,14 @@ __device__ __forceinline__ void product(const Product& p, int block, int blocks,
         for (int e = 0; e < 16; ++e) acc[f >> 1][f & 1][e] = 0.0f;
 
     load(begin);
+    if (threadIdx.x == 0) *inexact = p.K < 4;
+    __syncthreads();
     store(begin);
     __syncthreads();
+    uint32_t stop = 0;
     for (int k0 = begin; k0 < end; k0 += kStageK) {
         const bool more_stages = k0 + kStageK < end;
+        stop = *inexact;  // the same for all: written between the two barriers only
         if (more_stages) load(k0 + kStageK);
 #pragma unroll
         for (int s = 0; s < kStageK / 16; ++s) {
@@ -197,6 +286,8 @@ __device__ __forceinline__ void product(const Product& p, int block, int blocks,
                 for (int f = 0; f < 4; ++f)
                     acc[f >> 1][f & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kA[e]][f >> 1], b[kB[e]][f & 1], acc[f >> 1][f & 1], 0, 0, 0);
         }
+        stop = __builtin_amdgcn_readfirstlane(stop);
+        if (stop) break;
         __syncthreads();
         if (more_stages) {
             store(k0 + kStageK);
@@ -204,39 +295,23 @@ __device__ __forceinline__ void product(const Product& p, int block, int blocks,
         }
     }
 
-    // register e of a lane: slot 8 (e / 4) + 4 half + e % 4 of a fragment; row slot 32 f + s is row s of 32 rows (ALONG) or row 4 s + f,
-    // column slot 32 f + s column 4 s + f: the two column fragments are neighbours
-    const int n = n0 + 4 * i + 2 * wn;
-    float* const c = p.c + static_cast<size_t>(slice) * p.M * p.N;
-    if (n >= p.N) return;
-    const auto row_of = [&](int f, int e) {
-        const int in = 8 * (e >> 2) + 4 * half + (e & 3);
-        return m0 + (ALONG ? 32 * (2 * wm + f) + in : 4 * in + 2 * wm + f);
-    };
-    bool nan = false;
+    // parts that do not add up to their value, or a sum that is not finite (its product with zero is NaN)
+    float left = 0.0f;
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+    for (int f = 0; f < 4; ++f)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const fg_f2 sum = {acc[f][0][e], acc[f][1][e]};
-            const int m = row_of(f, e);
-            nan |= sum.x != sum.x || sum.y != sum.y;
-            if (m < p.M) *reinterpret_cast<fg_f2*>(c + static_cast<size_t>(m) * p.N + n) = sum;
-        }
-    // (apart from the stores: a call between them makes each wait for the one before it)
-    if (!nan) return;
-    for (int e = 0; e < 64; ++e) {
-        const int m = row_of(e >> 5, (e >> 1) & 15);
-        float* const at = c + static_cast<size_t>(m) * p.N + n + (e & 1);
-        if (m < p.M && *at != *at) *at = one_sum<ALONG>(p.a, p.b, p.M, p.N, p.K, m, n + (e & 1), begin, end);
-    }
+        for (int e = 0; e < 16; ++e) left = __builtin_fmaf(acc[f >> 1][f & 1][e], 0.0f, left);
+    const int again = __syncthreads_or(stop != 0 || left != left);
+    write_sums<ALONG>(p, at, wave, lane, acc);
+    if (__builtin_amdgcn_readfirstlane(again)) whole_product<ALONG>(p, at, lds);
 }
 
 __global__ __launch_bounds__(kThreads, 3) void f32_grads_kernel(const GradArgs args) {
     __shared__ __attribute__((aligned(16))) char lds[2 * kOperandBytes];
+    __shared__ uint32_t inexact;
     const int block = static_cast<int>(blockIdx.x);
-    if (block < args.first) product<true>(args.p[0], block, args.first, lds);
-    else product<false>(args.p[1], block - args.first, static_cast<int>(gridDim.x) - args.first, lds);
+    if (block < args.first) product<true>(args.p[0], block, args.first, lds, &inexact);
+    else product<false>(args.p[1], block - args.first, static_cast<int>(gridDim.x) - args.first, lds, &inexact);
 }
 
 struct Finish {

@@ -52,6 +52,47 @@ def test_wide_range_of_values_keeps_float32_precision():
     assert bool(((gx.double() - g.double() @ w.double()).abs() <= size * 2.0 ** -20).all())
 
 
+@pytest.mark.parametrize("power", [-104, -111, -118, -126, -134, -146])
+def test_tiny_values_keep_float32_precision(power):
+    """Values whose bfloat16 parts are subnormal, or nothing, in a few columns (the second stage of k and the last) and in all, against
+    partners of 2^100: the products are ordinary numbers."""
+    g, x, w = _case(40, 132, 260)
+    tiny = torch.randint(1 << 23, 1 << 24, g.shape, device="cuda").double() * 2.0 ** (power - 23)
+    for columns in (slice(40, 41), slice(257, 260), slice(None)):
+        a, b = g.clone(), w.clone()
+        a[:, columns] = tiny.float()[:, columns]
+        b[columns] *= 2.0 ** 100
+        a[:, 80:] *= (a[:, 80:].abs() < 1e-30).float()  # (columns of ordinary size would hide what the tiny ones add)
+        gx, gw = _grads(a, x, b)
+        for got, left, right in ((gx, a, b), (gw, a.T, x)):
+            want, size = left.double() @ right.double(), left.double().abs() @ right.double().abs()
+            terms = left.shape[1]
+            # a chain of float32 sums, its roundings in all directions, and float32's own smallest step for products below its range
+            bound = size * (3 * 2.0 ** -24 + 4 * terms ** 0.5 * 2.0 ** -24) + terms * 2.0 ** -149
+            assert bool(((got.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("terms", [1, 2, 3, 4])
+def test_sums_of_few_terms_round_once_a_term(terms):
+    g, x, w = _case(terms, 132, 260)
+    _, gw = _grads(g, x, w)
+    want, size = g.double().T @ x.double(), g.double().abs().T @ x.double().abs()
+    if terms < 4:  # float32: half a unit for each product and each sum
+        assert bool(((gw.double() - want).abs() <= size * terms * 2.0 ** -24).all())
+    assert (gw.double() - want).norm() <= 1.02 * ((g.T @ x).double() - want).norm()
+
+
+def test_products_next_to_the_largest_value():
+    """Factors that round up to 2^64 in bfloat16: the product of the rounded ones is infinite, theirs is not."""
+    g, x, w = _case(8, 64, 64)
+    g[2], w[:, 5] = 0.0, 0.0
+    g[2, 7] = w[7, 5] = 2.0 ** 64 * (1 - 2.0 ** -12)
+    gx, _ = _grads(g, x, w, want_weight=False)
+    want = g.double() @ w.double()
+    assert bool(gx.isfinite().all()) and float(gx[2, 5]) == float(want[2, 5].float())
+    assert bool(((gx.double() - want).abs() <= 1e-5 * (g.double().abs() @ w.double().abs())).all())
+
+
 def test_infinities_and_nan_as_in_float32():
     g, x, w = _case(40, 132, 260)
     g[3, 7], g[4, 8], g[5, 9], g[6, 1] = float("inf"), float("-inf"), float("nan"), 3.4e38
