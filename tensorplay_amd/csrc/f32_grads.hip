@@ -18,8 +18,10 @@
 //   * LDS: [part][chunk of 8 k][slot] of 16 bytes, a slot per row: fragment reads are 512 consecutive bytes, and so are the
 //     writes, row 4 i + e of a transposed operand having the slot 32 e + i.  A wavefront's two column fragments then lie at
 //     columns 4 i + 0, 1 (or 2, 3): a lane stores two neighbours;
-//   * the k range is cut into slices where tiles are few, so that workgroups of both products are about equally long; float32
-//     sums of slices meet in a second kernel, in slice order;
+//   * the k range is cut into slices where tiles are few, so that workgroups of both products are about equally long, up to all places for
+//     one tile (262144 rows, 64 -> 64: 512 slices, 128 us, at most eight slices 1915, the library products 554; 16 rows, 64 -> 65536
+//     32 / 454 / 97; 65536 rows, 128 -> 128 44 / 487 / 241; 32 rows, 512 -> 4096 15 / 36 / 37); their float32 sums, of a place a tile at
+//     most, meet in a second kernel, in slice order;
 //   * where that is not float32's result a tile's slice is formed again with float32 instructions: a value below 2^-110 whose lowest
 //     bits the parts lose (its l is a subnormal bfloat16; seen in the bits that l cuts off, half an instruction a value), a sum that is not
 //     finite (an infinite value has h = inf and m = NaN, one next to 2^64 can have h x h = inf), and sums of up to three terms, whose
@@ -318,22 +320,33 @@ struct Finish {
     const fg_f4* partial;
     fg_f4* out;
     int64_t quads;
-    int slices, blocks;
+    int slices, parts, blocks;  // parts: neighbouring slices go to one of this many threads
 };
 
-// the slices' sums, added in slice order; blocks of both products in one launch
+// The slices' sums, added in slice order; blocks of both products in one launch.  Many slices (an output of few tiles) are shared out over
+// parts of a workgroup, whose sums are then added in part order: 512 slices one after the other would be their requests' latency.
 __global__ __launch_bounds__(256) void f32_grads_finish_kernel(const Finish x, const Finish w) {
+    __shared__ fg_f4 sums[256];
     const bool second = static_cast<int>(blockIdx.x) >= x.blocks;
     const Finish f = second ? w : x;
-    const int64_t q = static_cast<int64_t>(static_cast<int>(blockIdx.x) - (second ? x.blocks : 0)) * 256 + threadIdx.x;
-    if (q >= f.quads) return;
-    fg_f4 sum = f.partial[q];
-    for (int s = 1; s < f.slices; ++s) sum += f.partial[s * f.quads + q];
-    f.out[q] = sum;
+    const int each = 256 / f.parts, part = static_cast<int>(threadIdx.x) / each;
+    const int64_t q = static_cast<int64_t>(static_cast<int>(blockIdx.x) - (second ? x.blocks : 0)) * each + static_cast<int>(threadIdx.x) % each;
+    const int per = (f.slices + f.parts - 1) / f.parts, first = part * per, last = first + per < f.slices ? first + per : f.slices;
+    fg_f4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (q < f.quads && first < last) {
+        sum = f.partial[first * f.quads + q];
+        for (int s = first + 1; s < last; ++s) sum += f.partial[s * f.quads + q];
+    }
+    if (f.parts > 1) {
+        sums[threadIdx.x] = sum;
+        __syncthreads();
+        for (int p = 1; p < f.parts && p * per < f.slices; ++p) sum += sums[(p * each + static_cast<int>(threadIdx.x)) & 255];
+    }
+    if (q < f.quads && part == 0) f.out[q] = sum;
 }
 
 constexpr int64_t kPlaces = 512;  // two workgroups on each of 256 compute units
-constexpr int kLeastStages = 4, kMostSlices = 8;
+constexpr int kLeastStages = 4;
 
 struct Plan {
     int64_t tiles_m, tiles_n, slices, stages;
@@ -343,7 +356,7 @@ Plan plan_of(int64_t M, int64_t N, int64_t K, int64_t stages_each) {
     Plan p{(M + kTile - 1) / kTile, (N + kTile - 1) / kTile, 1, 0};
     const int64_t stages = (K + kStageK - 1) / kStageK;
     int64_t slices = (stages + stages_each / 2) / stages_each;
-    slices = slices < 1 ? 1 : slices > kMostSlices ? kMostSlices : slices;
+    if (slices < 1) slices = 1;
     p.stages = (stages + slices - 1) / slices;
     p.slices = (stages + p.stages - 1) / p.stages;
     return p;
@@ -405,7 +418,8 @@ TPQ_EXPORT int tpq_f32_linear_grads(const float* grad, const float* x, const flo
         blocks[e] = plan[e].tiles_m * plan[e].tiles_n * plan[e].slices;
         if (p.slices > 1) {
             const int64_t quads = static_cast<int64_t>(p.M) * p.N / 4;
-            finish[e] = Finish{reinterpret_cast<const fg_f4*>(space), reinterpret_cast<fg_f4*>(p.c), quads, p.slices, static_cast<int>((quads + 255) / 256)};
+            const int parts = p.slices > 8 ? 16 : 1;
+            finish[e] = Finish{reinterpret_cast<const fg_f4*>(space), reinterpret_cast<fg_f4*>(p.c), quads, p.slices, parts, static_cast<int>((quads * parts + 255) / 256)};
             p.c = space;
             space += p.slices * quads * 4;
         }
