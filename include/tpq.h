@@ -68,13 +68,14 @@ int tpq_quantize_rowwise(const void* x, int x_dtype, int64_t M, int64_t K, float
  *         quantizers of a training linear (tensorplay/ao/quantization/int8_dyn_act_int4_weight.py:72-84);
  *   pad:  x as above and a copy of the int8 weight w [N, K] (any alignment).
  * M, N > 0, K % 4 == 0, 8 <= K <= 16384, the other operands 16-byte aligned; else TPQ_ERR_UNSUPPORTED.
+ * ..._takes: 1 where the sizes and the operands given (w NULL for pad) are such, before anything is allocated.  Host logic only.
  */
+int tpq_quantize_beside_takes(const void* x, const void* w, int64_t M, int64_t N, int64_t K, int64_t pitch);
 int tpq_quantize_both_rowwise(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K, int64_t pitch, float x_eps,
                               float w_eps, float w_divisor, int w_qmin, int w_qmax, int w_sign_mode, int8_t* x_codes,
                               float* x_scales, int8_t* w_codes, float* w_scales, void* stream);
 int tpq_quantize_rowwise_pad(const void* x, int dtype, int64_t M, int64_t K, float eps, const int8_t* w, int64_t N, int64_t pitch,
                              int8_t* codes, float* scales, int8_t* w_out, void* stream);
-
 
 /*
  * Integer matrix product C[M,N] (int32) = A[M,K] (int8, or uint8 when
@@ -392,7 +393,9 @@ int tpq_dense_mm(const void* x, int dtype, int64_t M, int64_t K, const void* w, 
  * contiguous and 16-byte aligned, K and N multiples of 4; TPQ_ERR_UNSUPPORTED otherwise, nothing written then.  workspace: at least
  * tpq_f32_linear_grads_workspace_bytes(M, K, N, grad_x wanted, grad_w wanted) bytes, no initial contents, free again when the
  * work enqueued here is done.
+ * ..._takes: 1 where these operands are such and M >= 4 (below, the separate products are the faster ones).  Host logic only.
  */
+int tpq_f32_linear_grads_takes(const float* grad, const float* x, const float* w, int64_t M, int64_t K, int64_t N);
 size_t tpq_f32_linear_grads_workspace_bytes(int64_t M, int64_t K, int64_t N, int want_x, int want_w);
 int tpq_f32_linear_grads(const float* grad, const float* x, const float* w, int64_t M, int64_t K, int64_t N, float* grad_x, float* grad_w,
                          void* workspace, size_t workspace_bytes, void* stream);

@@ -49,6 +49,7 @@ SIGNATURES = {
     "tpq_ternary_mm_ws": [_ptr, _ptr, _ptr, _f32, _ptr, _i64, _i64, _i64, _ptr, _int, _ptr, _ptr, _i64, _ptr],
     "tpq_ternary_linear_row": [_ptr, _int, _ptr, _f32, _ptr, _i64, _i64, _f32, _ptr, _ptr],
     "tpq_quantize_both_rowwise": [_ptr, _ptr, _int, _i64, _i64, _i64, _i64, _f32, _f32, _f32, _int, _int, _int, _ptr, _ptr, _ptr, _ptr, _ptr],
+    "tpq_quantize_beside_takes": [_ptr, _ptr, _i64, _i64, _i64, _i64],
     "tpq_quantize_rowwise_pad": [_ptr, _int, _i64, _i64, _f32, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr],
     "tpq_ternary_linear_workspace_bytes": [_i64, _i64, _i64],
     "tpq_ternary_linear": [_ptr, _int, _ptr, _f32, _ptr, _i64, _i64, _i64, _f32, _ptr, _ptr, _ptr, _ptr, _i64, _ptr],
@@ -58,6 +59,7 @@ SIGNATURES = {
     "tpq_int4_mm_swiglu_norm": [_ptr, _int, _i64, _i64, _ptr, _f32, _ptr, _ptr, _int, _i64, _i64, _ptr, _ptr, _ptr, _ptr],
     "tpq_rms_norm": [_ptr, _int, _i64, _i64, _ptr, _f32, _ptr, _ptr],
     "tpq_dense_mm": [_ptr, _int, _i64, _i64, _ptr, _i64, _ptr, _ptr],
+    "tpq_f32_linear_grads_takes": [_ptr, _ptr, _ptr, _i64, _i64, _i64],
     "tpq_f32_linear_grads_workspace_bytes": [_i64, _i64, _i64, _int, _int],
     "tpq_f32_linear_grads": [_ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr, _ptr, ctypes.c_size_t, _ptr],
     "tpq_packed_linear_workspace_bytes": [_i64, _i64, _i64, _int],

@@ -45,6 +45,7 @@ struct Library {
     TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
     TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine) \
     TPQ_ENTRY(tpq_f32_linear_grads_workspace_bytes) TPQ_ENTRY(tpq_f32_linear_grads) \
+    TPQ_ENTRY(tpq_f32_linear_grads_takes) TPQ_ENTRY(tpq_quantize_beside_takes) \
     TPQ_ENTRY(tpq_quantize_both_rowwise) TPQ_ENTRY(tpq_quantize_rowwise_pad)
     TPQ_ENTRIES
 #undef TPQ_ENTRY
@@ -268,7 +269,9 @@ TPQ_CALL(int8_linear, 7)
     const at::ScalarType type = reinterpret_cast<THPDtype*>(args[5])->scalar_type;
     const bool pad = K % 16 != 0 && M > ragged_rows;
     const int64_t pitch = pad ? code_pitch(K) : K;
-    if (float_tag(type) < 0 || !optional_vector(args[3], at::kFloat, N, *x, &bias)) Py_RETURN_NONE;
+    if (float_tag(type) < 0 || !optional_vector(args[3], at::kFloat, N, *x, &bias) ||
+        (pad && !lib.tpq_quantize_beside_takes(x->const_data_ptr(), nullptr, M, N, K, pitch)))
+        Py_RETURN_NONE;
     at::Tensor out;
     int status;
     {
@@ -303,6 +306,7 @@ TPQ_CALL(lowbit_linear, 8)
     const int64_t K = w->size(1), N = w->size(0), pitch = code_pitch(K);
     int64_t M;
     const auto sizes = product_sizes(*x, N, &M);
+    if (!lib.tpq_quantize_beside_takes(x->const_data_ptr(), w->const_data_ptr(), M, N, K, pitch)) Py_RETURN_NONE;
     at::Tensor out;
     int status;
     {
@@ -532,6 +536,7 @@ TPQ_CALL(linear_grads, 5)
         !same_device(*g, *x) || !same_device(*g, *w))
         Py_RETURN_NONE;
     const int64_t N = w->size(0), K = w->size(1), M = g->numel() / N;
+    if (!lib.tpq_f32_linear_grads_takes(ptr<float>(g), ptr<float>(x), ptr<float>(w), M, K, N)) Py_RETURN_NONE;
     const bool want_x = args[3] == Py_True, want_w = args[4] == Py_True;
     at::Tensor grad_x, grad_w;
     int status;

@@ -377,6 +377,21 @@ void plans(int64_t M, int64_t K, int64_t N, bool want_x, bool want_w, Plan (&pla
 
 using namespace tpq;
 
+namespace tpq {
+namespace {
+inline bool grads_sizes_ok(int64_t M, int64_t K, int64_t N) {
+    return M > 0 && K > 0 && N > 0 && K % 4 == 0 && N % 4 == 0 && M <= (1 << 24) && K <= (1 << 24) && N <= (1 << 24);
+}
+}  // namespace
+}  // namespace tpq
+
+// Up to three rows the tiles are padding but for those and grad_w is formed with float32 instructions too (us, this / library products:
+// 4096 x 4096 at 1, 2, 4 rows 55 / 41, 54 / 41, 38 / 40; 8192 x 8192 207 / 137, 199 / 137, 145 / 139; 4096 -> 11008 126 / 109, 138 / 109,
+// 94 / 110; small layers, where the calls are what counts, 2048 x 2048 21 / 40 at any of them).
+TPQ_EXPORT int tpq_f32_linear_grads_takes(const float* grad, const float* x, const float* w, int64_t M, int64_t K, int64_t N) {
+    return M >= 4 && grads_sizes_ok(M, K, N) && aligned(grad, 16) && aligned(x, 16) && aligned(w, 16);
+}
+
 TPQ_EXPORT size_t tpq_f32_linear_grads_workspace_bytes(int64_t M, int64_t K, int64_t N, int want_x, int want_w) {
     if (M <= 0 || K <= 0 || N <= 0) return 0;
     Plan plan[2];
@@ -390,7 +405,7 @@ TPQ_EXPORT size_t tpq_f32_linear_grads_workspace_bytes(int64_t M, int64_t K, int
 TPQ_EXPORT int tpq_f32_linear_grads(const float* grad, const float* x, const float* w, int64_t M, int64_t K, int64_t N, float* grad_x,
                                     float* grad_w, void* workspace, size_t workspace_bytes, void* stream) {
     TPQ_REQUIRE(M >= 0 && K >= 0 && N >= 0, TPQ_ERR_INVALID_VALUE, "tpq_f32_linear_grads: negative dimension");
-    TPQ_REQUIRE(M > 0 && K > 0 && N > 0 && K % 4 == 0 && N % 4 == 0 && M <= (1 << 24) && K <= (1 << 24) && N <= (1 << 24), TPQ_ERR_UNSUPPORTED,
+    TPQ_REQUIRE(grads_sizes_ok(M, K, N), TPQ_ERR_UNSUPPORTED,
                 "tpq_f32_linear_grads: sizes of 1 to 2^24, K and N multiples of 4");
     if (grad_x == nullptr && grad_w == nullptr) return TPQ_OK;
     TPQ_REQUIRE(grad && (grad_x == nullptr || w) && (grad_w == nullptr || x), TPQ_ERR_INVALID_VALUE, "tpq_f32_linear_grads: null pointer");

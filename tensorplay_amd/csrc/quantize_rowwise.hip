@@ -267,6 +267,10 @@ TPQ_EXPORT int tpq_quantize_rowwise(const void* x, int x_dtype, int64_t M, int64
     }
 }
 
+TPQ_EXPORT int tpq_quantize_beside_takes(const void* x, const void* w, int64_t M, int64_t N, int64_t K, int64_t pitch) {
+    return tpq::beside_takes(M, N, K, pitch) && tpq::aligned(x, 16) && tpq::aligned(w, 16);
+}
+
 TPQ_EXPORT int tpq_quantize_both_rowwise(const void* x, const void* w, int dtype, int64_t M, int64_t N, int64_t K, int64_t pitch, float x_eps, float w_eps,
                                          float w_divisor, int w_qmin, int w_qmax, int w_sign_mode, int8_t* x_codes, float* x_scales, int8_t* w_codes,
                                          float* w_scales, void* stream) {

@@ -950,8 +950,8 @@ _INT4_FUSED_ROWS = 32
 
 def linear_grads(grad: torch.Tensor, input: torch.Tensor, weight: torch.Tensor, want_input: bool = True, want_weight: bool = True):
     """Gradients of ``input @ weight.T`` for ``grad`` [..., N], input [..., K] and weight [N, K]: (grad @ weight like input, grad.T @ input
-    over all leading dims), None for one that is not wanted.  Contiguous float32 GPU tensors with N and K multiples of 4 run in
-    one kernel for both; anything else, and any call whose own gradient is recorded or carried along as a tangent, as the two products."""
+    over all leading dims), None for one that is not wanted.  Contiguous float32 GPU tensors of 4 rows and more with N and K multiples
+    of 4 run in one kernel for both; anything else, and any call whose own gradient is recorded or carried along as a tangent, as the two products."""
     calls = _lib.load().calls if grad.is_cuda else None
     if calls is not None and (pair := calls.linear_grads(grad, input, weight, bool(want_input), bool(want_weight))) is not None:
         return pair

@@ -199,3 +199,23 @@ def test_int4_workspace_lives_until_the_launch():
     with torch.no_grad():
         assert torch.equal(module(x), want)
     assert held() is None  # and no longer
+
+
+def test_refused_before_anything_is_allocated():
+    """Operands that the fused launches do not take: the native call returns to the Python form with nothing allocated."""
+    calls = _lib.load().calls
+    x = {k: torch.randn(48, k, device="cuda") for k in (516, 518, 16388, 4)}
+    w8 = {k: torch.ones(64, k, dtype=torch.int8, device="cuda") for k in x}
+    w = {k: torch.randn(64, k, device="cuda") for k in x}
+    scale, grad, few = torch.ones(64, device="cuda"), torch.randn(48, 64, device="cuda"), torch.randn(3, 64, device="cuda")
+    shifted = {k: _shifted(v) for k, v in x.items()}
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    for k in (518, 16388, 4):  # K % 4, above 16384 with K % 16, below 8
+        assert calls.int8_linear(x[k], w8[k], scale, None, 1e-5, torch.float32, 32) is None
+        assert calls.lowbit_linear(x[k], w[k], 1e-5, 1e-8, 7.0, -8, 7, 0) is None
+    assert calls.lowbit_linear(shifted[516], w[516], 1e-5, 1e-8, 7.0, -8, 7, 0) is None
+    with torch.no_grad():
+        assert calls.linear_grads(grad, x[518], w[518], True, True) is None
+        assert calls.linear_grads(grad, shifted[516], w[516], True, True) is None
+        assert calls.linear_grads(few, x[516][:3], w[516], True, True) is None  # up to three rows the products are the faster ones
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
