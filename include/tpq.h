@@ -242,7 +242,9 @@ int tpq_ternary_linear_row(const void* x, int x_dtype, const uint8_t* packed, fl
  * The same of M > 0 activation rows x [M, K] with the codes (int8 [M, K], 16-byte aligned) and scales (f32 [M]) of the rows in the
  * caller's memory: tpq_quantize_rowwise and tpq_ternary_mm_ws, with the same result bits.  Where the weight is written out as int8
  * rows first (a workspace of tpq_ternary_linear_workspace_bytes, K % 4 == 0, 8 <= K <= 16384, x 16-byte aligned), one launch does
- * that and quantizes the rows; what codes holds afterwards is unspecified then.
+ * that and quantizes the rows; what codes holds afterwards is unspecified then.  That workspace is a byte a code, four times the
+ * packed weight (8192 -> 28672: 235 MB), from 257 rows on where the weight has 2^24 codes and more (384, 512, 640 rows: smaller
+ * ones); with the workspace of tpq_ternary_mm_workspace_bytes the kernels of the packed weight run, which need none at 257..640 rows.
  */
 int64_t tpq_ternary_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int tpq_ternary_linear(const void* x, int x_dtype, const uint8_t* packed, float w_scale, const float* bias, int64_t M, int64_t N,

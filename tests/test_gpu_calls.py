@@ -219,3 +219,29 @@ def test_refused_before_anything_is_allocated():
         assert calls.linear_grads(grad, shifted[516], w[516], True, True) is None
         assert calls.linear_grads(few, x[516][:3], w[516], True, True) is None  # up to three rows the products are the faster ones
     assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+
+
+def test_a_full_card_leaves_the_routes_with_less_memory():
+    """Where the memory for the weight written out as int8 is not there, the kernels of the packed weight run, which need none."""
+    torch.manual_seed(0)
+    lin = _module("bitnet", 8192, 28672, torch.bfloat16, False)  # a workspace of 235 MB from 257 rows on
+    x = torch.randn(260, 8192, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        want = lin(x)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (120 << 20)) / total)
+        with torch.no_grad():
+            assert torch.equal(lin(x), want)
+            torch.cuda.empty_cache()
+            taken = []
+            with pytest.raises(torch.OutOfMemoryError):  # (64 of 8 MB are far more than is allowed)
+                for _ in range(64):
+                    taken.append(torch.empty(8 << 20, dtype=torch.uint8, device="cuda"))
+            with pytest.raises(torch.OutOfMemoryError):
+                lin(x)  # nothing left for the result, of 30 MB, either
+            del taken
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
