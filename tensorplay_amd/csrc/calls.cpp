@@ -40,7 +40,7 @@ struct Library {
 #define TPQ_ENTRY(NAME) decltype(&::NAME) NAME = nullptr;
 #define TPQ_ENTRIES                                                                                                       \
     TPQ_ENTRY(tpq_quantize_rowwise) TPQ_ENTRY(tpq_int8_mm_workspace_bytes) TPQ_ENTRY(tpq_int8_mm_dequant_ws)                \
-    TPQ_ENTRY(tpq_ternary_linear_workspace_bytes) TPQ_ENTRY(tpq_ternary_linear_row) TPQ_ENTRY(tpq_ternary_linear)                \
+    TPQ_ENTRY(tpq_ternary_mm_workspace_bytes) TPQ_ENTRY(tpq_ternary_linear_workspace_bytes) TPQ_ENTRY(tpq_ternary_linear_row) TPQ_ENTRY(tpq_ternary_linear)                \
     TPQ_ENTRY(tpq_int4_mm_ws)                                                                                             \
     TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
     TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
@@ -363,7 +363,9 @@ TPQ_CALL(ternary_linear, 6)
                                                 static_cast<float>(eps), out_ptr<float>(out), q.stream);
         }
         if (!one_launch || status != TPQ_OK) {
-            const Quantized room = room_for_codes(*x, M, K, lib.tpq_ternary_linear_workspace_bytes(M, N, K));
+            // rows off 16 bytes are quantized by themselves: the product behind them is that of the codes
+            const auto workspace_bytes = reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16 ? lib.tpq_ternary_mm_workspace_bytes : lib.tpq_ternary_linear_workspace_bytes;
+            const Quantized room = room_for_codes(*x, M, K, workspace_bytes(M, N, K));
             if (!one_launch) out = allocate(sizes, at::kFloat, *x);
             status = lib.tpq_ternary_linear(x->const_data_ptr(), float_tag(x->scalar_type()), ptr<uint8_t>(packed), static_cast<float>(w_scale), ptr<float>(bias), M, N, K,
                                             static_cast<float>(eps), room.codes, room.scales, out_ptr<float>(out), room.scratch, room.scratch_bytes, q.stream);

@@ -249,3 +249,31 @@ def test_rows_quantized_beside_the_expansion(m, k, n, dtype):
         want = ops.ternary_mm(codes, scale, packed, 0.037, k, bias=b)
         got = ops._ternary_linear(x, packed, 0.037, k, b, 1e-5)
         assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("m,k,n", [(256, 4096, 8192), (256, 8192, 4096), (256, 3072, 8192), (384, 4096, 4096), (384, 6912, 2560), (512, 1024, 4096), (512, 2560, 1640)])
+def test_linear_on_both_sides_of_the_expansion(m, k, n):
+    """One row more and the linear writes its weight out as int8; the product of the codes reads the packed weight on both sides, and so does
+    the linear of rows off 16 bytes, without the other's workspace.  The same bits."""
+    from tensorplay_amd import _lib, ops
+
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    packed = torch.randint(0, 256, (n, k // 4), device="cuda", generator=gen, dtype=torch.uint8)
+    bias = torch.randn(n, device="cuda", generator=gen)
+    for rows, expands in ((m, False), (m + 1, True)):
+        assert (lib.tpq_ternary_linear_workspace_bytes(rows, n, k) >= n * k) == expands and lib.tpq_ternary_mm_workspace_bytes(rows, n, k) < n * k
+        x = torch.randn(rows, k, device="cuda", generator=gen).bfloat16()
+        codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
+        want = ops.ternary_mm(codes, scale, packed, 0.037, k, bias=bias)
+        assert torch.equal(ops._ternary_linear(x, packed, 0.037, k, bias, 1e-5), want)
+        shifted = torch.empty(x.numel() + 1, dtype=x.dtype, device="cuda")[1:].view_as(x).copy_(x)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        assert torch.equal(ops._ternary_linear(shifted, packed, 0.037, k, bias, 1e-5), want)
+        torch.cuda.synchronize()
+        # codes, scales, the result and what comparing it takes
+        room = lib.tpq_ternary_mm_workspace_bytes(rows, n, k) + rows * k + 4 * rows + 5 * rows * n + (8 << 20)
+        if expands and n * k > room:
+            assert torch.cuda.max_memory_allocated() - before < n * k
