@@ -63,7 +63,7 @@ inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, bool may_slice, boo
 }
 
 template <class Tile>
-int launch_tiled(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t K, Tile tile, hipStream_t s, int slices = 1) {
+int launch_tiled(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t K, Tile tile, hipStream_t s, int slices = 1, bool weight_cached = false) {
     const char* env = tuning_env("TPQ_INT8_FORM");
     if (slices > 1) {
         if (env && env[0] == 's') return launch_stagger(a, w, M, N, K, tile, s, slices);
@@ -75,7 +75,7 @@ int launch_tiled(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t
         return launch_dma(a, w, M, N, K, tile, s, slices);
     }
     if (K >= (1 << 23) || (env && env[0] == 'd')) return launch_dma(a, w, M, N, K, tile, s, 1);
-    const bool use_short = env ? env[0] == 'h' : plan_tiled(M, N, K, false).form == kShort;
+    const bool use_short = env ? env[0] == 'h' : plan_tiled(M, N, K, false, weight_cached).form == kShort;
     if (K % kDmaRowBytes != 0) {
         if (use_short) return launch_stagger_as<ArithI8, 2, true>(a, w, M, N, K, tile, s, 1, "int8 mfma gemm (staggered, 128 rows, edge in k)");
         return launch_stagger_as<ArithI8, 4, true>(a, w, M, N, K, tile, s, 1, "int8 mfma gemm (staggered, edge in k)");
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) void int32_sum_slices_kernel(const int32_t* __
 }
 
 template <class Epilogue>
-int launch_best(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t K, Epilogue ep, hipStream_t s) {
+int launch_best(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t K, Epilogue ep, hipStream_t s, bool weight_cached = false) {
     const char* force = tuning_env("TPQ_INT8_KERNEL");  // "reg" keeps the register-staged kernel
     // a few rows: stream the weight once per 32 rows through the decode kernel.  K = N = 4096: 16 rows 6.9 us,
     // 32 rows 9.1 us, 64 rows 17.8 us, against 27.5 us for the tiled kernels below at any of these row counts
@@ -213,7 +213,7 @@ int launch_best(const int8_t* a, const int8_t* w, int64_t M, int64_t N, int64_t 
     // Rows that are no multiple of the 128-byte stage (K % 16 == 0 still) take the staggered kernel's edge stage from 65 rows
     // on: 473 rows of 1328 -> 3113 12.5 us (register-staged kernel 37.8); below, the 64 x 32 tiles of that one have the more
     // workgroups (48 rows of the same 8.7 us, staggered 9.6).
-    if ((K % kDmaRowBytes == 0 || (M > 64 && K < (1 << 23))) && !(force && force[0] == 'r')) return launch_tiled(a, w, M, N, K, to_tile(ep), s);
+    if ((K % kDmaRowBytes == 0 || (M > 64 && K < (1 << 23))) && !(force && force[0] == 'r')) return launch_tiled(a, w, M, N, K, to_tile(ep), s, 1, weight_cached);
     return launch_mfma(a, w, M, N, K, ep, s);
 }
 
@@ -322,9 +322,11 @@ TPQ_EXPORT int tpq_int_mm(const void* a, int a_unsigned, const int8_t* b, int64_
     return launch_generic(a, a_unsigned, b, b_stride_k, b_stride_n, M, K, N, ep, s);
 }
 
-TPQ_EXPORT int tpq_int8_mm_dequant(const int8_t* a, const int8_t* w, const float* row_scale,
-                                   const float* col_scale, const float* bias, void* out,
-                                   int out_dtype, int64_t M, int64_t N, int64_t K, void* stream) {
+namespace tpq {
+namespace {
+
+int int8_mm_dequant(const int8_t* a, const int8_t* w, const float* row_scale, const float* col_scale, const float* bias, void* out, int out_dtype,
+                    int64_t M, int64_t N, int64_t K, void* stream, bool weight_cached) {
     TPQ_REQUIRE(M >= 0 && N >= 0 && K >= 0, TPQ_ERR_INVALID_VALUE, "int8_mm_dequant: negative shape");
     TPQ_REQUIRE(out_dtype == TPQ_DTYPE_F32 || out_dtype == TPQ_DTYPE_F16 || out_dtype == TPQ_DTYPE_BF16,
                 TPQ_ERR_INVALID_TYPE, "int8_mm_dequant: unsupported output dtype");
@@ -338,7 +340,7 @@ TPQ_EXPORT int tpq_int8_mm_dequant(const int8_t* a, const int8_t* w, const float
     {                                                                                               \
         const EpilogueDequant<DT> ep{static_cast<typename Elem<DT>::storage*>(out), row_scale,      \
                                      col_scale, bias};                                              \
-        if (fast) return launch_best(a, w, M, N, K, ep, s);                                         \
+        if (fast) return launch_best(a, w, M, N, K, ep, s, weight_cached);                          \
         if (ragged) return launch_int8_decode_ragged(a, w, M, N, K, ep, [N](const EpilogueDequant<DT>& e, int64_t m0) { return rebase_rows(e, m0, N); }, s); \
         return launch_generic(a, 0, w, 1, K, M, K, N, ep, s);                                       \
     }
@@ -348,6 +350,15 @@ TPQ_EXPORT int tpq_int8_mm_dequant(const int8_t* a, const int8_t* w, const float
         default: TPQ_DISPATCH(TPQ_DTYPE_BF16)
     }
 #undef TPQ_DISPATCH
+}
+
+}  // namespace
+}  // namespace tpq
+
+TPQ_EXPORT int tpq_int8_mm_dequant(const int8_t* a, const int8_t* w, const float* row_scale,
+                                   const float* col_scale, const float* bias, void* out,
+                                   int out_dtype, int64_t M, int64_t N, int64_t K, void* stream) {
+    return int8_mm_dequant(a, w, row_scale, col_scale, bias, out, out_dtype, M, N, K, stream, false);
 }
 
 TPQ_EXPORT int tpq_int8_pad_rows(const int8_t* a, int64_t M, const int8_t* w, int64_t N, int64_t K, int8_t* a_out, int8_t* w_out,
@@ -378,7 +389,7 @@ int int8_mm_dequant_ws(const int8_t* a, const int8_t* w, const float* row_scale,
     const int slices = (M > 0 && N > 0 && K > 0 && a && w) ? int8_slices(a, w, M, N, K, weight_cached) : 1;
     if (slices < 2 || workspace == nullptr || workspace_bytes < slices * M * N * 4 || !aligned(workspace, 16) || (M * N) % 4 != 0 ||
         !aligned(col_scale, 16) || !aligned(bias, 16))
-        return tpq_int8_mm_dequant(a, w, row_scale, col_scale, bias, out, out_dtype, M, N, K, stream);
+        return int8_mm_dequant(a, w, row_scale, col_scale, bias, out, out_dtype, M, N, K, stream, weight_cached);
     TPQ_REQUIRE(out_dtype == TPQ_DTYPE_F32 || out_dtype == TPQ_DTYPE_F16 || out_dtype == TPQ_DTYPE_BF16,
                 TPQ_ERR_INVALID_TYPE, "int8_mm_dequant: unsupported output dtype");
     TPQ_REQUIRE(out && row_scale && col_scale, TPQ_ERR_INVALID_VALUE, "int8_mm_dequant: null pointer");

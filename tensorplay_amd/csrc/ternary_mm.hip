@@ -142,6 +142,11 @@ __global__ __launch_bounds__(256) void ternary_generic_kernel(const int8_t* __re
 inline int64_t ternary_padded_k(int64_t K) { return (K + 127) / 128 * 128; }
 inline int64_t round_up_256(int64_t v) { return (v + 255) / 256 * 256; }
 
+// The int8 rows come out of the last-level cache, as far as that holds them: the tiles of the product are planned for that.  Planned for a
+// weight from HBM / from the caches (us, the linear): 513 rows 5120 -> 11008 80 / 69, 577 rows 8192 -> 11008 116 / 104, 321 rows 11008 ->
+// 21760 (240 MB) 216 / 204, 12288 -> 21760 (267 MB) 224 / 218, 11008 -> 28672 (316 MB) 277 / 291.
+inline bool expanded_weight_cached(int64_t N, int64_t kp) { return N * kp <= (int64_t{1} << 28); }
+
 struct ExpandedPlan {
     int64_t kp, x_at, scale_at, gemm_at, gemm_bytes, total;  // byte offsets into the workspace, the weight at 0
 };
@@ -151,7 +156,7 @@ inline ExpandedPlan plan_expanded(int64_t M, int64_t N, int64_t K) {
     p.x_at = round_up_256(N * p.kp);
     p.scale_at = p.x_at + (p.kp == K ? 0 : round_up_256(M * p.kp));
     p.gemm_at = p.scale_at + round_up_256(N * 4);
-    p.gemm_bytes = int8_mm_workspace_bytes(M, N, p.kp, true);
+    p.gemm_bytes = int8_mm_workspace_bytes(M, N, p.kp, expanded_weight_cached(N, p.kp));
     p.total = p.gemm_at + p.gemm_bytes;
     return p;
 }
@@ -274,7 +279,7 @@ int launch_quantize_expand(const void* x, int64_t M, int64_t N, int64_t K, const
 int multiply_expanded(const int8_t* x, const float* row_scale, const float* bias, int64_t M, int64_t N, void* out, int out_dtype, const ExpandedPlan& p,
                       char* ws, hipStream_t s) {
     return int8_mm_dequant_ws(x, reinterpret_cast<const int8_t*>(ws), row_scale, reinterpret_cast<const float*>(ws + p.scale_at), bias, out, out_dtype, M, N, p.kp,
-                              p.gemm_bytes ? ws + p.gemm_at : nullptr, p.gemm_bytes, s, true);
+                              p.gemm_bytes ? ws + p.gemm_at : nullptr, p.gemm_bytes, s, expanded_weight_cached(N, p.kp));
 }
 
 int launch_ternary_expanded(const int8_t* x, const float* row_scale, const uint8_t* packed, float w_scale, const float* bias, int64_t M, int64_t N,

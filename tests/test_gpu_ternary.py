@@ -277,3 +277,16 @@ def test_linear_on_both_sides_of_the_expansion(m, k, n):
         room = lib.tpq_ternary_mm_workspace_bytes(rows, n, k) + rows * k + 4 * rows + 5 * rows * n + (8 << 20)
         if expands and n * k > room:
             assert torch.cuda.max_memory_allocated() - before < n * k
+
+
+@pytest.mark.parametrize("m,k,n", [(513, 5120, 11008), (577, 8192, 11008)])
+def test_linear_on_the_tiles_of_a_cached_weight(m, k, n):
+    """Sizes whose int8 product runs on 128-row tiles behind the expansion and on 256-row tiles where the weight comes from HBM: the same bits."""
+    from tensorplay_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    weight = torch.randint(-1, 2, (n, k), device="cuda", generator=gen, dtype=torch.int8)
+    x = torch.randn(m, k, device="cuda", generator=gen).half()
+    codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
+    want = ops.int8_mm_dequant(codes, weight, scale, torch.full((n,), 0.037, device="cuda"))
+    assert torch.equal(ops._ternary_linear(x, ops.pack_ternary(weight), 0.037, k, None, 1e-5), want)
