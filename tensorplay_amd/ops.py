@@ -984,7 +984,8 @@ def int4pack_mm_multi(input: torch.Tensor, mats, qGroupSize: int, scales_and_zer
 
     if len(ops) > 4 or len({inner for _, _, _, inner, _ in ops}) != 1 or x.dtype == torch.float32:
         return separate()
-    if g is not None and 16 < m <= _INT4_FUSED_ROWS:  # one launch for all rows behind the norm's, two with the norm folded in
+    # one launch for all rows behind the norm's, two with the norm folded in; an eps or addresses that that call refuses are left to it
+    if g is not None and 16 < m <= _INT4_FUSED_ROWS and eps >= 0 and (x.data_ptr() | g.data_ptr()) % 16 == 0:
         return separate()
     outs = [torch.empty((m, n), dtype=x.dtype, device=x.device) for _, _, _, _, n in ops]
     if m == 0:

@@ -506,6 +506,24 @@ def test_mm_multi_equals_separate_products(ops, tdt, tol, M, K, widths):
         assert_close_norm(y.float().cpu().numpy()[:, cols], want, 2 * tol)
 
 
+@pytest.mark.parametrize("M", [16, 20, 32, 33])
+def test_mm_multi_with_norm_refuses_at_any_row_count(ops, M):
+    """A negative or NaN eps, activations or a norm weight off 16 bytes: refused where the norm runs in a launch of its own (17 to 32 rows)
+    as where it is folded into the products."""
+    K, n = 4096, 136
+    codes, sz, x = _fused_case(np.random.default_rng(M), M, n, K, torch.float16)
+    packed = [ops._convert_weight_to_int4pack(torch.from_numpy(codes).to(DEV), 2)]
+    x, szs, g = x.to(DEV), [sz.to(DEV)], torch.ones(K, dtype=torch.float16, device=DEV)
+
+    def shifted(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view_as(t).copy_(t)
+
+    assert ops.int4pack_mm_multi(x, packed, 128, szs, norm_weight=g, eps=0.0)[0].shape == (M, n)
+    for act, weight, eps in ((x, g, -1e-5), (x, g, float("nan")), (shifted(x), g, 1e-5), (x, shifted(g), 1e-5)):
+        with pytest.raises(ValueError):
+            ops.int4pack_mm_multi(act, packed, 128, szs, norm_weight=weight, eps=eps)
+
+
 def _rms_norm_bits(x_bits, g_bits, tag, eps):
     """The reference's rms_norm in numpy float32 (tensorplay/nn/functional.py:2350-2372), rounded to the dtype."""
     x = oracle.to_f32(x_bits, tag)
