@@ -640,7 +640,7 @@ int launch_multi(const void* x, int64_t M, int count, const int32_t* const* pack
         const int shift = group == 128 ? 0 : 1;
 #define TPQ_MULTI(NBV, WV) int4_mfma_multi_kernel<DT, NBV, WV><<<dim3(blocks), dim3(WV * kWave), 0, s>>>(xp, set, rows, K, shift)
 #define TPQ_MULTI2(NBV, WV) int4_mfma_multi_kernel<DT, NBV, WV, 2><<<dim3(blocks), dim3(WV * kWave), 0, s>>>(xp, set, rows, K, shift)
-        if (rows > 16) { if (nb == 1) TPQ_MULTI2(1, 8); else if (nb == 2 && waves == 8) TPQ_MULTI2(2, 8); else if (nb == 2) TPQ_MULTI2(2, 4); else TPQ_MULTI2(4, 4); }
+        if (rows > 16) { if (nb == 1) TPQ_MULTI2(1, 8); else if (nb == 2) TPQ_MULTI2(2, 8); else TPQ_MULTI2(4, 4); }  // (two: below 10240 channels, eight wavefronts)
         else if (waves == 8) { if (nb == 1) TPQ_MULTI(1, 8); else if (nb == 2) TPQ_MULTI(2, 8); else TPQ_MULTI(4, 8); }
         else { if (nb == 2) TPQ_MULTI(2, 4); else TPQ_MULTI(4, 4); }
 #undef TPQ_MULTI2

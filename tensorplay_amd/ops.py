@@ -90,6 +90,17 @@ def _dynamic_lowbit_linear(input: torch.Tensor, weight: torch.Tensor, weight_eps
     return None if calls is None else calls.lowbit_linear(input, weight, 1e-5, weight_eps, divisor, qmin, qmax, int(sign_mode))
 
 
+def linear_grads(grad: torch.Tensor, input: torch.Tensor, weight: torch.Tensor, want_input: bool = True, want_weight: bool = True):
+    """Gradients of ``input @ weight.T`` for ``grad`` [..., N], input [..., K] and weight [N, K]: (grad @ weight like input, grad.T @ input
+    over all leading dims), None for one that is not wanted.  Contiguous float32 GPU tensors of 4 rows and more with N and K multiples
+    of 4 run in one kernel for both; anything else, and any call whose own gradient is recorded or carried along as a tangent, as the two products."""
+    calls = _lib.load().calls if grad.is_cuda else None
+    if calls is not None and (pair := calls.linear_grads(grad, input, weight, bool(want_input), bool(want_weight))) is not None:
+        return pair
+    grad_weight = grad.reshape(-1, weight.shape[0]).T @ input.reshape(-1, weight.shape[1]) if want_weight else None
+    return (grad @ weight.to(grad.dtype) if want_input else None), grad_weight
+
+
 def _check_int_mm_operands(self, mat2):
     if self.dim() != 2 or mat2.dim() != 2:
         raise RuntimeError(f"_int_mm: expected two matrices but got {self.dim()}-D and {mat2.dim()}-D tensors")
@@ -948,21 +959,10 @@ def _norm_operand(x: torch.Tensor, norm_weight: torch.Tensor, what: str) -> torc
 _INT4_FUSED_ROWS = 32
 
 
-def linear_grads(grad: torch.Tensor, input: torch.Tensor, weight: torch.Tensor, want_input: bool = True, want_weight: bool = True):
-    """Gradients of ``input @ weight.T`` for ``grad`` [..., N], input [..., K] and weight [N, K]: (grad @ weight like input, grad.T @ input
-    over all leading dims), None for one that is not wanted.  Contiguous float32 GPU tensors of 4 rows and more with N and K multiples
-    of 4 run in one kernel for both; anything else, and any call whose own gradient is recorded or carried along as a tangent, as the two products."""
-    calls = _lib.load().calls if grad.is_cuda else None
-    if calls is not None and (pair := calls.linear_grads(grad, input, weight, bool(want_input), bool(want_weight))) is not None:
-        return pair
-    grad_weight = grad.reshape(-1, weight.shape[0]).T @ input.reshape(-1, weight.shape[1]) if want_weight else None
-    return (grad @ weight.to(grad.dtype) if want_input else None), grad_weight
-
-
 def int4pack_mm_multi(input: torch.Tensor, mats, qGroupSize: int, scales_and_zeros, norm_weight: Optional[torch.Tensor] = None,
                       eps: float = 1e-5) -> list:
     """``[_weight_int4pack_mm(input, w, qGroupSize, sz) for w, sz in zip(mats, scales_and_zeros)]`` with one launch
-    per 16 rows for up to four weights (q, k, v of a decoder layer).  Shapes the fused kernel does not take, and more
+    per 32 rows (16 with the norm inside) for up to four weights (q, k, v of a decoder layer).  Shapes the fused kernel does not take, and more
     than four weights, run the separate op.  With ``norm_weight`` the products are taken of ``rms_norm(input,
     norm_weight, eps)``, normalized inside the same launch where the kernel is built for it."""
     mats, scales_and_zeros = list(mats), list(scales_and_zeros)
