@@ -93,10 +93,13 @@ def _dynamic_lowbit_linear(input: torch.Tensor, weight: torch.Tensor, weight_eps
 def linear_grads(grad: torch.Tensor, input: torch.Tensor, weight: torch.Tensor, want_input: bool = True, want_weight: bool = True):
     """Gradients of ``input @ weight.T`` for ``grad`` [..., N], input [..., K] and weight [N, K]: (grad @ weight like input, grad.T @ input
     over all leading dims), None for one that is not wanted.  Contiguous float32 GPU tensors of 4 rows and more with N and K multiples
-    of 4 run in one kernel for both; anything else, and any call whose own gradient is recorded or carried along as a tangent, as the two products."""
+    of 4 run in one kernel for both; anything else, and any call whose own gradient is recorded or carried along as a tangent, as the two
+    products.  Types that the product for the weight refuses are refused without it too."""
     calls = _lib.load().calls if grad.is_cuda else None
     if calls is not None and (pair := calls.linear_grads(grad, input, weight, bool(want_input), bool(want_weight))) is not None:
         return pair
+    if not want_weight and grad.dtype != input.dtype and not torch.is_autocast_enabled(grad.device.type):
+        raise RuntimeError(f"linear_grads: expected grad and input of the same dtype, but got {grad.dtype} and {input.dtype}")
     grad_weight = grad.reshape(-1, weight.shape[0]).T @ input.reshape(-1, weight.shape[1]) if want_weight else None
     return (grad @ weight.to(grad.dtype) if want_input else None), grad_weight
 

@@ -140,6 +140,16 @@ def test_forms_that_stay_with_the_plain_products():
     assert torch.allclose(second, 2 * (g @ lin.weight) @ lin.weight.T, rtol=1e-4, atol=1e-7)
 
 
+@pytest.mark.parametrize("frozen", [False, True])
+def test_a_16_bit_layer_refuses_its_backward(frozen):
+    """Its output and the gradient of that are float32: no product with 16-bit operands, with the weight's gradient wanted or not."""
+    lin = q.Int8DynActInt4WeightLinear(64, 32, bias=False, device="cuda").bfloat16()
+    lin.weight.requires_grad_(not frozen)
+    x = torch.randn(16, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    with pytest.raises(RuntimeError):
+        lin(x).sum().backward()
+
+
 def test_tangents_pass_through_the_backward():
     """The derivative of the gradients along a direction of the output's gradient, in forward mode."""
     import torch.autograd.forward_ad as fwad
