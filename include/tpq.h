@@ -263,6 +263,8 @@ int tpq_ternary_linear(const void* x, int x_dtype, const uint8_t* packed, float 
  * slices are added in a fixed order.
  */
 int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
+/* Activation rows of a workgroup's tile with that workspace, where the weight is rounded once.  Host logic only. */
+int tpq_packed_rows_tile_rows(int dtype, int64_t M, int64_t N, int64_t K);
 /*
  * 1 where _weight_int4pack_mm (innerKTiles = 2) and the n-bit linear run the products below, 0 where another kernel is the
  * faster one or these do not take the operands (type, sizes, alignment).  Host logic only.

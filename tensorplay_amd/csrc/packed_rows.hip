@@ -97,6 +97,10 @@ TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t
     return p.slices > 1 ? static_cast<int64_t>(p.slices) * M * N * 4 : 0;
 }
 
+TPQ_EXPORT int tpq_packed_rows_tile_rows(int dtype, int64_t M, int64_t N, int64_t K) {
+    return M <= 0 || N <= 0 || K <= 0 ? 0 : 16 * packed_rows_plan(dtype, M, N, K, int64_t{1} << 60).mb;
+}
+
 TPQ_EXPORT int tpq_int4_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, int64_t N, int64_t group,
                                 const void* scales_and_zeros, void* out, void* workspace, int64_t workspace_bytes, void* stream) {
     return tpq_int4_mm_rows_bias(x, dtype, M, K, packed, N, group, scales_and_zeros, nullptr, out, workspace, workspace_bytes, stream);

@@ -80,6 +80,27 @@ def test_lowbit_rows(dtype, bits, lsb_first, M, N, K, group):
     _check(out, x, w, bias, 0.011 * (1 + (1 << bits) / 8), dtype)
 
 
+# (M, N, K, group, rows of a tile, slices of k): two to four tiles of rows, the last one partly empty, whole k and cut
+TALL = [(257, 6664, 256, 64, 80, 1), (241, 8200, 256, 32, 96, 1), (289, 8200, 256, 128, 112, 1), (225, 11016, 256, 64, 128, 1),
+        (257, 1096, 5248, 128, 80, 7), (241, 1544, 7296, 64, 96, 6), (289, 1608, 7296, 128, 112, 6), (241, 2824, 7296, 128, 128, 5),
+        (203, 11008, 4096, 128, 112, 1)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [0, 1, 2, 8])  # 0: the int4 layout
+@pytest.mark.parametrize("M,N,K,group,rows,slices", TALL)
+def test_tall_tiles(dtype, bits, M, N, K, group, rows, slices):
+    from tensorplay_amd import _lib, ops
+
+    lib, tag = _lib.load(), ops._DT[dtype]
+    assert lib.tpq_packed_rows_tile_rows(tag, M, N, K) == rows
+    assert lib.tpq_packed_rows_workspace_bytes(tag, M, N, K) == (0 if slices == 1 else 4 * slices * M * N)
+    if bits:
+        test_lowbit_rows(dtype, bits, False, M, N, K, group)
+    else:
+        test_int4_rows(dtype, M, N, K, group)
+
+
 def _fragment(kind, M, N, K, group, bits, dtype, change=lambda x, sz: None):
     """(result, exact float64 result) on weights whose (scale, zero) have no short form in 16 bits.  change: of x and the pairs, in
     place, before the call (sz [K / group, N, 2], of the type that the call takes)."""
