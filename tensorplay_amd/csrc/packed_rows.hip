@@ -9,13 +9,14 @@ namespace {
 template <int DT>
 int run_int4(const PackedRowsArgs& a, const PackedRowsPlan& p, hipStream_t s) { return launch_packed_rows<DT, SourceInt4>(a, p, s); }
 
-// Between the decode kernels and the dense route.  Upper limit, measured (us, this kernel / what runs above it): float16 and
-// bfloat16 alike, N < 16384: 384 rows of 4096 -> 11008 69 / 70, 8192 x 8192 78 / 104, 5120 -> 13824 84 / 97, 3072 -> 7088 33 / 39;
-// 512 rows of 8192 x 8192 90 / 103, 14336 -> 4096 71 / 110, 4096 x 4096 24 / 41, but 5120 -> 13824 111 / 99; 768 rows of
-// 4096 x 4096 42 / 43, 2048 x 2048 14 / 24, but 8192 x 8192 128 / 125.  Wider weights: bfloat16 4096 -> 32000 at 384 rows
-// 142 / 165, at 512 195 / 180; float16 (the tiled kernel of packed weights) at 256 rows 98 / 102, at 384 148 / 132.  float32: 192
-// rows of 4096 -> 11008 193 / 223, 4096 -> 16384 232 / 250, at 256 rows 309 / 305.  K that is no multiple of 128 has the narrow
-// tiles only: 4768 -> 13544 at 256 rows 120 / 106 (float32 at 96 rows 176 / 182, at 128 244 / 215).
+// Between the decode kernels and the dense route.  Upper limit, measured (us, this kernel / what runs above it, groups of 128, weights
+// from HBM): float16, N < 16384: up to 2^24 weights, 768 rows of 4096 x 4096 30 / 44, 1024 rows 41 / 47; up to 2^26, 512 rows of 4096 ->
+// 11008 66 / 67, 8192 x 8192 71 / 102, 14336 -> 4096 69 / 111, 768 rows 109 / 122 and 91 / 119; beyond, 384 rows of 5120 -> 13824 69 /
+// 98, 512 rows 90 / 100.  Wider weights, 4096 -> 32000: 256, 384, 512 rows 81 / 112, 120 / 137, 158 / 154; bfloat16 384 and 512 rows
+// 119 / 172, 155 / 182.  So the lines lie where a tile of 64 rows, which this kernel had when they were drawn, stopped paying; with the
+// tiles of up to 128 rows the first rows above most of them are the shorter ones here too.  float32: 192 rows of 4096 -> 11008 217 / 228,
+// 4096 -> 16384 257 / 251, at 256 rows of the first 256 / 222.  K that is no multiple of 128 has the narrow tiles only: 4768 -> 13544 at 192
+// rows 111, at 256 150 (float32 at 96 rows 185 / 182, at 128 258 / 215).
 int64_t rows_limit(int64_t N, int64_t K, int dtype) {
     if (dtype == TPQ_DTYPE_F32) return K % 128 ? 96 : 192;
     if (K % 128) return 192;
@@ -47,8 +48,8 @@ using namespace tpq;
 // 33 of 4096 x 4096 10.8 / 15.1, 48 of 4096 -> 11008 18.5 / 20.2; groups of 64, 17 rows:
 // 11008 -> 4096 12.0 / 23.1, 16 rows 11.3 / 12.0.  K % 128 != 0 (slabs of four rows): 4768 -> 13544 at 3 / 33 rows 19.4 /
 // 92, 31 / 868.  float32: 4096 -> 11008 at 1, 2, 64 rows 24.4 / 24.2, 24.7 / 45, 68 / 110; 2048 x 2048 at 1 and 2 rows
-// 8.1 / 7.2, 8.2 / 7.4.  bfloat16 stops at 256 rows although this kernel is the faster one beyond (384 rows of 8192 x 8192 78 / 104, 512 of
-// 4096 x 4096 24 / 41): from 257 rows on the results are those of the dense route, the reference's device formulation with a weight
+// 8.1 / 7.2, 8.2 / 7.4.  bfloat16 stops at 256 rows although this kernel is the faster one beyond (384 rows of 8192 x 8192 52 / 104, 512 of
+// 4096 x 4096 24 / 42): from 257 rows on the results are those of the dense route, the reference's device formulation with a weight
 // rounded to bfloat16 twice, and are held to it within 1e-2, element by element, by tests.  A weight rounded once lies closer to
 // the exact product and misses that on single elements; below 257 rows, where the tiled kernel and the slabs ran, the comparison
 // is with the exact product.
@@ -67,8 +68,8 @@ TPQ_EXPORT int tpq_int4_mm_rows_takes(const void* x, int dtype, int64_t M, int64
 // home: 4096 x 4096 at 19 rows, 1 / 2 / 4 / 8 bits 10.7 / 10.0, 10.8 / 10.5, 11.4 / 11.9, 13.1 / 16.9; 4096 -> 11008, 2 bits, 24 / 32 /
 // 40 rows 21.7 / 20.6, 21.6 / 21.5, 20 / 31; 1024 -> 512 at 18 rows 7.3 / 6.0.  Other groups, 4096 x 4096 in groups of 32, 2 bits:
 // 1 / 16 / 80 rows 10.1 / 25, 10.4 / 46, 17.6 / 175; one row of 4 bits stays with the row kernel (8.6 / 6.1).  float32
-// 4096 -> 11008: 1 / 8 / 64 rows 33 / 35, 33 / 57, 84 / 99.  8 bits are twice the bytes: 4096 -> 11008 at 300 rows 74 / 85, at
-// 512 111 / 83; 4096 x 4096 at 512 33 / 42.
+// 4096 -> 11008: 1 / 8 / 64 rows 33 / 35, 33 / 57, 84 / 99.  8 bits are twice the bytes: 4096 -> 11008 at 300 rows 75 / 86, at
+// 384 81 / 85, at 512 90 / 84; 4096 x 4096 at 512 31 / 42.
 TPQ_EXPORT int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int bits, int lsb_first, int64_t group,
                                         const uint8_t* packed, const float* scales_and_zeros) {
     if (M <= 0 || N <= 0 || K <= 0 || group <= 0 || (bits != 1 && bits != 2 && bits != 4 && bits != 8) || (lsb_first && bits != 1)) return 0;
