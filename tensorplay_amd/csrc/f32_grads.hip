@@ -19,20 +19,20 @@
 //     writes, row 4 i + e of a transposed operand having the slot 32 e + i.  A wavefront's two column fragments then lie at
 //     columns 4 i + 0, 1 (or 2, 3): a lane stores two neighbours;
 //   * the k range is cut into slices where tiles are few, so that workgroups of both products are about equally long, up to all places for
-//     one tile (262144 rows, 64 -> 64: 512 slices, 128 us, at most eight slices 1915, the library products 554; 16 rows, 64 -> 65536
-//     32 / 454 / 97; 65536 rows, 128 -> 128 44 / 487 / 241; 32 rows, 512 -> 4096 15 / 36 / 37); their float32 sums, of a place a tile at
-//     most, meet in a second kernel, in slice order;
+//     one tile (262144 rows, 64 -> 64: 328 slices, 128 us, at most eight slices 1915, the library products 554; 16 rows, 64 -> 65536
+//     32 / 454 / 97; 65536 rows, 128 -> 128 44 / 487 / 241; 32 rows, 512 -> 4096 15 / 36 / 37); their float32 sums, about a tile for each
+//     place, meet in a second kernel, in slice order;
 //   * where that is not float32's result a tile's slice is formed again with float32 instructions: a value below 2^-110 whose lowest
 //     bits the parts lose (its l is a subnormal bfloat16; seen in the bits that l cuts off, half an instruction a value), a sum that is not
 //     finite (an infinite value has h = inf and m = NaN, one next to 2^64 can have h x h = inf), and sums of up to three terms, whose
 //     error is that of a term (against float64, one / two / three terms: six products 3.7e-8 / 3.7e-8 / 3.6e-8, float32 2.5e-8 / 3.1e-8 /
-//     3.5e-8; from four on the six products have the smaller one).  512 rows, 2048 -> 4096 with such a value in every stage 166 us (the
-//     library products 131),
-//     with a row of infinities, seen at the end only, 240; the test for them costs the others 2 of 98.
-// Measured (us, both gradients with the adding launch, float32 library products before): 512 rows, 2048 -> 4096 140 -> 103 (matrix cores
-// busy for 41 of them; the write-back of 32 MB at the end of the launch takes 7, the rest is stages in which the workgroups of a unit
-// wait for each other's phases), 295 rows, 808 -> 3840 49 -> 41, 128 rows, 2048 -> 2048 38 -> 27, 72 rows, 1280 -> 712 39 -> 15.  Error against
-// float64 at the first: 3.5e-7 (grad_x) and 3.4e-7, the products before 1.15e-6 and 4.05e-7.  float32 values kept in LDS and taken apart
+//     3.5e-8; from four on the six products have the smaller one).  512 rows, 2048 -> 4096 with such a value in every stage 166 us, with
+//     a row of infinities, which only the end shows, 240 (the library products 131); the test for them costs the others 3 of 98.
+// Measured (us, both gradients with the adding launch / float32 library products): 512 rows, 2048 -> 4096 101 / 131 (the matrix cores are
+// busy for 55 % of it by the counters; the write-back of 32 MB at the end of the launch takes 7, the rest is stages in which the workgroups
+// of a unit wait for each other's phases), 295 rows, 808 -> 3840 38 / 48, 128 rows, 2048 -> 2048 28 / 37, 72 rows, 1280 -> 712 15 / 37, 4096
+// rows, 4096 -> 4096 1450 / 1840, 8 rows of the same 38 / 40.  Error against float64 at the first: 3.4e-7 (grad_x 3.5e-7), the products 4.0e-7
+// (1.15e-6).  float32 values kept in LDS and taken apart
 // by the wavefronts that multiply them (no barrier between the two, each value twice): 113 - 130.
 // Rows behind the operand's end repeat its last ones and are not stored; k behind the end is cleared in both operands.
 #include "tpq_common.h"
@@ -250,7 +250,7 @@ __device__ __forceinline__ void product(const Product& p, int block, int blocks,
         uint32_t cut = 0;
         if (first_operand) put<ALONG>(v, lds, t, cut);
         else put<false>(v, lds_b, t, cut);
-        if (cut & 0xFFFFu) *inexact = 1;
+        return (cut & 0xFFFFu) != 0;
     };
 
     fg_f16 acc[2][2];
@@ -261,13 +261,12 @@ __device__ __forceinline__ void product(const Product& p, int block, int blocks,
 
     load(begin);
     if (threadIdx.x == 0) *inexact = p.K < 4;
+    const bool first_cut = store(begin);
     __syncthreads();
-    store(begin);
-    __syncthreads();
-    uint32_t stop = 0;
+    if (first_cut) *inexact = 1;
+    uint32_t stop = 0;  // what *inexact was between the two barriers before a stage, the same for all of the workgroup
     for (int k0 = begin; k0 < end; k0 += kStageK) {
         const bool more_stages = k0 + kStageK < end;
-        stop = *inexact;  // the same for all: written between the two barriers only
         if (more_stages) load(k0 + kStageK);
 #pragma unroll
         for (int s = 0; s < kStageK / 16; ++s) {
@@ -289,21 +288,23 @@ __device__ __forceinline__ void product(const Product& p, int block, int blocks,
                     acc[f >> 1][f & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kA[e]][f >> 1], b[kB[e]][f & 1], acc[f >> 1][f & 1], 0, 0, 0);
         }
         stop = __builtin_amdgcn_readfirstlane(stop);
-        if (stop) break;
+        if (stop || !more_stages) break;
         __syncthreads();
-        if (more_stages) {
-            store(k0 + kStageK);
-            __syncthreads();
-        }
+        if (store(k0 + kStageK)) *inexact = 1;
+        __syncthreads();
+        stop = *inexact;
     }
 
     // parts that do not add up to their value, or a sum that is not finite (its product with zero is NaN)
-    float left = 0.0f;
+    float left[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int f = 0; f < 4; ++f)
+    for (int e = 0; e < 16; ++e)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) left = __builtin_fmaf(acc[f >> 1][f & 1][e], 0.0f, left);
-    const int again = __syncthreads_or(stop != 0 || left != left);
+        for (int f = 0; f < 4; ++f) left[f] = __builtin_fmaf(acc[f >> 1][f & 1][e], 0.0f, left[f]);
+    const float any = (left[0] + left[1]) + (left[2] + left[3]);
+    if (any != any) *inexact = 1;
+    __syncthreads();
+    const uint32_t again = *inexact;
     write_sums<ALONG>(p, at, wave, lane, acc);
     if (__builtin_amdgcn_readfirstlane(again)) whole_product<ALONG>(p, at, lds);
 }
@@ -323,8 +324,10 @@ struct Finish {
     int slices, parts, blocks;  // parts: neighbouring slices go to one of this many threads
 };
 
-// The slices' sums, added in slice order; blocks of both products in one launch.  Many slices (an output of few tiles) are shared out over
-// parts of a workgroup, whose sums are then added in part order: 512 slices one after the other would be their requests' latency.
+// The slices' sums, added in slice order; blocks of both products in one launch.  Many slices of a small output, whose quads are too few
+// threads for the chip, are shared out over parts of a workgroup, whose sums are then added in part order: 512 slices one after the other
+// would be their requests' latency.  A larger output (more than 128 workgroups of quads) is the slower that way (256 rows, 1648 -> 2560, nine
+// slices: 40 / 36 us).
 __global__ __launch_bounds__(256) void f32_grads_finish_kernel(const Finish x, const Finish w) {
     __shared__ fg_f4 sums[256];
     const bool second = static_cast<int>(blockIdx.x) >= x.blocks;
@@ -347,6 +350,7 @@ __global__ __launch_bounds__(256) void f32_grads_finish_kernel(const Finish x, c
 
 constexpr int64_t kPlaces = 512;  // two workgroups on each of 256 compute units
 constexpr int kLeastStages = 4;
+constexpr int64_t kFewQuads = 128 * 256;
 
 struct Plan {
     int64_t tiles_m, tiles_n, slices, stages;
@@ -362,14 +366,23 @@ Plan plan_of(int64_t M, int64_t N, int64_t K, int64_t stages_each) {
     return p;
 }
 
-// plans of grad_x and grad_w: about the stages that each place gets if all are shared out evenly
+// Plans of grad_x and grad_w: about the stages that each place gets if all are shared out evenly.  Nine to sixteen slices of a product only
+// where all workgroups find a place at once: the few that would not start when the others end, and then take as long (248 rows, 1536 ->
+// 2944: 516 workgroups 47 us, 468 37; 180 rows, 1408 -> 3584 44 / 39).  With more slices they are short (55 rows, 1408 -> 3584: 616 workgroups,
+// 28 slices, 22 us, 517 23), and where the tiles fill the places by themselves there is nothing to lose.
 void plans(int64_t M, int64_t K, int64_t N, bool want_x, bool want_w, Plan (&plan)[2]) {
     const auto tiles = [](int64_t a, int64_t b) { return ((a + kTile - 1) / kTile) * ((b + kTile - 1) / kTile); };
-    const int64_t all = (want_x ? tiles(M, K) * ((N + kStageK - 1) / kStageK) : 0) + (want_w ? tiles(N, K) * ((M + kStageK - 1) / kStageK) : 0);
+    const int64_t tiles_x = want_x ? tiles(M, K) : 0, tiles_w = want_w ? tiles(N, K) : 0;
+    const int64_t all = tiles_x * ((N + kStageK - 1) / kStageK) + tiles_w * ((M + kStageK - 1) / kStageK);
     int64_t each = (all + kPlaces - 1) / kPlaces;
     if (each < kLeastStages) each = kLeastStages;
-    plan[0] = plan_of(M, K, N, each);
-    plan[1] = plan_of(N, K, M, each);
+    const auto settled = [](const Plan& p) { return p.slices <= 8 || p.slices > 16; };
+    for (;; each += each / 8 + 1) {
+        plan[0] = plan_of(M, K, N, each);
+        plan[1] = plan_of(N, K, M, each);
+        const int64_t x = tiles_x * plan[0].slices, w = tiles_w * plan[1].slices;
+        if ((settled(plan[0]) && settled(plan[1])) || tiles_x + tiles_w >= kPlaces || x + w <= kPlaces) return;
+    }
 }
 
 }  // namespace
@@ -433,7 +446,7 @@ TPQ_EXPORT int tpq_f32_linear_grads(const float* grad, const float* x, const flo
         blocks[e] = plan[e].tiles_m * plan[e].tiles_n * plan[e].slices;
         if (p.slices > 1) {
             const int64_t quads = static_cast<int64_t>(p.M) * p.N / 4;
-            const int parts = p.slices > 8 ? 16 : 1;
+            const int parts = p.slices > 8 && quads <= kFewQuads ? 16 : 1;
             finish[e] = Finish{reinterpret_cast<const fg_f4*>(space), reinterpret_cast<fg_f4*>(p.c), quads, p.slices, parts, static_cast<int>((quads * parts + 255) / 256)};
             p.c = space;
             space += p.slices * quads * 4;
