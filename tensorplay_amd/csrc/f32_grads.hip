@@ -30,10 +30,10 @@
 //     a row of infinities, which only the end shows, 240 (the library products 131); the test for them costs the others 3 of 98.
 // Measured (us, both gradients with the adding launch / float32 library products): 512 rows, 2048 -> 4096 101 / 131 (the matrix cores are
 // busy for 55 % of it by the counters; the write-back of 32 MB at the end of the launch takes 7, the rest is stages in which the workgroups
-// of a unit wait for each other's phases), 295 rows, 808 -> 3840 38 / 48, 128 rows, 2048 -> 2048 28 / 37, 72 rows, 1280 -> 712 15 / 37, 4096
-// rows, 4096 -> 4096 1450 / 1840, 8 rows of the same 38 / 40.  Error against float64 at the first: 3.4e-7 (grad_x 3.5e-7), the products 4.0e-7
-// (1.15e-6).  float32 values kept in LDS and taken apart
-// by the wavefronts that multiply them (no barrier between the two, each value twice): 113 - 130.
+// of a unit wait for each other's phases), 295 rows, 808 -> 3840 38 / 48, 128 rows, 2048 -> 2048 28 / 37, 72 rows, 1280 -> 712 15 / 37, 1024
+// rows, 4096 -> 4096 360 / 468, 8 rows of the same 38 / 38.  Error against float64 at the first: 3.4e-7 (grad_x 3.5e-7), the products 4.0e-7
+// (1.15e-6).  float32 values kept in LDS and taken apart by the wavefronts that multiply them (no barrier between the two, each value
+// twice): 113 - 130.
 // Rows behind the operand's end repeat its last ones and are not stored; k behind the end is cleared in both operands.
 #include "tpq_common.h"
 
@@ -452,7 +452,7 @@ TPQ_EXPORT int tpq_f32_linear_grads(const float* grad, const float* x, const flo
             space += p.slices * quads * 4;
         }
     }
-    TPQ_REQUIRE(blocks[0] + blocks[1] <= (1 << 24), TPQ_ERR_UNSUPPORTED, "tpq_f32_linear_grads: too many tiles");
+    TPQ_REQUIRE(blocks[0] + blocks[1] < (1 << 24), TPQ_ERR_UNSUPPORTED, "tpq_f32_linear_grads: too many tiles");
     args.first = static_cast<int>(blocks[0]);
     hipStream_t s = static_cast<hipStream_t>(stream);
     f32_grads_kernel<<<dim3(static_cast<unsigned>(blocks[0] + blocks[1])), dim3(kThreads), 0, s>>>(args);

@@ -22,9 +22,10 @@ def _grads(g, x, w, **want):
 
 
 # one value, edges of the 128 x 128 tiles and of the 32 k stages, several slices of k on either product, many more rows than columns;
-# 9, 46, 129 and 400 slices of one product (a workgroup's parts of one, 3, 9 and 25 of them, the last ones short or empty)
+# 9, 46, 129 and 400 slices of one product (a workgroup's parts of one, 3, 9 and 25 of them, the last ones short or empty), and 12 of one
+# that is added without parts
 SIZES = [(1, 4, 4), (4, 4, 260), (5, 132, 260), (31, 128, 124), (33, 1280, 712), (128, 512, 512), (129, 260, 132), (72, 1280, 4096), (295, 808, 3840), (2100, 96, 64),
-         (1150, 64, 68), (40, 68, 7300), (16500, 60, 124), (64000, 4, 8)]
+         (1150, 64, 68), (129, 1040, 2304), (40, 68, 7300), (16500, 60, 124), (64000, 4, 8)]
 
 
 @pytest.mark.parametrize("m,k,n", SIZES)
