@@ -75,6 +75,29 @@ def test_tiny_values_keep_float32_precision(power):
             assert bool(((got.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("value", [1.1e-39, float("inf")])
+def test_one_such_value_changes_its_own_tiles_only(value):
+    """Several tiles of rows and columns and slices of k in both products, the value in a tile and a slice in the middle."""
+    g, x, w = _case(650, 520, 1100)
+    before = _grads(g, x, w)
+    g[300, 500] = value
+    gx, gw = _grads(g, x, w)
+    rows = torch.ones(650, dtype=torch.bool, device="cuda")
+    rows[256:384] = False  # grad_x: the tile of row 300
+    channels = torch.ones(1100, dtype=torch.bool, device="cuda")
+    channels[384:512] = False  # grad_w: the tile of channel 500
+    assert torch.equal(gx[rows], before[0][rows]) and torch.equal(gw[channels], before[1][channels])
+    rows[300] = channels[500] = True
+    for got, a, b, own, others in ((gx, g, w, 300, ~rows), (gw, g.T, x, 500, ~channels)):
+        want, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+        bound = size * (3 * 2.0 ** -24 + 4 * a.shape[1] ** 0.5 * 2.0 ** -24)
+        assert bool(((got.double() - want).abs() <= bound)[others].all())
+        if value > 1:
+            assert torch.equal(got[own].double(), want[own]) and bool(got[own].isinf().all())
+        else:
+            assert bool(((got.double() - want).abs() <= bound)[own].all())
+
+
 @pytest.mark.parametrize("terms", [1, 2, 3, 4])
 def test_sums_of_few_terms_round_once_a_term(terms):
     from tensorplay_amd import _lib
