@@ -239,6 +239,19 @@ int tpq_ternary_linear_row(const void* x, int x_dtype, const uint8_t* packed, fl
                            int64_t K, float eps, float* out, void* stream);
 
 /*
+ * Dynamically quantized linears of up to 16 activation rows x [M, K] in one launch, with the bits of tpq_quantize_rowwise (divisor 127,
+ * codes -127 .. 127) followed by tpq_int8_mm_dequant (out [M, N] of out_dtype) or by tpq_ternary_mm (out [M, N] float32).  The `_takes` forms
+ * say (1 / 0) whether a shape and its operands are taken: K % 16 == 0 (ternary: 64), M ceil(K / 512) <= 64, at most 2^25 weights
+ * with a compute unit's share in its registers, x and the weight 16-byte aligned; else TPQ_ERR_UNSUPPORTED.
+ */
+int tpq_int8_linear_few_takes(const void* x, const int8_t* w, int64_t M, int64_t N, int64_t K);
+int tpq_int8_linear_few(const void* x, int x_dtype, const int8_t* w, const float* col_scale, const float* bias, int64_t M, int64_t N,
+                        int64_t K, float eps, void* out, int out_dtype, void* stream);
+int tpq_ternary_linear_few_takes(const void* x, const uint8_t* packed, int64_t M, int64_t N, int64_t K);
+int tpq_ternary_linear_few(const void* x, int x_dtype, const uint8_t* packed, float w_scale, const float* bias, int64_t M, int64_t N,
+                           int64_t K, float eps, float* out, void* stream);
+
+/*
  * The same of M > 0 activation rows x [M, K] with the codes (int8 [M, K], 16-byte aligned) and scales (f32 [M]) of the rows in the
  * caller's memory: tpq_quantize_rowwise and tpq_ternary_mm_ws, with the same result bits.  Where the weight is written out as int8
  * rows first (a workspace of tpq_ternary_linear_workspace_bytes, K % 4 == 0, 8 <= K <= 16384, x 16-byte aligned), one launch does

@@ -47,6 +47,7 @@ struct Library {
     TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine) \
     TPQ_ENTRY(tpq_f32_linear_grads_workspace_bytes) TPQ_ENTRY(tpq_f32_linear_grads) \
     TPQ_ENTRY(tpq_f32_linear_grads_takes) TPQ_ENTRY(tpq_quantize_beside_takes) \
+    TPQ_ENTRY(tpq_int8_linear_few_takes) TPQ_ENTRY(tpq_int8_linear_few) TPQ_ENTRY(tpq_ternary_linear_few_takes) TPQ_ENTRY(tpq_ternary_linear_few) \
     TPQ_ENTRY(tpq_quantize_both_rowwise) TPQ_ENTRY(tpq_quantize_rowwise_pad)
     TPQ_ENTRIES
 #undef TPQ_ENTRY
@@ -281,6 +282,16 @@ TPQ_CALL(int8_linear, 7)
         Py_RETURN_NONE;
     at::Tensor out;
     int status;
+    if (lib.tpq_int8_linear_few_takes(x->const_data_ptr(), ptr<int8_t>(w), M, N, K)) {
+        {
+            Enqueue q(*x);
+            out = allocate(sizes, type, *x);
+            status = lib.tpq_int8_linear_few(x->const_data_ptr(), float_tag(x->scalar_type()), ptr<int8_t>(w), ptr<float>(cs), ptr<float>(bias), M, N, K,
+                                             static_cast<float>(eps), out.data_ptr(), float_tag(type), q.stream);
+        }
+        if (status != TPQ_OK) Py_RETURN_NONE;
+        return THPVariable_Wrap(std::move(out));
+    }
     {
         Enqueue q(*x);
         const Quantized room = room_for_codes(*x, M, pitch, lib.tpq_int8_mm_workspace_bytes(M, N, pitch));
@@ -332,8 +343,8 @@ TPQ_CALL(lowbit_linear, 8)
     return THPVariable_Wrap(std::move(out));
 TPQ_CALL_END
 
-// One row of a weight of up to this many codes: the product quantizes the row itself.  Each of its workgroups reads and quantizes
-// the whole row, so beyond, the quantizer's launch and codes in memory are the cheaper way.  Measured (us, weights from HBM,
+// One row of a weight of up to this many codes: the row kernel quantizes the row itself.  Each of its workgroups reads and quantizes
+// the whole row, so beyond, the kernel of few rows, one workgroup per compute unit, or the quantizer's launch and codes in memory are the cheaper way.  Measured (us, weights from HBM,
 // float16, one launch / two): 2560 -> 6912 5.49 / 6.06, 4096 x 4096 5.34 / 6.02, 2560 -> 9216 5.67 / 5.91, 4096 -> 6144 6.01 / 5.98,
 // 5120 x 5120 6.23 / 6.41 (float32 7.30 / 6.62), 2560 -> 10240 6.39 / 6.16, 4096 -> 8192 7.23 / 6.75, 4096 -> 14336 10.2 / 7.6,
 // 8192 -> 28672 35.7 / 17.3.
@@ -356,9 +367,12 @@ TPQ_CALL(ternary_linear, 6)
     int status = TPQ_ERR_UNSUPPORTED;
     {
         Enqueue q(*x);
-        const bool one_launch = M == 1 && N * K <= kRowQuantizedInProduct;
-        if (one_launch) {
-            out = allocate(sizes, at::kFloat, *x);
+        const bool row = M == 1 && N * K <= kRowQuantizedInProduct, one_launch = row || lib.tpq_ternary_linear_few_takes(x->const_data_ptr(), ptr<uint8_t>(packed), M, N, K);
+        if (one_launch) out = allocate(sizes, at::kFloat, *x);
+        if (one_launch && !row)
+            status = lib.tpq_ternary_linear_few(x->const_data_ptr(), float_tag(x->scalar_type()), ptr<uint8_t>(packed), static_cast<float>(w_scale), ptr<float>(bias), M, N, K,
+                                                static_cast<float>(eps), out_ptr<float>(out), q.stream);
+        if (row) {
             status = lib.tpq_ternary_linear_row(x->const_data_ptr(), float_tag(x->scalar_type()), ptr<uint8_t>(packed), static_cast<float>(w_scale), ptr<float>(bias), N, K,
                                                 static_cast<float>(eps), out_ptr<float>(out), q.stream);
         }

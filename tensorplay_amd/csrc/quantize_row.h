@@ -68,9 +68,9 @@ __device__ __forceinline__ void quantize_eight_packed(const float (&v)[kVec], fl
 // (rint(divisor (1 + 2^-20)) <= qmax and >= -qmin, true for the usual divisor = qmax = -qmin = 127): no clamp is
 // needed, and the code is read off the mantissa.  t = fma(v, 1/scale, 1.5 * 2^23) rounds the exact product to the
 // nearest integer (ties to even) and leaves it in two's complement in the low mantissa bits; c = t - 1.5 * 2^23 is that
-// integer, r = fma(v, 1/scale, -c) its distance from the product.  The product is within 2^-16 of the correctly rounded
-// quotient the reference rounds, so |r| <= 1/2 - 2^-13 proves both round to c; anything else (also NaN) is redone with
-// the division.  Five instructions per code and three byte permutes per four codes.
+// integer, r = fma(v, 1/scale, -c) its distance from the product, rounded by 2^-25 at most.  The product is within 2^-16 of the
+// correctly rounded quotient the reference rounds (two roundings of 2^-24 relative, |quotient| <= 128), so |r| <= 1/2 - 2^-15 proves both
+// round to c; anything else (also NaN) is redone with the division: one element in 16 000, a wavefront in 30 where a limit of 2^-13 sent one in 8.  Five instructions per code and three byte permutes per four codes.
 __device__ __forceinline__ void quantize_eight_lean(const float (&v)[kVec], float scale, float inv_scale, const QParams& p,
                                                     uint32_t& lo, uint32_t& hi) {
     constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
@@ -81,7 +81,7 @@ __device__ __forceinline__ void quantize_eight_lean(const float (&v)[kVec], floa
         const float tf = __builtin_fmaf(v[i], inv_scale, kMagic);
         const float c = tf - kMagic;
         const float r = __builtin_fmaf(v[i], inv_scale, -c);
-        redo |= !(fabsf(r) <= 0.5f - 0x1p-13f);
+        redo |= !(fabsf(r) <= 0.5f - 0x1p-15f);
         t[i] = __builtin_bit_cast(uint32_t, tf);
     }
     // v_perm_b32(a, b, sel): selector bytes 0..3 take bytes of b, 4..7 of a, 0x0c a zero byte
