@@ -16,8 +16,11 @@
 //     its channels once for more rows, and 203 rows of 4096 -> 11008 are 172 tiles of 112 rows in one round of workgroups instead of 344 of 64
 //     in two (2 bits 48.5 -> 32, int4 41 -> 28 us; int4 at 256 rows 43 -> 34, at 384 66 -> 53);
 //   * its eight multiplying wavefronts are CW channel positions x KW steps of 128 k: a round of the loop covers KW steps, whose
-//     activations two more wavefronts fetch by direct global -> LDS loads (whole lines, one copy per workgroup, double
-//     buffered, the swizzle of the fragment reads applied on the global side) while the round before is multiplied.  A direct
+//     activations two more wavefronts fetch by direct global -> LDS loads (whole lines, one copy per workgroup, the
+//     swizzle of the fragment reads applied on the global side) into a ring of two to three rounds while the rounds before are multiplied:
+//     with two, a round's loads were all waited for before the next ones were asked for (us, two rounds / as many as fit: 85 rows of
+//     2240 -> 2560 in groups of 64 16.2 / 12.4, 150 and 256 rows of 4096 x 4096 14.4 / 12.7 and 15.6 / 14.0, 240 rows of 4096 -> 11008 34.5 / 31.9, 48
+//     rows of 11008 -> 4096 15.7 / 15.4; tiles of one and two blocks of rows keep two: nothing gained).  A direct
 //     load blocks the wavefront that issues it until the memory path accepts it, and vector loads return in order, so in a
 //     multiplying wavefront it would stand in front of the products and tie the weights' prefetch to the activations';
 //   * packed weights and parameters are loaded two rounds ahead, into registers (four rounds: the same times, 40 registers
@@ -256,18 +259,24 @@ __device__ float one_sum(const PackedRowsArgs& a, int m, int n, int k0, int k1) 
     return sum;
 }
 
+// Slots of one step of activations each in a workgroup's ring: two rounds of the small ones, up to three of those from 12 KB on, as far as a
+// compute unit's LDS holds them
+constexpr int rows_ring_slots(int slot_bytes, int kw) {
+    const int most = 160 * 1024 / slot_bytes, wanted = slot_bytes >= 12 * 1024 ? 3 * kw : 2 * kw;
+    return most < wanted ? most : wanted;
+}
+
 template <int DT, class Source, int MB, int CW, bool EDGE, bool SPLIT>
 __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedRowsArgs a) {
     using A = RowsArith<DT>;
     using P = RowsParams<DT, Source::kTypedParams>;
     using storage = typename Elem<DT>::storage;
     constexpr int KW = 8 / CW, NB = kRowsNB, kRows = 16 * MB, kStepBytes = A::kChunks * 16;
-    constexpr int kRoundLoads = KW * kRows * kStepBytes / 1024, kMine = kRoundLoads / kRowsProducers;  // 1 KB loads of a round, a requesting wavefront's
-    constexpr int kLoadsPerStep = kRows * kStepBytes / 1024, kRowsPerLoad = 64 / A::kChunks;
-    constexpr int kBuffer = kRoundLoads * 1024;
+    constexpr int kLoadsPerStep = kRows * kStepBytes / 1024, kMine = kLoadsPerStep / kRowsProducers;  // 1 KB loads of a step, a requesting wavefront's
+    constexpr int kRowsPerLoad = 64 / A::kChunks, kSlot = kLoadsPerStep * 1024, kSlots = rows_ring_slots(kSlot, KW);
     static_assert(!SPLIT || DT != TPQ_DTYPE_F32, "float32 weights are not rounded");
-    static_assert(kRoundLoads % kRowsProducers == 0, "every wavefront loads the same number of pieces");
-    extern __shared__ uint4 pr_lds[];  // [2][KW][kRows][kStepBytes], later the partial sums [CW][NB][MB][KW][64 lanes]
+    static_assert(kLoadsPerStep % kRowsProducers == 0 && kSlots >= 2 * KW, "every wavefront loads the same number of pieces");
+    extern __shared__ uint4 pr_lds[];  // [kSlots][kRows][kStepBytes], later the partial sums [CW][NB][MB][KW][64 lanes]
     char* const lds = reinterpret_cast<char*>(pr_lds);
 
     const int lane = threadIdx.x & (kWave - 1);
@@ -287,43 +296,67 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     // LDS traffic only: the loads of weights stay in flight
     auto lds_barrier = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
-    // ---- the requesting wavefronts: pieces of 1 KB, kRowsPerLoad rows of a step each; one barrier per round
+    // ---- the requesting wavefronts: pieces of 1 KB, kRowsPerLoad rows of a step each; step t of the slice in slot t % kSlots, one barrier
+    // per round.  One round is asked for at first (more would stand in front of the first weights: 232 rows of 6656 -> 576, two rounds of
+    // the loop, 13.3 -> 13.7 us), and from the first barrier on what the ring holds, so that loads are under way while a round is waited for.
     if (wave >= 8) {
         const uint32_t row_bytes = static_cast<uint32_t>(a.K) * A::kElem;
         const char* const x_base = static_cast<const char*>(a.x) + static_cast<size_t>(m0) * row_bytes;
         const uint32_t ring_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((pr_lds_ptr)pr_lds));
         const int first = (wave - 8) * kMine;
         uint32_t x_off[kMine];  // byte offset of the lane's chunk in step 0
+        auto chunk_of = [&](int j) __attribute__((always_inline)) { return (lane % A::kChunks) ^ (((first + j) * kRowsPerLoad + lane / A::kChunks) & 15); };
 #pragma unroll
         for (int j = 0; j < kMine; ++j) {
-            const int row = (first + j) % kLoadsPerStep * kRowsPerLoad + lane / A::kChunks;
-            x_off[j] = static_cast<uint32_t>(m0 + row < a.M ? row : a.M - 1 - m0) * row_bytes + static_cast<uint32_t>((lane % A::kChunks) ^ (row & 15)) * 16;
+            const int row = (first + j) * kRowsPerLoad + lane / A::kChunks;
+            x_off[j] = static_cast<uint32_t>(m0 + row < a.M ? row : a.M - 1 - m0) * row_bytes + static_cast<uint32_t>(chunk_of(j)) * 16;
         }
-        for (int round = 0; round < rounds; ++round) {
-            const uint32_t buffer_addr = ring_addr + (round & 1) * kBuffer;
-#pragma unroll
-            for (int j = 0; j < kMine; ++j) {
-                const int step = step_of(round, (first + j) / kLoadsPerStep);
-                uint32_t off = x_off[j];
-                if constexpr (EDGE) {  // the last chunk of the row in place of the ones behind it
-                    const int chunk = (lane % A::kChunks) ^ (((first + j) % kLoadsPerStep * kRowsPerLoad + lane / A::kChunks) & 15);
-                    const int behind = chunk - ((step == steps_all - 1 ? edge_chunks : A::kChunks) - 1);
-                    off -= static_cast<uint32_t>(behind > 0 ? behind : 0) * 16;
-                }
+        const int total = rounds * KW;
+        int asked = 0, fill = 0;  // steps asked for; the slot of the next one
+        auto ask_up_to = [&](int limit) __attribute__((always_inline)) {
+            for (limit = limit < total ? limit : total; asked < limit; ++asked) {
+                const int step = step_of(0, asked);
                 const char* const from = x_base + static_cast<size_t>(step) * kStepBytes;
-                const uint32_t to = buffer_addr + (first + j) * 1024;
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(from) : "memory", "m0");
-            }
-            __builtin_amdgcn_s_waitcnt(pr_vmcnt(0));
-            if constexpr (EDGE) {  // zeros over what was fetched in place of chunks behind K
 #pragma unroll
                 for (int j = 0; j < kMine; ++j) {
-                    const int chunk = (lane % A::kChunks) ^ (((first + j) % kLoadsPerStep * kRowsPerLoad + lane / A::kChunks) & 15);
-                    if (step_of(round, (first + j) / kLoadsPerStep) == steps_all - 1 && chunk >= edge_chunks)
-                        *reinterpret_cast<uint4*>(lds + (round & 1) * kBuffer + (first + j) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+                    uint32_t off = x_off[j];
+                    if constexpr (EDGE) {  // the last chunk of the row in place of the ones behind it
+                        const int behind = chunk_of(j) - ((step == steps_all - 1 ? edge_chunks : A::kChunks) - 1);
+                        off -= static_cast<uint32_t>(behind > 0 ? behind : 0) * 16;
+                    }
+                    const uint32_t to = ring_addr + fill * kSlot + (first + j) * 1024;
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(from) : "memory", "m0");
+                }
+                fill = fill + 1 == kSlots ? 0 : fill + 1;
+            }
+        };
+        // all but the loads of the last `steps` steps have landed
+        auto wait_but = [&](int steps) __attribute__((always_inline)) {
+            bool done = false;
+            pr_static_for<0, kSlots - KW + 1>([&](auto e) __attribute__((always_inline)) {
+                constexpr int N = kSlots - KW - decltype(e)::value, kCount = N * kMine < 63 ? N * kMine : 63;  // (the counter ends at 63: a wait for more)
+                if (!done && steps >= N) {
+                    __builtin_amdgcn_s_waitcnt(pr_vmcnt(kCount));
+                    done = true;
+                }
+            });
+        };
+        ask_up_to(KW);
+        for (int round = 0; round < rounds; ++round) {
+            wait_but(asked - (round + 1) * KW);
+            if constexpr (EDGE) {  // zeros over what was fetched in place of chunks behind K
+#pragma unroll
+                for (int k = 0; k < KW; ++k) {
+                    if (step_of(round, k) == steps_all - 1) {
+                        char* const slot = lds + static_cast<uint32_t>(round * KW + k) % static_cast<uint32_t>(kSlots) * kSlot;
+#pragma unroll
+                        for (int j = 0; j < kMine; ++j)
+                            if (chunk_of(j) >= edge_chunks) *reinterpret_cast<uint4*>(slot + (first + j) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+                    }
                 }
             }
             lds_barrier();  // round `round` is there, and everybody is done with the round before it
+            ask_up_to(kSlots + round * KW);
         }
         __syncthreads();  // the products of the last round are done
         __syncthreads();  // the sums are in LDS
@@ -447,12 +480,13 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
 
     // A step's products in pieces: piece c = u MB + r is chunk u of the lane's activations for row block r
     constexpr int kU = A::kChunks / 4, kPieces = kU * MB, kFragments = kPieces < 3 ? kPieces : 3;
-    const char* const frag_base = lds + kk * (kLoadsPerStep * 1024) + i * kStepBytes;
+    const char* const frag_base = lds + i * kStepBytes;
+    int slot = kk;  // of this wavefront's step in the current round
     pr_word4 frag[kFragments];
-    auto read_piece = [&](int buffer, auto c) __attribute__((always_inline)) {
+    auto read_piece = [&](const char* from, auto c) __attribute__((always_inline)) {
         constexpr int C = decltype(c)::value;
         if constexpr (C < kPieces)
-            frag[C % kFragments] = *reinterpret_cast<const pr_word4*>(frag_base + buffer * kBuffer + (C % MB) * (16 * kStepBytes) + (((kU * q + C / MB)) ^ i) * 16);
+            frag[C % kFragments] = *reinterpret_cast<const pr_word4*>(from + (C % MB) * (16 * kStepBytes) + ((kU * q + C / MB) ^ i) * 16);
     };
     // float32: a piece's own sum, added to its step's while the next piece multiplies
     float4_t piece[DT == TPQ_DTYPE_F32 ? 2 : 1][NB], step_sum[NB][DT == TPQ_DTYPE_F32 ? MB : 1];
@@ -499,15 +533,17 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     // afterwards.  The last chunk prepares the first one of the next step (next; NEXT), and the ring slot is asked for again
     // as soon as its last codes are used.
     constexpr int kShare = NB * kChunkPairs;
-    auto products = [&](Loaded& d, const Loaded& next, int buffer, int load_round, auto has_next, auto load_c) __attribute__((always_inline)) {
+    auto products = [&](Loaded& d, const Loaded& next, int load_round, auto has_next, auto load_c) __attribute__((always_inline)) {
         constexpr bool NEXT = decltype(has_next)::value, LOAD = decltype(load_c)::value;
-        pr_static_for<0, kFragments - 1>([&](auto c) __attribute__((always_inline)) { read_piece(buffer, c); });
+        const char* const from = frag_base + slot * kSlot;
+        slot = slot + KW >= kSlots ? slot + KW - kSlots : slot + KW;
+        pr_static_for<0, kFragments - 1>([&](auto c) __attribute__((always_inline)) { read_piece(from, c); });
         pr_static_for<0, kPieces>([&](auto c) __attribute__((always_inline)) {
             constexpr int C = decltype(c)::value, U = C / MB, r = C % MB;
             constexpr std::integral_constant<int, r * kShare / MB> first{};
             constexpr std::integral_constant<int, (r + 1) * kShare / MB> last{};
             constexpr std::integral_constant<int, (U + 1) % kU> following{};
-            read_piece(buffer, std::integral_constant<int, C + kFragments - 1>{});
+            read_piece(from, std::integral_constant<int, C + kFragments - 1>{});
             multiply_piece(c);
             if constexpr (U + 1 < kU) dequantize(d, following, first, last);
             else if constexpr (NEXT) dequantize(next, following, first, last);
@@ -520,7 +556,7 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     Loaded ring[kRowsAhead];
     auto phase = [&](int round, auto slot_c, auto load_c) __attribute__((always_inline)) {  // a round that is not the last; slot_c = round % kRowsAhead
         constexpr int SLOT = decltype(slot_c)::value;
-        products(ring[SLOT], ring[(SLOT + 1) % kRowsAhead], SLOT & 1, round + kRowsAhead, std::true_type{}, load_c);
+        products(ring[SLOT], ring[(SLOT + 1) % kRowsAhead], round + kRowsAhead, std::true_type{}, load_c);
         lds_barrier();
     };
     pr_static_for<0, kRowsAhead>([&](auto r) __attribute__((always_inline)) { load_w(decltype(r)::value, ring[decltype(r)::value]); });
@@ -544,7 +580,7 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     pr_last_rounds<0, kRowsAhead>(rounds - round, [&](auto r) __attribute__((always_inline)) { phase(round + decltype(r)::value, r, std::false_type{}); },
                                   [&](auto r) __attribute__((always_inline)) {
                                       constexpr int SLOT = decltype(r)::value;
-                                      if (s_begin + (round + SLOT) * KW + kk < s_end) products(ring[SLOT], ring[SLOT], SLOT & 1, 0, std::false_type{}, std::false_type{});
+                                      if (s_begin + (round + SLOT) * KW + kk < s_end) products(ring[SLOT], ring[SLOT], 0, std::false_type{}, std::false_type{});
                                   });
     __syncthreads();
 
@@ -640,7 +676,7 @@ inline int64_t ceil_div(int64_t a, int64_t b) {
 }
 
 // Tile height, channels per workgroup and slices of K by an estimate (us) fitted to a sweep of 1 .. 8 slices and both widths
-// over six shapes and 16 .. 256 rows (128 channels and 5 .. 8 blocks of rows, on the same line: 1.36 and 1.49 us a round at 7 and 8): 4 for
+// over six shapes and 16 .. 256 rows (128 channels and 5 .. 8 blocks of rows, on the same line: 1.36 and 1.49 us a round at 7 and 8; unrounded weights 1.29, 1.43, 1.66 and 1.86 us at 1 .. 4 blocks): 4 for
 // the launch, the first loads and the epilogue, per round what the comment on the kernel says, per round of workgroups over the compute
 // units, and 2 + the bytes of the slices' sums (written and read) at 4 TB/s for the second kernel.  Within 5 % of the sweep's best nearly
 // everywhere (11008 -> 4096 at 128 rows 24.8, best 22.7).  A call plans twice (workspace, launch), so what the heights have in common, the
@@ -672,7 +708,7 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
             const int64_t row_tiles = ceil_div(blocks, mb);
             if (ceil_div(blocks, row_tiles) != mb) continue;
             const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
-            const double round_us = wide ? 0.2 + 2.1 * mb : cw == 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb;
+            const double round_us = wide ? 0.2 + 2.1 * mb : p.split ? 1.08 + 0.19 * mb : cw == 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb;
             for (int c = 0; c < cuts; ++c) {
                 const int64_t z = slices_of[c], rounds = (steps_of[c] + (1 << kw_shift) - 1) >> kw_shift;
                 const double waves = static_cast<double>((tiles * z + 255) >> 8);  // 256 compute units
@@ -691,7 +727,8 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
 template <int DT, class Source, int MB, int CW, bool EDGE, bool SPLIT>
 int launch_packed_rows_shape(const PackedRowsArgs& a, int slices, hipStream_t s) {
     constexpr int KW = 8 / CW, NB = kRowsNB;
-    constexpr size_t stage = 2 * static_cast<size_t>(KW) * 16 * MB * RowsArith<DT>::kChunks * 16, sums = static_cast<size_t>(8) * NB * MB * 1024;
+    constexpr int kSlot = 16 * MB * RowsArith<DT>::kChunks * 16;
+    constexpr size_t stage = static_cast<size_t>(rows_ring_slots(kSlot, KW)) * kSlot, sums = static_cast<size_t>(8) * NB * MB * 1024;
     constexpr size_t smem = stage > sums ? stage : sums;
     static_assert(smem <= 160 * 1024, "LDS of one compute unit");
     auto kernel = packed_rows_kernel<DT, Source, MB, CW, EDGE, SPLIT>;
