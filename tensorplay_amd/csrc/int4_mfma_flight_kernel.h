@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kFlightWaves* kWave) void int4_mfma_flight_kernel(c
     extern __shared__ __align__(16) unsigned char flight_lds[];
     unsigned char* const xbuf = flight_lds;
     uint32_t* const par = reinterpret_cast<uint32_t*>(flight_lds + static_cast<size_t>(kFlightWaves) * XS * XR * kFlightRowStride);
-    float* const red = reinterpret_cast<float*>(par + kFlightWaves * SPW * PW * kWave);  // [wave][NB][4][4 XR]
+    float4_t* const red = reinterpret_cast<float4_t*>(par + kFlightWaves * SPW * PW * kWave);  // [wave][NB][4 XR]: four channels of a row
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -265,10 +265,9 @@ __global__ __launch_bounds__(kFlightWaves* kWave) void int4_mfma_flight_kernel(c
         }
     }
 
-    // constant A of the correction MFMA: row 0 = offset + 8 of the pair parity, row 1 = ones
-    uint32_t a_corr_even = 0, a_corr_odd = 0;
-    if (i == 0) { a_corr_even = ML::kOffEven; a_corr_odd = ML::kOffOdd; }
-    if (i == 1) { a_corr_even = ML::kOnes; a_corr_odd = ML::kOnes; }
+    // constant A of the correction MFMA: even rows = offset + 8 of the pair parity, odd rows = ones, so that every lane gets the two sums of
+    // its column in its own registers 0 and 1 (in rows 0 and 1 alone they had to come through LDS, twice a step)
+    const uint32_t a_corr_even = i & 1 ? ML::kOnes : ML::kOffEven, a_corr_odd = i & 1 ? ML::kOnes : ML::kOffOdd;
     uint32_t magic_even, magic_odd;  // kept in VGPRs behind an opaque move: v_and_or_b32 takes one literal only
     asm volatile("v_mov_b32 %0, %1" : "=v"(magic_even) : "s"(L::kMagicEven));
     asm volatile("v_mov_b32 %0, %1" : "=v"(magic_odd) : "s"(L::kMagicOdd));
@@ -282,7 +281,7 @@ __global__ __launch_bounds__(kFlightWaves* kWave) void int4_mfma_flight_kernel(c
 #pragma unroll
         for (int h = 0; h < PW; ++h) my_par[(j * PW + h) * kWave + lane] = pw[j][h];
 
-    float* const ssq = red + kFlightWaves * NB * 4 * (4 * XR);  // [wave][XR], NORM only
+    float* const ssq = reinterpret_cast<float*>(red + kFlightWaves * NB * (4 * XR));  // [wave][XR], NORM only
     float* const undo = ssq + kFlightWaves * XR;                // [wave][XR], NORM with fp16: 2^(ex + eg) of the row's products
     if constexpr (NORM) {
         // lane (i, q) holds eight k of row 4 t + q per step: squares added per row, the values multiplied by g in place.
@@ -310,11 +309,7 @@ __global__ __launch_bounds__(kFlightWaves* kWave) void int4_mfma_flight_kernel(c
                     mag = mag > hi ? mag : hi;
                 }
             }
-#pragma unroll
-            for (int off = 8; off > 0; off >>= 1) {
-                const uint32_t other = __shfl_xor(mag, off, kWave);
-                mag = mag > other ? mag : other;
-            }
+            over_16_lanes(mag, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
             eg = static_cast<int>(mag >> 10) - 14;  // |g| < 2^eg (biased exponent - 15 + 1)
             eg = eg < -15 ? -15 : eg > 16 ? 16 : eg;
             const half2_t gs = __builtin_bit_cast(half2_t, pow2_half2(-eg));
@@ -336,8 +331,7 @@ __global__ __launch_bounds__(kFlightWaves* kWave) void int4_mfma_flight_kernel(c
                 for (int e = 0; e < 4; ++e)
                     if (j < SPW - 1 || last_counts) acc = L::dot(xw[e], xw[e], acc);  // a step past the end was read twice
             }
-#pragma unroll
-            for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
+            over_16_lanes(acc, [](float a, float b) { return a + b; });
             if (i == 0) ssq[wave * XR + 4 * t + q] = acc;  // read behind the barrier at the end
             [[maybe_unused]] half2_t xs;
             if constexpr (DT == TPQ_DTYPE_F16) {
@@ -403,8 +397,7 @@ __global__ __launch_bounds__(kFlightWaves* kWave) void int4_mfma_flight_kernel(c
 #pragma unroll
             for (int u = 0; u < 4; ++u) d[b] = ML::mfma(word4_t{v[0][u], v[1][u], v[2][u], v[3][u]}, xb[u], d[b]);
         }
-        // rows 0 and 1 of the correction product sit in lanes 0..15, registers 0 and 1
-        const float corr = __shfl(aux[0], i, kWave), sx = __shfl(aux[1], i, kWave);
+        const float corr = aux[0], sx = aux[1];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const uint4 p = *reinterpret_cast<const uint4*>(my_par + j * PW * kWave + 16 * b + 4 * q);
@@ -473,12 +466,14 @@ __global__ __launch_bounds__(kFlightWaves* kWave) void int4_mfma_flight_kernel(c
     if (i < XR) {
 #pragma unroll
         for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                float part = yacc[rb][b][v];
-                if constexpr (NORM && DT == TPQ_DTYPE_F16) part *= undo[wave * XR + i];  // this wavefront's own write, same row: exact
-                red[((wave * NB + b) * 4 + v) * (4 * XR) + slot] = part;
+        {
+            float4_t part = {yacc[rb][b][0], yacc[rb][b][1], yacc[rb][b][2], yacc[rb][b][3]};
+            if constexpr (NORM && DT == TPQ_DTYPE_F16) {  // this wavefront's own write, same row: exact
+                const float back = undo[wave * XR + i];
+                part = float4_t{part[0] * back, part[1] * back, part[2] * back, part[3] * back};
             }
+            red[(wave * NB + b) * (4 * XR) + slot] = part;
+        }
     }
     __syncthreads();
     const int out_row = XR * rb + i;  // RB = 1: i
@@ -490,13 +485,16 @@ __global__ __launch_bounds__(kFlightWaves* kWave) void int4_mfma_flight_kernel(c
         if (n >= out.N) continue;  // N % 8 == 0 and n % 4 == 0: all four channels exist
         float sum[PAIR ? 2 : 1][4];
 #pragma unroll
-        for (int h = 0; h < (PAIR ? 2 : 1); ++h)
+        for (int h = 0; h < (PAIR ? 2 : 1); ++h) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                sum[h][v] = 0.0f;
+            for (int v = 0; v < 4; ++v) sum[h][v] = 0.0f;
+#pragma unroll 8  // (all sixteen reads at once are 64 registers a sum: the narrow forms lose their second workgroup per compute unit)
+            for (int ww = 0; ww < kFlightWaves; ++ww) {
+                const float4_t part = red[(ww * NB + b + h * C) * (4 * XR) + slot];
 #pragma unroll
-                for (int ww = 0; ww < kFlightWaves; ++ww) sum[h][v] += red[((ww * NB + b + h * C) * 4 + v) * (4 * XR) + slot];
+                for (int v = 0; v < 4; ++v) sum[h][v] += part[v];
             }
+        }
         if constexpr (NORM) {  // the row's factor rsqrt(mean(x^2) + eps)
             float total = 0.0f;
 #pragma unroll

@@ -132,10 +132,9 @@ __device__ __forceinline__ void int4_mfma_body(
     unsigned char* const xch_put = lds_raw + wave * kXBytes + (lane >> 4) * kXPitch + (lane & 15) * 16;  // + 4 c rows
     const unsigned char* const xch_get = lds_raw + wave * kXBytes + i * kXPitch + q * 64;                 // + 16 c
 
-    // constant A of the correction MFMA: row 0 = offset + 8 of the pair parity, row 1 = ones
-    uint32_t a_corr_even = 0, a_corr_odd = 0;
-    if (i == 0) { a_corr_even = ML::kOffEven; a_corr_odd = ML::kOffOdd; }
-    if (i == 1) { a_corr_even = ML::kOnes; a_corr_odd = ML::kOnes; }
+    // constant A of the correction MFMA: even rows = offset + 8 of the pair parity, odd rows = ones, so that every lane gets the two sums of
+    // its column in its own registers 0 and 1
+    const uint32_t a_corr_even = i & 1 ? ML::kOnes : ML::kOffEven, a_corr_odd = i & 1 ? ML::kOnes : ML::kOffOdd;
     uint32_t magic_even, magic_odd;  // kept in VGPRs behind an opaque move: v_and_or_b32 takes one literal only
     asm volatile("v_mov_b32 %0, %1" : "=v"(magic_even) : "s"(L::kMagicEven));
     asm volatile("v_mov_b32 %0, %1" : "=v"(magic_odd) : "s"(L::kMagicOdd));
@@ -261,8 +260,7 @@ __device__ __forceinline__ void int4_mfma_body(
         }
 #pragma unroll
         for (int r = 0; r < MB; ++r) {
-            // rows 0 and 1 of the correction product sit in lanes 0..15, registers 0 and 1
-            const float corr = __shfl(aux[r][0], i, kWave), sx = __shfl(aux[r][1], i, kWave);
+            const float corr = aux[r][0], sx = aux[r][1];
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
 #pragma unroll

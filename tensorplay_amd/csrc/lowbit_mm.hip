@@ -141,13 +141,14 @@ __global__ __launch_bounds__(WAVES * kWave) void lowbit_mfma_kernel(
     unsigned char* const xch_put = xch + (lane / kPiecesPerRow) * kPitch + (lane % kPiecesPerRow) * 16;  // + kRowsPerLoad j rows
     const unsigned char* const xch_get = xch + i * kPitch + q * (F::kCodes * 2);                        // + 16 c
 
-    // constant A of the offset MFMA: row 0 = the offsets of the eight k of an MFMA (pairs 0..3 of the
-    // lane's codes: the pattern repeats every byte, so every MFMA has the same), row 1 = ones
+    // constant A of the offset MFMA: even rows = the offsets of the eight k of an MFMA (pairs 0..3 of the
+    // lane's codes: the pattern repeats every byte, so every MFMA has the same), odd rows = ones, so that every lane gets the two sums of its
+    // column in its own registers 0 and 1
     uint32_t a_corr[4];
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
-        if constexpr (DT == TPQ_DTYPE_F16) a_corr[h] = i == 0 ? F::magic(h) : i == 1 ? 0x3C003C00u : 0u;
-        else a_corr[h] = (i == 0 && kFieldsInPlace) ? F::magic_bf(h) : i == 1 ? 0x3F803F80u : 0u;
+        if constexpr (DT == TPQ_DTYPE_F16) a_corr[h] = i & 1 ? 0x3C003C00u : F::magic(h);
+        else a_corr[h] = i & 1 ? 0x3F803F80u : kFieldsInPlace ? F::magic_bf(h) : 0u;
     }
     uint32_t magic[F::kMagics];  // kept in VGPRs behind opaque moves: v_and_or_b32 takes one scalar operand
 #pragma unroll
@@ -225,8 +226,7 @@ __global__ __launch_bounds__(WAVES * kWave) void lowbit_mfma_kernel(
             // 9.6 / 9.9 / 10.6 -> 9.0 / 9.7 / 10.2 us; at 2 and 4 rows it costs 0.2 - 0.4).
             if constexpr (kFieldsInPlace && (DT != TPQ_DTYPE_F16 || XL == 2)) __builtin_amdgcn_sched_barrier(0);
         }
-        // rows 0 and 1 of the offset product sit in lanes 0..15, registers 0 and 1
-        const float corr = __shfl(aux[0], i, kWave), sx = __shfl(aux[1], i, kWave);
+        const float corr = aux[0], sx = aux[1];
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll

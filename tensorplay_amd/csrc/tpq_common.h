@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "../../include/tpq.h"
 
@@ -186,21 +187,36 @@ __device__ __forceinline__ void load_eight(const typename Elem<DT>::storage* p, 
     }
 }
 
-// ---- 64-lane reductions -----------------------------------------------------
+// ---- reductions over lanes -----------------------------------------------------
 
+// v := op over the sixteen neighbouring lanes that share a quarter of the wavefront, in each of them: four moves between lanes, where
+// __shfl_xor is a trip through LDS each.  All lanes of the wavefront take part.
+template <class T, class Op>
+__device__ __forceinline__ void over_16_lanes(T& v, Op op) {
+    auto moved = [&](auto control) { return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(control)::value, 0xF, 0xF, true)); };
+    v = op(v, moved(std::integral_constant<int, 0xB1>{}));   // quad_perm [1, 0, 3, 2]
+    v = op(v, moved(std::integral_constant<int, 0x4E>{}));   // quad_perm [2, 3, 0, 1]
+    v = op(v, moved(std::integral_constant<int, 0x141>{}));  // row_half_mirror
+    v = op(v, moved(std::integral_constant<int, 0x140>{}));  // row_mirror
+}
+template <class T>
+__device__ __forceinline__ T from_lane(T v, int lane) { return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); }
+
+// over all 64 lanes, for operations whose result does not depend on the order
+template <class T, class Op>
+__device__ __forceinline__ T over_wave(T v, Op op) {
+    over_16_lanes(v, op);
+    return op(op(from_lane(v, 0), from_lane(v, 16)), op(from_lane(v, 32), from_lane(v, 48)));
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, kWave));
-    return v;
+    return over_wave(v, [](float a, float b) { return fmaxf(a, b); });
 }
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-    return v;
-}
-
 __device__ __forceinline__ int wave_sum(int v) {
+    return over_wave(v, [](int a, int b) { return a + b; });
+}
+
+// a butterfly: the order of the sums is part of the results
+__device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
     return v;
