@@ -21,16 +21,6 @@
 namespace tpq {
 namespace {
 
-// The greatest of sixteen neighbouring lanes' values, in each of them (four DPP moves; __shfl_xor is a trip through LDS each)
-__device__ __forceinline__ float max_of_16_lanes(float v) {
-    auto moved = [&](auto control) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(control)::value, 0xF, 0xF, true)); };
-    v = fmaxf(v, moved(std::integral_constant<int, 0xB1>{}));   // quad_perm [1, 0, 3, 2]
-    v = fmaxf(v, moved(std::integral_constant<int, 0x4E>{}));   // quad_perm [2, 3, 0, 1]
-    v = fmaxf(v, moved(std::integral_constant<int, 0x141>{}));  // row_half_mirror
-    return fmaxf(v, moved(std::integral_constant<int, 0x140>{}));  // row_mirror
-}
-__device__ __forceinline__ uint32_t lane_bits(float v, int lane) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); }
-
 constexpr int kFewWaves = 16, kFewRows = 16, kFewSegment = kWave * kVec, kFewSegments = 4 * kFewWaves, kFewMaxSteps = 4;
 
 struct FewRowsOut {
@@ -134,11 +124,7 @@ __global__ __launch_bounds__(kFewWaves * kWave) void few_rows_kernel(const typen
         float most = 0.0f;
 #pragma unroll
         for (int e = 0; e < kVec; ++e) most = fmaxf(most, fabsf(v[j][e]));
-        most = max_of_16_lanes(most);
-        // no value is negative or NaN, so their bits order them
-        const uint32_t a = lane_bits(most, 0), b = lane_bits(most, 16), c = lane_bits(most, 32), d = lane_bits(most, 48);
-        const uint32_t ab = a > b ? a : b, cd = c > d ? c : d;
-        most = __builtin_bit_cast(float, ab > cd ? ab : cd);
+        most = wave_max(most);
         if (lane == 0 && wave + j * kFewWaves < segs) seg_most[wave + j * kFewWaves] = most;
     }
     for (int t = threadIdx.x, spare = (pitch - 16 - K) / 16; t < M * spare; t += kFewWaves * kWave) {  // zeros behind K
@@ -150,13 +136,15 @@ __global__ __launch_bounds__(kFewWaves * kWave) void few_rows_kernel(const typen
     static_assert(SEGS <= 4, "a group of sixteen lanes per segment");
     const int my = q < SEGS ? q : 0, my_seg = wave + my * kFewWaves < segs ? wave + my * kFewWaves : segs - 1;
     const int my_row = row_of(my_seg);
-    const RowScale mine = scale_of_row(max_of_16_lanes(seg_most[my_row * segs_per_row + (i < segs_per_row ? i : 0)]), quantizer);
+    float row_most = seg_most[my_row * segs_per_row + (i < segs_per_row ? i : 0)];
+    over_16_lanes(row_most, [](float a, float b) { return fmaxf(a, b); });
+    const RowScale mine = scale_of_row(row_most, quantizer);
 #pragma unroll
     for (int j = 0; j < SEGS; ++j) {
         if (wave + j * kFewWaves < segs) {
             RowScale r;
-            r.scale = __builtin_bit_cast(float, lane_bits(mine.scale, 16 * j));
-            r.inverse = __builtin_bit_cast(float, lane_bits(mine.inverse, 16 * j));
+            r.scale = from_lane(mine.scale, 16 * j);
+            r.inverse = from_lane(mine.inverse, 16 * j);
             r.shortcut = __builtin_amdgcn_readlane(mine.shortcut, 16 * j) != 0;
             r.lean = __builtin_amdgcn_readlane(mine.lean, 16 * j) != 0;
             uint32_t lo, hi;

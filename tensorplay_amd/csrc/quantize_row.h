@@ -15,12 +15,17 @@ struct QParams {
     int no_clamp;  // no quotient |v| / scale, |v| <= absmax, can round outside [qmin, qmax]
 };
 
-__device__ __forceinline__ int quantize_one(float v, float scale, const QParams& p) {
-    if (p.sign_mode) return v >= 0.0f ? p.qmax : p.qmin;
+// (apart from the sign mode's form: asked for together with it, eight comparisons and selections of that form were made in front of
+// every branch)
+__device__ __forceinline__ int quantize_divided(float v, float scale, const QParams& p) {
     // __fdiv_rn: correctly rounded division regardless of compiler flags
     float q = rintf(__fdiv_rn(v, scale));
     q = fminf(fmaxf(q, static_cast<float>(p.qmin)), static_cast<float>(p.qmax));
     return static_cast<int>(q);
+}
+__device__ __forceinline__ int quantize_one(float v, float scale, const QParams& p) {
+    if (p.sign_mode) return v >= 0.0f ? p.qmax : p.qmin;
+    return quantize_divided(v, scale, p);
 }
 
 // Eight codes with one reciprocal instead of eight divisions, same bits as quantize_one.
@@ -57,8 +62,8 @@ __device__ __forceinline__ void quantize_eight_packed(const float (&v)[kVec], fl
             lo = hi = 0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                lo |= (static_cast<uint32_t>(quantize_one(v[i], divisor, p)) & 0xFFu) << (8 * i);
-                hi |= (static_cast<uint32_t>(quantize_one(v[i + 4], divisor, p)) & 0xFFu) << (8 * i);
+                lo |= (static_cast<uint32_t>(quantize_divided(v[i], divisor, p)) & 0xFFu) << (8 * i);
+                hi |= (static_cast<uint32_t>(quantize_divided(v[i + 4], divisor, p)) & 0xFFu) << (8 * i);
             }
         }
     }
@@ -97,8 +102,8 @@ __device__ __forceinline__ void quantize_eight_lean(const float (&v)[kVec], floa
             lo = hi = 0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                lo |= (static_cast<uint32_t>(quantize_one(v[i], divisor, p)) & 0xFFu) << (8 * i);
-                hi |= (static_cast<uint32_t>(quantize_one(v[i + 4], divisor, p)) & 0xFFu) << (8 * i);
+                lo |= (static_cast<uint32_t>(quantize_divided(v[i], divisor, p)) & 0xFFu) << (8 * i);
+                hi |= (static_cast<uint32_t>(quantize_divided(v[i + 4], divisor, p)) & 0xFFu) << (8 * i);
             }
         }
     }
@@ -175,10 +180,9 @@ __device__ __forceinline__ void load_chunk(const typename Elem<DT>::storage* p, 
     unpack_chunk<DT>(load_raw<DT, NT>(p), v);
 }
 
-// Block-wide max over THREADS threads; every thread gets the result.
+// The greatest of the wavefronts' maxima over a workgroup of THREADS threads; every thread gets the result.
 template <int THREADS>
 __device__ __forceinline__ float block_max(float v, float* smem) {
-    v = wave_max(v);
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
     if (lane == 0) smem[wave] = v;
     __syncthreads();

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(THREADS) void quantize_rows_cached(
 }
 
 // Short rows (8 <= K <= LANES * CHUNKS * 8, K % 4 == 0): LANES lanes of a wavefront per row, so a workgroup
-// takes 256 / LANES rows and no lane idles; the maximum is a butterfly inside the lane group, no LDS.
+// takes 256 / LANES rows and no lane idles; the maximum is found inside the lane group.
 template <int DT, int LANES, int CHUNKS>
 __global__ __launch_bounds__(kThreads) void quantize_rows_subwave(
     const typename Elem<DT>::storage* __restrict__ x, int8_t* __restrict__ codes,
@@ -91,8 +91,16 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_subwave(
 #pragma unroll
             for (int i = 0; i < kVec; ++i) absmax = fmaxf(absmax, fabsf(v[c][i]));
     }
+    if constexpr (LANES == kWave) {
+        absmax = wave_max(absmax);
+    } else if constexpr (LANES >= 16) {
+        over_16_lanes(absmax, [](float a, float b) { return fmaxf(a, b); });
 #pragma unroll
-    for (int off = LANES / 2; off >= 1; off >>= 1) absmax = fmaxf(absmax, __shfl_xor(absmax, off));
+        for (int off = LANES / 2; off >= 16; off >>= 1) absmax = fmaxf(absmax, __shfl_xor(absmax, off));
+    } else {
+#pragma unroll
+        for (int off = LANES / 2; off >= 1; off >>= 1) absmax = fmaxf(absmax, __shfl_xor(absmax, off));
+    }
     const RowScale r = scale_of_row(absmax, p);
     if (live && sub == 0) scales[row] = r.scale;
 
@@ -188,7 +196,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_streaming(
     int8_t* cr = codes + row * K;
     float absmax = 0.0f;
     for (int64_t k = threadIdx.x; k < K; k += kThreads) absmax = fmaxf(absmax, fabsf(Elem<DT>::load(xr[k])));
-    absmax = block_max<kThreads>(absmax, smem);
+    absmax = block_max<kThreads>(wave_max(absmax), smem);
     const float scale = __fdiv_rn(fmaxf(absmax, p.eps), p.divisor);
     if (threadIdx.x == 0) scales[row] = scale;
     for (int64_t k = threadIdx.x; k < K; k += kThreads)

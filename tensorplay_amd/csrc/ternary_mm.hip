@@ -443,10 +443,9 @@ TPQ_EXPORT int tpq_ternary_linear_row(const void* x, int x_dtype, const uint8_t*
     TPQ_REQUIRE(x && packed && out, TPQ_ERR_INVALID_VALUE, "ternary_linear_row: null pointer");
     const int rows_wg = ternary_row_rows_per_workgroup(1, N, K);
     TPQ_REQUIRE(rows_wg > 0 && aligned(x, 16) && aligned(packed, 16), TPQ_ERR_UNSUPPORTED, "ternary_linear_row: K must be a multiple of 64 up to %d, operands 16-byte aligned", kTernaryRowMaxK);
-    const QParams quantizer = row_quantizer(eps, 127.0f, -127, 127, 0);
     const EpilogueTernary<TPQ_DTYPE_F32> ep{out, nullptr, nullptr, bias, w_scale};
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (x_dtype == TPQ_DTYPE_F32) return launch_ternary_row<TPQ_DTYPE_F32>(x, packed, N, K, rows_wg, ep, s, quantizer);
-    if (x_dtype == TPQ_DTYPE_F16) return launch_ternary_row<TPQ_DTYPE_F16>(x, packed, N, K, rows_wg, ep, s, quantizer);
-    return launch_ternary_row<TPQ_DTYPE_BF16>(x, packed, N, K, rows_wg, ep, s, quantizer);
+    if (x_dtype == TPQ_DTYPE_F32) return launch_ternary_row<TPQ_DTYPE_F32>(x, packed, N, K, rows_wg, ep, s, eps);
+    if (x_dtype == TPQ_DTYPE_F16) return launch_ternary_row<TPQ_DTYPE_F16>(x, packed, N, K, rows_wg, ep, s, eps);
+    return launch_ternary_row<TPQ_DTYPE_BF16>(x, packed, N, K, rows_wg, ep, s, eps);
 }

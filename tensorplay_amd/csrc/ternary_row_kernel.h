@@ -39,7 +39,7 @@ __host__ __device__ constexpr int ternary_row_x_slots(int K) { return (K >> 4) +
 constexpr int kTernaryRowCodes = -1;
 template <class Epilogue, int XDT>
 __global__ __launch_bounds__(kTernaryRowMaxThreads) void ternary_row_kernel(const void* __restrict__ x, const uint8_t* __restrict__ packed, int N,
-                                                                           int K, int rows_wg, float inv_chunks_per_row, QParams quantizer, Epilogue ep) {
+                                                                           int K, int rows_wg, float inv_chunks_per_row, float eps, Epilogue ep) {
     // [K / 16 + K / 256]: slot 4 c + d + c / 4 holds the transposed piece d of chunk c (one slot of padding per four
     // chunks: the sixteen lanes a 16-byte read serves together, chunks c .. c + 15, then hit sixteen different groups of
     // four banks; without it chunks four apart met in the same banks and most of the kernel's LDS cycles were conflicts)
@@ -82,8 +82,10 @@ __global__ __launch_bounds__(kTernaryRowMaxThreads) void ternary_row_kernel(cons
         absmax = wave_max(absmax);
         if ((t & (kWave - 1)) == 0) most[t >> 6] = absmax;
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        absmax = most[0];
-        for (int i = 1; i < static_cast<int>(blockDim.x) / kWave; ++i) absmax = fmaxf(absmax, most[i]);
+        const int waves = static_cast<int>(blockDim.x) / kWave, mine = t & 15;  // at most 16
+        absmax = most[mine < waves ? mine : 0];
+        over_16_lanes(absmax, [](float a, float b) { return fmaxf(a, b); });
+        const QParams quantizer{eps, 127.0f, -127, 127, 0, 1};  // constants: what other parameters would need is not compiled in
         const RowScale r = scale_of_row(absmax, quantizer);
         row_scale = r.scale;
         quantize_eight(xv[0], r, quantizer, xr.x, xr.y);
@@ -154,13 +156,13 @@ inline int ternary_row_rows_per_workgroup(int64_t M, int64_t N, int64_t K, int c
 }
 
 template <int XDT = kTernaryRowCodes, class Epilogue>
-int launch_ternary_row(const void* x, const uint8_t* packed, int64_t N, int64_t K, int rows_wg, Epilogue ep, hipStream_t s, const QParams& quantizer = {}) {
+int launch_ternary_row(const void* x, const uint8_t* packed, int64_t N, int64_t K, int rows_wg, Epilogue ep, hipStream_t s, float eps = 0.0f) {
     const int64_t cpr = K / 64, threads = (rows_wg * cpr + 63) / 64 * 64;
     TPQ_REQUIRE(K % 64 == 0 && K <= kTernaryRowMaxK && rows_wg >= 4 && threads <= kTernaryRowMaxThreads && threads >= K / 16 && threads >= rows_wg,
                 TPQ_ERR_INVALID_VALUE, "ternary row kernel: workgroup shape");
     const size_t smem = 16 * static_cast<size_t>(ternary_row_x_slots(static_cast<int>(K))) + 4 * static_cast<size_t>(rows_wg);
     ternary_row_kernel<Epilogue, XDT><<<static_cast<unsigned>((N + rows_wg - 1) / rows_wg), static_cast<unsigned>(threads), smem, s>>>(
-        x, packed, static_cast<int>(N), static_cast<int>(K), rows_wg, 1.0f / static_cast<float>(cpr), quantizer, ep);
+        x, packed, static_cast<int>(N), static_cast<int>(K), rows_wg, 1.0f / static_cast<float>(cpr), eps, ep);
     return check_launch("tpq_ternary_mm (one row)");
 }
 
