@@ -272,10 +272,11 @@ int tpq_ternary_linear(const void* x, int x_dtype, const uint8_t* packed, float 
  * groups of 128 on the slab kernels; n-bit: up to 56 rows, 80 for small weights), multiplied in two parts of that type that hold it
  * to 2^-22 (bfloat16: 2^-17).  The bytes of the weight and of scales_and_zeros: up to 4 GB.  x, packed: 16-byte aligned; out: 8 bytes (float32: 16);
  * lowbit: N % 4 == 0.  workspace (16-byte aligned, contents undefined, may be NULL): with
- * tpq_packed_rows_workspace_bytes bytes the k range can be cut into slices where the channels do not fill the chip; the
- * slices are added in a fixed order.
+ * tpq_packed_rows_workspace_bytes bytes (n-bit rows: tpq_lowbit_mm_rows_workspace_bytes, whose rounds of the loop are longer) the k range
+ * can be cut into slices where the channels do not fill the chip; the slices are added in a fixed order.
  */
 int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
+int64_t tpq_lowbit_mm_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
 /* Activation rows of a workgroup's tile with that workspace, where the weight is rounded once.  Host logic only. */
 int tpq_packed_rows_tile_rows(int dtype, int64_t M, int64_t N, int64_t K);
 /*

@@ -43,7 +43,7 @@ struct Library {
     TPQ_ENTRY(tpq_ternary_mm_workspace_bytes) TPQ_ENTRY(tpq_ternary_linear_workspace_bytes) TPQ_ENTRY(tpq_ternary_linear_row) TPQ_ENTRY(tpq_ternary_linear)                \
     TPQ_ENTRY(tpq_int4_mm_ws)                                                                                             \
     TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
-    TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
+    TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
     TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine) \
     TPQ_ENTRY(tpq_f32_linear_grads_workspace_bytes) TPQ_ENTRY(tpq_f32_linear_grads) \
     TPQ_ENTRY(tpq_f32_linear_grads_takes) TPQ_ENTRY(tpq_quantize_beside_takes) \
@@ -472,7 +472,7 @@ TPQ_CALL(lowbit_mm, 7)
         Enqueue q(*x);
         out = allocate(sizes, x->scalar_type(), *x);
         if (rows) {
-            const int64_t bytes = lib.tpq_packed_rows_workspace_bytes(tag, M, N, K);
+            const int64_t bytes = lib.tpq_lowbit_mm_rows_workspace_bytes(tag, M, N, K);
             const at::Tensor part = bytes ? allocate({bytes}, at::kByte, *x) : at::Tensor();
             status = lib.tpq_lowbit_mm_rows(x->const_data_ptr(), tag, M, K, ptr<uint8_t>(packed), static_cast<int>(bits), lsb_first, N, group, ptr<float>(sz), ptr<float>(bias),
                                             out.data_ptr(), bytes ? part.data_ptr() : nullptr, bytes, q.stream);

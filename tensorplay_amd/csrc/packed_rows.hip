@@ -92,10 +92,16 @@ TPQ_EXPORT int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int
     return M >= (bits == 8 ? 17 : 33) || !at_home;
 }
 
-TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
+static int64_t rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, RowsWeights weights) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, int64_t{1} << 60);
+    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, int64_t{1} << 60, weights);
     return p.slices > 1 ? static_cast<int64_t>(p.slices) * M * N * 4 : 0;
+}
+
+TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) { return rows_workspace_bytes(dtype, M, N, K, kRowsRounded); }
+
+TPQ_EXPORT int64_t tpq_lowbit_mm_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
+    return rows_workspace_bytes(dtype, M, N, K, lowbit_rows_weights(M, N, K));
 }
 
 TPQ_EXPORT int tpq_packed_rows_tile_rows(int dtype, int64_t M, int64_t N, int64_t K) {
@@ -120,7 +126,8 @@ TPQ_EXPORT int tpq_int4_mm_rows_bias(const void* x, int dtype, int64_t M, int64_
     TPQ_REQUIRE(aligned(x, 16) && aligned(packed, 16) && aligned(scales_and_zeros, wide ? 8 : 4) && aligned(out, wide ? 16 : 8) && aligned(bias, wide ? 4 : 2), TPQ_ERR_UNSUPPORTED,
                 "int4_mm_rows: unaligned operand");
     const bool room = workspace != nullptr && aligned(workspace, 16);
-    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, room ? workspace_bytes / 4 : 0, int4_weights_unrounded(dtype, M, N, K, group));
+    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, room ? workspace_bytes / 4 : 0,
+                                              int4_weights_unrounded(dtype, M, N, K, group) ? kRowsUnrounded : kRowsRounded);
     PackedRowsArgs a{};
     a.x = x; a.w = packed; a.sz = scales_and_zeros; a.y = out; a.after = bias; a.partial = static_cast<float*>(workspace);
     a.M = static_cast<int>(M); a.N = static_cast<int>(N); a.K = static_cast<int>(K); a.tiles_per_group = static_cast<int>(group / 32);

@@ -21,12 +21,13 @@ int packed_rows_bits_bf16(const PackedRowsBits& call);
 
 namespace {
 
+// up to these rows the decode kernels ran, which apply the scales to sums of whole codes: no weight is rounded to 16 bits; above, the
+// dense route's 16-bit weight
+inline RowsWeights lowbit_rows_weights(int64_t M, int64_t N, int64_t K) { return M <= (N * K <= (int64_t{1} << 24) ? 80 : 56) ? kRowsUnroundedBits : kRowsRounded; }
+
 template <int DT>
 int run_packed_rows_bits(const PackedRowsBits& c) {
-    // up to these rows the decode kernels ran, which apply the scales to sums of whole codes: no weight is rounded to 16 bits; above, the
-    // dense route's 16-bit weight
-    const bool split = c.M <= (c.N * c.K <= (int64_t{1} << 24) ? 80 : 56);
-    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats, split);
+    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats, lowbit_rows_weights(c.M, c.N, c.K));
     PackedRowsArgs a{};
     a.x = c.x; a.w = c.packed; a.sz = c.sz; a.bias = c.bias; a.y = c.out; a.partial = static_cast<float*>(c.workspace);
     a.M = static_cast<int>(c.M); a.N = static_cast<int>(c.N); a.K = static_cast<int>(c.K); a.tiles_per_group = static_cast<int>(c.group / 32);

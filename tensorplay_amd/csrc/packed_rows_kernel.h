@@ -65,7 +65,7 @@ typedef __bf16 pr_bf8 __attribute__((ext_vector_type(8)));
 
 constexpr int pr_vmcnt(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }  // s_waitcnt immediate, vmcnt only
 
-// a workgroup's eight multiplying wavefronts: CW (2 or 4) positions of two blocks of 16 channels x 8 / CW steps of k,
+// a workgroup's eight multiplying wavefronts: CW (1, 2 or 4) positions of two blocks of 16 channels x 8 / CW steps of k,
 constexpr int kRowsNB = 2;
 // and two more that only request activations
 constexpr int kRowsProducers = 2, kRowsThreads = (8 + kRowsProducers) * kWave;
@@ -603,10 +603,15 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     __syncthreads();
     for (int t = wave; t < CW * NB * MB; t += 8) {
         float4_t s = sums[(t * KW) * kWave + lane];
+        auto add = [](const float4_t& a, const float4_t& b) { return float4_t{a[0] + b[0], a[1] + b[1], a[2] + b[2], a[3] + b[3]}; };
+        if constexpr (KW == 8) {  // by halves: eight in a row are 8 % more error in float32 than the four of two slices had
+            float4_t part[KW];
 #pragma unroll
-        for (int k = 1; k < KW; ++k) {
-            const float4_t more = sums[(t * KW + k) * kWave + lane];
-            s = float4_t{s[0] + more[0], s[1] + more[1], s[2] + more[2], s[3] + more[3]};
+            for (int k = 0; k < KW; ++k) part[k] = sums[(t * KW + k) * kWave + lane];
+            s = add(add(add(part[0], part[1]), add(part[2], part[3])), add(add(part[4], part[5]), add(part[6], part[7])));
+        } else {
+#pragma unroll
+            for (int k = 1; k < KW; ++k) s = add(s, sums[(t * KW + k) * kWave + lane]);
         }
         const int block = t / MB, r = t % MB;
         const int m = m0 + 16 * r + i, n = blockIdx.x * (16 * NB * CW) + block * 16 + 4 * q;
@@ -664,7 +669,8 @@ __global__ __launch_bounds__(256) void packed_rows_finish_kernel(const float* __
 // ---- launch ------------------------------------------------------------------------------------------
 struct PackedRowsPlan {
     int mb;        // blocks of 16 rows per workgroup: 1 .. 4, with 128 channels 3 .. 8 (float32: 1, 2)
-    int cw;        // channel positions: 2 (64 channels per workgroup) or 4 (128; 16-bit, three blocks of rows and more, K % 128 == 0)
+    int cw;        // channel positions: 2 (64 channels per workgroup), 4 (128; 16-bit, three blocks of rows and more, K % 128 == 0) or 1 (32; up to
+                   // 32 rows, float32 16)
     int slices, steps_per_slice;
     bool split;    // the weights' remainders multiplied too (64 channels per workgroup)
 };
@@ -676,14 +682,21 @@ inline int64_t ceil_div(int64_t a, int64_t b) {
 }
 
 // Tile height, channels per workgroup and slices of K by an estimate (us) fitted to a sweep of 1 .. 8 slices and both widths
-// over six shapes and 16 .. 256 rows (128 channels and 5 .. 8 blocks of rows, on the same line: 1.36 and 1.49 us a round at 7 and 8; unrounded weights 1.29, 1.43, 1.66 and 1.86 us at 1 .. 4 blocks): 4 for
-// the launch, the first loads and the epilogue, per round what the comment on the kernel says, per round of workgroups over the compute
-// units, and 2 + the bytes of the slices' sums (written and read) at 4 TB/s for the second kernel.  Within 5 % of the sweep's best nearly
-// everywhere (11008 -> 4096 at 128 rows 24.8, best 22.7).  A call plans twice (workspace, launch), so what the heights have in common, the
+// over six shapes and 16 .. 256 rows (128 channels and 5 .. 8 blocks of rows, on the same line: 1.36 and 1.49 us a round at 7 and 8; unrounded
+// weights 1.29, 1.43, 1.66 and 1.86 us at 1 .. 4 blocks, n-bit rows 1.4 times that): 4 for the launch, the first loads and the epilogue, per
+// round what the comment on the kernel says, per round of workgroups over the compute units, and for the second kernel 2.5 + the bytes of
+// the slices' sums (written and read) at 4 TB/s.  Within 5 % of the sweep's best nearly everywhere (11008 -> 4096 at 128 rows 24.8, best 22.7).
+// Few rows: 32 channels per workgroup, eight steps of k a round.  Half the rounds on twice the compute units, so a few thousand k
+// need no slices, and where the card would be as fast with them the host saves a launch and an allocation (us, slices / this, eager and then
+// in a graph: int4 in groups of 64, 28 rows 4096 x 4096 11.2 / 7.6, 8.4 / 7.6; 20 rows 2048 x 2048 10.9 / 7.0, 6.7 / 5.2; 32 rows 3072 -> 8192
+// 8.7 / 7.4, 9.0 / 7.7; float32, nine rows 1408 x 1408 11.0 / 8.0, 8.2 / 7.8; 2 bits in groups of 64, three rows 2944 -> 5832 15.4 / 9.9, 15.8 / 10.2).
+// A call plans twice (workspace, launch), so what the heights have in common, the
 // divisions above all, is worked out once: 203 rows of 4096 -> 11008 0.12 us of host time instead of 0.83.
-inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, bool split = false) {
+enum RowsWeights { kRowsRounded, kRowsUnrounded, kRowsUnroundedBits };  // (16-bit) weights rounded, int4 or n-bit weights not rounded
+
+inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, RowsWeights weights = kRowsRounded) {
     PackedRowsPlan p;
-    p.split = split && dtype != TPQ_DTYPE_F32;
+    p.split = weights != kRowsRounded && dtype != TPQ_DTYPE_F32;
     const bool wide = dtype == TPQ_DTYPE_F32;
     const int64_t blocks = (M + 15) / 16, steps = (K + 127) / 128;
     int64_t best = 1;
@@ -699,20 +712,22 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
         slices_of[cuts] = z;
         steps_of[cuts++] = per;
     }
-    for (int cw = 2; cw <= (K % 128 == 0 && !p.split && !wide ? 4 : 2); cw += 2) {
-        // 64 channels: tiles of equal height, as few as the tallest allows; 128 channels: any height that tiles of equal height can have
-        const int kw_shift = cw == 2 ? 2 : 1, most = wide ? 2 : cw == 2 ? 4 : 8;
+    for (int cw = blocks <= (wide ? 1 : 2) ? 1 : 2; cw <= (K % 128 == 0 && !p.split && !wide ? 4 : 2); cw *= 2) {
+        // 32 and 64 channels: tiles of equal height, as few as the tallest allows; 128 channels: any height that tiles of equal height can have
+        const int kw_shift = cw == 1 ? 3 : cw == 2 ? 2 : 1, most = wide ? 2 : cw <= 2 ? 4 : 8;
         const int64_t fewest = ceil_div(blocks, most);
         const int tallest = static_cast<int>(ceil_div(blocks, fewest));
-        for (int mb = tallest; mb >= (cw == 2 ? tallest : 3); --mb) {
+        for (int mb = tallest; mb >= (cw <= 2 ? tallest : 3); --mb) {
             const int64_t row_tiles = ceil_div(blocks, mb);
             if (ceil_div(blocks, row_tiles) != mb) continue;
             const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
-            const double round_us = wide ? 0.2 + 2.1 * mb : p.split ? 1.08 + 0.19 * mb : cw == 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb;
+            const double round_us = (wide ? 0.2 + 2.1 * mb : p.split ? (1.08 + 0.19 * mb) * (weights == kRowsUnroundedBits ? 1.4 : 1.0) : cw <= 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb) +
+                                    (cw == 1 ? 0.2 * mb : 0.0);
             for (int c = 0; c < cuts; ++c) {
+                if (cw == 1 && c > 0) break;  // no slices is what they are for
                 const int64_t z = slices_of[c], rounds = (steps_of[c] + (1 << kw_shift) - 1) >> kw_shift;
                 const double waves = static_cast<double>((tiles * z + 255) >> 8);  // 256 compute units
-                const double us = waves * (4.0 + round_us * static_cast<double>(rounds)) + (z == 1 ? 0.0 : 2.0 + static_cast<double>(z * M * N) * 8.0 / 4e6);
+                const double us = waves * ((cw == 1 ? 3.4 : 4.0) + round_us * static_cast<double>(rounds)) + (z == 1 ? 0.0 : 2.5 + static_cast<double>(z * M * N) * 8.0 / 4e6);
                 if (us < best_us) { best_us = us; best = z; p.cw = cw; p.mb = mb; }
             }
         }
@@ -741,7 +756,7 @@ int launch_packed_rows_shape(const PackedRowsArgs& a, int slices, hipStream_t s)
 
 template <int DT, class Source, int MB, int CW>
 int launch_packed_rows_as(const PackedRowsArgs& a, const PackedRowsPlan& p, hipStream_t s) {
-    if constexpr (CW == 2) {
+    if constexpr (CW <= 2) {
         if constexpr (DT != TPQ_DTYPE_F32) {
             if (p.split) return a.K % 128 != 0 ? launch_packed_rows_shape<DT, Source, MB, CW, true, true>(a, p.slices, s)
                                                : launch_packed_rows_shape<DT, Source, MB, CW, false, true>(a, p.slices, s);
@@ -758,9 +773,11 @@ int launch_packed_rows(PackedRowsArgs a, const PackedRowsPlan& p, hipStream_t s)
     if (p.slices == 1) a.partial = nullptr;
     int rc;
     const bool wide = p.cw == 4;
-    if (p.mb == 1) rc = launch_packed_rows_as<DT, Source, 1, 2>(a, p, s);
-    else if (p.mb == 2) rc = launch_packed_rows_as<DT, Source, 2, 2>(a, p, s);
-    else {
+    if (p.mb == 1) rc = p.cw == 1 ? launch_packed_rows_as<DT, Source, 1, 1>(a, p, s) : launch_packed_rows_as<DT, Source, 1, 2>(a, p, s);
+    else if (p.mb == 2) {
+        if constexpr (DT == TPQ_DTYPE_F32) rc = launch_packed_rows_as<DT, Source, 2, 2>(a, p, s);
+        else rc = p.cw == 1 ? launch_packed_rows_as<DT, Source, 2, 1>(a, p, s) : launch_packed_rows_as<DT, Source, 2, 2>(a, p, s);
+    } else {
         if constexpr (DT == TPQ_DTYPE_F32) rc = fail(TPQ_ERR_RUNTIME, "packed rows: no such tile");
         else if (p.mb == 8) rc = launch_packed_rows_shape<DT, Source, 8, 4, false, false>(a, p.slices, s);
         else if (p.mb == 7) rc = launch_packed_rows_shape<DT, Source, 7, 4, false, false>(a, p.slices, s);

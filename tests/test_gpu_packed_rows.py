@@ -224,3 +224,40 @@ def test_float16_weights_of_any_size_are_not_rounded(kind, M, N, K, group, bits,
     assert bool((exact.abs() > 2.0 ** -14).float().mean() > 0.9)  # the result's own rounding is a normal one
     moved = (got.cpu() != exact.to(torch.float16)).float().mean().item()
     assert moved < 0.05, moved
+
+
+# (rows, N, K, group): few rows on 32 channels a workgroup and eight steps of k a round: one, two and four rounds, the last one and the last
+# step partial, channels that leave a tile partly empty, one tile and more than the compute units
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,group", [(1, 8, 1024, 32), (16, 40, 1152, 64), (5, 1160, 1376, 32), (32, 72, 2048, 64), (17, 8200, 928, 32), (29, 2056, 4096, 64)])
+def test_few_rows_without_slices(dtype, M, N, K, group):
+    from tensorplay_amd import _lib, ops
+
+    if dtype == torch.float32 and M > 16:
+        pytest.skip("two blocks of float32 rows do not fit a round of eight steps")
+    lib, tag = _lib.load(), ops._DT[dtype]
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(dtype)
+    codes = torch.randint(0, 16, (N, K), dtype=torch.int32, device=DEV, generator=gen)
+    sz = torch.stack([torch.rand(K // group, N, device=DEV, generator=gen) * 0.01 + 1e-3, torch.randn(K // group, N, device=DEV, generator=gen) * 0.01], -1).to(dtype).contiguous()
+    packed = ops._convert_weight_to_int4pack(codes, 2)
+    w = (codes - 8).double() * sz[..., 0].double().t().repeat_interleave(group, 1) + sz[..., 1].double().t().repeat_interleave(group, 1)
+    out = torch.empty(M, N, dtype=dtype, device=DEV)
+    ops._check(lib.tpq_int4_mm_rows(x.data_ptr(), tag, M, K, packed.data_ptr(), N, group, sz.data_ptr(), out.data_ptr(), None, 0, ops._stream(x)))
+    _check(out, x, w, None, 0.011, dtype)
+    sz = torch.stack([torch.rand(K // group, N, device=DEV, generator=gen) * 0.01 + 1e-3, torch.randint(0, 4, (K // group, N), device=DEV, generator=gen).float()], -1).contiguous()
+    codes = torch.randint(0, 4, (N, K), dtype=torch.int32, device=DEV, generator=gen)
+    packed = ((codes.view(N, K // 4, 4) << torch.tensor([6, 4, 2, 0], device=DEV, dtype=torch.int32)).sum(-1)).to(torch.uint8).contiguous()
+    w = (codes.double() - sz[..., 1].double().t().repeat_interleave(group, 1)) * sz[..., 0].double().t().repeat_interleave(group, 1)
+    ops._check(lib.tpq_lowbit_mm_rows(x.data_ptr(), tag, M, K, packed.data_ptr(), 2, 0, N, group, sz.data_ptr(), None, out.data_ptr(), None, 0, ops._stream(x)))
+    _check(out, x, w, None, 0.011, dtype)
+
+
+def test_few_rows_take_no_workspace():
+    """The plan's side of it: no slices where a few thousand k go to 32 channels a workgroup, slices beyond."""
+    from tensorplay_amd import _lib, ops
+
+    lib, f16 = _lib.load(), ops._DT[torch.float16]
+    assert lib.tpq_packed_rows_workspace_bytes(f16, 28, 4096, 4096) == 0 and lib.tpq_packed_rows_workspace_bytes(f16, 20, 2048, 2048) == 0
+    assert lib.tpq_packed_rows_workspace_bytes(f16, 33, 2048, 2048) > 0 and lib.tpq_packed_rows_workspace_bytes(f16, 28, 4096, 11008) > 0
+    assert lib.tpq_lowbit_mm_rows_workspace_bytes(f16, 3, 5832, 2944) == 0
