@@ -47,8 +47,9 @@ using namespace tpq;
 // Lower limit, measured (us, this kernel / decode kernels): groups of 128 (weights unrounded): 24 rows of 4096 -> 16384 17.5 / 15.4,
 // 33 of 4096 x 4096 10.8 / 15.1, 48 of 4096 -> 11008 18.5 / 20.2; groups of 64, 17 rows:
 // 11008 -> 4096 12.0 / 23.1, 16 rows 11.3 / 12.0.  K % 128 != 0 (slabs of four rows): 4768 -> 13544 at 3 / 33 rows 19.4 /
-// 92, 31 / 868.  float32: 4096 -> 11008 at 1, 2, 64 rows 24.4 / 24.2, 24.7 / 45, 68 / 110; 2048 x 2048 at 1 and 2 rows
-// 8.1 / 7.2, 8.2 / 7.4.  bfloat16 stops at 256 rows although this kernel is the faster one beyond (384 rows of 8192 x 8192 52 / 104, 512 of
+// 92, 31 / 868.  float32, all rows (up to eight in blocks of four): one row of 2048 x 2048
+// 5.7 / 7.2, 4096 x 4096 9.2 / 14.3, 8192 x 8192 15.5 / 29.5, 4768 -> 1264 6.8 / 15.2, 1024 x 1024 4.4 / 4.7 (in a graph); 4096 -> 11008 at 2
+// and 64 rows 15 / 45, 68 / 110.  bfloat16 stops at 256 rows although this kernel is the faster one beyond (384 rows of 8192 x 8192 52 / 104, 512 of
 // 4096 x 4096 24 / 42): from 257 rows on the results are those of the dense route, the reference's device formulation with a weight
 // rounded to bfloat16 twice, and are held to it within 1e-2, element by element, by tests.  A weight rounded once lies closer to
 // the exact product and misses that on single elements; below 257 rows, where the tiled kernel and the slabs ran, the comparison
@@ -59,7 +60,7 @@ TPQ_EXPORT int tpq_int4_mm_rows_takes(const void* x, int dtype, int64_t M, int64
     if (M <= 0 || N <= 0 || K <= 0 || K % 32 || N % 8 || N * K >= (int64_t{1} << 33) || K >= (1 << 24) || M > rows_limit(N, K, dtype)) return 0;
     if (!aligned(x, 16) || !aligned(packed, 16) || !aligned(scales_and_zeros, dtype == TPQ_DTYPE_F32 ? 8 : 4)) return 0;
     if (dtype == TPQ_DTYPE_BF16 && M > 256) return 0;
-    if (dtype == TPQ_DTYPE_F32) return M >= 2 || (N * K >= (1 << 24) && K > 4096);
+    if (dtype == TPQ_DTYPE_F32) return 1;
     if (K % 128) return 1;
     return M >= (group < 128 ? 17 : 33);
 }
@@ -68,7 +69,7 @@ TPQ_EXPORT int tpq_int4_mm_rows_takes(const void* x, int dtype, int64_t M, int64
 // home: 4096 x 4096 at 19 rows, 1 / 2 / 4 / 8 bits 10.7 / 10.0, 10.8 / 10.5, 11.4 / 11.9, 13.1 / 16.9; 4096 -> 11008, 2 bits, 24 / 32 /
 // 40 rows 21.7 / 20.6, 21.6 / 21.5, 20 / 31; 1024 -> 512 at 18 rows 7.3 / 6.0.  Other groups, 4096 x 4096 in groups of 32, 2 bits:
 // 1 / 16 / 80 rows 10.1 / 25, 10.4 / 46, 17.6 / 175; one row of 4 bits stays with the row kernel (8.6 / 6.1).  float32
-// 4096 -> 11008: 1 / 8 / 64 rows 33 / 35, 33 / 57, 84 / 99.  8 bits are twice the bytes: 4096 -> 11008 at 300 rows 75 / 86, at
+// 4096 -> 11008: 8 / 64 rows 26 / 57, 84 / 99.  8 bits are twice the bytes: 4096 -> 11008 at 300 rows 75 / 86, at
 // 384 81 / 85, at 512 90 / 84; 4096 x 4096 at 512 31 / 42.
 TPQ_EXPORT int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int64_t N, int64_t K, int bits, int lsb_first, int64_t group,
                                         const uint8_t* packed, const float* scales_and_zeros) {
@@ -105,7 +106,9 @@ TPQ_EXPORT int64_t tpq_lowbit_mm_rows_workspace_bytes(int dtype, int64_t M, int6
 }
 
 TPQ_EXPORT int tpq_packed_rows_tile_rows(int dtype, int64_t M, int64_t N, int64_t K) {
-    return M <= 0 || N <= 0 || K <= 0 ? 0 : 16 * packed_rows_plan(dtype, M, N, K, int64_t{1} << 60).mb;
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, int64_t{1} << 60);
+    return p.quads ? 4 * p.quads : 16 * p.mb;
 }
 
 TPQ_EXPORT int tpq_int4_mm_rows(const void* x, int dtype, int64_t M, int64_t K, const int32_t* packed, int64_t N, int64_t group,
@@ -128,6 +131,9 @@ TPQ_EXPORT int tpq_int4_mm_rows_bias(const void* x, int dtype, int64_t M, int64_
     const bool room = workspace != nullptr && aligned(workspace, 16);
     const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, room ? workspace_bytes / 4 : 0,
                                               int4_weights_unrounded(dtype, M, N, K, group) ? kRowsUnrounded : kRowsRounded);
+    if (p.quads)
+        return packed_rows_quads({x, packed, scales_and_zeros, nullptr, bias, out, workspace, M, N, K, group, 0, 0, 0, static_cast<hipStream_t>(stream)}, p.quads, p.cw >> 1,
+                                 p.slices, p.steps_per_slice);
     PackedRowsArgs a{};
     a.x = x; a.w = packed; a.sz = scales_and_zeros; a.y = out; a.after = bias; a.partial = static_cast<float*>(workspace);
     a.M = static_cast<int>(M); a.N = static_cast<int>(N); a.K = static_cast<int>(K); a.tiles_per_group = static_cast<int>(group / 32);
@@ -152,7 +158,7 @@ TPQ_EXPORT int tpq_lowbit_mm_rows(const void* x, int dtype, int64_t M, int64_t K
     TPQ_REQUIRE(aligned(x, 16) && aligned(packed, 16) && aligned(scales_and_zeros, 8) && aligned(out, dtype == TPQ_DTYPE_F32 ? 16 : 8), TPQ_ERR_UNSUPPORTED,
                 "lowbit_mm_rows: unaligned operand");
     const bool room = workspace != nullptr && aligned(workspace, 16);
-    const PackedRowsBits call{x, packed, scales_and_zeros, bias, out, workspace, M, N, K, group, room ? workspace_bytes / 4 : 0, bits, lsb_first,
+    const PackedRowsBits call{x, packed, scales_and_zeros, bias, nullptr, out, workspace, M, N, K, group, room ? workspace_bytes / 4 : 0, bits, lsb_first,
                               static_cast<hipStream_t>(stream)};
     if (dtype == TPQ_DTYPE_F32) return packed_rows_bits_f32(call);
     return dtype == TPQ_DTYPE_F16 ? packed_rows_bits_f16(call) : packed_rows_bits_bf16(call);

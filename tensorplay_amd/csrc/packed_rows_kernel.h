@@ -43,8 +43,8 @@
 //   * the KW partial sums of a tile meet in LDS at the end.
 // Measured (us, weights from HBM, this kernel / what ran before): int4, bfloat16, 11008 -> 4096 in groups of 64: 24 / 48 / 128 / 256
 // rows 12.4 / 22.8, 14.8 / 39, 24 / 43, 36 / 71; 4096 x 4096 in groups of 128: 33 rows (SPLIT) 10.8 / 12.5, 64 / 256 rows 11.2 / 20, 15.8 / 34;
-// 4768 -> 13544 in groups of 32 (K % 128 != 0): 3 / 33 rows (SPLIT) 19.4 / 92, 31 / 868.  float32 4096 x 4096: 3 / 19 / 64 rows 12.4 / 22, 18 / 38,
-// 29 / 47 (bound by its MFMAs, 32 clocks for 16 x 16 x 4).  2 bits: 4096 -> 11008 at 203 rows 32 /
+// 4768 -> 13544 in groups of 32 (K % 128 != 0): 3 / 33 rows (SPLIT) 19.4 / 92, 31 / 868.  float32 4096 x 4096: 19 / 64 rows 16.5 / 38,
+// 28 / 47 (bound by its MFMAs, 32 clocks for 16 x 16 x 4; up to eight rows: packed_rows_quads.hip).  2 bits: 4096 -> 11008 at 203 rows 32 /
 // 67, (SPLIT) at 40 rows 20 / 31; 4096 x 4096 in groups of 32 (SPLIT): 1 / 16 / 80 rows 10.1 / 25, 10.4 / 46, 17.6 / 175.
 // Rows >= M repeat row M - 1, steps of k behind the end of the slice are loaded (from the last step) and not multiplied, the
 // chunks of a last partial step behind K are cleared in LDS.
@@ -85,6 +85,17 @@ struct PackedRowsArgs {
     int M, N, K, tiles_per_group, steps_per_slice;
     float inv_tiles_per_group;
 };
+
+// code - zero, rounded once (one instruction instead of a conversion and a subtraction)
+template <int HALF>
+__device__ __forceinline__ float less_zero(half2_t codes, float zero) {
+    float out;
+    if constexpr (HALF == 0)
+        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(out) : "v"(codes), "v"(zero));
+    else
+        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(out) : "v"(codes), "v"(zero));
+    return out;
+}
 
 // ---- the two weight sources ------------------------------------------------------------------------------
 // codes(): the lane's 32 codes as 16 pairs under fp16 exponents, pair p = codes 2 p, 2 p + 1 in k order
@@ -422,8 +433,8 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
                 lo = __builtin_fmaf(static_cast<float>(h.x), scale, zero);
                 hi = __builtin_fmaf(static_cast<float>(h.y), scale, zero);
             } else {  // zero points are whole numbers as a rule: one rounding
-                lo = (static_cast<float>(h.x) - zero) * scale;
-                hi = (static_cast<float>(h.y) - zero) * scale;
+                lo = less_zero<0>(h, zero) * scale;
+                hi = less_zero<1>(h, zero) * scale;
             }
         } else {  // the offset folded into the constant: an error of 2^-24 x 1032 scale at most, below the operand type's rounding
             const float z_lo = Source::kTypedParams ? zero - Source::offset(p, 0) * scale : -(zero + Source::offset(p, 0)) * scale;
@@ -671,7 +682,8 @@ struct PackedRowsPlan {
     int mb;        // blocks of 16 rows per workgroup: 1 .. 4, with 128 channels 3 .. 8 (float32: 1, 2)
     int cw;        // channel positions: 2 (64 channels per workgroup), 4 (128; 16-bit, three blocks of rows and more, K % 128 == 0) or 1 (32; up to
                    // 32 rows, float32 16)
-    int slices, steps_per_slice;
+    int slices, steps_per_slice;  // (steps of 128 k)
+    int quads;     // float32: blocks of four rows per workgroup (of 32 cw channels), 0: the blocks of 16 above
     bool split;    // the weights' remainders multiplied too (64 channels per workgroup)
 };
 
@@ -694,8 +706,43 @@ inline int64_t ceil_div(int64_t a, int64_t b) {
 // divisions above all, is worked out once: 203 rows of 4096 -> 11008 0.12 us of host time instead of 0.83.
 enum RowsWeights { kRowsRounded, kRowsUnrounded, kRowsUnroundedBits };  // (16-bit) weights rounded, int4 or n-bit weights not rounded
 
+// float32, up to eight rows: blocks of four.  The estimate (us): 2 for the launch, then for every workgroup that a compute unit gets 1 and its rounds of the
+// loop, 1.6 with one block of rows, 2.6 with two (int4 1.5 and 2.4, 8 bits 2.4 and 3.1); slices 3.5 and their bytes: on the device less, but the host pays
+// the second launch and an allocation.  Against the blocks of 16 (us, those / these, eager): four rows, 2 bits 4864 -> 9728 34.8 / 20.8; int4
+// 1408 -> 1152 7.7 / 7.6 (in a graph 7.8 / 5.2), 4096 x 4096 11.8 / 9.3; two rows of 4096 -> 11008 28.2 / 15; one row, 2 bits, 5248 -> 3104 15.9 / 11.4; eight rows,
+// 4 bits, 4096 -> 11008 30.5 / 26.4, 2048 x 2048 10.9 / 9.5, int4 4096 x 4096 12.1 / 11.3; six rows, 8 bits, 4864 -> 10880 37.9 / 33.5.  From three
+// blocks on the two kinds cost the same (12 rows of 11008 -> 4096 24.4 / 24.4, 16 rows of 4096 x 4096 12.3 / 14.1): a product of sixteen 4 x 4
+// blocks takes half the clocks of 16 x 16 x 4.
+constexpr int64_t kQuadRows = 8;
+
+inline PackedRowsPlan packed_quads_plan(int64_t M, int64_t N, int64_t K, int64_t room_floats) {
+    PackedRowsPlan p{};
+    p.quads = static_cast<int>((M + 3) / 4);
+    const int64_t steps = (K + 127) / 128;
+    double best_us = 1e30;
+    for (int64_t z = 1; z <= 16 && z <= steps; ++z) {
+        if (z > 1 && z * M * N > room_floats) break;
+        const int64_t per = ceil_div(steps, z);
+        if (ceil_div(steps, per) != z) continue;
+        for (int shift = 0; shift < 2; ++shift) {
+            const int64_t workgroups = ((N + (32 << shift) - 1) >> (5 + shift)) * z, rounds = (per + (8 >> shift) - 1) >> (3 - shift);
+            const double us = 2.0 + static_cast<double>((workgroups + 255) >> 8) * (1.0 + (p.quads == 1 ? 1.6 : 2.6) * static_cast<double>(rounds)) +
+                              (z == 1 ? 0.0 : 3.5 + static_cast<double>(z * M * N) * 8.0 / 4e6);
+            if (us < best_us) {
+                best_us = us;
+                p.cw = 1 << shift;
+                p.slices = static_cast<int>(z);
+                p.steps_per_slice = static_cast<int>(per);
+            }
+        }
+    }
+    return p;
+}
+
 inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, RowsWeights weights = kRowsRounded) {
+    if (dtype == TPQ_DTYPE_F32 && M <= kQuadRows) return packed_quads_plan(M, N, K, room_floats);
     PackedRowsPlan p;
+    p.quads = 0;
     p.split = weights != kRowsRounded && dtype != TPQ_DTYPE_F32;
     const bool wide = dtype == TPQ_DTYPE_F32;
     const int64_t blocks = (M + 15) / 16, steps = (K + 127) / 128;

@@ -261,3 +261,60 @@ def test_few_rows_take_no_workspace():
     assert lib.tpq_packed_rows_workspace_bytes(f16, 28, 4096, 4096) == 0 and lib.tpq_packed_rows_workspace_bytes(f16, 20, 2048, 2048) == 0
     assert lib.tpq_packed_rows_workspace_bytes(f16, 33, 2048, 2048) > 0 and lib.tpq_packed_rows_workspace_bytes(f16, 28, 4096, 11008) > 0
     assert lib.tpq_lowbit_mm_rows_workspace_bytes(f16, 3, 5832, 2944) == 0
+
+
+# (M, N, K, group): float32 in blocks of four rows: one and two blocks, full and not; steps of 128 k of which the last one has one to three tiles, fewer
+# steps than wavefronts, more than they have in flight; a part of 32 and of 64 channels; slices of k
+QUADS = [(1, 4, 32, 32), (3, 40, 96, 96), (4, 32, 160, 32), (5, 68, 1088, 64), (8, 200, 4096, 128), (4, 1160, 8224, 32), (7, 9736, 4864, 128), (2, 8200, 3072, 64)]
+
+
+@pytest.mark.parametrize("bits,lsb_first", [(0, False), (1, False), (1, True), (2, False), (4, False), (8, False)])  # 0: the int4 layout
+@pytest.mark.parametrize("M,N,K,group", QUADS)
+def test_blocks_of_four_rows(M, N, K, group, bits, lsb_first):
+    """Against float64, element by element, and beside the blocks of 16 rows: the same rows among nine, whose bound is the same."""
+    from tensorplay_amd import _lib, ops
+
+    lib, tag = _lib.load(), ops._DT[torch.float32]
+    N, group = (N + 7) // 8 * 8 if bits == 0 else N, group if bits or group in (32, 64, 128) else 32
+    assert lib.tpq_packed_rows_tile_rows(tag, M, N, K) == 4 * -(-M // 4) and lib.tpq_packed_rows_tile_rows(tag, 9, N, K) == 16
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K + bits)
+    x = torch.randn(9, K, device=DEV, generator=gen)
+    bias = torch.randn(N, device=DEV, generator=gen)
+    codes = torch.randint(0, 1 << (bits or 4), (N, K), dtype=torch.int32, device=DEV, generator=gen)
+    scale, zero = torch.rand(K // group, N, device=DEV, generator=gen) * 0.01 + 1e-3, torch.randn(K // group, N, device=DEV, generator=gen)
+    sz = torch.stack([scale, zero * (1.0 if bits else 0.01)], -1).contiguous()
+    s64, z64 = (sz[..., i].double().t().repeat_interleave(group, 1) for i in (0, 1))
+    if bits == 0:
+        packed = ops._convert_weight_to_int4pack(codes, 2)
+        w = (codes - 8).double() * s64 + z64
+    else:
+        codes = codes - 128 if bits == 8 else codes
+        per = 8 // bits
+        order = [i * bits if lsb_first else 8 - (i + 1) * bits for i in range(per)]
+        packed = ((codes & 255).view(N, K // per, per) << torch.tensor(order, device=DEV, dtype=torch.int32)).sum(-1).to(torch.uint8).contiguous()
+        w = (codes.double() - z64) * s64
+    results = {}
+    for m in (M, 9):
+        sizes = {int((lib.tpq_lowbit_mm_rows_workspace_bytes if bits else lib.tpq_packed_rows_workspace_bytes)(tag, m, N, K)), 0}
+        for need in sizes:  # with its slices, and without a workspace
+            out = torch.full((m, N), float("nan"), device=DEV)
+            ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
+            at = [x.data_ptr(), tag, m, K, packed.data_ptr()], [bias.data_ptr(), out.data_ptr(), ws.data_ptr() if need else None, need, ops._stream(x)]
+            if bits:
+                ops._check(lib.tpq_lowbit_mm_rows(*at[0], bits, int(lsb_first), N, group, sz.data_ptr(), *at[1]))
+            else:
+                ops._check(lib.tpq_int4_mm_rows_bias(*at[0], N, group, sz.data_ptr(), *at[1]))
+            _check(out, x[:m], w, bias, 0.011, torch.float32)
+            results[m] = out[:M]
+    size = x[:M].double().abs() @ w.abs().t() + bias.double().abs()
+    assert bool(((results[M] - results[9]).double().abs() <= 2 * (K + 17) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("kind,bits", [("int4", 4), ("lowbit", 1), ("lowbit", 8)])
+def test_blocks_of_four_rows_not_finite(kind, bits):
+    """Infinite activations and zero points, in the last tile of a K that ends inside a step of 128."""
+    def change(x, sz):
+        x[0, 5], x[1, -1], x[2, 3], x[2, 40] = float("inf"), float("-inf"), float("inf"), float("nan")
+        sz[-1, 7, 1] = float("inf")
+
+    _assert_same_classes(*_fragment(kind, 6, 72, 544, 32, bits, torch.float32, change))
