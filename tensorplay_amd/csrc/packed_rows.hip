@@ -132,7 +132,7 @@ TPQ_EXPORT int tpq_int4_mm_rows_bias(const void* x, int dtype, int64_t M, int64_
     const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, room ? workspace_bytes / 4 : 0,
                                               int4_weights_unrounded(dtype, M, N, K, group) ? kRowsUnrounded : kRowsRounded);
     if (p.quads)
-        return packed_rows_quads({x, packed, scales_and_zeros, nullptr, bias, out, workspace, M, N, K, group, 0, 0, 0, static_cast<hipStream_t>(stream)}, p.quads, p.cw >> 1,
+        return packed_rows_f32({x, packed, scales_and_zeros, nullptr, bias, out, workspace, M, N, K, group, 0, 0, 0, static_cast<hipStream_t>(stream)}, p.quads, p.cw,
                                  p.slices, p.steps_per_slice);
     PackedRowsArgs a{};
     a.x = x; a.w = packed; a.sz = scales_and_zeros; a.y = out; a.after = bias; a.partial = static_cast<float*>(workspace);

@@ -19,7 +19,7 @@ struct PackedRowsBits {
 int packed_rows_bits_f32(const PackedRowsBits& call);
 int packed_rows_bits_f16(const PackedRowsBits& call);
 int packed_rows_bits_bf16(const PackedRowsBits& call);
-int packed_rows_quads(const PackedRowsBits& call, int quads, int cw_shift, int slices, int steps_per_slice);  // float32, blocks of four rows
+int packed_rows_f32(const PackedRowsBits& call, int quads, int cw, int slices, int steps_per_slice);  // float32, the kernels without LDS for the activations
 
 namespace {
 
@@ -31,7 +31,7 @@ template <int DT>
 int run_packed_rows_bits(const PackedRowsBits& c) {
     const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats, lowbit_rows_weights(c.M, c.N, c.K));
     if constexpr (DT == TPQ_DTYPE_F32)
-        if (p.quads) return packed_rows_quads(c, p.quads, p.cw >> 1, p.slices, p.steps_per_slice);
+        if (p.quads) return packed_rows_f32(c, p.quads, p.cw, p.slices, p.steps_per_slice);
     PackedRowsArgs a{};
     a.x = c.x; a.w = c.packed; a.sz = c.sz; a.bias = c.bias; a.y = c.out; a.partial = static_cast<float*>(c.workspace);
     a.M = static_cast<int>(c.M); a.N = static_cast<int>(c.N); a.K = static_cast<int>(c.K); a.tiles_per_group = static_cast<int>(c.group / 32);

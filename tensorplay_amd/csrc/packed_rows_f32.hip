@@ -1,4 +1,4 @@
-// Packed weights against up to eight rows of float32 activations, in blocks of FOUR (int4 layout and n-bit rows, as packed_rows_kernel.h, whose
+// Packed weights against float32 activations without LDS for those.  First, up to eight rows in blocks of FOUR (int4 layout and n-bit rows, as packed_rows_kernel.h, whose
 // blocks of 16 rows multiply padding where the rows do not fill them: one row costs what sixteen do).
 //
 // What bounds it: about evenly the float32 matrix instructions (some 16 clocks each) and the dequantization (2.3 to 4 vector instructions a
@@ -194,14 +194,182 @@ __global__ __launch_bounds__(8 * kWave) void packed_quads_kernel(const PackedRow
     }
 }
 
+// ---- more rows: a lane per channel ----------------------------------------------------------------------------
+// From nine rows on, where that is the faster way (packed_lanes_plan).  What bounds it: the matrix instructions, 32 clocks for 16 rows x 64 channels x one k
+// (v_mfma_f32_16x16x1, four blocks of 16 channels), and the dequantization behind them.  What the kernel with its activations in LDS spends beside those, barriers between
+// its rounds and wavefronts that only fetch, is not here: a wavefront takes tiles of 32 k for itself, MB blocks of 16 rows and, QB, one of four rows (v_mfma_f32_4x4x1 with
+// the channels of a lane side by side), so that 19 rows cost 20 and not 32.
+//   * lane n is channel n: its 32 codes of a tile, dequantized, are the second operand as they are, its (scale, zero) one load.  n-bit rows are read a line per lane: with so
+//     many rows to multiply that is still the smaller part;
+//   * activations, first operand, reach all four blocks from one (cbsz 2): lane (row, b) loads eight k of its row, 8 b .. + 7, register v, block abid hold k = 8 abid + v;
+//     of the block of four (cbsz 4), lane (row, b) holds k = 2 b, + 1;
+//   * sums as above; the eight wavefronts' meet in LDS, 16 rows at a time.
+// Measured (us, before / with this, in a graph): int4 19 rows 4096 x 4096 17.4 / 13.4, 35 rows 26.5 / 19.2, 17 rows 11008 -> 4096 35.5 / 25.6; 8 bits, 36 rows 4096 x 4096 30 / 24.8.
+typedef float float16_t __attribute__((ext_vector_type(16)));
+constexpr int kLanesPitch = kWave + 4;  // of a row of sums in LDS: the four rows that a wavefront stores at once lie 16 banks apart
+
+template <class Source, int MB, int QB>
+__global__ __launch_bounds__(8 * kWave) void packed_lanes_kernel(const PackedRowsArgs a) {
+    using P = RowsParams<TPQ_DTYPE_F32, Source::kTypedParams>;
+    constexpr int kDepth = MB == 1 ? 4 : MB == 2 ? 3 : 2, kChains = MB == 1 ? 2 : 1;
+    __shared__ float sums[8][16][kLanesPitch];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = blockIdx.x * kWave + lane, m0 = blockIdx.y * (16 * MB + 4 * QB);
+    const int tiles = a.K / 32, begin = blockIdx.z * a.steps_per_slice;  // (steps_per_slice: tiles)
+    const int end = tiles < begin + a.steps_per_slice ? tiles : begin + a.steps_per_slice;
+    const int count = end - begin > wave ? (end - begin - wave + 7) / 8 : 0;  // tiles of this wavefront
+
+    const uint32_t w_off = Source::lane_offset(a, n, 0);
+    const uint32_t p_off = static_cast<uint32_t>(n < a.N ? n : a.N - 1) * 8u, group_bytes = static_cast<uint32_t>(a.N) * 8u;
+    const char* x_row[MB];
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+        const int row = m0 + 16 * b + (lane & 15);
+        x_row[b] = static_cast<const char*>(a.x) + (static_cast<size_t>(row < a.M ? row : a.M - 1) * a.K + 8 * (lane >> 4)) * 4;  // rows past M: the last one again, dropped
+    }
+    const int quad_row = m0 + 16 * MB + (lane & 3);
+    const char* const x_quad = static_cast<const char*>(a.x) + (static_cast<size_t>(quad_row < a.M ? quad_row : a.M - 1) * a.K + 2 * (lane >> 2)) * 4;
+    struct Tile {
+        typename Source::Words w;
+        typename P::raw_t p;
+        pr_word4 x[MB][2];
+        pr_word2 x_quad;
+    };
+    auto load = [&](int j, Tile& d) __attribute__((always_inline)) {
+        const int tile = begin + wave + 8 * (j < count ? j : count - 1);  // past the last: that one again
+        const uint32_t group = static_cast<uint32_t>((static_cast<float>(tile) + 0.5f) * a.inv_tiles_per_group);  // exact: tile < 2^20
+        auto from = (TPQ_GLOBAL char*)a.w + static_cast<size_t>(tile) * (Source::kStepBytes / 4);
+        auto params = (TPQ_GLOBAL char*)a.sz;
+        asm volatile("" : "+s"(from), "+s"(params));  // the loads stay here (see pinned_global)
+        const pr_word2 t = *(TPQ_GLOBAL pr_word2*)(params + (group * group_bytes + p_off));
+        d.p.x = t.x; d.p.y = t.y;
+        Source::load(from, w_off, d.w);
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) d.x[b][h] = *((TPQ_GLOBAL pr_word4*)pinned_global(x_row[b] + static_cast<size_t>(tile) * 128) + h);
+        if constexpr (QB) d.x_quad = *(TPQ_GLOBAL pr_word2*)pinned_global(x_quad + static_cast<size_t>(tile) * 128);
+    };
+
+    float16_t acc[MB] = {};
+    float4_t acc_quad = {};
+    uint32_t magic[2] = {Source::kMagic0, Source::kMagic1};
+    asm volatile("" : "+v"(magic[0]), "+v"(magic[1]));
+    auto multiply = [&](const Tile& d) __attribute__((always_inline)) {
+        const float scale = P::scale(d.p), zero = P::zero(d.p);
+        float16_t piece[kChains][MB];
+        float4_t piece_quad[kChains];
+        pr_static_for<0, 16>([&](auto pair_c) __attribute__((always_inline)) {
+            constexpr int kPair = decltype(pair_c)::value;
+            constexpr int kAt = kChains == 2 ? (kPair >> 1) + 8 * (kPair & 1) : kPair, kChain = kChains == 2 ? kPair & 1 : 0;
+            constexpr bool kFirst = kChains == 2 ? kPair < 2 : (kPair & 7) == 0, kLast = kChains == 2 ? kPair >= 14 : (kPair & 7) == 7;
+            const half2_t h = __builtin_bit_cast(half2_t, Source::pair(d.w, kAt, magic)) -
+                              half2_t{static_cast<_Float16>(Source::offset(kAt, 0)), static_cast<_Float16>(Source::offset(kAt, 1))};
+            float w[2];
+            if constexpr (Source::kTypedParams) {
+                w[0] = __builtin_fmaf(static_cast<float>(h.x), scale, zero);
+                w[1] = __builtin_fmaf(static_cast<float>(h.y), scale, zero);
+            } else {
+                w[0] = less_zero<0>(h, zero) * scale;
+                w[1] = less_zero<1>(h, zero) * scale;
+            }
+            pr_static_for<0, 2>([&](auto v_c) __attribute__((always_inline)) {
+                constexpr int kV = decltype(v_c)::value, kIn = (2 * kAt + kV) & 7, kBlock = (2 * kAt) >> 3;
+#pragma unroll
+                for (int b = 0; b < MB; ++b) {
+                    const uint32_t bits = d.x[b][kIn >> 2][kIn & 3];
+                    piece[kChain][b] = __builtin_amdgcn_mfma_f32_16x16x1f32(__builtin_bit_cast(float, bits), w[kV], kFirst && kV == 0 ? float16_t{} : piece[kChain][b], 2, kBlock, 0);
+                }
+                if constexpr (QB) {
+                    const uint32_t bits = kV ? d.x_quad.y : d.x_quad.x;
+                    piece_quad[kChain] = __builtin_amdgcn_mfma_f32_4x4x1f32(__builtin_bit_cast(float, bits), w[kV], kFirst && kV == 0 ? float4_t{} : piece_quad[kChain], 4, kAt, 0);
+                }
+            });
+            if constexpr (kLast) {
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[b][e] += piece[kChain][b][e];
+                if constexpr (QB) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc_quad[e] += piece_quad[kChain][e];
+                }
+            }
+        });
+    };
+
+    if (count > 0) {
+        Tile ring[kDepth];
+        pr_static_for<0, kDepth>([&](auto d) __attribute__((always_inline)) { load(decltype(d)::value, ring[decltype(d)::value]); });
+        int j = 0;
+        for (; j + kDepth < count; j += kDepth)
+            pr_static_for<0, kDepth>([&](auto d) __attribute__((always_inline)) {
+                multiply(ring[decltype(d)::value]);
+                load(j + kDepth + decltype(d)::value, ring[decltype(d)::value]);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        pr_static_for<0, kDepth>([&](auto d) __attribute__((always_inline)) {
+            if (j + decltype(d)::value < count) multiply(ring[decltype(d)::value]);
+        });
+    }
+
+    auto store = [&](int row, int m) __attribute__((always_inline)) {
+        if (m >= a.M || n >= a.N) return;
+        float part[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) part[k] = sums[k][row][lane];
+        float s = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+        const size_t at = static_cast<size_t>(m) * a.N + n;
+        if (a.partial != nullptr) {
+            a.partial[static_cast<size_t>(blockIdx.z) * a.M * a.N + at] = s;
+            return;
+        }
+        if (a.bias != nullptr) s += a.bias[n];
+        if (a.after != nullptr) s += static_cast<const float*>(a.after)[n];
+        static_cast<float*>(a.y)[at] = s;
+    };
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+        if (b > 0) __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sums[wave][4 * (lane >> 4) + e][16 * c + (lane & 15)] = acc[b][4 * c + e];
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) store(wave + 8 * h, m0 + 16 * b + wave + 8 * h);
+    }
+    if constexpr (QB) {
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sums[wave][e][lane] = acc_quad[e];
+        __syncthreads();
+        if (wave < 4) store(wave, m0 + 16 * MB + wave);
+    }
+}
+
 template <class Source>
-int launch_packed_quads(PackedRowsArgs a, int quads, int cw_shift, int slices, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>((a.N + (32 << cw_shift) - 1) / (32 << cw_shift)), static_cast<unsigned>((a.M + 4 * quads - 1) / (4 * quads)), static_cast<unsigned>(slices));
-    if (quads == 1)
-        packed_quads_kernel<Source, 1><<<grid, 8 * kWave, 0, s>>>(a, cw_shift);
-    else
-        packed_quads_kernel<Source, 2><<<grid, 8 * kWave, 0, s>>>(a, cw_shift);
-    if (int rc = check_launch("packed rows (blocks of four)")) return rc;
+int launch_packed_f32(PackedRowsArgs a, int quads, int cw, int slices, hipStream_t s) {
+    const int channels = cw == 0 ? kWave : 32 * cw;
+    const dim3 grid(static_cast<unsigned>((a.N + channels - 1) / channels), static_cast<unsigned>((a.M + 4 * quads - 1) / (4 * quads)), static_cast<unsigned>(slices));
+    if (cw > 0) {
+        if (quads == 1)
+            packed_quads_kernel<Source, 1><<<grid, 8 * kWave, 0, s>>>(a, cw >> 1);
+        else
+            packed_quads_kernel<Source, 2><<<grid, 8 * kWave, 0, s>>>(a, cw >> 1);
+    } else {
+        switch (quads) {
+            case 4: packed_lanes_kernel<Source, 1, 0><<<grid, 8 * kWave, 0, s>>>(a); break;
+            case 5: packed_lanes_kernel<Source, 1, 1><<<grid, 8 * kWave, 0, s>>>(a); break;
+            case 8: packed_lanes_kernel<Source, 2, 0><<<grid, 8 * kWave, 0, s>>>(a); break;
+            case 9: packed_lanes_kernel<Source, 2, 1><<<grid, 8 * kWave, 0, s>>>(a); break;
+            case 12: packed_lanes_kernel<Source, 3, 0><<<grid, 8 * kWave, 0, s>>>(a); break;
+            case 13: packed_lanes_kernel<Source, 3, 1><<<grid, 8 * kWave, 0, s>>>(a); break;
+            default: packed_lanes_kernel<Source, 4, 0><<<grid, 8 * kWave, 0, s>>>(a); break;
+        }
+    }
+    if (int rc = check_launch("packed rows (float32)")) return rc;
     if (a.partial == nullptr) return TPQ_OK;
     const int64_t quarters = static_cast<int64_t>(a.M) * a.N / 4;
     packed_rows_finish_kernel<TPQ_DTYPE_F32><<<static_cast<unsigned>((quarters + 255) / 256), 256, 0, s>>>(
@@ -211,7 +379,7 @@ int launch_packed_quads(PackedRowsArgs a, int quads, int cw_shift, int slices, h
 
 }  // namespace
 
-int packed_rows_quads(const PackedRowsBits& c, int quads, int cw_shift, int slices, int steps_per_slice) {
+int packed_rows_f32(const PackedRowsBits& c, int quads, int cw, int slices, int steps_per_slice) {
     PackedRowsArgs a{};
     a.x = c.x; a.w = c.packed; a.sz = c.sz; a.bias = c.bias; a.after = c.after; a.y = c.out; a.partial = slices > 1 ? static_cast<float*>(c.workspace) : nullptr;
     a.M = static_cast<int>(c.M); a.N = static_cast<int>(c.N); a.K = static_cast<int>(c.K);
@@ -219,11 +387,11 @@ int packed_rows_quads(const PackedRowsBits& c, int quads, int cw_shift, int slic
     a.inv_tiles_per_group = 1.0f / static_cast<float>(a.tiles_per_group);
     a.steps_per_slice = steps_per_slice;
     switch (c.bits) {
-        case 0: return launch_packed_quads<SourceInt4>(a, quads, cw_shift, slices, c.stream);
-        case 1: return c.lsb_first ? launch_packed_quads<SourceBits<1, true>>(a, quads, cw_shift, slices, c.stream) : launch_packed_quads<SourceBits<1, false>>(a, quads, cw_shift, slices, c.stream);
-        case 2: return launch_packed_quads<SourceBits<2, false>>(a, quads, cw_shift, slices, c.stream);
-        case 4: return launch_packed_quads<SourceBits<4, false>>(a, quads, cw_shift, slices, c.stream);
-        default: return launch_packed_quads<SourceBits<8, false>>(a, quads, cw_shift, slices, c.stream);
+        case 0: return launch_packed_f32<SourceInt4>(a, quads, cw, slices, c.stream);
+        case 1: return c.lsb_first ? launch_packed_f32<SourceBits<1, true>>(a, quads, cw, slices, c.stream) : launch_packed_f32<SourceBits<1, false>>(a, quads, cw, slices, c.stream);
+        case 2: return launch_packed_f32<SourceBits<2, false>>(a, quads, cw, slices, c.stream);
+        case 4: return launch_packed_f32<SourceBits<4, false>>(a, quads, cw, slices, c.stream);
+        default: return launch_packed_f32<SourceBits<8, false>>(a, quads, cw, slices, c.stream);
     }
 }
 

@@ -43,8 +43,8 @@
 //   * the KW partial sums of a tile meet in LDS at the end.
 // Measured (us, weights from HBM, this kernel / what ran before): int4, bfloat16, 11008 -> 4096 in groups of 64: 24 / 48 / 128 / 256
 // rows 12.4 / 22.8, 14.8 / 39, 24 / 43, 36 / 71; 4096 x 4096 in groups of 128: 33 rows (SPLIT) 10.8 / 12.5, 64 / 256 rows 11.2 / 20, 15.8 / 34;
-// 4768 -> 13544 in groups of 32 (K % 128 != 0): 3 / 33 rows (SPLIT) 19.4 / 92, 31 / 868.  float32 4096 x 4096: 19 / 64 rows 16.5 / 38,
-// 28 / 47 (bound by its MFMAs, 32 clocks for 16 x 16 x 4; up to eight rows: packed_rows_quads.hip).  2 bits: 4096 -> 11008 at 203 rows 32 /
+// 4768 -> 13544 in groups of 32 (K % 128 != 0): 3 / 33 rows (SPLIT) 19.4 / 92, 31 / 868.  float32 4096 x 4096: 64 rows 26.7 /
+// 47 (bound by its MFMAs, 32 clocks for 16 x 16 x 4; most shapes of fewer rows: packed_rows_f32.hip).  2 bits: 4096 -> 11008 at 203 rows 32 /
 // 67, (SPLIT) at 40 rows 20 / 31; 4096 x 4096 in groups of 32 (SPLIT): 1 / 16 / 80 rows 10.1 / 25, 10.4 / 46, 17.6 / 175.
 // Rows >= M repeat row M - 1, steps of k behind the end of the slice are loaded (from the last step) and not multiplied, the
 // chunks of a last partial step behind K are cleared in LDS.
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(kRowsThreads) void packed_rows_kernel(const PackedR
     }
 }
 
-// y = round(sum over the slices, in slice order (+ bias)); a thread takes four consecutive elements (N % 4 == 0)
+// y = round(sum over the slices, in a fixed order (+ bias)); a thread takes four consecutive elements (N % 4 == 0)
 template <int DT>
 __global__ __launch_bounds__(256) void packed_rows_finish_kernel(const float* __restrict__ partial, int slices, int64_t quads, const float* __restrict__ bias,
                                                                  const typename Elem<DT>::storage* __restrict__ after, int quads_per_row,
@@ -665,9 +665,17 @@ __global__ __launch_bounds__(256) void packed_rows_finish_kernel(const float* __
         float4_t more[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) more[j] = reinterpret_cast<const float4_t*>(partial)[static_cast<int64_t>(z0 + j < slices ? z0 + j : slices - 1) * quads + e];
+        if constexpr (DT == TPQ_DTYPE_F32) {  // four by halves: in one chain, eleven slices' roundings show (40 rows of 11008 -> 1024 1.23e-7 of the result for 1.19e-7)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (z0 + j < slices) sum = float4_t{sum[0] + more[j][0], sum[1] + more[j][1], sum[2] + more[j][2], sum[3] + more[j][3]};
+            for (int v = 0; v < 4; ++v) {
+                const float m1 = z0 + 1 < slices ? more[1][v] : 0.0f, m2 = z0 + 2 < slices ? more[2][v] : 0.0f, m3 = z0 + 3 < slices ? more[3][v] : 0.0f;
+                sum[v] += (more[0][v] + m1) + (m2 + m3);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (z0 + j < slices) sum = float4_t{sum[0] + more[j][0], sum[1] + more[j][1], sum[2] + more[j][2], sum[3] + more[j][3]};
+        }
     }
     const int n = bias != nullptr || after != nullptr ? static_cast<int>(static_cast<uint32_t>(e) % static_cast<uint32_t>(quads_per_row)) * 4 : 0;
     if (bias != nullptr) {
@@ -683,7 +691,8 @@ struct PackedRowsPlan {
     int cw;        // channel positions: 2 (64 channels per workgroup), 4 (128; 16-bit, three blocks of rows and more, K % 128 == 0) or 1 (32; up to
                    // 32 rows, float32 16)
     int slices, steps_per_slice;  // (steps of 128 k)
-    int quads;     // float32: blocks of four rows per workgroup (of 32 cw channels), 0: the blocks of 16 above
+    int quads;     // float32, kernels without LDS for the activations: a quarter of the rows per workgroup (of 32 cw channels; cw 0: a lane per channel,
+                   // steps_per_slice in tiles of 32 k); 0: the kernel above
     bool split;    // the weights' remainders multiplied too (64 channels per workgroup)
 };
 
@@ -712,8 +721,14 @@ enum RowsWeights { kRowsRounded, kRowsUnrounded, kRowsUnroundedBits };  // (16-b
 // 1408 -> 1152 7.7 / 7.6 (in a graph 7.8 / 5.2), 4096 x 4096 11.8 / 9.3; two rows of 4096 -> 11008 28.2 / 15; one row, 2 bits, 5248 -> 3104 15.9 / 11.4; eight rows,
 // 4 bits, 4096 -> 11008 30.5 / 26.4, 2048 x 2048 10.9 / 9.5, int4 4096 x 4096 12.1 / 11.3; six rows, 8 bits, 4864 -> 10880 37.9 / 33.5.  From three
 // blocks on the two kinds cost the same (12 rows of 11008 -> 4096 24.4 / 24.4, 16 rows of 4096 x 4096 12.3 / 14.1): a product of sixteen 4 x 4
-// blocks takes half the clocks of 16 x 16 x 4.
+// blocks takes half the clocks of one of 16 x 16.
 constexpr int64_t kQuadRows = 8;
+
+// With the second kernel for z slices; a call of two launches and an allocation keeps the host for 10.8 us.
+inline double sliced_us(double us, int64_t z, int64_t M, int64_t N) {
+    us += 2.5 + static_cast<double>(z * M * N) * 8.0 / 4e6;
+    return us < 10.8 ? 10.8 : us;
+}
 
 inline PackedRowsPlan packed_quads_plan(int64_t M, int64_t N, int64_t K, int64_t room_floats) {
     PackedRowsPlan p{};
@@ -737,6 +752,33 @@ inline PackedRowsPlan packed_quads_plan(int64_t M, int64_t N, int64_t K, int64_t
         }
     }
     return p;
+}
+
+// float32, a lane per channel: 16 to 64 rows a workgroup, and where one to four rows are left over by blocks of 16, those as a block of four.  The estimate (us): 3 and
+// half a microsecond for each block of rows (launch, first loads, sums in LDS), per round of eight tiles of k 0.35 + 1.01 a block + 0.33 for the block of four, for every
+// workgroup that a compute unit gets (one block: two are there at once; more: a microsecond a block between them), and the slices' second kernel as above.  Against the kernel with its activations in LDS (us, that one / this): int4 19 rows 4096 x 4096
+// 17.8 / 13.6, 35 rows 26.2 / 19.3, 48 rows 26.4 / 22.1, 80 rows 42.9 / 35.4, 17 rows 11008 -> 4096 35.2 / 25.8, 14 rows 4096 -> 11008 26.7 / 22.2; 36 rows with 8 bits 29.8 / 24.7;
+// but 64 rows 2048 -> 8192 23.9 / 27.6, 50 rows 2048 x 2048 with 1 bit 12.4 / 13.6, 32 rows 4096 x 4096 17.3 / 17.5.
+inline bool packed_lanes_plan(int64_t M, int64_t N, int64_t K, int64_t room_floats, double& best_us, PackedRowsPlan& p) {
+    const int64_t blocks = (M + 15) / 16, row_tiles = ceil_div(blocks, 4), tiles = K / 32, columns = (N + 63) / 64;
+    const bool four = row_tiles == 1 && M > 16 && M % 16 >= 1 && M % 16 <= 4;
+    const int64_t sixteens = four ? blocks - 1 : ceil_div(blocks, row_tiles);
+    const double fixed_us = 3.0 + 0.5 * static_cast<double>(sixteens), round_us = 0.35 + 1.01 * static_cast<double>(sixteens) + (four ? 0.33 : 0.0);
+    bool taken = false;
+    for (int64_t z = 1; z <= 16 && z <= tiles; ++z) {
+        if (z > 1 && z * M * N > room_floats) break;
+        const int64_t per = ceil_div(tiles, z);
+        if (ceil_div(tiles, per) != z) continue;
+        const int64_t turns = (columns * row_tiles * z + 255) >> 8;
+        double us = fixed_us + round_us * static_cast<double>(turns * ((per + 7) >> 3)) + static_cast<double>((turns - 1) * (sixteens - 1));
+        if (z > 1) us = sliced_us(us, z, M, N);
+        if (us < best_us) {
+            best_us = us;
+            p = PackedRowsPlan{0, 0, static_cast<int>(z), static_cast<int>(per), static_cast<int>(4 * sixteens + (four ? 1 : 0)), false};
+            taken = true;
+        }
+    }
+    return taken;
 }
 
 inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, RowsWeights weights = kRowsRounded) {
@@ -768,16 +810,21 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
             const int64_t row_tiles = ceil_div(blocks, mb);
             if (ceil_div(blocks, row_tiles) != mb) continue;
             const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
-            const double round_us = (wide ? 0.2 + 2.1 * mb : p.split ? (1.08 + 0.19 * mb) * (weights == kRowsUnroundedBits ? 1.4 : 1.0) : cw <= 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb) +
+            const double round_us = (wide ? 0.3 + 2.3 * mb : p.split ? (1.08 + 0.19 * mb) * (weights == kRowsUnroundedBits ? 1.4 : 1.0) : cw <= 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb) +
                                     (cw == 1 ? 0.2 * mb : 0.0);
             for (int c = 0; c < cuts; ++c) {
                 if (cw == 1 && c > 0) break;  // no slices is what they are for
                 const int64_t z = slices_of[c], rounds = (steps_of[c] + (1 << kw_shift) - 1) >> kw_shift;
                 const double waves = static_cast<double>((tiles * z + 255) >> 8);  // 256 compute units
-                const double us = waves * ((cw == 1 ? 3.4 : 4.0) + round_us * static_cast<double>(rounds)) + (z == 1 ? 0.0 : 2.5 + static_cast<double>(z * M * N) * 8.0 / 4e6);
+                double us = waves * ((cw == 1 ? 3.4 : 4.0) + round_us * static_cast<double>(rounds));
+                if (z > 1) us = wide ? sliced_us(us, z, M, N) : us + 2.5 + static_cast<double>(z * M * N) * 8.0 / 4e6;
                 if (us < best_us) { best_us = us; best = z; p.cw = cw; p.mb = mb; }
             }
         }
+    }
+    if (wide) {
+        PackedRowsPlan lanes;
+        if (packed_lanes_plan(M, N, K, room_floats, best_us, lanes)) return lanes;
     }
     if (const char* e = tuning_env("TPQ_ROWS_SLICES")) best = std::atoi(e);
     if (const char* e = tuning_env("TPQ_ROWS_CW")) p.cw = std::atoi(e);

@@ -268,17 +268,13 @@ def test_few_rows_take_no_workspace():
 QUADS = [(1, 4, 32, 32), (3, 40, 96, 96), (4, 32, 160, 32), (5, 68, 1088, 64), (8, 200, 4096, 128), (4, 1160, 8224, 32), (7, 9736, 4864, 128), (2, 8200, 3072, 64)]
 
 
-@pytest.mark.parametrize("bits,lsb_first", [(0, False), (1, False), (1, True), (2, False), (4, False), (8, False)])  # 0: the int4 layout
-@pytest.mark.parametrize("M,N,K,group", QUADS)
-def test_blocks_of_four_rows(M, N, K, group, bits, lsb_first):
-    """Against float64, element by element, and beside the blocks of 16 rows: the same rows among nine, whose bound is the same."""
+def _float32_products(counts, N, K, group, bits, lsb_first):
+    """The first rows of one x, as many as each count says, with a bias, with the plan's slices and without a workspace, every element within its bound of float64: ({count: result}, |x| |w|)."""
     from tensorplay_amd import _lib, ops
 
-    lib, tag = _lib.load(), ops._DT[torch.float32]
-    N, group = (N + 7) // 8 * 8 if bits == 0 else N, group if bits or group in (32, 64, 128) else 32
-    assert lib.tpq_packed_rows_tile_rows(tag, M, N, K) == 4 * -(-M // 4) and lib.tpq_packed_rows_tile_rows(tag, 9, N, K) == 16
-    gen = torch.Generator(device=DEV).manual_seed(M + N + K + bits)
-    x = torch.randn(9, K, device=DEV, generator=gen)
+    lib, tag, most = _lib.load(), ops._DT[torch.float32], max(counts)
+    gen = torch.Generator(device=DEV).manual_seed(most + N + K + bits)
+    x = torch.randn(most, K, device=DEV, generator=gen)
     bias = torch.randn(N, device=DEV, generator=gen)
     codes = torch.randint(0, 1 << (bits or 4), (N, K), dtype=torch.int32, device=DEV, generator=gen)
     scale, zero = torch.rand(K // group, N, device=DEV, generator=gen) * 0.01 + 1e-3, torch.randn(K // group, N, device=DEV, generator=gen)
@@ -294,9 +290,9 @@ def test_blocks_of_four_rows(M, N, K, group, bits, lsb_first):
         packed = ((codes & 255).view(N, K // per, per) << torch.tensor(order, device=DEV, dtype=torch.int32)).sum(-1).to(torch.uint8).contiguous()
         w = (codes.double() - z64) * s64
     results = {}
-    for m in (M, 9):
+    for m in counts:
         sizes = {int((lib.tpq_lowbit_mm_rows_workspace_bytes if bits else lib.tpq_packed_rows_workspace_bytes)(tag, m, N, K)), 0}
-        for need in sizes:  # with its slices, and without a workspace
+        for need in sizes:
             out = torch.full((m, N), float("nan"), device=DEV)
             ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
             at = [x.data_ptr(), tag, m, K, packed.data_ptr()], [bias.data_ptr(), out.data_ptr(), ws.data_ptr() if need else None, need, ops._stream(x)]
@@ -305,16 +301,50 @@ def test_blocks_of_four_rows(M, N, K, group, bits, lsb_first):
             else:
                 ops._check(lib.tpq_int4_mm_rows_bias(*at[0], N, group, sz.data_ptr(), *at[1]))
             _check(out, x[:m], w, bias, 0.011, torch.float32)
-            results[m] = out[:M]
-    size = x[:M].double().abs() @ w.abs().t() + bias.double().abs()
-    assert bool(((results[M] - results[9]).double().abs() <= 2 * (K + 17) * 2.0 ** -24 * size).all())
+            results[m] = out
+    return results, x.double().abs() @ w.abs().t() + bias.double().abs()
+
+
+WIDTHS = [(0, False), (1, False), (1, True), (2, False), (4, False), (8, False)]  # (bits, lsb_first), 0: the int4 layout
+
+
+@pytest.mark.parametrize("bits,lsb_first", WIDTHS)
+@pytest.mark.parametrize("M,N,K,group", QUADS)
+def test_blocks_of_four_rows(M, N, K, group, bits, lsb_first):
+    """Against float64, element by element, and beside the blocks of 16 rows: the same rows among nine, whose bound is the same."""
+    from tensorplay_amd import _lib, ops
+
+    lib, tag = _lib.load(), ops._DT[torch.float32]
+    N, group = (N + 7) // 8 * 8 if bits == 0 else N, group if bits or group in (32, 64, 128) else 32
+    assert lib.tpq_packed_rows_tile_rows(tag, M, N, K) == 4 * -(-M // 4) and lib.tpq_packed_rows_tile_rows(tag, 9, N, K) == 16
+    results, size = _float32_products((M, 9), N, K, group, bits, lsb_first)
+    assert bool(((results[M] - results[9][:M]).double().abs() <= 2 * (K + 17) * 2.0 ** -24 * size[:M]).all())
+
+
+# (M, N, K, group, rows of a tile): float32 with a lane per channel: one to four blocks of 16 rows, with a block of four behind one to three of them, full and
+# not, two and three tiles of rows; fewer tiles of k than wavefronts, more than they have in flight; channels that leave a part partly empty
+LANES = [(17, 8200, 96, 32, 20), (20, 8200, 1088, 32, 20), (17, 68, 11008, 128, 20), (35, 1032, 4128, 32, 36), (52, 1032, 2080, 32, 52), (14, 11008, 4096, 128, 16),
+         (40, 4096, 4096, 128, 48), (60, 4096, 4096, 64, 64), (96, 2056, 2080, 32, 48), (130, 1032, 4096, 64, 48)]
+
+
+@pytest.mark.parametrize("bits,lsb_first", WIDTHS)
+@pytest.mark.parametrize("M,N,K,group,rows", LANES)
+def test_lane_per_channel(M, N, K, group, rows, bits, lsb_first):
+    """Against float64, element by element, and beside the blocks of four: the first eight rows by themselves."""
+    from tensorplay_amd import _lib, ops
+
+    N = (N + 7) // 8 * 8 if bits == 0 else N
+    assert _lib.load().tpq_packed_rows_tile_rows(ops._DT[torch.float32], M, N, K) == rows
+    results, size = _float32_products((M, 8), N, K, group, bits, lsb_first)
+    assert bool(((results[M][:8] - results[8]).double().abs() <= 2 * (K + 17) * 2.0 ** -24 * size[:8]).all())
 
 
 @pytest.mark.parametrize("kind,bits", [("int4", 4), ("lowbit", 1), ("lowbit", 8)])
-def test_blocks_of_four_rows_not_finite(kind, bits):
+@pytest.mark.parametrize("M", [6, 19])  # blocks of four; a lane per channel
+def test_float32_rows_not_finite(M, kind, bits):
     """Infinite activations and zero points, in the last tile of a K that ends inside a step of 128."""
     def change(x, sz):
         x[0, 5], x[1, -1], x[2, 3], x[2, 40] = float("inf"), float("-inf"), float("inf"), float("nan")
         sz[-1, 7, 1] = float("inf")
 
-    _assert_same_classes(*_fragment(kind, 6, 72, 544, 32, bits, torch.float32, change))
+    _assert_same_classes(*_fragment(kind, M, 72, 544, 32, bits, torch.float32, change))
