@@ -190,14 +190,15 @@ __device__ __forceinline__ void load_eight(const typename Elem<DT>::storage* p, 
 // ---- reductions over lanes -----------------------------------------------------
 
 // v := op over the sixteen neighbouring lanes that share a quarter of the wavefront, in each of them: four moves between lanes, where
-// __shfl_xor is a trip through LDS each.  All lanes of the wavefront take part.
+// __shfl_xor is a trip through LDS each.  Lanes 8, 4, 2, 1 apart meet in this order, as in a butterfly (once lanes eight apart are alike, a
+// turn by four is an exchange of those four apart, and so on), so float sums have a butterfly's bits.  All lanes of the wavefront take part.
 template <class T, class Op>
 __device__ __forceinline__ void over_16_lanes(T& v, Op op) {
     auto moved = [&](auto control) { return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(control)::value, 0xF, 0xF, true)); };
-    v = op(v, moved(std::integral_constant<int, 0xB1>{}));   // quad_perm [1, 0, 3, 2]
-    v = op(v, moved(std::integral_constant<int, 0x4E>{}));   // quad_perm [2, 3, 0, 1]
-    v = op(v, moved(std::integral_constant<int, 0x141>{}));  // row_half_mirror
-    v = op(v, moved(std::integral_constant<int, 0x140>{}));  // row_mirror
+    v = op(v, moved(std::integral_constant<int, 0x128>{}));  // row_ror:8
+    v = op(v, moved(std::integral_constant<int, 0x124>{}));  // row_ror:4
+    v = op(v, moved(std::integral_constant<int, 0x122>{}));  // row_ror:2
+    v = op(v, moved(std::integral_constant<int, 0x121>{}));  // row_ror:1
 }
 template <class T>
 __device__ __forceinline__ T from_lane(T v, int lane) { return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); }

@@ -588,6 +588,32 @@ def test_mm_multi_with_rms_norm_row_magnitudes(ops, tdt, tol, K, widths):
             assert_close_norm(y[r:r + 1], want[r:r + 1], 2 * tol, "row of magnitude %g" % scales[r])
 
 
+def test_rms_norm_in_the_products_adds_a_rows_squares_by_halves(ops):
+    """The order of a row's float32 sum of squares is part of the results: of a step's sixteen lanes (eight k each) those eight apart meet
+    first.  The rows come in pairs: beside one large square, whose last place is 2, both hold two ones.  In the first row they lie in lanes 1
+    and 9, which make 2 in that order, while each by itself is rounded away beside the large one; in the second they lie in one lane and count
+    in any order.  All weights but those of k = 0, where a pair is alike, are zero, so a pair's outputs are the same bits where its factors
+    are (with the last place of the factor one output in 12 000 or so changes: some fifty a pair).
+    """
+    K, n, pairs = 2048, 16384, 8
+    rng = np.random.default_rng(5)
+    x = np.zeros((2 * pairs, K), dtype=np.float16)
+    x[:, 0] = np.repeat(4096 + 4 * rng.permutation(400)[:pairs], 2)  # squares between 2^24 and 2^25, multiples of 16
+    x[:, 8] = 1
+    x[0::2, 8 * 9], x[1::2, 9] = -1, -1
+    g = torch.ones(K, dtype=torch.float16, device=DEV)
+    packed, szs = [], []
+    for _ in range(4):
+        codes = np.full((n, K), 8, dtype=np.int32)
+        codes[:, 0] = rng.integers(0, 16, n)
+        packed.append(ops._convert_weight_to_int4pack(torch.from_numpy(codes).to(DEV), 2))
+        sz = np.zeros((K // 128, n, 2), dtype=np.float16)
+        sz[:, :, 0] = rng.uniform(0.01, 0.04, n)
+        szs.append(torch.from_numpy(sz).to(DEV))
+    for y in ops.int4pack_mm_multi(torch.from_numpy(x).to(DEV), packed, 128, szs, norm_weight=g, eps=0.0):
+        assert torch.equal(y[0::2], y[1::2])
+
+
 @pytest.mark.parametrize("tdt,tol", [(torch.float16, 2e-3), (torch.bfloat16, 1.6e-2)])
 @pytest.mark.parametrize("M,N,K", [(8, 11008, 4096), (2, 72, 4096), (5, 136, 2048), (12, 200, 4096), (3, 64, 512)])
 def test_mm_swiglu_with_rms_norm_against_oracle(ops, tdt, tol, M, N, K):
