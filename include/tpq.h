@@ -272,8 +272,19 @@ int tpq_ternary_linear(const void* x, int x_dtype, const uint8_t* packed, float 
  * groups of 128 on the slab kernels; n-bit: up to 56 rows, 80 for small weights), multiplied in two parts of that type that hold it
  * to 2^-22 (bfloat16: 2^-17).  The bytes of the weight and of scales_and_zeros: up to 4 GB.  x, packed: 16-byte aligned; out: 8 bytes (float32: 16);
  * lowbit: N % 4 == 0.  workspace (16-byte aligned, contents undefined, may be NULL): with
- * tpq_packed_rows_workspace_bytes bytes (n-bit rows: tpq_lowbit_mm_rows_workspace_bytes, whose rounds of the loop are longer) the k range
- * can be cut into slices where the channels do not fill the chip; the slices are added in a fixed order.
+ * tpq_packed_rows_call_workspace_bytes bytes (bits 0: the int4 layout) the k range can be cut into slices where the channels do not fill
+ * the chip; the slices are added in a fixed order.  A smaller one makes fewer slices.
+ */
+int64_t tpq_packed_rows_call_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group);
+/*
+ * What such a call runs with workspace_bytes (below 0: with any it asks for): plan[4] = kernel, activation rows of a workgroup's tile, its
+ * channels, slices of k.  Kernels: activations staged in LDS; float32 in blocks of four rows, or with a lane per channel.  Host logic only.
+ */
+enum { TPQ_ROWS_STAGED = 0, TPQ_ROWS_QUADS = 1, TPQ_ROWS_LANES = 2 };
+int tpq_packed_rows_call_plan(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group, int64_t workspace_bytes, int32_t* plan);
+/*
+ * Workspaces without the group or the width: of int4 calls whose weight is rounded once, and of n-bit calls.  A call whose own plan wants
+ * more slices than that makes fewer.
  */
 int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
 int64_t tpq_lowbit_mm_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);

@@ -38,6 +38,8 @@ SIGNATURES = {
     "tpq_int4_mm_rows_workspace_bytes": [_i64, _i64, _i64],
     "tpq_packed_rows_workspace_bytes": [_int, _i64, _i64, _i64],
     "tpq_lowbit_mm_rows_workspace_bytes": [_int, _i64, _i64, _i64],
+    "tpq_packed_rows_call_workspace_bytes": [_int, _i64, _i64, _i64, _int, _i64],
+    "tpq_packed_rows_call_plan": [_int, _i64, _i64, _i64, _int, _i64, _i64, _ptr],
     "tpq_packed_rows_tile_rows": [_int, _i64, _i64, _i64],
     "tpq_int4_mm_rows_takes": [_ptr, _int, _i64, _i64, _i64, _i64, _ptr, _ptr],
     "tpq_lowbit_mm_rows_takes": [_ptr, _int, _i64, _i64, _i64, _int, _int, _i64, _ptr, _ptr],

@@ -42,8 +42,8 @@ struct Library {
     TPQ_ENTRY(tpq_quantize_rowwise) TPQ_ENTRY(tpq_int8_mm_workspace_bytes) TPQ_ENTRY(tpq_int8_mm_dequant_ws)                \
     TPQ_ENTRY(tpq_ternary_mm_workspace_bytes) TPQ_ENTRY(tpq_ternary_linear_workspace_bytes) TPQ_ENTRY(tpq_ternary_linear_row) TPQ_ENTRY(tpq_ternary_linear)                \
     TPQ_ENTRY(tpq_int4_mm_ws)                                                                                             \
-    TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
-    TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
+    TPQ_ENTRY(tpq_int4_mm_rows_workspace_bytes) TPQ_ENTRY(tpq_packed_rows_call_workspace_bytes) TPQ_ENTRY(tpq_int4_mm_rows_bias) \
+    TPQ_ENTRY(tpq_int4_mm_rows_takes) TPQ_ENTRY(tpq_lowbit_mm_rows) TPQ_ENTRY(tpq_lowbit_mm_rows_takes)                     \
     TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine) \
     TPQ_ENTRY(tpq_f32_linear_grads_workspace_bytes) TPQ_ENTRY(tpq_f32_linear_grads) \
     TPQ_ENTRY(tpq_f32_linear_grads_takes) TPQ_ENTRY(tpq_quantize_beside_takes) \
@@ -412,7 +412,7 @@ TPQ_CALL(int4_mm, 6)
     at::Tensor workspace;
     int64_t workspace_bytes = 0;
     if (rows) {
-        workspace_bytes = lib.tpq_packed_rows_workspace_bytes(tag, M, N, K);
+        workspace_bytes = lib.tpq_packed_rows_call_workspace_bytes(tag, M, N, K, 0, group);
     } else {
         const int64_t stream = static_cast<int64_t>(reinterpret_cast<intptr_t>(c10::hip::getCurrentHIPStream(x->device().index()).stream()));
         PyObject* key = Py_BuildValue("(iL)", static_cast<int>(x->device().index()), static_cast<long long>(stream));
@@ -472,7 +472,7 @@ TPQ_CALL(lowbit_mm, 7)
         Enqueue q(*x);
         out = allocate(sizes, x->scalar_type(), *x);
         if (rows) {
-            const int64_t bytes = lib.tpq_lowbit_mm_rows_workspace_bytes(tag, M, N, K);
+            const int64_t bytes = lib.tpq_packed_rows_call_workspace_bytes(tag, M, N, K, static_cast<int>(bits), group);
             const at::Tensor part = bytes ? allocate({bytes}, at::kByte, *x) : at::Tensor();
             status = lib.tpq_lowbit_mm_rows(x->const_data_ptr(), tag, M, K, ptr<uint8_t>(packed), static_cast<int>(bits), lsb_first, N, group, ptr<float>(sz), ptr<float>(bias),
                                             out.data_ptr(), bytes ? part.data_ptr() : nullptr, bytes, q.stream);

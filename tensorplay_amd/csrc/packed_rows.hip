@@ -93,10 +93,15 @@ TPQ_EXPORT int tpq_lowbit_mm_rows_takes(const void* x, int dtype, int64_t M, int
     return M >= (bits == 8 ? 17 : 33) || !at_home;
 }
 
+static PackedRowsPlan int4_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t group, int64_t room_floats) {
+    return packed_rows_plan(dtype, M, N, K, room_floats, int4_weights_unrounded(dtype, M, N, K, group) ? kRowsUnrounded : kRowsRounded);
+}
+
+static int64_t slices_bytes(const PackedRowsPlan& p, int64_t M, int64_t N) { return p.slices > 1 ? static_cast<int64_t>(p.slices) * M * N * 4 : 0; }
+
 static int64_t rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, RowsWeights weights) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, int64_t{1} << 60, weights);
-    return p.slices > 1 ? static_cast<int64_t>(p.slices) * M * N * 4 : 0;
+    return slices_bytes(packed_rows_plan(dtype, M, N, K, kRowsAnyRoom, weights), M, N);
 }
 
 TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) { return rows_workspace_bytes(dtype, M, N, K, kRowsRounded); }
@@ -105,9 +110,28 @@ TPQ_EXPORT int64_t tpq_lowbit_mm_rows_workspace_bytes(int dtype, int64_t M, int6
     return rows_workspace_bytes(dtype, M, N, K, lowbit_rows_weights(M, N, K));
 }
 
+// The plan of a call (bits 0: the int4 layout): what the launches below go by, so a workspace of its size is what they cut k for.
+static PackedRowsPlan call_plan(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group, int64_t room_floats) {
+    return bits == 0 ? int4_rows_plan(dtype, M, N, K, group, room_floats) : packed_rows_plan(dtype, M, N, K, room_floats, lowbit_rows_weights(M, N, K));
+}
+
+TPQ_EXPORT int64_t tpq_packed_rows_call_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group) {
+    return M <= 0 || N <= 0 || K <= 0 ? 0 : slices_bytes(call_plan(dtype, M, N, K, bits, group, kRowsAnyRoom), M, N);
+}
+
+TPQ_EXPORT int tpq_packed_rows_call_plan(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group, int64_t workspace_bytes, int32_t* plan) {
+    TPQ_REQUIRE(M > 0 && N > 0 && K > 0 && plan, TPQ_ERR_INVALID_VALUE, "packed_rows_call_plan: bad shape or null pointer");
+    const PackedRowsPlan p = call_plan(dtype, M, N, K, bits, group, workspace_bytes < 0 ? kRowsAnyRoom : workspace_bytes / 4);
+    plan[0] = p.quads == 0 ? TPQ_ROWS_STAGED : p.cw == 0 ? TPQ_ROWS_LANES : TPQ_ROWS_QUADS;
+    plan[1] = p.quads ? 4 * p.quads : 16 * p.mb;
+    plan[2] = p.quads && p.cw == 0 ? kWave : 32 * p.cw;
+    plan[3] = p.slices;
+    return TPQ_OK;
+}
+
 TPQ_EXPORT int tpq_packed_rows_tile_rows(int dtype, int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, int64_t{1} << 60);
+    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, kRowsAnyRoom);
     return p.quads ? 4 * p.quads : 16 * p.mb;
 }
 
@@ -129,8 +153,7 @@ TPQ_EXPORT int tpq_int4_mm_rows_bias(const void* x, int dtype, int64_t M, int64_
     TPQ_REQUIRE(aligned(x, 16) && aligned(packed, 16) && aligned(scales_and_zeros, wide ? 8 : 4) && aligned(out, wide ? 16 : 8) && aligned(bias, wide ? 4 : 2), TPQ_ERR_UNSUPPORTED,
                 "int4_mm_rows: unaligned operand");
     const bool room = workspace != nullptr && aligned(workspace, 16);
-    const PackedRowsPlan p = packed_rows_plan(dtype, M, N, K, room ? workspace_bytes / 4 : 0,
-                                              int4_weights_unrounded(dtype, M, N, K, group) ? kRowsUnrounded : kRowsRounded);
+    const PackedRowsPlan p = int4_rows_plan(dtype, M, N, K, group, room ? workspace_bytes / 4 : 0);
     if (p.quads)
         return packed_rows_f32({x, packed, scales_and_zeros, nullptr, bias, out, workspace, M, N, K, group, 0, 0, 0, static_cast<hipStream_t>(stream)}, p.quads, p.cw,
                                  p.slices, p.steps_per_slice);

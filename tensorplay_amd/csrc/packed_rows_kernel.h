@@ -711,6 +711,9 @@ inline int64_t ceil_div(int64_t a, int64_t b) {
 // need no slices, and where the card would be as fast with them the host saves a launch and an allocation (us, slices / this, eager and then
 // in a graph: int4 in groups of 64, 28 rows 4096 x 4096 11.2 / 7.6, 8.4 / 7.6; 20 rows 2048 x 2048 10.9 / 7.0, 6.7 / 5.2; 32 rows 3072 -> 8192
 // 8.7 / 7.4, 9.0 / 7.7; float32, nine rows 1408 x 1408 11.0 / 8.0, 8.2 / 7.8; 2 bits in groups of 64, three rows 2944 -> 5832 15.4 / 9.9, 15.8 / 10.2).
+// Unrounded int4 weights, whose few rows of an odd k come here: 3 for the second kernel (us, one slice / sliced, eager and then in a graph: two rows
+// 3776 -> 616 9.0 / 11.6, 8.8 / 6.6; 31 rows 4800 -> 3584 14.1 / 11.8, 14.2 / 11.3; 46 rows 1824 -> 1688 11.2 / 11.4, 11.2 / 9.6; and where half a
+// microsecond of the device would cost an eager call four: two rows 2272 -> 512 7.5 / 11.7, 7.2 / 6.5; 79 rows 1280 -> 1024 8.6 / 11.5, 8.5 / 8.2).
 // A call plans twice (workspace, launch), so what the heights have in common, the
 // divisions above all, is worked out once: 203 rows of 4096 -> 11008 0.12 us of host time instead of 0.83.
 enum RowsWeights { kRowsRounded, kRowsUnrounded, kRowsUnroundedBits };  // (16-bit) weights rounded, int4 or n-bit weights not rounded
@@ -723,6 +726,8 @@ enum RowsWeights { kRowsRounded, kRowsUnrounded, kRowsUnroundedBits };  // (16-b
 // blocks on the two kinds cost the same (12 rows of 11008 -> 4096 24.4 / 24.4, 16 rows of 4096 x 4096 12.3 / 14.1): a product of sixteen 4 x 4
 // blocks takes half the clocks of one of 16 x 16.
 constexpr int64_t kQuadRows = 8;
+
+constexpr int64_t kRowsAnyRoom = int64_t{1} << 60;  // floats of a workspace that holds the slices of any plan
 
 // With the second kernel for z slices; a call of two launches and an allocation keeps the host for 10.8 us.
 inline double sliced_us(double us, int64_t z, int64_t M, int64_t N) {
@@ -788,6 +793,7 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
     p.split = weights != kRowsRounded && dtype != TPQ_DTYPE_F32;
     const bool wide = dtype == TPQ_DTYPE_F32;
     const int64_t blocks = (M + 15) / 16, steps = (K + 127) / 128;
+    const double second_us = weights == kRowsUnrounded ? 3.0 : 2.5;
     int64_t best = 1;
     double best_us = 1e30;
     p.cw = 2;
@@ -817,7 +823,7 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
                 const int64_t z = slices_of[c], rounds = (steps_of[c] + (1 << kw_shift) - 1) >> kw_shift;
                 const double waves = static_cast<double>((tiles * z + 255) >> 8);  // 256 compute units
                 double us = waves * ((cw == 1 ? 3.4 : 4.0) + round_us * static_cast<double>(rounds));
-                if (z > 1) us = wide ? sliced_us(us, z, M, N) : us + 2.5 + static_cast<double>(z * M * N) * 8.0 / 4e6;
+                if (z > 1) us = wide ? sliced_us(us, z, M, N) : us + second_us + static_cast<double>(z * M * N) * 8.0 / 4e6;
                 if (us < best_us) { best_us = us; best = z; p.cw = cw; p.mb = mb; }
             }
         }

@@ -408,10 +408,8 @@ def _dense_mm(x: torch.Tensor, dense: torch.Tensor, out: torch.Tensor) -> torch.
 
 # ---- packed weights, a block of activation rows (tpq_int4_mm_rows, tpq_lowbit_mm_rows): the library says for which
 
-def _rows_workspace(dtype: torch.dtype, m: int, n: int, k: int, device: torch.device, lowbit: bool = False) -> torch.Tensor:
-    lib = _lib.load()
-    need = (lib.tpq_lowbit_mm_rows_workspace_bytes if lowbit else lib.tpq_packed_rows_workspace_bytes)(_DT[dtype], m, n, k)
-    return torch.empty(int(need), dtype=torch.uint8, device=device)
+def _rows_workspace(dtype: torch.dtype, m: int, n: int, k: int, bits: int, group: int, device: torch.device) -> torch.Tensor:
+    return torch.empty(int(_lib.load().tpq_packed_rows_call_workspace_bytes(_DT[dtype], m, n, k, bits, group)), dtype=torch.uint8, device=device)
 
 
 def _int4_dequantize(packed: torch.Tensor, inner: int, n: int, k: int, group: int, sz: torch.Tensor) -> torch.Tensor:
@@ -458,7 +456,7 @@ def _weight_int4pack_mm(self: torch.Tensor, mat2: torch.Tensor, qGroupSize: int,
     sz = qScaleAndZeros.to(self.dtype).contiguous()
     if inner == 2 and _lib.load().tpq_int4_mm_rows_takes(_ptr(x), _DT[x.dtype], m, n, k, qGroupSize, _ptr(w), _ptr(sz)):
         with torch.cuda.device(self.device):
-            ws = _rows_workspace(self.dtype, m, n, k, self.device)
+            ws = _rows_workspace(self.dtype, m, n, k, 0, qGroupSize, self.device)
             _check(_lib.load().tpq_int4_mm_rows(_ptr(x), _DT[x.dtype], m, k, _ptr(w), n, qGroupSize, _ptr(sz), _ptr(out), _ptr(ws),
                                                 ws.numel(), _stream(self)))
         return out
@@ -849,7 +847,7 @@ def _lowbit_mm(input: torch.Tensor, packed: torch.Tensor, bits: int, columns: in
     if m and _lib.load().tpq_lowbit_mm_rows_takes(_ptr(x), _DT[x.dtype], m, n, columns, bits, int(lsb_first), group, _ptr(w), _ptr(sz)):
         out = torch.empty((m, n), dtype=x.dtype, device=x.device)
         with torch.cuda.device(x.device):
-            ws = _rows_workspace(x.dtype, m, n, columns, x.device, lowbit=True)
+            ws = _rows_workspace(x.dtype, m, n, columns, bits, group, x.device)
             _check(_lib.load().tpq_lowbit_mm_rows(_ptr(x), _DT[x.dtype], m, columns, _ptr(w), bits, int(lsb_first), n, group, _ptr(sz), _ptr(b),
                                                   _ptr(out), _ptr(ws), ws.numel(), _stream(x)))
         return out

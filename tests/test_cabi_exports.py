@@ -162,3 +162,32 @@ def test_quantizer_beside_the_other_operand_refuses_more_rows_than_a_launch_hold
     for m, n in ((1 << 24, 16), (16, 1 << 24)):
         assert lib.tpq_quantize_both_rowwise(256, 256, _lib.F32, m, n, 64, 64, 1e-5, 1e-8, 7.0, -8, 7, 0, 256, 256, 256, 256, None) == _lib.TPQ_ERR_UNSUPPORTED
         assert lib.tpq_quantize_rowwise_pad(256, _lib.F32, m, 36, 1e-5, 256, n, 128, 256, 256, 256, None) == _lib.TPQ_ERR_UNSUPPORTED
+
+
+def test_packed_rows_workspace_is_that_of_the_calls_plan():
+    """A packed-weight call on a block of rows cuts k as it does with any room once it has the workspace that it is told: int4 with its weight
+    rounded once or not (K % 128 != 0, groups of 128 on few rows), n-bit rows, all types, over a grid of sizes."""
+    import itertools
+
+    from tensorplay_amd import _lib
+
+    lib = _lib.load()
+
+    def plan(*call):
+        out = (ctypes.c_int32 * 4)()
+        assert lib.tpq_packed_rows_call_plan(*call, ctypes.cast(out, ctypes.c_void_p)) == _lib.TPQ_OK
+        return list(out)
+
+    sliced = 0
+    for dtype, M, N, K, (bits, group) in itertools.product((0, 1, 2), (1, 2, 9, 17, 33, 46, 80, 129, 300), (520, 1184, 3032, 5720, 11008), (1664, 1824, 4096, 4640, 10432),
+                                                           ((0, 32), (0, 64), (0, 128), (1, 32), (2, 64), (4, 128), (8, 32))):
+        if K % group:
+            continue
+        room = lib.tpq_packed_rows_call_workspace_bytes(dtype, M, N, K, bits, group)
+        want = plan(dtype, M, N, K, bits, group, -1)
+        assert plan(dtype, M, N, K, bits, group, room) == want, (dtype, M, N, K, bits, group)
+        assert room == (0 if want[3] == 1 else 4 * want[3] * M * N)
+        sliced += want[3] > 1
+    assert sliced > 500
+    assert plan(1, 46, 1688, 1824, 0, 32, 0)[3] == 1 and plan(1, 46, 1688, 1824, 0, 32, -1)[3] > 1
+    assert lib.tpq_packed_rows_call_plan(1, 0, 8, 32, 0, 32, -1, None) == _lib.TPQ_ERR_INVALID_VALUE

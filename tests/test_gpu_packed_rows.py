@@ -263,6 +263,33 @@ def test_few_rows_take_no_workspace():
     assert lib.tpq_lowbit_mm_rows_workspace_bytes(f16, 3, 5832, 2944) == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,group", [(46, 1688, 1824, 32), (2, 3032, 4640, 32), (11, 1184, 3136, 64), (33, 1024, 4096, 128)])
+def test_calls_have_the_slices_that_their_weight_wants(dtype, M, N, K, group):
+    """A weight that is not rounded (K % 128 != 0, groups of 128 on few rows) has longer rounds of the loop than one that is, and slices where
+    that has none: the Python entry gives the library room for them (one slice adds k in another order: some outputs in a thousand differ)."""
+    import ctypes
+
+    from tensorplay_amd import _lib, ops
+
+    lib, tag = _lib.load(), ops._DT[dtype]
+    need, plan = int(lib.tpq_packed_rows_call_workspace_bytes(tag, M, N, K, 0, group)), (ctypes.c_int32 * 4)()
+    ops._check(lib.tpq_packed_rows_call_plan(tag, M, N, K, 0, group, need, ctypes.cast(plan, ctypes.c_void_p)))
+    assert need == 4 * plan[3] * M * N and plan[3] > 1
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    packed = ops._convert_weight_to_int4pack(torch.randint(0, 16, (N, K), dtype=torch.int32, device=DEV, generator=gen), 2)
+    sz = (torch.rand(K // group, N, 2, device=DEV, generator=gen) * 0.01 + 1e-3).to(dtype)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(dtype)
+    assert lib.tpq_int4_mm_rows_takes(x.data_ptr(), tag, M, N, K, group, packed.data_ptr(), sz.data_ptr())
+    results = []
+    for room in (need, 0):
+        out, ws = torch.empty(M, N, dtype=dtype, device=DEV), torch.empty(max(room, 16), dtype=torch.uint8, device=DEV)
+        ops._check(lib.tpq_int4_mm_rows(x.data_ptr(), tag, M, K, packed.data_ptr(), N, group, sz.data_ptr(), out.data_ptr(), ws.data_ptr() if room else None, room, ops._stream(x)))
+        results.append(out)
+    assert not torch.equal(*results)
+    assert torch.equal(ops._weight_int4pack_mm(x, packed, group, sz), results[0])
+
+
 # (M, N, K, group): float32 in blocks of four rows: one and two blocks, full and not; steps of 128 k of which the last one has one to three tiles, fewer
 # steps than wavefronts, more than they have in flight; a part of 32 and of 64 channels; slices of k
 QUADS = [(1, 4, 32, 32), (3, 40, 96, 96), (4, 32, 160, 32), (5, 68, 1088, 64), (8, 200, 4096, 128), (4, 1160, 8224, 32), (7, 9736, 4864, 128), (2, 8200, 3072, 64)]
