@@ -1,4 +1,6 @@
 // Entry points of the packed-weight products for a block of activation rows (packed_rows_kernel.h).
+#include <algorithm>
+
 #include "int4_gemm_kernel.h"
 #include "packed_rows_bits.h"
 
@@ -99,20 +101,17 @@ static PackedRowsPlan int4_rows_plan(int dtype, int64_t M, int64_t N, int64_t K,
 
 static int64_t slices_bytes(const PackedRowsPlan& p, int64_t M, int64_t N) { return p.slices > 1 ? static_cast<int64_t>(p.slices) * M * N * 4 : 0; }
 
-static int64_t rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, RowsWeights weights) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    return slices_bytes(packed_rows_plan(dtype, M, N, K, kRowsAnyRoom, weights), M, N);
+TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
+    return M <= 0 || N <= 0 || K <= 0 ? 0 : slices_bytes(packed_rows_plan(dtype, M, N, K, kRowsAnyRoom), M, N);
 }
 
-TPQ_EXPORT int64_t tpq_packed_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) { return rows_workspace_bytes(dtype, M, N, K, kRowsRounded); }
-
-TPQ_EXPORT int64_t tpq_lowbit_mm_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
-    return rows_workspace_bytes(dtype, M, N, K, lowbit_rows_weights(M, N, K));
+TPQ_EXPORT int64_t tpq_lowbit_mm_rows_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {  // of any width: those that cost alike
+    return std::max(tpq_packed_rows_call_workspace_bytes(dtype, M, N, K, 1, 32), tpq_packed_rows_call_workspace_bytes(dtype, M, N, K, 8, 32));
 }
 
 // The plan of a call (bits 0: the int4 layout): what the launches below go by, so a workspace of its size is what they cut k for.
 static PackedRowsPlan call_plan(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group, int64_t room_floats) {
-    return bits == 0 ? int4_rows_plan(dtype, M, N, K, group, room_floats) : packed_rows_plan(dtype, M, N, K, room_floats, lowbit_rows_weights(M, N, K));
+    return bits == 0 ? int4_rows_plan(dtype, M, N, K, group, room_floats) : packed_rows_plan(dtype, M, N, K, room_floats, lowbit_rows_weights(M, N, K), bits);
 }
 
 TPQ_EXPORT int64_t tpq_packed_rows_call_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group) {

@@ -29,7 +29,7 @@ inline RowsWeights lowbit_rows_weights(int64_t M, int64_t N, int64_t K) { return
 
 template <int DT>
 int run_packed_rows_bits(const PackedRowsBits& c) {
-    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats, lowbit_rows_weights(c.M, c.N, c.K));
+    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats, lowbit_rows_weights(c.M, c.N, c.K), c.bits);
     if constexpr (DT == TPQ_DTYPE_F32)
         if (p.quads) return packed_rows_f32(c, p.quads, p.cw, p.slices, p.steps_per_slice);
     PackedRowsArgs a{};

@@ -702,6 +702,105 @@ inline int64_t ceil_div(int64_t a, int64_t b) {
     return up <= 0x7FFFFFFF ? static_cast<uint32_t>(up) / static_cast<uint32_t>(b) : up / b;
 }
 
+enum RowsWeights { kRowsRounded, kRowsUnrounded, kRowsUnroundedBits };  // (16-bit) weights rounded, int4 or n-bit weights not rounded
+
+constexpr int64_t kRowsAnyRoom = int64_t{1} << 60;  // floats of a workspace that holds the slices of any plan
+
+// ---- float32 ---------------------------------------------------------------------------------------------
+// Three kernels, one of which a call runs, by estimates (us).
+// Fitted to the device times of all plans of 85 shapes (k 1024 .. 8192, channels 512 .. 11008) at 25 row counts up to 64, in groups of 32, 64 and
+// 128; the plan that they take is 2 % (8 bits 4 %) above the best on average, with one cost for all widths it was 4 (9, up to 124).  What a round of the loop costs depends on the width of the codes: int4 (one instruction from pair to floats), 1, 2 and 4 bits (an instruction more a
+// code), 8 bits (twice the bytes, and with a lane per channel a line per lane and tile).  A workgroup that a compute unit gets after its first (a turn) costs its rounds
+// again, and what does not hide behind the one before it.  (10.4 and 98.5: int4 takes no staged tile of 16 rows, and 1 to 4 bits none in turns; the others were never slower.)
+struct RowsF32Cost {
+    double quads, quads_turn, quads_round[2], quads_slices, quads_mb;                // blocks of four rows: one, two of them
+    double narrow, narrow_turn, narrow_round;                                        // activations staged, 32 channels per workgroup
+    double staged, staged_round[2], staged_turn[2], staged_slices, staged_mb;        // 64 channels; one block of 16 rows, two
+    double lanes, lanes_round, lanes_block, lanes_four, lanes_turn, lanes_short, lanes_slices, lanes_mb;  // a lane per channel: a round, a block of 16, one of four
+};
+constexpr RowsF32Cost kRowsF32Costs[3] = {
+    {2.0, 1.0, {1.6, 2.4}, 2.0, 2.0, 3.9, 0.0, 2.25, 3.5, {10.4, 4.3}, {0.2, 0.9}, 1.3, 1.6, 3.3, 0.2, 0.9, 0.5, 0.0, 0.3, 1.8, 1.45},        // int4
+    {1.0, 1.2, {1.9, 2.4}, 1.0, 3.0, 3.8, 0.45, 2.85, 2.7, {2.45, 5.05}, {98.5, 4.7}, 3.0, 0.55, 4.25, 0.3, 1.0, 0.5, 1.7, 0.3, 1.85, 1.4},  // 1, 2, 4 bits
+    {1.8, 2.5, {1.4, 2.0}, 1.3, 0.4, 4.6, 0.4, 2.65, 3.4, {2.45, 4.8}, {3.55, 5.15}, 2.65, 0.95, 4.15, 1.3, 0.8, 0.0, 2.4, 0.0, 2.55, 0.95},  // 8 bits
+};
+
+// The best plan so far.  A call is replayed in a graph as well as made eagerly, where the host needs 7.2 us for one launch and 10.8 for two and an
+// allocation: the sum of both times decides (us, eager and in a graph: nine rows, int4 2048 -> 2048 one slice 9.5, 9.5, eight slices 10.8, 7.2; 1280 -> 768 8.0, 8.0 and
+// 10.8, 6.5).
+struct RowsF32Choice {
+    PackedRowsPlan plan{};
+    double best = 1e30;
+    void offer(double us, int quads, int mb, int cw, int64_t slices, int64_t steps_per_slice) {
+        const double host = slices > 1 ? 10.8 : 7.2, both = us + (us > host ? us : host);
+        if (both >= best) return;
+        best = both;
+        plan = PackedRowsPlan{mb, cw, static_cast<int>(slices), static_cast<int>(steps_per_slice), quads, false};
+    }
+};
+
+// every number of slices that `units` can be cut into: (slices, units of one, megabytes of their sums written and read)
+template <class F>
+inline void rows_slices(int64_t units, int64_t M, int64_t N, int64_t room_floats, F&& each) {
+    for (int64_t z = 1; z <= 16 && z <= units; ++z) {
+        if (z > 1 && z * M * N > room_floats) break;
+        const int64_t per = ceil_div(units, z);
+        if (ceil_div(units, per) == z) each(z, per, z > 1 ? static_cast<double>(z * M * N) * 8.0 / 4e6 : 0.0);
+    }
+}
+
+// Up to eight rows: blocks of four.  Against the blocks of 16 (us, those / these, eager): four rows, 2 bits 4864 -> 9728 34.8 / 20.8; int4
+// 1408 -> 1152 7.7 / 7.6 (in a graph 7.8 / 5.2), 4096 x 4096 11.8 / 9.3; two rows of 4096 -> 11008 28.2 / 15; one row, 2 bits, 5248 -> 3104 15.9 / 11.4; eight rows,
+// 4 bits, 4096 -> 11008 30.5 / 26.4, 2048 x 2048 10.9 / 9.5, int4 4096 x 4096 12.1 / 11.3; six rows, 8 bits, 4864 -> 10880 37.9 / 33.5.  From three
+// blocks on the two kinds cost the same (12 rows of 11008 -> 4096 24.4 / 24.4, 16 rows of 4096 x 4096 12.3 / 14.1): a product of sixteen 4 x 4
+// blocks takes half the clocks of one of 16 x 16.
+constexpr int64_t kQuadRows = 8;
+
+// From nine rows on: activations staged in LDS, or a lane per channel: 16 to 64 rows a workgroup, and where one to four rows are left over by blocks of 16, those as a
+// block of four.  Slices so short that a wavefront's four tiles in flight are not filled, on workgroups that take turns, are the worst of both kinds (10 rows 3968 -> 4864
+// with 1 bit in 16 slices 25, in three 17; 16 rows 5632 -> 8480 with 8 bits in eleven 65, three 40): the estimates of turns keep calls away from them.
+// Staged / a lane per channel, us in a graph: int4 19 rows 4096 x 4096 17.8 / 13.6, 35 rows 26.2 / 19.3, 80 rows 42.9 / 35.4, 17 rows 11008 -> 4096 35.2 / 25.8; 36 rows
+// with 8 bits 29.8 / 24.7; but 64 rows 2048 -> 8192 23.9 / 27.6, 50 rows 2048 x 2048 with 1 bit 12.4 / 13.6, 14 rows 8064 -> 1536 with 8 bits 15.6 / 17.5, 20 rows
+// 2560 -> 8192 with 8 bits 25 / 31.
+inline PackedRowsPlan packed_rows_f32_plan(int64_t M, int64_t N, int64_t K, int64_t room_floats, int bits) {
+    const RowsF32Cost& cost = kRowsF32Costs[bits == 0 ? 0 : bits == 8 ? 2 : 1];
+    RowsF32Choice choice;
+    auto turns_of = [](int64_t workgroups) { return static_cast<double>((workgroups + 255) >> 8); };  // 256 compute units
+    const int64_t steps = (K + 127) / 128, tiles = K / 32, blocks = (M + 15) / 16, columns = (N + 63) / 64;
+    if (M <= kQuadRows) {
+        const int quads = static_cast<int>((M + 3) / 4);
+        rows_slices(steps, M, N, room_floats, [&](int64_t z, int64_t per, double mb) {
+            for (int shift = 0; shift < 2; ++shift) {
+                const double turns = turns_of(((N + (32 << shift) - 1) >> (5 + shift)) * z), rounds = static_cast<double>((per + (8 >> shift) - 1) >> (3 - shift));
+                choice.offer(cost.quads + turns * (cost.quads_turn + cost.quads_round[quads - 1] * rounds) + (z > 1 ? cost.quads_slices + cost.quads_mb * mb : 0.0), quads, 0, 1 << shift, z, per);
+            }
+        });
+        return choice.plan;
+    }
+    if (blocks == 1) {  // no slices is what the narrow tiles are for
+        const double turns = turns_of((N + 31) / 32);
+        choice.offer(cost.narrow + cost.narrow_turn * (turns - 1.0) + cost.narrow_round * turns * static_cast<double>((steps + 7) >> 3), 0, 1, 1, 1, steps);
+    }
+    const int64_t staged_tiles = ceil_div(blocks, 2);
+    const int mb16 = static_cast<int>(ceil_div(blocks, staged_tiles));
+    rows_slices(steps, M, N, room_floats, [&](int64_t z, int64_t per, double mb) {
+        if (z > 1 && per < 4) return;  // less than a round of the loop
+        const double turns = turns_of(columns * staged_tiles * z), rounds = static_cast<double>((per + 3) >> 2);
+        choice.offer(cost.staged + turns * rounds * cost.staged_round[mb16 - 1] + (turns - 1.0) * cost.staged_turn[mb16 - 1] + (z > 1 ? cost.staged_slices + cost.staged_mb * mb : 0.0), 0, mb16, 2, z, per);
+    });
+    const int64_t lanes_tiles = ceil_div(blocks, 4);
+    const bool four = lanes_tiles == 1 && M > 16 && M % 16 >= 1 && M % 16 <= 4;
+    const int sixteens = static_cast<int>(four ? blocks - 1 : ceil_div(blocks, lanes_tiles));
+    const double round_us = cost.lanes_round + cost.lanes_block * sixteens + (four ? cost.lanes_four : 0.0);
+    rows_slices(tiles, M, N, room_floats, [&](int64_t z, int64_t per, double mb) {
+        const double turns = turns_of(columns * lanes_tiles * z), rounds = static_cast<double>((per + 7) >> 3);
+        choice.offer(cost.lanes + (sixteens > 3 ? 0.3 : 0.0) + turns * rounds * round_us + (turns - 1.0) * (cost.lanes_turn + cost.lanes_short * (rounds < 4.0 ? 4.0 - rounds : 0.0)) +
+                         (z > 1 ? cost.lanes_slices + cost.lanes_mb * mb : 0.0),
+                     4 * sixteens + (four ? 1 : 0), 0, 0, z, per);
+    });
+    return choice.plan;
+}
+
+// ---- float16, bfloat16 ----------------------------------------------------------------------------------
 // Tile height, channels per workgroup and slices of K by an estimate (us) fitted to a sweep of 1 .. 8 slices and both widths
 // over six shapes and 16 .. 256 rows (128 channels and 5 .. 8 blocks of rows, on the same line: 1.36 and 1.49 us a round at 7 and 8; unrounded
 // weights 1.29, 1.43, 1.66 and 1.86 us at 1 .. 4 blocks, n-bit rows 1.4 times that): 4 for the launch, the first loads and the epilogue, per
@@ -710,88 +809,17 @@ inline int64_t ceil_div(int64_t a, int64_t b) {
 // Few rows: 32 channels per workgroup, eight steps of k a round.  Half the rounds on twice the compute units, so a few thousand k
 // need no slices, and where the card would be as fast with them the host saves a launch and an allocation (us, slices / this, eager and then
 // in a graph: int4 in groups of 64, 28 rows 4096 x 4096 11.2 / 7.6, 8.4 / 7.6; 20 rows 2048 x 2048 10.9 / 7.0, 6.7 / 5.2; 32 rows 3072 -> 8192
-// 8.7 / 7.4, 9.0 / 7.7; float32, nine rows 1408 x 1408 11.0 / 8.0, 8.2 / 7.8; 2 bits in groups of 64, three rows 2944 -> 5832 15.4 / 9.9, 15.8 / 10.2).
+// 8.7 / 7.4, 9.0 / 7.7; 2 bits in groups of 64, three rows 2944 -> 5832 15.4 / 9.9, 15.8 / 10.2).
 // Unrounded int4 weights, whose few rows of an odd k come here: 3 for the second kernel (us, one slice / sliced, eager and then in a graph: two rows
 // 3776 -> 616 9.0 / 11.6, 8.8 / 6.6; 31 rows 4800 -> 3584 14.1 / 11.8, 14.2 / 11.3; 46 rows 1824 -> 1688 11.2 / 11.4, 11.2 / 9.6; and where half a
 // microsecond of the device would cost an eager call four: two rows 2272 -> 512 7.5 / 11.7, 7.2 / 6.5; 79 rows 1280 -> 1024 8.6 / 11.5, 8.5 / 8.2).
 // A call plans twice (workspace, launch), so what the heights have in common, the
 // divisions above all, is worked out once: 203 rows of 4096 -> 11008 0.12 us of host time instead of 0.83.
-enum RowsWeights { kRowsRounded, kRowsUnrounded, kRowsUnroundedBits };  // (16-bit) weights rounded, int4 or n-bit weights not rounded
-
-// float32, up to eight rows: blocks of four.  The estimate (us): 2 for the launch, then for every workgroup that a compute unit gets 1 and its rounds of the
-// loop, 1.6 with one block of rows, 2.6 with two (int4 1.5 and 2.4, 8 bits 2.4 and 3.1); slices 3.5 and their bytes: on the device less, but the host pays
-// the second launch and an allocation.  Against the blocks of 16 (us, those / these, eager): four rows, 2 bits 4864 -> 9728 34.8 / 20.8; int4
-// 1408 -> 1152 7.7 / 7.6 (in a graph 7.8 / 5.2), 4096 x 4096 11.8 / 9.3; two rows of 4096 -> 11008 28.2 / 15; one row, 2 bits, 5248 -> 3104 15.9 / 11.4; eight rows,
-// 4 bits, 4096 -> 11008 30.5 / 26.4, 2048 x 2048 10.9 / 9.5, int4 4096 x 4096 12.1 / 11.3; six rows, 8 bits, 4864 -> 10880 37.9 / 33.5.  From three
-// blocks on the two kinds cost the same (12 rows of 11008 -> 4096 24.4 / 24.4, 16 rows of 4096 x 4096 12.3 / 14.1): a product of sixteen 4 x 4
-// blocks takes half the clocks of one of 16 x 16.
-constexpr int64_t kQuadRows = 8;
-
-constexpr int64_t kRowsAnyRoom = int64_t{1} << 60;  // floats of a workspace that holds the slices of any plan
-
-// With the second kernel for z slices; a call of two launches and an allocation keeps the host for 10.8 us.
-inline double sliced_us(double us, int64_t z, int64_t M, int64_t N) {
-    us += 2.5 + static_cast<double>(z * M * N) * 8.0 / 4e6;
-    return us < 10.8 ? 10.8 : us;
-}
-
-inline PackedRowsPlan packed_quads_plan(int64_t M, int64_t N, int64_t K, int64_t room_floats) {
-    PackedRowsPlan p{};
-    p.quads = static_cast<int>((M + 3) / 4);
-    const int64_t steps = (K + 127) / 128;
-    double best_us = 1e30;
-    for (int64_t z = 1; z <= 16 && z <= steps; ++z) {
-        if (z > 1 && z * M * N > room_floats) break;
-        const int64_t per = ceil_div(steps, z);
-        if (ceil_div(steps, per) != z) continue;
-        for (int shift = 0; shift < 2; ++shift) {
-            const int64_t workgroups = ((N + (32 << shift) - 1) >> (5 + shift)) * z, rounds = (per + (8 >> shift) - 1) >> (3 - shift);
-            const double us = 2.0 + static_cast<double>((workgroups + 255) >> 8) * (1.0 + (p.quads == 1 ? 1.6 : 2.6) * static_cast<double>(rounds)) +
-                              (z == 1 ? 0.0 : 3.5 + static_cast<double>(z * M * N) * 8.0 / 4e6);
-            if (us < best_us) {
-                best_us = us;
-                p.cw = 1 << shift;
-                p.slices = static_cast<int>(z);
-                p.steps_per_slice = static_cast<int>(per);
-            }
-        }
-    }
-    return p;
-}
-
-// float32, a lane per channel: 16 to 64 rows a workgroup, and where one to four rows are left over by blocks of 16, those as a block of four.  The estimate (us): 3 and
-// half a microsecond for each block of rows (launch, first loads, sums in LDS), per round of eight tiles of k 0.35 + 1.01 a block + 0.33 for the block of four, for every
-// workgroup that a compute unit gets (one block: two are there at once; more: a microsecond a block between them), and the slices' second kernel as above.  Against the kernel with its activations in LDS (us, that one / this): int4 19 rows 4096 x 4096
-// 17.8 / 13.6, 35 rows 26.2 / 19.3, 48 rows 26.4 / 22.1, 80 rows 42.9 / 35.4, 17 rows 11008 -> 4096 35.2 / 25.8, 14 rows 4096 -> 11008 26.7 / 22.2; 36 rows with 8 bits 29.8 / 24.7;
-// but 64 rows 2048 -> 8192 23.9 / 27.6, 50 rows 2048 x 2048 with 1 bit 12.4 / 13.6, 32 rows 4096 x 4096 17.3 / 17.5.
-inline bool packed_lanes_plan(int64_t M, int64_t N, int64_t K, int64_t room_floats, double& best_us, PackedRowsPlan& p) {
-    const int64_t blocks = (M + 15) / 16, row_tiles = ceil_div(blocks, 4), tiles = K / 32, columns = (N + 63) / 64;
-    const bool four = row_tiles == 1 && M > 16 && M % 16 >= 1 && M % 16 <= 4;
-    const int64_t sixteens = four ? blocks - 1 : ceil_div(blocks, row_tiles);
-    const double fixed_us = 3.0 + 0.5 * static_cast<double>(sixteens), round_us = 0.35 + 1.01 * static_cast<double>(sixteens) + (four ? 0.33 : 0.0);
-    bool taken = false;
-    for (int64_t z = 1; z <= 16 && z <= tiles; ++z) {
-        if (z > 1 && z * M * N > room_floats) break;
-        const int64_t per = ceil_div(tiles, z);
-        if (ceil_div(tiles, per) != z) continue;
-        const int64_t turns = (columns * row_tiles * z + 255) >> 8;
-        double us = fixed_us + round_us * static_cast<double>(turns * ((per + 7) >> 3)) + static_cast<double>((turns - 1) * (sixteens - 1));
-        if (z > 1) us = sliced_us(us, z, M, N);
-        if (us < best_us) {
-            best_us = us;
-            p = PackedRowsPlan{0, 0, static_cast<int>(z), static_cast<int>(per), static_cast<int>(4 * sixteens + (four ? 1 : 0)), false};
-            taken = true;
-        }
-    }
-    return taken;
-}
-
-inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, RowsWeights weights = kRowsRounded) {
-    if (dtype == TPQ_DTYPE_F32 && M <= kQuadRows) return packed_quads_plan(M, N, K, room_floats);
+inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, RowsWeights weights = kRowsRounded, int bits = 0) {
+    if (dtype == TPQ_DTYPE_F32) return packed_rows_f32_plan(M, N, K, room_floats, bits);
     PackedRowsPlan p;
     p.quads = 0;
-    p.split = weights != kRowsRounded && dtype != TPQ_DTYPE_F32;
-    const bool wide = dtype == TPQ_DTYPE_F32;
+    p.split = weights != kRowsRounded;
     const int64_t blocks = (M + 15) / 16, steps = (K + 127) / 128;
     const double second_us = weights == kRowsUnrounded ? 3.0 : 2.5;
     int64_t best = 1;
@@ -807,30 +835,26 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
         slices_of[cuts] = z;
         steps_of[cuts++] = per;
     }
-    for (int cw = blocks <= (wide ? 1 : 2) ? 1 : 2; cw <= (K % 128 == 0 && !p.split && !wide ? 4 : 2); cw *= 2) {
+    for (int cw = blocks <= 2 ? 1 : 2; cw <= (K % 128 == 0 && !p.split ? 4 : 2); cw *= 2) {
         // 32 and 64 channels: tiles of equal height, as few as the tallest allows; 128 channels: any height that tiles of equal height can have
-        const int kw_shift = cw == 1 ? 3 : cw == 2 ? 2 : 1, most = wide ? 2 : cw <= 2 ? 4 : 8;
+        const int kw_shift = cw == 1 ? 3 : cw == 2 ? 2 : 1, most = cw <= 2 ? 4 : 8;
         const int64_t fewest = ceil_div(blocks, most);
         const int tallest = static_cast<int>(ceil_div(blocks, fewest));
         for (int mb = tallest; mb >= (cw <= 2 ? tallest : 3); --mb) {
             const int64_t row_tiles = ceil_div(blocks, mb);
             if (ceil_div(blocks, row_tiles) != mb) continue;
             const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
-            const double round_us = (wide ? 0.3 + 2.3 * mb : p.split ? (1.08 + 0.19 * mb) * (weights == kRowsUnroundedBits ? 1.4 : 1.0) : cw <= 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb) +
+            const double round_us = (p.split ? (1.08 + 0.19 * mb) * (weights == kRowsUnroundedBits ? 1.4 : 1.0) : cw <= 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb) +
                                     (cw == 1 ? 0.2 * mb : 0.0);
             for (int c = 0; c < cuts; ++c) {
                 if (cw == 1 && c > 0) break;  // no slices is what they are for
                 const int64_t z = slices_of[c], rounds = (steps_of[c] + (1 << kw_shift) - 1) >> kw_shift;
                 const double waves = static_cast<double>((tiles * z + 255) >> 8);  // 256 compute units
                 double us = waves * ((cw == 1 ? 3.4 : 4.0) + round_us * static_cast<double>(rounds));
-                if (z > 1) us = wide ? sliced_us(us, z, M, N) : us + second_us + static_cast<double>(z * M * N) * 8.0 / 4e6;
+                if (z > 1) us += second_us + static_cast<double>(z * M * N) * 8.0 / 4e6;
                 if (us < best_us) { best_us = us; best = z; p.cw = cw; p.mb = mb; }
             }
         }
-    }
-    if (wide) {
-        PackedRowsPlan lanes;
-        if (packed_lanes_plan(M, N, K, room_floats, best_us, lanes)) return lanes;
     }
     if (const char* e = tuning_env("TPQ_ROWS_SLICES")) best = std::atoi(e);
     if (const char* e = tuning_env("TPQ_ROWS_CW")) p.cw = std::atoi(e);

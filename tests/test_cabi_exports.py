@@ -191,3 +191,29 @@ def test_packed_rows_workspace_is_that_of_the_calls_plan():
     assert sliced > 500
     assert plan(1, 46, 1688, 1824, 0, 32, 0)[3] == 1 and plan(1, 46, 1688, 1824, 0, 32, -1)[3] > 1
     assert lib.tpq_packed_rows_call_plan(1, 0, 8, 32, 0, 32, -1, None) == _lib.TPQ_ERR_INVALID_VALUE
+
+
+def test_float32_packed_rows_plan_by_width_and_without_short_turns():
+    """float32 rows against packed weights: workgroups that take turns on the compute units have at least a round of the loop each with something
+    behind it (a wavefront's tiles in flight filled: 8 bits, 16 rows of 5632 -> 8480 took 65 us in eleven slices of one round, 40 in three), the kernel depends on
+    the width of the codes, and between plans that an eager call cannot tell apart the shorter one on the device is taken."""
+    import itertools
+
+    from tensorplay_amd import _lib
+
+    lib = _lib.load()
+    staged, lanes = 0, 2
+
+    def plan(M, K, N, bits, group):
+        out = (ctypes.c_int32 * 4)()
+        assert lib.tpq_packed_rows_call_plan(0, M, N, K, bits, group, -1, ctypes.cast(out, ctypes.c_void_p)) == _lib.TPQ_OK
+        return list(out)
+
+    for M, K, N, bits in itertools.product((9, 13, 16, 20, 35, 64, 150), (1664, 2432, 3328, 3968, 5632, 8192), (520, 3776, 4368, 4864, 6264, 8480, 11008), (0, 1, 4, 8)):
+        kernel, rows, _, slices = plan(M, K, N, bits, 32)
+        turns = -(-(-(-N // 64) * -(-M // rows) * slices) // 256)
+        if kernel == lanes and slices > 1 and turns > 1:
+            assert -(-(K // 32) // slices) > 8, (M, K, N, bits)
+    assert [plan(14, 8064, 1536, bits, 64)[0] for bits in (0, 8)] == [lanes, staged]
+    assert plan(16, 5632, 8480, 8, 32)[0] == staged and plan(10, 3968, 4864, 1, 64)[0] == staged
+    assert plan(12, 4096, 1024, 0, 128)[0] == lanes and plan(9, 2336, 520, 0, 32)[0] == lanes
