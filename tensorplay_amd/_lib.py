@@ -53,6 +53,8 @@ SIGNATURES = {
     "tpq_ternary_mm_ws": [_ptr, _ptr, _ptr, _f32, _ptr, _i64, _i64, _i64, _ptr, _int, _ptr, _ptr, _i64, _ptr],
     "tpq_ternary_linear_row": [_ptr, _int, _ptr, _f32, _ptr, _i64, _i64, _f32, _ptr, _ptr],
     "tpq_int8_linear_few_takes": [_ptr, _ptr, _i64, _i64, _i64],
+    "tpq_int8_linear_few_pays": [_i64, _i64, _i64],
+    "tpq_ternary_linear_few_pays": [_i64, _i64, _i64],
     "tpq_int8_linear_few": [_ptr, _int, _ptr, _ptr, _ptr, _i64, _i64, _i64, _f32, _ptr, _int, _ptr],
     "tpq_ternary_linear_few_takes": [_ptr, _ptr, _i64, _i64, _i64],
     "tpq_ternary_linear_few": [_ptr, _int, _ptr, _f32, _ptr, _i64, _i64, _i64, _f32, _ptr, _ptr],

@@ -26,6 +26,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 #include <c10/util/Exception.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
@@ -47,7 +48,7 @@ struct Library {
     TPQ_ENTRY(tpq_lowbit_mm) TPQ_ENTRY(tpq_quantize_affine) TPQ_ENTRY(tpq_dequantize_affine) \
     TPQ_ENTRY(tpq_f32_linear_grads_workspace_bytes) TPQ_ENTRY(tpq_f32_linear_grads) \
     TPQ_ENTRY(tpq_f32_linear_grads_takes) TPQ_ENTRY(tpq_quantize_beside_takes) \
-    TPQ_ENTRY(tpq_int8_linear_few_takes) TPQ_ENTRY(tpq_int8_linear_few) TPQ_ENTRY(tpq_ternary_linear_few_takes) TPQ_ENTRY(tpq_ternary_linear_few) \
+    TPQ_ENTRY(tpq_int8_linear_few_pays) TPQ_ENTRY(tpq_ternary_linear_few_pays) TPQ_ENTRY(tpq_int8_linear_few_takes) TPQ_ENTRY(tpq_int8_linear_few) TPQ_ENTRY(tpq_ternary_linear_few_takes) TPQ_ENTRY(tpq_ternary_linear_few) \
     TPQ_ENTRY(tpq_quantize_both_rowwise) TPQ_ENTRY(tpq_quantize_rowwise_pad)
     TPQ_ENTRIES
 #undef TPQ_ENTRY
@@ -261,6 +262,15 @@ TPQ_CALL_END
 // Rows of codes that a product of more than ragged_rows rows reads: the next multiple of 128 where K is none of 16
 int64_t code_pitch(int64_t K) { return K % 16 ? (K + 127) / 128 * 128 : K; }
 
+// A launch saved that makes the device's part longer (the library's answer 1) is saved in eager calls only; the bits are the same either way.
+bool pays_here(int pays, const at::Tensor& x) {
+    if (pays != 1) return pays != 0;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream(x.device().index()).stream(), &capture) == hipSuccess) return capture == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // the default stream beside a capture that waits for it: not captured itself
+    return true;
+}
+
 // int8_linear(x [..., K] float, w int8 [N, K], col_scale, bias or None, eps, out_dtype, ragged_rows): quantize + product.  Above ragged_rows
 // rows with K % 16 != 0 the quantizer's launch copies the weight to padded rows as well.
 TPQ_CALL(int8_linear, 7)
@@ -282,7 +292,7 @@ TPQ_CALL(int8_linear, 7)
         Py_RETURN_NONE;
     at::Tensor out;
     int status;
-    if (lib.tpq_int8_linear_few_takes(x->const_data_ptr(), ptr<int8_t>(w), M, N, K)) {
+    if (lib.tpq_int8_linear_few_takes(x->const_data_ptr(), ptr<int8_t>(w), M, N, K) && pays_here(lib.tpq_int8_linear_few_pays(M, N, K), *x)) {
         {
             Enqueue q(*x);
             out = allocate(sizes, type, *x);
@@ -367,7 +377,8 @@ TPQ_CALL(ternary_linear, 6)
     int status = TPQ_ERR_UNSUPPORTED;
     {
         Enqueue q(*x);
-        const bool row = M == 1 && N * K <= kRowQuantizedInProduct, one_launch = row || lib.tpq_ternary_linear_few_takes(x->const_data_ptr(), ptr<uint8_t>(packed), M, N, K);
+        const bool row = M == 1 && N * K <= kRowQuantizedInProduct;
+        const bool one_launch = row || (lib.tpq_ternary_linear_few_takes(x->const_data_ptr(), ptr<uint8_t>(packed), M, N, K) && pays_here(lib.tpq_ternary_linear_few_pays(M, N, K), *x));
         if (one_launch) out = allocate(sizes, at::kFloat, *x);
         if (one_launch && !row)
             status = lib.tpq_ternary_linear_few(x->const_data_ptr(), float_tag(x->scalar_type()), ptr<uint8_t>(packed), static_cast<float>(w_scale), ptr<float>(bias), M, N, K,

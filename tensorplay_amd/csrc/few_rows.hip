@@ -211,6 +211,23 @@ inline FewRowsPlan few_rows_plan(int64_t M, int64_t N, int64_t K, int step, int 
     return p;
 }
 
+// For whom a call that the kernel takes should go to it: 2 everybody, 1 who makes it eagerly (the host saves a launch and a buffer, the device is
+// longer by the vector work of the rows in every workgroup, so the two launches are the shorter ones to replay), 0 nobody.  us, two launches / one, in a
+// graph and eager:
+//   four segments: int8 with two steps a wavefront, eight rows 3968 -> 1708 9.0 / 9.5, 10.7 / 9.7, 11 rows 2528 -> 2460 8.1 / 9.6, 9.4 / 9.8; with one, 16 rows 1984 -> 2272 8.1 /
+//     8.7, 10.6 / 8.7, but up to 48 of the 64 filled, 12 rows 1936 -> 3832 8.4 / 8.1.  Ternary with K % 256 == 0, two linears: 16 rows 2048 x 2048 15.6 / 17.4, 25.9 / 17.5; other K,
+//     whose product of codes is the slower one, 16 rows 1984 x 1984 22.4 / 17.8
+//   int8 rows off 64 bytes, whose steps touch twice the lines: four steps a wavefront, one row 7392 -> 1348 10.2 / 11.6, 10.8 / 11.7, two rows 6160 -> 820 9.8 / 11.7, 10.6 /
+//     11.8; three steps and two segments, three rows 4272 -> 924 9.2 / 10.5, 10.6 / 10.6 (one segment, 3 rows in four are shorter)
+inline int few_rows_pays(const FewRowsPlan& p, int64_t M, int64_t K, int step) {
+    if (!p.segments) return 0;
+    if (step != FewInt8::kStep) return p.segments == 4 && K % step == 0 ? 1 : 2;
+    const bool off_lines = K % 64 != 0;
+    if (off_lines && p.steps_per_wave == 4) return 0;
+    const bool full = p.segments == 4 && (p.steps_per_wave > 1 || M * ((K + kFewSegment - 1) / kFewSegment) > 48);
+    return full || (off_lines && p.segments == 2 && p.steps_per_wave == 3) ? 1 : 2;
+}
+
 template <class Source, int XDT>
 int launch_few_rows(const void* x, const uint8_t* w, int64_t M, int64_t N, int64_t K, const FewRowsPlan& p, float eps, const FewRowsOut& o, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(((N + 15) / 16 + (1 << p.nb_shift) - 1) >> p.nb_shift));
@@ -257,6 +274,8 @@ TPQ_EXPORT int tpq_int8_linear_few_takes(const void* x, const int8_t* w, int64_t
     return few_rows_plan(M, N, K, FewInt8::kStep, 16).segments && aligned(x, 16) && aligned(w, 16);
 }
 
+TPQ_EXPORT int tpq_int8_linear_few_pays(int64_t M, int64_t N, int64_t K) { return few_rows_pays(few_rows_plan(M, N, K, FewInt8::kStep, 16), M, K, FewInt8::kStep); }
+
 TPQ_EXPORT int tpq_int8_linear_few(const void* x, int x_dtype, const int8_t* w, const float* col_scale, const float* bias, int64_t M, int64_t N, int64_t K, float eps,
                                    void* out, int out_dtype, void* stream) {
     TPQ_REQUIRE(float_dtype(x_dtype) && float_dtype(out_dtype), TPQ_ERR_INVALID_TYPE, "int8_linear_few: unsupported dtype");
@@ -267,6 +286,8 @@ TPQ_EXPORT int tpq_int8_linear_few(const void* x, int x_dtype, const int8_t* w, 
 TPQ_EXPORT int tpq_ternary_linear_few_takes(const void* x, const uint8_t* packed, int64_t M, int64_t N, int64_t K) {
     return few_rows_plan(M, N, K, FewTernary::kStep, 64).segments && aligned(x, 16) && aligned(packed, 16);
 }
+
+TPQ_EXPORT int tpq_ternary_linear_few_pays(int64_t M, int64_t N, int64_t K) { return few_rows_pays(few_rows_plan(M, N, K, FewTernary::kStep, 64), M, K, FewTernary::kStep); }
 
 TPQ_EXPORT int tpq_ternary_linear_few(const void* x, int x_dtype, const uint8_t* packed, float w_scale, const float* bias, int64_t M, int64_t N, int64_t K, float eps,
                                       float* out, void* stream) {

@@ -102,3 +102,49 @@ def test_linears_on_both_sides_of_the_line_in_a_graph():
             codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
             want = ops.int8_mm_dequant(codes, module.weight, scale, module.weight_scale, bias=module.bias, out_dtype=torch.float16)
             assert torch.equal(out, want) and torch.equal(module(x), want)
+
+
+# (kind, rows, k, n): where the one launch is the longer one on the device and on both sides of that line
+PAYS = [("int8", 8, 4096, 4096, 1), ("int8", 11, 2528, 2460, 1), ("int8", 16, 1984, 2272, 1), ("int8", 12, 1984, 2272, 2), ("int8", 2, 4096, 4096, 2), ("int8", 1, 7392, 1348, 0),
+        ("int8", 1, 7424, 1348, 2), ("int8", 3, 4272, 924, 1), ("int8", 3, 4288, 924, 2), ("int8", 17, 1024, 64, 0), ("ternary", 16, 2048, 2048, 1), ("ternary", 16, 1984, 2048, 2),
+        ("ternary", 8, 2048, 2048, 2)]
+
+
+@pytest.mark.parametrize("kind,m,k,n,pays", PAYS)
+def test_one_launch_where_it_pays(kind, m, k, n, pays):
+    """Eager calls save a launch and its buffer wherever the device is not longer by more; a captured call takes the shorter way on the device.  The same
+    bits either way, eager, captured and replayed; the way shows in the allocations (the result, and the codes that two launches need)."""
+    from tensorplay_amd import _lib, ops
+    from tensorplay_amd.ao import quantization as q
+
+    lib = _lib.load()
+    assert (lib.tpq_int8_linear_few_pays if kind == "int8" else lib.tpq_ternary_linear_few_pays)(m, n, k) == pays
+    lin = torch.nn.Linear(k, n, bias=False, device="cuda", dtype=torch.float16)
+    module = q.Int8DynamicLinear.from_float(lin, out_dtype=torch.float16) if kind == "int8" else q.BitNetPacked2bitLinear.from_float(lin)
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    x = torch.randn(m, k, device="cuda", generator=gen).half()
+
+    def codes_and_product():
+        codes, scale = ops._quantize_int8_rowwise(x, 1e-5)
+        if kind == "int8":
+            return ops.int8_mm_dequant(codes, module.weight, scale, module.weight_scale, bias=module.bias, out_dtype=torch.float16)
+        return ops.ternary_mm(codes, scale, module.int_data, float(module.scale), k, bias=module.bias)
+
+    def allocations(call):
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        out = call()
+        return out, torch.cuda.memory_stats()["allocation.all.allocated"] - before
+
+    with torch.no_grad():
+        module(x)
+        torch.cuda.synchronize()
+        _, eager = allocations(lambda: module(x))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out, captured = allocations(lambda: module(x))
+        assert (eager > 1, captured > 1) == (pays == 0, pays < 2)
+        for _ in range(3):
+            x.copy_(torch.randn(m, k, device="cuda", generator=gen))
+            graph.replay()
+            want = codes_and_product()
+            assert torch.equal(out, want) and torch.equal(module(x), want)
