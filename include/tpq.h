@@ -241,8 +241,9 @@ int tpq_ternary_linear_row(const void* x, int x_dtype, const uint8_t* packed, fl
 /*
  * Dynamically quantized linears of up to 16 activation rows x [M, K] in one launch, with the bits of tpq_quantize_rowwise (divisor 127,
  * codes -127 .. 127) followed by tpq_int8_mm_dequant (out [M, N] of out_dtype) or by tpq_ternary_mm (out [M, N] float32).  The `_takes` forms
- * say (1 / 0) whether a shape and its operands are taken: K % 16 == 0 (ternary: 64), M ceil(K / 512) <= 64, at most 2^25 weights
- * with a compute unit's share in its registers, x and the weight 16-byte aligned; else TPQ_ERR_UNSUPPORTED.  The `_pays` forms say for whom a
+ * say (1 / 0) whether a shape and its operands are taken, else TPQ_ERR_UNSUPPORTED: K % 16 == 0 (ternary: 64), K <= 8192, N <= 32768,
+ * M ceil(K / 512) <= 64, at most 2^25 weights with a compute unit's share in its registers, x and the weight 16-byte aligned, and for int8
+ * rows with M ceil(K / 512) > 32 half of that share and K within 15 / 16 of a multiple of 512.  The `_pays` forms say for whom a
  * shape that is taken should go this way: 2 everybody, 1 eager calls but no captured ones (the two launches are the shorter ones on the
  * device), 0 nobody.  Host logic only.
  */

@@ -21,7 +21,8 @@
 namespace tpq {
 namespace {
 
-constexpr int kFewWaves = 16, kFewRows = 16, kFewSegment = kWave * kVec, kFewSegments = 4 * kFewWaves, kFewMaxSteps = 4;
+constexpr int kFewWaves = 16, kFewRows = 16, kFewSegment = kWave * kVec, kFewSegments = 4 * kFewWaves, kFewMaxSteps = 4,
+              kFewFullSteps = 2;  // int8 rows in four segments
 
 struct FewRowsOut {
     void* out;           // [M][N]
@@ -206,7 +207,7 @@ inline FewRowsPlan few_rows_plan(int64_t M, int64_t N, int64_t K, int step, int 
     while (((N + 15) / 16 + (1 << p.nb_shift) - 1) >> p.nb_shift > 256) ++p.nb_shift;
     const int64_t shares = (((K + step - 1) / step << p.nb_shift) + kFewWaves - 1) / kFewWaves;
     if (shares > kFewMaxSteps) return none;
-    if (step == FewInt8::kStep && p.segments == 4 && (shares > 2 || M * K * 16 < segs * kFewSegment * 15)) return none;
+    if (step == FewInt8::kStep && p.segments == 4 && (shares > kFewFullSteps || M * K * 16 < segs * kFewSegment * 15)) return none;
     p.steps_per_wave = static_cast<int>(shares);
     return p;
 }
@@ -239,11 +240,12 @@ int launch_few_rows(const void* x, const uint8_t* w, int64_t M, int64_t N, int64
             per_row, 1.0f / static_cast<float>(per_row), eps, o);
     };
     auto with_segments = [&](auto segs) {
-        switch (p.steps_per_wave) {
-            case 1: run(segs, std::integral_constant<int, 1>{}); break;
-            case 2: run(segs, std::integral_constant<int, 2>{}); break;
-            case 3: run(segs, std::integral_constant<int, 3>{}); break;
-            default: run(segs, std::integral_constant<int, 4>{}); break;
+        constexpr int kMost = Source::kStep == FewInt8::kStep && decltype(segs)::value == 4 ? kFewFullSteps : kFewMaxSteps;
+        if (p.steps_per_wave == 1) run(segs, std::integral_constant<int, 1>{});
+        else if (p.steps_per_wave == 2) run(segs, std::integral_constant<int, 2>{});
+        else if constexpr (kMost > kFewFullSteps) {
+            if (p.steps_per_wave == 3) run(segs, std::integral_constant<int, 3>{});
+            else run(segs, std::integral_constant<int, 4>{});
         }
     };
     if (p.segments == 1) with_segments(std::integral_constant<int, 1>{});
