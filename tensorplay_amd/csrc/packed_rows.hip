@@ -111,7 +111,7 @@ TPQ_EXPORT int64_t tpq_lowbit_mm_rows_workspace_bytes(int dtype, int64_t M, int6
 
 // The plan of a call (bits 0: the int4 layout): what the launches below go by, so a workspace of its size is what they cut k for.
 static PackedRowsPlan call_plan(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group, int64_t room_floats) {
-    return bits == 0 ? int4_rows_plan(dtype, M, N, K, group, room_floats) : packed_rows_plan(dtype, M, N, K, room_floats, lowbit_rows_weights(M, N, K), bits);
+    return bits == 0 ? int4_rows_plan(dtype, M, N, K, group, room_floats) : packed_rows_plan(dtype, M, N, K, room_floats, lowbit_rows_weights(M, N, K, bits), bits);
 }
 
 TPQ_EXPORT int64_t tpq_packed_rows_call_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int bits, int64_t group) {

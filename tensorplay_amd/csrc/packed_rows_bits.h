@@ -25,11 +25,13 @@ namespace {
 
 // up to these rows the decode kernels ran, which apply the scales to sums of whole codes: no weight is rounded to 16 bits; above, the
 // dense route's 16-bit weight
-inline RowsWeights lowbit_rows_weights(int64_t M, int64_t N, int64_t K) { return M <= (N * K <= (int64_t{1} << 24) ? 80 : 56) ? kRowsUnroundedBits : kRowsRounded; }
+inline RowsWeights lowbit_rows_weights(int64_t M, int64_t N, int64_t K, int bits) {
+    return M <= (N * K <= (int64_t{1} << 24) ? 80 : 56) ? kRowsUnroundedBits : bits == 8 ? kRowsRoundedBytes : kRowsRoundedBits;
+}
 
 template <int DT>
 int run_packed_rows_bits(const PackedRowsBits& c) {
-    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats, lowbit_rows_weights(c.M, c.N, c.K), c.bits);
+    const PackedRowsPlan p = packed_rows_plan(DT, c.M, c.N, c.K, c.room_floats, lowbit_rows_weights(c.M, c.N, c.K, c.bits), c.bits);
     if constexpr (DT == TPQ_DTYPE_F32)
         if (p.quads) return packed_rows_f32(c, p.quads, p.cw, p.slices, p.steps_per_slice);
     PackedRowsArgs a{};

@@ -702,7 +702,8 @@ inline int64_t ceil_div(int64_t a, int64_t b) {
     return up <= 0x7FFFFFFF ? static_cast<uint32_t>(up) / static_cast<uint32_t>(b) : up / b;
 }
 
-enum RowsWeights { kRowsRounded, kRowsUnrounded, kRowsUnroundedBits };  // (16-bit) weights rounded, int4 or n-bit weights not rounded
+// (16-bit) weights rounded once: int4, n-bit, 8-bit; not rounded: int4, n-bit
+enum RowsWeights { kRowsRounded, kRowsRoundedBits, kRowsRoundedBytes, kRowsUnrounded, kRowsUnroundedBits };
 
 constexpr int64_t kRowsAnyRoom = int64_t{1} << 60;  // floats of a workspace that holds the slices of any plan
 
@@ -713,10 +714,10 @@ constexpr int64_t kRowsAnyRoom = int64_t{1} << 60;  // floats of a workspace tha
 // code), 8 bits (twice the bytes, and with a lane per channel a line per lane and tile).  A workgroup that a compute unit gets after its first (a turn) costs its rounds
 // again, and what does not hide behind the one before it.  (10.4 and 98.5: int4 takes no staged tile of 16 rows, and 1 to 4 bits none in turns; the others were never slower.)
 struct RowsF32Cost {
-    double quads, quads_turn, quads_round[2], quads_slices, quads_mb;                // blocks of four rows: one, two of them
+    double quads, quads_turn, quads_round[2], quads_slices, quads_bytes;                // blocks of four rows: one, two of them
     double narrow, narrow_turn, narrow_round;                                        // activations staged, 32 channels per workgroup
-    double staged, staged_round[2], staged_turn[2], staged_slices, staged_mb;        // 64 channels; one block of 16 rows, two
-    double lanes, lanes_round, lanes_block, lanes_four, lanes_turn, lanes_short, lanes_slices, lanes_mb;  // a lane per channel: a round, a block of 16, one of four
+    double staged, staged_round[2], staged_turn[2], staged_slices, staged_bytes;        // 64 channels; one block of 16 rows, two
+    double lanes, lanes_round, lanes_block, lanes_four, lanes_turn, lanes_short, lanes_slices, lanes_bytes;  // a lane per channel: a round, a block of 16, one of four
 };
 constexpr RowsF32Cost kRowsF32Costs[3] = {
     {2.0, 1.0, {1.6, 2.4}, 2.0, 2.0, 3.9, 0.0, 2.25, 3.5, {10.4, 4.3}, {0.2, 0.9}, 1.3, 1.6, 3.3, 0.2, 0.9, 0.5, 0.0, 0.3, 1.8, 1.45},        // int4
@@ -738,7 +739,7 @@ struct RowsF32Choice {
     }
 };
 
-// every number of slices that `units` can be cut into: (slices, units of one, megabytes of their sums written and read)
+// every number of slices that `units` can be cut into: (slices, units of one, us of their sums written and read at 4 TB/s)
 template <class F>
 inline void rows_slices(int64_t units, int64_t M, int64_t N, int64_t room_floats, F&& each) {
     for (int64_t z = 1; z <= 16 && z <= units; ++z) {
@@ -768,10 +769,10 @@ inline PackedRowsPlan packed_rows_f32_plan(int64_t M, int64_t N, int64_t K, int6
     const int64_t steps = (K + 127) / 128, tiles = K / 32, blocks = (M + 15) / 16, columns = (N + 63) / 64;
     if (M <= kQuadRows) {
         const int quads = static_cast<int>((M + 3) / 4);
-        rows_slices(steps, M, N, room_floats, [&](int64_t z, int64_t per, double mb) {
+        rows_slices(steps, M, N, room_floats, [&](int64_t z, int64_t per, double sums_us) {
             for (int shift = 0; shift < 2; ++shift) {
                 const double turns = turns_of(((N + (32 << shift) - 1) >> (5 + shift)) * z), rounds = static_cast<double>((per + (8 >> shift) - 1) >> (3 - shift));
-                choice.offer(cost.quads + turns * (cost.quads_turn + cost.quads_round[quads - 1] * rounds) + (z > 1 ? cost.quads_slices + cost.quads_mb * mb : 0.0), quads, 0, 1 << shift, z, per);
+                choice.offer(cost.quads + turns * (cost.quads_turn + cost.quads_round[quads - 1] * rounds) + (z > 1 ? cost.quads_slices + cost.quads_bytes * sums_us : 0.0), quads, 0, 1 << shift, z, per);
             }
         });
         return choice.plan;
@@ -782,19 +783,19 @@ inline PackedRowsPlan packed_rows_f32_plan(int64_t M, int64_t N, int64_t K, int6
     }
     const int64_t staged_tiles = ceil_div(blocks, 2);
     const int mb16 = static_cast<int>(ceil_div(blocks, staged_tiles));
-    rows_slices(steps, M, N, room_floats, [&](int64_t z, int64_t per, double mb) {
+    rows_slices(steps, M, N, room_floats, [&](int64_t z, int64_t per, double sums_us) {
         if (z > 1 && per < 4) return;  // less than a round of the loop
         const double turns = turns_of(columns * staged_tiles * z), rounds = static_cast<double>((per + 3) >> 2);
-        choice.offer(cost.staged + turns * rounds * cost.staged_round[mb16 - 1] + (turns - 1.0) * cost.staged_turn[mb16 - 1] + (z > 1 ? cost.staged_slices + cost.staged_mb * mb : 0.0), 0, mb16, 2, z, per);
+        choice.offer(cost.staged + turns * rounds * cost.staged_round[mb16 - 1] + (turns - 1.0) * cost.staged_turn[mb16 - 1] + (z > 1 ? cost.staged_slices + cost.staged_bytes * sums_us : 0.0), 0, mb16, 2, z, per);
     });
     const int64_t lanes_tiles = ceil_div(blocks, 4);
     const bool four = lanes_tiles == 1 && M > 16 && M % 16 >= 1 && M % 16 <= 4;
     const int sixteens = static_cast<int>(four ? blocks - 1 : ceil_div(blocks, lanes_tiles));
     const double round_us = cost.lanes_round + cost.lanes_block * sixteens + (four ? cost.lanes_four : 0.0);
-    rows_slices(tiles, M, N, room_floats, [&](int64_t z, int64_t per, double mb) {
+    rows_slices(tiles, M, N, room_floats, [&](int64_t z, int64_t per, double sums_us) {
         const double turns = turns_of(columns * lanes_tiles * z), rounds = static_cast<double>((per + 7) >> 3);
         choice.offer(cost.lanes + (sixteens > 3 ? 0.3 : 0.0) + turns * rounds * round_us + (turns - 1.0) * (cost.lanes_turn + cost.lanes_short * (rounds < 4.0 ? 4.0 - rounds : 0.0)) +
-                         (z > 1 ? cost.lanes_slices + cost.lanes_mb * mb : 0.0),
+                         (z > 1 ? cost.lanes_slices + cost.lanes_bytes * sums_us : 0.0),
                      4 * sixteens + (four ? 1 : 0), 0, 0, z, per);
     });
     return choice.plan;
@@ -805,7 +806,9 @@ inline PackedRowsPlan packed_rows_f32_plan(int64_t M, int64_t N, int64_t K, int6
 // over six shapes and 16 .. 256 rows (128 channels and 5 .. 8 blocks of rows, on the same line: 1.36 and 1.49 us a round at 7 and 8; unrounded
 // weights 1.29, 1.43, 1.66 and 1.86 us at 1 .. 4 blocks, n-bit rows 1.4 times that): 4 for the launch, the first loads and the epilogue, per
 // round what the comment on the kernel says, per round of workgroups over the compute units, and for the second kernel 2.5 + the bytes of
-// the slices' sums (written and read) at 4 TB/s.  Within 5 % of the sweep's best nearly everywhere (11008 -> 4096 at 128 rows 24.8, best 22.7).
+// the slices' sums (written and read) at 4 TB/s.  Rounded n-bit weights by all plans of 50 shapes at 16 row counts: rounds of 8 bits are twice as long
+// (us, with the costs of int4 / with their own: 8 bits 132 rows 2560 -> 1152 16.3 / 11.8, 129 rows 1920 -> 896 12.6 / 10.5; 2 bits 154 rows 5888 -> 6272
+// 31 / 26), and the plans taken with 8 bits are 1.6 % above the best on average, 4.1 before.  Within 5 % of the sweep's best nearly everywhere (11008 -> 4096 at 128 rows 24.8, best 22.7).
 // Few rows: 32 channels per workgroup, eight steps of k a round.  Half the rounds on twice the compute units, so a few thousand k
 // need no slices, and where the card would be as fast with them the host saves a launch and an allocation (us, slices / this, eager and then
 // in a graph: int4 in groups of 64, 28 rows 4096 x 4096 11.2 / 7.6, 8.4 / 7.6; 20 rows 2048 x 2048 10.9 / 7.0, 6.7 / 5.2; 32 rows 3072 -> 8192
@@ -815,13 +818,22 @@ inline PackedRowsPlan packed_rows_f32_plan(int64_t M, int64_t N, int64_t K, int6
 // microsecond of the device would cost an eager call four: two rows 2272 -> 512 7.5 / 11.7, 7.2 / 6.5; 79 rows 1280 -> 1024 8.6 / 11.5, 8.5 / 8.2).
 // A call plans twice (workspace, launch), so what the heights have in common, the
 // divisions above all, is worked out once: 203 rows of 4096 -> 11008 0.12 us of host time instead of 0.83.
+struct RowsCost {
+    double round, block, wide_round, wide_block;  // a round of the loop and a block of 16 rows in it: up to 64 channels, 128
+    double second, bytes;                         // slices: the second kernel; factor of what their sums, written and read, take at 4 TB/s
+    int tall;                                     // from this many blocks on a workgroup costs 2 us more
+};
+constexpr RowsCost kRowsCosts[5] = {
+    {0.5, 0.18, 0.45, 0.13, 2.5, 1.0, 9}, {0.55, 0.19, 0.55, 0.14, 2.3, 1.0, 7}, {1.3, 0.18, 1.08, 0.2, 1.6, 1.4, 6},
+    {1.08, 0.19, 0.0, 0.0, 3.0, 1.0, 9}, {1.51, 0.27, 0.0, 0.0, 2.5, 1.0, 9},
+};
 inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int64_t room_floats, RowsWeights weights = kRowsRounded, int bits = 0) {
     if (dtype == TPQ_DTYPE_F32) return packed_rows_f32_plan(M, N, K, room_floats, bits);
     PackedRowsPlan p;
     p.quads = 0;
-    p.split = weights != kRowsRounded;
+    p.split = weights >= kRowsUnrounded;
+    const RowsCost& cost = kRowsCosts[weights];
     const int64_t blocks = (M + 15) / 16, steps = (K + 127) / 128;
-    const double second_us = weights == kRowsUnrounded ? 3.0 : 2.5;
     int64_t best = 1;
     double best_us = 1e30;
     p.cw = 2;
@@ -844,14 +856,14 @@ inline PackedRowsPlan packed_rows_plan(int dtype, int64_t M, int64_t N, int64_t 
             const int64_t row_tiles = ceil_div(blocks, mb);
             if (ceil_div(blocks, row_tiles) != mb) continue;
             const int64_t tiles = ((N + 32 * cw - 1) / (32 * cw)) * row_tiles;
-            const double round_us = (p.split ? (1.08 + 0.19 * mb) * (weights == kRowsUnroundedBits ? 1.4 : 1.0) : cw <= 2 ? 0.5 + 0.18 * mb : 0.45 + 0.13 * mb) +
-                                    (cw == 1 ? 0.2 * mb : 0.0);
+            const double round_us = (cw <= 2 ? cost.round + cost.block * mb : cost.wide_round + cost.wide_block * mb) + (cw == 1 ? 0.2 * mb : 0.0);
+            const double fixed_us = cw == 1 ? 3.4 : mb >= cost.tall ? 6.0 : 4.0;
             for (int c = 0; c < cuts; ++c) {
                 if (cw == 1 && c > 0) break;  // no slices is what they are for
                 const int64_t z = slices_of[c], rounds = (steps_of[c] + (1 << kw_shift) - 1) >> kw_shift;
                 const double waves = static_cast<double>((tiles * z + 255) >> 8);  // 256 compute units
-                double us = waves * ((cw == 1 ? 3.4 : 4.0) + round_us * static_cast<double>(rounds));
-                if (z > 1) us += second_us + static_cast<double>(z * M * N) * 8.0 / 4e6;
+                double us = waves * (fixed_us + round_us * static_cast<double>(rounds));
+                if (z > 1) us += cost.second + cost.bytes * (static_cast<double>(z * M * N) * 8.0 / 4e6);
                 if (us < best_us) { best_us = us; best = z; p.cw = cw; p.mb = mb; }
             }
         }

@@ -217,3 +217,19 @@ def test_float32_packed_rows_plan_by_width_and_without_short_turns():
     assert [plan(14, 8064, 1536, bits, 64)[0] for bits in (0, 8)] == [lanes, staged]
     assert plan(16, 5632, 8480, 8, 32)[0] == staged and plan(10, 3968, 4864, 1, 64)[0] == staged
     assert plan(12, 4096, 1024, 0, 128)[0] == lanes and plan(9, 2336, 520, 0, 32)[0] == lanes
+
+
+def test_packed_rows_plan_of_16_bit_rows_knows_the_width():
+    """Rounded n-bit weights: a round of the loop takes 8 bits twice as long as int4, so k is cut where int4 keeps one slice (132 rows 2560 -> 1152 with 8 bits
+    16.3 us in one, 11.8 in three; two bits, 154 rows 5888 -> 6272, 31 and 26)."""
+    from tensorplay_amd import _lib
+
+    lib = _lib.load()
+
+    def slices(M, K, N, bits, group):
+        out = (ctypes.c_int32 * 4)()
+        assert lib.tpq_packed_rows_call_plan(1, M, N, K, bits, group, -1, ctypes.cast(out, ctypes.c_void_p)) == _lib.TPQ_OK
+        return out[3]
+
+    assert slices(132, 2560, 1152, 0, 64) == 1 and slices(132, 2560, 1152, 8, 128) == 3
+    assert slices(129, 1920, 896, 8, 128) > 1 and slices(154, 5888, 6272, 2, 128) == 2
