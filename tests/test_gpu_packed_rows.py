@@ -1,5 +1,7 @@
 """GPU: packed weights against a block of activation rows (tpq_int4_mm_rows, tpq_lowbit_mm_rows), every element within the
 bound that its roundings give, against float64 on the same quantized operands."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -7,6 +9,18 @@ import torch
 from gpu_util import DEV
 
 pytestmark = pytest.mark.gpu
+
+STAGED, QUADS_OF_ROWS, LANES_OF_CHANNELS = 0, 1, 2  # the kernels: activations staged in LDS; float32 in blocks of four rows, with a lane per channel
+
+
+def _plan(dtype, M, N, K, bits, group, room=-1):
+    """[kernel, rows of a tile, its channels, slices of k] of a call with a workspace of `room` bytes (-1: what it asks for); bits 0: the int4 layout."""
+    from tensorplay_amd import _lib, ops
+
+    out = (ctypes.c_int32 * 4)()
+    ops._check(_lib.load().tpq_packed_rows_call_plan(ops._DT[dtype], M, N, K, bits, group, room, ctypes.cast(out, ctypes.c_void_p)))
+    return list(out)
+
 
 UNIT = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
 # (M, N, K, group): one and two rounds of four steps of 128 k, rounds of which the last is partial, several slices of k, rows at
@@ -45,7 +59,7 @@ def test_int4_rows(dtype, M, N, K, group):
     x = torch.randn(M, K, device=DEV, generator=gen).to(dtype)
     w = (codes - 8).double() * sz[..., 0].double().t().repeat_interleave(group, 1) + sz[..., 1].double().t().repeat_interleave(group, 1)
     lib = _lib.load()
-    need = int(lib.tpq_packed_rows_workspace_bytes(ops._DT[dtype], M, N, K))
+    need = int(lib.tpq_packed_rows_call_workspace_bytes(ops._DT[dtype], M, N, K, 0, group))
     for room in {need, 0}:  # with its slices, and without a workspace
         out = torch.empty(M, N, dtype=dtype, device=DEV)
         ws = torch.empty(max(room, 1), dtype=torch.uint8, device=DEV)
@@ -72,7 +86,8 @@ def test_lowbit_rows(dtype, bits, lsb_first, M, N, K, group):
     w = (value - zero) * scale
     out = torch.empty(M, N, dtype=dtype, device=DEV)
     lib = _lib.load()
-    need = int(lib.tpq_packed_rows_workspace_bytes(ops._DT[dtype], M, N, K))
+    need = int(lib.tpq_packed_rows_call_workspace_bytes(ops._DT[dtype], M, N, K, bits, group))
+    assert need > 0 or (M, N, K) not in ((33, 264, 1056), (64, 200, 4096))  # slices with a last step that is partial, and many
     ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
     ops._check(lib.tpq_lowbit_mm_rows(x.data_ptr(), ops._DT[dtype], M, K, packed.data_ptr(), bits, int(lsb_first), N, group, sz.data_ptr(),
                                       bias.data_ptr(), out.data_ptr(), ws.data_ptr(), need, ops._stream(x)))
@@ -80,21 +95,19 @@ def test_lowbit_rows(dtype, bits, lsb_first, M, N, K, group):
     _check(out, x, w, bias, 0.011 * (1 + (1 << bits) / 8), dtype)
 
 
-# (M, N, K, group, rows of a tile, slices of k): two to four tiles of rows, the last one partly empty, whole k and cut
-TALL = [(257, 6664, 256, 64, 80, 1), (241, 8200, 256, 32, 96, 1), (289, 8200, 256, 128, 112, 1), (225, 11016, 256, 64, 128, 1),
-        (257, 1096, 5248, 128, 80, 7), (241, 1544, 7296, 64, 96, 6), (289, 1608, 7296, 128, 112, 6), (241, 2824, 7296, 128, 128, 5),
-        (203, 11008, 4096, 128, 112, 1)]
+# (M, N, K, group, (rows of a tile, slices of k) for int4, 1 to 4 and 8 bits): two to four tiles of rows, the last one partly empty, whole k and cut
+TALL = [(257, 6664, 256, 64, (80, 1), (80, 1), (80, 1)), (241, 8200, 256, 32, (96, 1), (96, 1), (96, 1)), (289, 8200, 256, 128, (112, 1), (112, 1), (112, 1)),
+        (225, 11016, 256, 64, (128, 1), (128, 1), (128, 1)), (257, 1096, 5248, 128, (80, 7), (80, 7), (80, 7)), (241, 1544, 7296, 64, (96, 6), (96, 6), (64, 2)),
+        (289, 1608, 7296, 128, (112, 6), (80, 4), (80, 4)), (241, 2824, 7296, 128, (128, 5), (64, 1), (128, 5)), (203, 11008, 4096, 128, (112, 1), (112, 1), (112, 1)),
+        (193, 4104, 3840, 128, (48, 1), (48, 1), (112, 3)), (257, 2056, 7296, 128, (96, 5), (96, 5), (96, 5))]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bits", [0, 1, 2, 8])  # 0: the int4 layout
-@pytest.mark.parametrize("M,N,K,group,rows,slices", TALL)
-def test_tall_tiles(dtype, bits, M, N, K, group, rows, slices):
-    from tensorplay_amd import _lib, ops
-
-    lib, tag = _lib.load(), ops._DT[dtype]
-    assert lib.tpq_packed_rows_tile_rows(tag, M, N, K) == rows
-    assert lib.tpq_packed_rows_workspace_bytes(tag, M, N, K) == (0 if slices == 1 else 4 * slices * M * N)
+@pytest.mark.parametrize("M,N,K,group,int4,few_bits,byte", TALL)
+def test_tall_tiles(dtype, bits, M, N, K, group, int4, few_bits, byte):
+    kernel, rows, _, slices = _plan(dtype, M, N, K, bits, group)
+    assert kernel == STAGED and (rows, slices) == {0: int4, 8: byte}.get(bits, few_bits)
     if bits:
         test_lowbit_rows(dtype, bits, False, M, N, K, group)
     else:
@@ -229,12 +242,18 @@ def test_float16_weights_of_any_size_are_not_rounded(kind, M, N, K, group, bits,
 # (rows, N, K, group): few rows on 32 channels a workgroup and eight steps of k a round: one, two and four rounds, the last one and the last
 # step partial, channels that leave a tile partly empty, one tile and more than the compute units
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("M,N,K,group", [(1, 8, 1024, 32), (16, 40, 1152, 64), (5, 1160, 1376, 32), (32, 72, 2048, 64), (17, 8200, 928, 32), (29, 2056, 4096, 64)])
+@pytest.mark.parametrize("M,N,K,group", [(1, 8, 1024, 32), (16, 40, 1152, 64), (5, 1160, 1376, 32), (32, 72, 2048, 64), (17, 8168, 928, 32), (17, 8200, 928, 32), (29, 2056, 4096, 64)])
 def test_few_rows_without_slices(dtype, M, N, K, group):
     from tensorplay_amd import _lib, ops
 
     if dtype == torch.float32 and M > 16:
         pytest.skip("two blocks of float32 rows do not fit a round of eight steps")
+    for bits in (0, 2):
+        kernel, rows, channels, slices = _plan(dtype, M, N, K, bits, group, 0)
+        if dtype == torch.float32 and M <= 8:
+            assert kernel == QUADS_OF_ROWS
+        else:  # (8200 channels are a tile of 32 more than there are compute units)
+            assert (kernel, rows, channels, slices) == (STAGED, -(-M // 16) * 16, 64 if N == 8200 else 32, 1)
     lib, tag = _lib.load(), ops._DT[dtype]
     gen = torch.Generator(device=DEV).manual_seed(M + N + K)
     x = torch.randn(M, K, device=DEV, generator=gen).to(dtype)
@@ -268,14 +287,12 @@ def test_few_rows_take_no_workspace():
 def test_calls_have_the_slices_that_their_weight_wants(dtype, M, N, K, group):
     """A weight that is not rounded (K % 128 != 0, groups of 128 on few rows) has longer rounds of the loop than one that is, and slices where
     that has none: the Python entry gives the library room for them (one slice adds k in another order: some outputs in a thousand differ)."""
-    import ctypes
-
     from tensorplay_amd import _lib, ops
 
     lib, tag = _lib.load(), ops._DT[dtype]
-    need, plan = int(lib.tpq_packed_rows_call_workspace_bytes(tag, M, N, K, 0, group)), (ctypes.c_int32 * 4)()
-    ops._check(lib.tpq_packed_rows_call_plan(tag, M, N, K, 0, group, need, ctypes.cast(plan, ctypes.c_void_p)))
-    assert need == 4 * plan[3] * M * N and plan[3] > 1
+    need = int(lib.tpq_packed_rows_call_workspace_bytes(tag, M, N, K, 0, group))
+    slices = _plan(dtype, M, N, K, 0, group, need)[3]
+    assert need == 4 * slices * M * N and slices > 1
     gen = torch.Generator(device=DEV).manual_seed(M + N + K)
     packed = ops._convert_weight_to_int4pack(torch.randint(0, 16, (N, K), dtype=torch.int32, device=DEV, generator=gen), 2)
     sz = (torch.rand(K // group, N, 2, device=DEV, generator=gen) * 0.01 + 1e-3).to(dtype)
@@ -318,7 +335,7 @@ def _float32_products(counts, N, K, group, bits, lsb_first):
         w = (codes.double() - z64) * s64
     results = {}
     for m in counts:
-        sizes = {int((lib.tpq_lowbit_mm_rows_workspace_bytes if bits else lib.tpq_packed_rows_workspace_bytes)(tag, m, N, K)), 0}
+        sizes = {int(lib.tpq_packed_rows_call_workspace_bytes(tag, m, N, K, bits, group)), 0}
         for need in sizes:
             out = torch.full((m, N), float("nan"), device=DEV)
             ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
@@ -338,30 +355,26 @@ WIDTHS = [(0, False), (1, False), (1, True), (2, False), (4, False), (8, False)]
 @pytest.mark.parametrize("bits,lsb_first", WIDTHS)
 @pytest.mark.parametrize("M,N,K,group", QUADS)
 def test_blocks_of_four_rows(M, N, K, group, bits, lsb_first):
-    """Against float64, element by element, and beside the blocks of 16 rows: the same rows among nine, whose bound is the same."""
-    from tensorplay_amd import _lib, ops
-
-    lib, tag = _lib.load(), ops._DT[torch.float32]
+    """Against float64, element by element, and beside the kernels of 16 rows: the same rows among nine, whose bound is the same."""
     N, group = (N + 7) // 8 * 8 if bits == 0 else N, group if bits or group in (32, 64, 128) else 32
-    assert lib.tpq_packed_rows_tile_rows(tag, M, N, K) == 4 * -(-M // 4) and lib.tpq_packed_rows_tile_rows(tag, 9, N, K) == 16
+    assert _plan(torch.float32, M, N, K, bits, group)[:2] == [QUADS_OF_ROWS, 4 * -(-M // 4)] and _plan(torch.float32, 9, N, K, bits, group)[0] != QUADS_OF_ROWS
     results, size = _float32_products((M, 9), N, K, group, bits, lsb_first)
     assert bool(((results[M] - results[9][:M]).double().abs() <= 2 * (K + 17) * 2.0 ** -24 * size[:M]).all())
 
 
-# (M, N, K, group, rows of a tile): float32 with a lane per channel: one to four blocks of 16 rows, with a block of four behind one to three of them, full and
-# not, two and three tiles of rows; fewer tiles of k than wavefronts, more than they have in flight; channels that leave a part partly empty
-LANES = [(17, 8200, 96, 32, 20), (20, 8200, 1088, 32, 20), (17, 68, 11008, 128, 20), (35, 1032, 4128, 32, 36), (52, 1032, 2080, 32, 52), (14, 11008, 4096, 128, 16),
-         (40, 4096, 4096, 128, 48), (60, 4096, 4096, 64, 64), (96, 2056, 2080, 32, 48), (130, 1032, 4096, 64, 48)]
+# (M, N, K, group, rows of a tile, widths whose plan it is): float32 with a lane per channel: one to four blocks of 16 rows, with a block of four behind one to three of
+# them, full and not, two and three tiles of rows; fewer tiles of k than wavefronts, more than they have in flight; channels that leave a part partly empty
+ALL, INT4, BITS, BYTE = (0, 1, 2, 4, 8), (0,), (1, 2, 4), (8,)
+LANES = [(17, 8200, 96, 32, 20, ALL), (20, 8200, 1088, 32, 20, ALL), (17, 68, 11008, 128, 20, ALL), (35, 1032, 4128, 32, 36, ALL), (52, 1032, 2080, 32, 52, INT4 + BYTE),
+         (14, 11008, 4096, 128, 16, INT4), (40, 4096, 4096, 128, 48, ALL), (60, 4096, 4096, 64, 64, INT4 + BITS), (96, 2056, 2080, 32, 48, ALL), (130, 1032, 4096, 64, 48, INT4 + BITS),
+         (14, 68, 1088, 32, 16, BITS + BYTE), (29, 68, 544, 32, 32, ALL), (50, 68, 544, 32, 52, ALL), (60, 68, 544, 32, 64, ALL)]
 
 
-@pytest.mark.parametrize("bits,lsb_first", WIDTHS)
-@pytest.mark.parametrize("M,N,K,group,rows", LANES)
+@pytest.mark.parametrize("M,N,K,group,rows,bits,lsb_first", [(*shape, bits, lsb_first) for *shape, widths in LANES for bits, lsb_first in WIDTHS if bits in widths])
 def test_lane_per_channel(M, N, K, group, rows, bits, lsb_first):
     """Against float64, element by element, and beside the blocks of four: the first eight rows by themselves."""
-    from tensorplay_amd import _lib, ops
-
     N = (N + 7) // 8 * 8 if bits == 0 else N
-    assert _lib.load().tpq_packed_rows_tile_rows(ops._DT[torch.float32], M, N, K) == rows
+    assert _plan(torch.float32, M, N, K, bits, group)[:2] == [LANES_OF_CHANNELS, rows]
     results, size = _float32_products((M, 8), N, K, group, bits, lsb_first)
     assert bool(((results[M][:8] - results[8]).double().abs() <= 2 * (K + 17) * 2.0 ** -24 * size[:8]).all())
 
