@@ -10,8 +10,8 @@
 //     LDS, and 128 k of four rows are two 16-byte loads a lane;
 //   * a wavefront is 32 channels and R blocks of four rows; a workgroup's eight wavefronts are CW x 32 channels times 8 / CW steps of 128 k at a
 //     time, and slices of K (summed by packed_rows_finish_kernel) fill the chip where the channels do not;
-//   * sums go over 16 k, two of them over a tile, the tiles over the wavefront's share; a tile's four q meet by two swaps between lanes, which
-//     leave row q in lane group q, the wavefronts meet in LDS by halves;
+//   * sums go over 16 k and those over the wavefront's share (a quarter of its tiles each of the four q); the four q meet by two swaps between lanes,
+//     which leave row q in lane group q, the wavefronts meet in LDS by halves;
 //   * a last step that is partial repeats the last tile with scale, zero and activations cleared: zeros that meet finite numbers only.
 // Measured (us, this kernel / what ran before, in a graph): int4, one row of 4096 x 4096 9.2 / 14.3, 8192 x 8192 15.5 / 29.5; two rows of 2048 x 2048
 // 5.9 / 8.5; seven of 8192 x 8192 22 / 30; n-bit rows, 4 rows of 11008 -> 4096 with 8 bits 20 / 28, 2 rows of 5120 -> 13824 with 1 bit 21.5 / 37.5, 7 rows of
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(8 * kWave) void packed_quads_kernel(const PackedRow
                 for (int h = 0; h < 2; ++h) d.x[r][h] = d.live ? d.x[r][h] : pr_word4{0u, 0u, 0u, 0u};
         }
         float4_t piece[kChains][NB][R];
-        // a chain is 16 k; up to two blocks of rows both halves of the tile are under way (a product waits for the one before it)
+        // a chain is 16 k; with one block of rows both halves of the tile are under way (a product waits for the one before it)
         pr_static_for<0, 16>([&](auto pair_c) __attribute__((always_inline)) {
             constexpr int kPair = decltype(pair_c)::value;
             constexpr int kAt = kChains == 2 ? (kPair >> 1) + 8 * (kPair & 1) : kPair, kChain = kChains == 2 ? kPair & 1 : 0;
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(8 * kWave) void packed_quads_kernel(const PackedRow
 }
 
 // ---- more rows: a lane per channel ----------------------------------------------------------------------------
-// From nine rows on, where that is the faster way (packed_lanes_plan).  What bounds it: the matrix instructions, 32 clocks for 16 rows x 64 channels x one k
+// From nine rows on, where that is the faster way (packed_rows_f32_plan).  What bounds it: the matrix instructions, 32 clocks for 16 rows x 64 channels x one k
 // (v_mfma_f32_16x16x1, four blocks of 16 channels), and the dequantization behind them.  What the kernel with its activations in LDS spends beside those, barriers between
 // its rounds and wavefronts that only fetch, is not here: a wavefront takes tiles of 32 k for itself, MB blocks of 16 rows and, QB, one of four rows (v_mfma_f32_4x4x1 with
 // the channels of a lane side by side), so that 19 rows cost 20 and not 32.
@@ -203,16 +203,28 @@ __global__ __launch_bounds__(8 * kWave) void packed_quads_kernel(const PackedRow
 //     many rows to multiply that is still the smaller part;
 //   * activations, first operand, reach all four blocks from one (cbsz 2): lane (row, b) loads eight k of its row, 8 b .. + 7, register v, block abid hold k = 8 abid + v;
 //     of the block of four (cbsz 4), lane (row, b) holds k = 2 b, + 1;
-//   * sums as above; the eight wavefronts' meet in LDS, 16 rows at a time.
+//   * sums go over 16 k, those over a group of three or four tiles, the groups over the wavefront's share: in one chain over 2944 k the error against float64 is 1.14 times that of
+//     the staged kernel, whose steps of 128 k are summed first.  Three blocks of rows and more have no registers for both: the groups' sum lies in LDS, each lane's own words
+//     (read, added to and written once in four tiles; slices of up to 48 tiles, where one chain is as precise by the variances of the roundings - (1 / 256 - 1 / 1024) K <= 4.5 -
+//     go without).  The eight wavefronts' sums meet in LDS by halves, up to two blocks 16 rows at a time.
 // Measured (us, before / with this, in a graph): int4 19 rows 4096 x 4096 17.4 / 13.4, 35 rows 26.5 / 19.2, 17 rows 11008 -> 4096 35.5 / 25.6; 8 bits, 36 rows 4096 x 4096 30 / 24.8.
 typedef float float16_t __attribute__((ext_vector_type(16)));
+constexpr int kLanesGroupBlocks = 2, kLanesOneChain = 48;  // blocks of 16 rows whose groups are summed in registers; tiles of a slice without groups in LDS
 constexpr int kLanesPitch = kWave + 4;  // of a row of sums in LDS: the four rows that a wavefront stores at once lie 16 banks apart
 
+constexpr int lanes_words(int mb, int qb) { return mb <= kLanesGroupBlocks ? 16 : 16 * mb + 4 * qb; }  // of LDS a lane of each wavefront
+
+// one block of rows, up to 4 bits: two workgroups on a compute unit, three tiles in flight each
 template <class Source, int MB, int QB>
-__global__ __launch_bounds__(8 * kWave) void packed_lanes_kernel(const PackedRowsArgs a) {
+constexpr bool lanes_in_pairs() { return MB == 1 && QB == 0 && sizeof(typename Source::Words) <= 16; }
+
+template <class Source, int MB, int QB>
+__global__ __launch_bounds__(8 * kWave, (lanes_in_pairs<Source, MB, QB>() ? 4 : 2)) void packed_lanes_kernel(const PackedRowsArgs a) {
     using P = RowsParams<TPQ_DTYPE_F32, Source::kTypedParams>;
-    constexpr int kDepth = MB == 1 ? 4 : MB == 2 ? 3 : 2, kChains = MB == 1 ? 2 : 1;
-    __shared__ float sums[8][16][kLanesPitch];
+    constexpr int kDepth = lanes_in_pairs<Source, MB, QB>() ? 3 : MB == 1 ? 4 : MB == 2 ? 3 : 2, kChains = MB == 1 ? 2 : 1;
+    constexpr bool kGroups = MB <= kLanesGroupBlocks;
+    extern __shared__ float lanes_sums[];  // [8][lanes_words(MB, QB)][kLanesPitch]
+    auto sums = reinterpret_cast<float(*)[lanes_words(MB, QB)][kLanesPitch]>(lanes_sums);
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = blockIdx.x * kWave + lane, m0 = blockIdx.y * (16 * MB + 4 * QB);
@@ -252,8 +264,42 @@ __global__ __launch_bounds__(8 * kWave) void packed_lanes_kernel(const PackedRow
         if constexpr (QB) d.x_quad = *(TPQ_GLOBAL pr_word2*)pinned_global(x_quad + static_cast<size_t>(tile) * 128);
     };
 
-    float16_t acc[MB] = {};
-    float4_t acc_quad = {};
+    float16_t acc[MB] = {}, group_sum[kGroups ? MB : 1] = {};
+    float4_t acc_quad = {}, group_quad = {};
+    auto flush = [&]() __attribute__((always_inline)) {
+        if constexpr (kGroups) {
+#pragma unroll
+            for (int b = 0; b < MB; ++b) {
+                acc[b] += group_sum[b];
+                group_sum[b] = float16_t{};
+            }
+            if constexpr (QB) {
+                acc_quad += group_quad;
+                group_quad = float4_t{};
+            }
+        }
+    };
+    // kGroups: nothing; else the lane's words of LDS := the same (first) or += acc, and acc := 0
+    auto to_lds = [&](bool first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                float& at = sums[wave][16 * b + e][lane];
+                at = first ? acc[b][e] : at + acc[b][e];
+                acc[b][e] = 0.0f;
+            }
+        if constexpr (QB) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float& at = sums[wave][16 * MB + e][lane];
+                at = first ? acc_quad[e] : at + acc_quad[e];
+                acc_quad[e] = 0.0f;
+            }
+        }
+    };
+    bool first_group = true;
+    const bool in_groups = end - begin > kLanesOneChain;
     uint32_t magic[2] = {Source::kMagic0, Source::kMagic1};
     asm volatile("" : "+v"(magic[0]), "+v"(magic[1]));
     auto multiply = [&](const Tile& d) __attribute__((always_inline)) {
@@ -290,10 +336,16 @@ __global__ __launch_bounds__(8 * kWave) void packed_lanes_kernel(const PackedRow
 #pragma unroll
                 for (int b = 0; b < MB; ++b)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) acc[b][e] += piece[kChain][b][e];
+                    for (int e = 0; e < 16; ++e) {
+                        if constexpr (kGroups) group_sum[b][e] += piece[kChain][b][e];
+                        else acc[b][e] += piece[kChain][b][e];
+                    }
                 if constexpr (QB) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc_quad[e] += piece_quad[kChain][e];
+                    for (int e = 0; e < 4; ++e) {
+                        if constexpr (kGroups) group_quad[e] += piece_quad[kChain][e];
+                        else acc_quad[e] += piece_quad[kChain][e];
+                    }
                 }
             }
         });
@@ -303,22 +355,36 @@ __global__ __launch_bounds__(8 * kWave) void packed_lanes_kernel(const PackedRow
         Tile ring[kDepth];
         pr_static_for<0, kDepth>([&](auto d) __attribute__((always_inline)) { load(decltype(d)::value, ring[decltype(d)::value]); });
         int j = 0;
-        for (; j + kDepth < count; j += kDepth)
+        for (; j + kDepth < count; j += kDepth) {
             pr_static_for<0, kDepth>([&](auto d) __attribute__((always_inline)) {
                 multiply(ring[decltype(d)::value]);
                 load(j + kDepth + decltype(d)::value, ring[decltype(d)::value]);
+                if constexpr (decltype(d)::value == kDepth - 1) flush();
                 __builtin_amdgcn_sched_barrier(0);
             });
+            if constexpr (!kGroups) {
+                static_assert(kDepth == 2, "a group of four tiles is two turns of the ring");
+                if (in_groups && (j & 2)) {
+                    to_lds(first_group);
+                    first_group = false;
+                }
+            }
+        }
         pr_static_for<0, kDepth>([&](auto d) __attribute__((always_inline)) {
             if (j + decltype(d)::value < count) multiply(ring[decltype(d)::value]);
         });
+        flush();
     }
 
-    auto store = [&](int row, int m) __attribute__((always_inline)) {
+    if constexpr (!kGroups) {
+        to_lds(first_group);
+        __syncthreads();
+    }
+    auto store = [&](int row, int at_lane, int m) __attribute__((always_inline)) {  // row: of words in LDS
         if (m >= a.M || n >= a.N) return;
         float part[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) part[k] = sums[k][row][lane];
+        for (int k = 0; k < 8; ++k) part[k] = sums[k][row][at_lane];
         float s = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
         const size_t at = static_cast<size_t>(m) * a.N + n;
         if (a.partial != nullptr) {
@@ -329,24 +395,46 @@ __global__ __launch_bounds__(8 * kWave) void packed_lanes_kernel(const PackedRow
         if (a.after != nullptr) s += static_cast<const float*>(a.after)[n];
         static_cast<float*>(a.y)[at] = s;
     };
+    if constexpr (kGroups) {
 #pragma unroll
-    for (int b = 0; b < MB; ++b) {
-        if (b > 0) __syncthreads();
+        for (int b = 0; b < MB; ++b) {
+            if (b > 0) __syncthreads();
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+            for (int c = 0; c < 4; ++c)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sums[wave][4 * (lane >> 4) + e][16 * c + (lane & 15)] = acc[b][4 * c + e];
-        __syncthreads();
+                for (int e = 0; e < 4; ++e) sums[wave][4 * (lane >> 4) + e][16 * c + (lane & 15)] = acc[b][4 * c + e];
+            __syncthreads();
 #pragma unroll
-        for (int h = 0; h < 2; ++h) store(wave + 8 * h, m0 + 16 * b + wave + 8 * h);
+            for (int h = 0; h < 2; ++h) store(wave + 8 * h, lane, m0 + 16 * b + wave + 8 * h);
+        }
+        if constexpr (QB) {
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sums[wave][e][lane] = acc_quad[e];
+            __syncthreads();
+            if (wave < 4) store(wave, lane, m0 + 16 * MB + wave);
+        }
+    } else {  // as the products left them: row 4 q + e of a block, channel 16 c + i in word 4 c + e of lane (i, q)
+#pragma unroll
+        for (int h = 0; h < 2 * MB; ++h) {
+            const int row = wave + 8 * h, in_block = row & 15;
+            store((row & ~15) + 4 * (lane >> 4) + (in_block & 3), (in_block >> 2) * 16 + (lane & 15), m0 + row);
+        }
+        if constexpr (QB) {
+            if (wave < 4) store(16 * MB + wave, lane, m0 + 16 * MB + wave);
+        }
     }
-    if constexpr (QB) {
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sums[wave][e][lane] = acc_quad[e];
-        __syncthreads();
-        if (wave < 4) store(wave, m0 + 16 * MB + wave);
-    }
+}
+
+template <class Source, int MB, int QB>
+int launch_packed_lanes(const PackedRowsArgs& a, const dim3& grid, hipStream_t s) {
+    constexpr size_t smem = static_cast<size_t>(8) * lanes_words(MB, QB) * kLanesPitch * sizeof(float);
+    static_assert(smem <= 160 * 1024, "LDS of one compute unit");
+    auto kernel = packed_lanes_kernel<Source, MB, QB>;
+    static std::atomic<uint64_t> configured{0};
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), smem, configured, "packed rows (float32)")) return rc;
+    kernel<<<grid, 8 * kWave, smem, s>>>(a);
+    return TPQ_OK;
 }
 
 template <class Source>
@@ -359,15 +447,17 @@ int launch_packed_f32(PackedRowsArgs a, int quads, int cw, int slices, hipStream
         else
             packed_quads_kernel<Source, 2><<<grid, 8 * kWave, 0, s>>>(a, cw >> 1);
     } else {
+        int rc;
         switch (quads) {
-            case 4: packed_lanes_kernel<Source, 1, 0><<<grid, 8 * kWave, 0, s>>>(a); break;
-            case 5: packed_lanes_kernel<Source, 1, 1><<<grid, 8 * kWave, 0, s>>>(a); break;
-            case 8: packed_lanes_kernel<Source, 2, 0><<<grid, 8 * kWave, 0, s>>>(a); break;
-            case 9: packed_lanes_kernel<Source, 2, 1><<<grid, 8 * kWave, 0, s>>>(a); break;
-            case 12: packed_lanes_kernel<Source, 3, 0><<<grid, 8 * kWave, 0, s>>>(a); break;
-            case 13: packed_lanes_kernel<Source, 3, 1><<<grid, 8 * kWave, 0, s>>>(a); break;
-            default: packed_lanes_kernel<Source, 4, 0><<<grid, 8 * kWave, 0, s>>>(a); break;
+            case 4: rc = launch_packed_lanes<Source, 1, 0>(a, grid, s); break;
+            case 5: rc = launch_packed_lanes<Source, 1, 1>(a, grid, s); break;
+            case 8: rc = launch_packed_lanes<Source, 2, 0>(a, grid, s); break;
+            case 9: rc = launch_packed_lanes<Source, 2, 1>(a, grid, s); break;
+            case 12: rc = launch_packed_lanes<Source, 3, 0>(a, grid, s); break;
+            case 13: rc = launch_packed_lanes<Source, 3, 1>(a, grid, s); break;
+            default: rc = launch_packed_lanes<Source, 4, 0>(a, grid, s); break;
         }
+        if (rc) return rc;
     }
     if (int rc = check_launch("packed rows (float32)")) return rc;
     if (a.partial == nullptr) return TPQ_OK;

@@ -758,7 +758,7 @@ constexpr int64_t kQuadRows = 8;
 
 // From nine rows on: activations staged in LDS, or a lane per channel: 16 to 64 rows a workgroup, and where one to four rows are left over by blocks of 16, those as a
 // block of four.  Slices so short that a wavefront's four tiles in flight are not filled, on workgroups that take turns, are the worst of both kinds (10 rows 3968 -> 4864
-// with 1 bit in 16 slices 25, in three 17; 16 rows 5632 -> 8480 with 8 bits in eleven 65, three 40): the estimates of turns keep calls away from them.
+// with 1 bit in 16 slices 25, in three 17; 16 rows 5632 -> 8480 with 8 bits in eleven 65, three 40): the estimates of turns keep calls away from them, and a round is the least.
 // Staged / a lane per channel, us in a graph: int4 19 rows 4096 x 4096 17.8 / 13.6, 35 rows 26.2 / 19.3, 80 rows 42.9 / 35.4, 17 rows 11008 -> 4096 35.2 / 25.8; 36 rows
 // with 8 bits 29.8 / 24.7; but 64 rows 2048 -> 8192 23.9 / 27.6, 50 rows 2048 x 2048 with 1 bit 12.4 / 13.6, 14 rows 8064 -> 1536 with 8 bits 15.6 / 17.5, 20 rows
 // 2560 -> 8192 with 8 bits 25 / 31.
@@ -794,6 +794,7 @@ inline PackedRowsPlan packed_rows_f32_plan(int64_t M, int64_t N, int64_t K, int6
     const double round_us = cost.lanes_round + cost.lanes_block * sixteens + (four ? cost.lanes_four : 0.0);
     rows_slices(tiles, M, N, room_floats, [&](int64_t z, int64_t per, double sums_us) {
         const double turns = turns_of(columns * lanes_tiles * z), rounds = static_cast<double>((per + 7) >> 3);
+        if (z > 1 && turns > 1.0 && per <= 8) return;
         choice.offer(cost.lanes + (sixteens > 3 ? 0.3 : 0.0) + turns * rounds * round_us + (turns - 1.0) * (cost.lanes_turn + cost.lanes_short * (rounds < 4.0 ? 4.0 - rounds : 0.0)) +
                          (z > 1 ? cost.lanes_slices + cost.lanes_bytes * sums_us : 0.0),
                      4 * sixteens + (four ? 1 : 0), 0, 0, z, per);
