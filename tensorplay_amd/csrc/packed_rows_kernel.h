@@ -9,9 +9,9 @@
 // KB, 1400), the fragment reads from LDS (1024 + 512 for writing them), the dequantization (1280) and the products (1024).
 // Taken out one at a time they all shorten the loop, none by much (4096 x 4096 at 256 rows, bfloat16: 17.0 us, without
 // activations 13.3, without dequantization 16.5, without products 15.4, loads of weights and barriers alone 8.9).  Hence
-//   * a workgroup owns 64 channels (128 where that still fills the chip: half the activation bytes per product) and a slice of
-//     K (a few slices of K fill the chip where N / 64 workgroups do not; their fp32 sums meet in a second kernel, added in
-//     slice order);
+//   * a workgroup owns 64 channels (128 where that still fills the chip: half the activation bytes per product; 32 with few rows, which then
+//     need no slices) and a slice of K (a few slices of K fill the chip where N / 64 workgroups do not; their fp32 sums meet in a second kernel,
+//     added in slice order, float32 four at a time by halves);
 //   * up to 64 rows, with 128 channels up to 128 (whose two rounds of activations fill 128 KB of LDS): a taller tile dequantizes
 //     its channels once for more rows, and 203 rows of 4096 -> 11008 are 172 tiles of 112 rows in one round of workgroups instead of 344 of 64
 //     in two (2 bits 48.5 -> 32, int4 41 -> 28 us; int4 at 256 rows 43 -> 34, at 384 66 -> 53);

@@ -92,7 +92,7 @@ __device__ __forceinline__ void quantize_eight_lean(const float (&v)[kVec], floa
     // v_perm_b32(a, b, sel): selector bytes 0..3 take bytes of b, 4..7 of a, 0x0c a zero byte
     lo = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0400u) | __builtin_amdgcn_perm(t[3], t[2], 0x04000c0cu);
     hi = __builtin_amdgcn_perm(t[5], t[4], 0x0c0c0400u) | __builtin_amdgcn_perm(t[7], t[6], 0x04000c0cu);
-    // Rare (one element in a few thousand).  Behind a branch the whole wavefront takes or skips, and with the divisor
+    // Rare (one element in 16 000).  Behind a branch the whole wavefront takes or skips, and with the divisor
     // passed through a statement the compiler may not move: as a plain "if", the eight divisions were hoisted above the
     // branch, computed for every chunk and selected away.
     if (__builtin_amdgcn_ballot_w64(redo) != 0) {
